@@ -57,6 +57,16 @@ hipEvent_t prof_phase(Server *s, hipStream_t st, int *open, int next_kind) {
   return e;
 }
 
+// Single batches: remembers whether the caller takes them one after the other (Pipe::taken_in_order).
+static void single_issued(Server *s, int pipe) {
+  s->pipes[pipe].taken_in_order = s->last_taken;
+  s->last_pipe = pipe;
+  s->last_taken = false;
+}
+static void single_taken(Server *s, int pipe, hipStream_t st) {
+  if (pipe == s->last_pipe && s->pipes[pipe].last_stream == st) s->last_taken = true;
+}
+
 // Start of a batch, or of a group of n batches served together: decides whether it is profiled.
 static void prof_batch(Server *s, int n = 1) {
   s->prof_on = s->prof_level != 0 && (s->prof_seq++ % std::max(1, s->prof_every)) == 0;
@@ -769,6 +779,7 @@ int lmi_op_batch_generate(lmi_server *h, int pipe, void *stream, const int32_t *
   hipStream_t st = (hipStream_t)stream;
   BatchParams bp{};
   prof_batch(s);
+  single_issued(s, pipe);
   LMI_TRY(pipe_join(p, st));
   pipe_begin(p, st);
   LMI_TRY(batch_params(s, p, st, seeds, n, seeds_location, batch_counter, mode, rng_seed, &bp));
@@ -908,7 +919,7 @@ static int run_group(Server *s, Pipe *const *pp, const BatchParams *bps, int n, 
     // misses start over the host link while the later hops are still being sampled
     split = s->split_lookup && s->cfg.hops >= 2 && s->feat_loc == LMI_LOC_HOST && s->split_miss == 1 &&
             (s->cache_kind == LMI_CACHE_STATIC || s->cache_kind == LMI_CACHE_INT8) &&
-            (s->split_lookup == 1 || (s->split_lookup == 2 && n > 1));
+            (s->split_lookup == 1 || (s->split_lookup == 2 && n > 1)) && !gather_in_line(s, pp, n, s->cfg.hops);
     LMI_TRY(launch_batch_generate(s, pp, bps, n, st, false));
     for (int k = 0; k < s->cfg.hops; ++k) {
       LMI_TRY(launch_hop(s, pp, n, st, k, true, true));
@@ -934,6 +945,7 @@ int lmi_run_once(lmi_server *h, int pipe, void *stream, const int32_t *seeds, in
   hipStream_t st = (hipStream_t)stream;
   BatchParams bp{};
   prof_batch(s);
+  single_issued(s, pipe);
   // a pipe's previous batch may still be gathering misses, or sit on another stream: only behind it may
   // this batch's first command, the copy of host seeds into the pipe's staging buffer, be queued
   LMI_TRY(pipes_join(pp, 1, st));
@@ -960,6 +972,9 @@ int lmi_run_group(lmi_server *h, int n_batches, const int32_t *pipes, void *stre
     pp[k] = &s->pipes[pipes[k]];
   }
   prof_batch(s, n_batches);
+  s->last_pipe = -1;  // a group is prefetched: its misses overlap the next group's sampling
+  s->last_taken = false;
+  for (int k = 0; k < n_batches; ++k) pp[k]->taken_in_order = false;
   LMI_TRY(pipes_join(pp, n_batches, st));  // before the seeds are staged: see lmi_run_once
   for (int k = 0; k < n_batches; ++k)
     LMI_TRY(batch_params(s, *pp[k], st, seeds ? seeds[k] : nullptr, (seeds && n_seeds) ? n_seeds[k] : 0, seeds_location,
@@ -1083,6 +1098,7 @@ static int fault_status_once(Server *s) {
 int lmi_batch_wait(lmi_server *h, int pipe, void *stream) {
   Server *s = reinterpret_cast<Server *>(h);
   LMI_TRY(check_pipe(s, pipe));
+  single_taken(s, pipe, (hipStream_t)stream);
   LMI_TRY(pipe_join(s->pipes[pipe], (hipStream_t)stream));
   return fault_status_once(s);
 }
@@ -1114,6 +1130,7 @@ int lmi_batch_counters(lmi_server *h, int pipe, void *stream, int32_t node_count
   Server *s = reinterpret_cast<Server *>(h);
   LMI_TRY(check_pipe(s, pipe));
   DevState hs;
+  single_taken(s, pipe, (hipStream_t)stream);
   LMI_TRY(pipe_join(s->pipes[pipe], (hipStream_t)stream));
   LMI_HIP(hipStreamSynchronize((hipStream_t)stream));
   LMI_HIP(hipMemcpy(&hs, s->pipes[pipe].st, sizeof(DevState), hipMemcpyDeviceToHost));

@@ -37,6 +37,7 @@ namespace lmi {
 struct MoveRow {
   const int2 *list;
   const int32_t *first_ptr, *n_ptr, *src_index, *dst_index;
+  const int32_t *ids;  // gather_rows_flat_kernel<.., MISSES>: node id per row
   uint8_t *dst;
 };
 struct MoveGroup {
@@ -236,8 +237,8 @@ static __global__ __launch_bounds__(256) void move_rows_tiled_kernel(
   }
 }
 
-// The HBM gather of cache hits, for fp32 / fp16 rows of every size from 16 bytes up.  Output rows [first, n)
-// directly, source row = src_index[row] (a cache slot; negative = a miss, skipped).  A block takes a
+// The HBM gather, for fp32 / fp16 rows of every size from 16 bytes up.  Output rows [first, n)
+// directly, source row = src_index[row] (a cache slot; outside [0, n_src) = nothing to move).  A block takes a
 // tile of consecutive rows and its 256 threads walk the tile's 16-byte units in flat order -- unit f is
 // piece f % upr of row f / upr -- U units per lane and pass: the U slots (lanes of one row read the
 // same word: one cache line per wavefront), then the U row pieces, then the U stores, each step
@@ -248,17 +249,22 @@ static __global__ __launch_bounds__(256) void move_rows_tiled_kernel(
 // tile's rows through LDS first kept 70 %.  A row that is no multiple of 16 bytes ends with a unit
 // that overlaps the one before it (both write the same bytes), so every access is 16 bytes wide, at
 // 4-byte alignment when the row length demands it (V16 says which).
+// MISSES: a row without a slot is read from the feature table by its node id in the same pass (gather_in_line says
+// when).  The table may lie behind the host link: the wavefronts that hold such rows then wait for the link, which
+// bounds the launch, while the hits of all others stream past.
 // rows_seen (pinned host memory, or null): the launch leaves each pipe's row count there for the host
 // to size later grids by (see launch_gather_flat).
-template <typename V16, int U, bool NT>
+template <typename V16, int U, bool NT, bool MISSES>
 static __global__ __launch_bounds__(256) void gather_rows_flat_kernel(MoveGroup g, const uint8_t *__restrict__ src,
-                                                                      int upr, int last_off, int rows_per_tile,
-                                                                      int64_t src_pitch, int64_t dst_pitch,
-                                                                      unsigned long long *row_counter,
+                                                                      uint32_t n_src, const uint8_t *__restrict__ table,
+                                                                      uint32_t n_table, int upr, int last_off,
+                                                                      int rows_per_tile, int64_t src_pitch,
+                                                                      int64_t dst_pitch, unsigned long long *row_counter,
                                                                       int32_t *rows_seen) {
   LMI_GRID_ROW(g.n);
   const MoveRow &r = g.p[row];
   const int32_t *__restrict__ src_index = r.src_index;
+  const int32_t *__restrict__ ids = r.ids;
   uint8_t *__restrict__ dst = r.dst;
   const int n = *r.n_ptr;
   const int first = r.first_ptr ? *r.first_ptr : 0;
@@ -275,13 +281,17 @@ static __global__ __launch_bounds__(256) void gather_rows_flat_kernel(MoveGroup 
     const int lim = nr * upr;
     int rr = r0, uu = u0;
     for (int f0 = threadIdx.x; f0 < lim; f0 += 256 * U) {
-      int slot[U], off[U];
+      int slot[U], id[U], off[U];
       int64_t da[U];
       V16 v[U];
 #pragma unroll
       for (int k = 0; k < U; ++k) {
         const int i = row0 + rr;
-        slot[k] = f0 + 256 * k < lim ? src_index[i] : -1;
+        slot[k] = id[k] = -1;
+        if (f0 + 256 * k < lim) {
+          slot[k] = src_index[i];
+          if (MISSES) id[k] = ids[i];  // beside the slot, not behind it: a miss waits for one read, not for two
+        }
         off[k] = (uu == upr - 1) ? last_off : 16 * uu;
         da[k] = (int64_t)i * dst_pitch + off[k];
         uu += dr;
@@ -291,13 +301,18 @@ static __global__ __launch_bounds__(256) void gather_rows_flat_kernel(MoveGroup 
           ++rr;
         }
       }
+      const uint8_t *at[U];
+#pragma unroll
+      for (int k = 0; k < U; ++k) {
+        at[k] = (uint32_t)slot[k] < n_src ? src + (int64_t)slot[k] * src_pitch + off[k] : nullptr;
+        if (MISSES && !at[k] && (uint32_t)id[k] < n_table) at[k] = table + (int64_t)id[k] * src_pitch + off[k];
+      }
 #pragma unroll
       for (int k = 0; k < U; ++k)
-        if (slot[k] >= 0)
-          v[k] = __builtin_nontemporal_load(reinterpret_cast<const V16 *>(src + (int64_t)slot[k] * src_pitch + off[k]));
+        if (at[k]) v[k] = __builtin_nontemporal_load(reinterpret_cast<const V16 *>(at[k]));
 #pragma unroll
       for (int k = 0; k < U; ++k)
-        if (slot[k] >= 0) {
+        if (at[k]) {
           V16 *d = reinterpret_cast<V16 *>(dst + da[k]);
           if (NT) __builtin_nontemporal_store(v[k], d);
           else *d = v[k];
@@ -332,6 +347,10 @@ struct MoveArgs {
   unsigned long long *row_counter;  // device counter that receives the number of work items, or null
   hipEvent_t ev_start, ev_stop;     // stamped with the kernel's begin and end when not null (profiling)
   const uint8_t *src;
+  int64_t n_src;                    // rows of src (flat gather: indexes at or beyond it move nothing)
+  const uint8_t *table;             // flat gather: the feature table rows without a slot are read from, or null
+  int64_t n_table;                  // node ids below this have a row there
+  bool note_rows;                   // flat gather: leave the row counts for later grids (a batch, not a cache being filled)
   int64_t src_row_bytes, dst_row_bytes, row_bytes;  // row_bytes = bytes moved per row
   int64_t n_max;   // per pipe
 };
@@ -435,21 +454,23 @@ static int launch_gather_flat(Server *s, hipStream_t st, const MoveArgs &a, bool
   const int U = u_want >= 4 ? 4 : u_want >= 2 ? 2 : 1;
   int rpt = (int)std::max<int64_t>(2, std::min<int64_t>(64, 8192 / a.row_bytes));
   if (s->gather_tile_rows > 0) rpt = std::min(s->gather_tile_rows, 256);
-  const int64_t want = ceil_div(hinted_rows(s, a.n_max), rpt);
+  const int64_t want = ceil_div(a.note_rows ? hinted_rows(s, a.n_max) : a.n_max, rpt);
   const int64_t cap = a.max_blocks > 0 ? a.max_blocks : s->gather_blocks > 0 ? s->gather_blocks : (int64_t)s->n_cu * 64;
   const int grid = (int)std::max<int64_t>(1, std::min(want, cap));
-#define LMI_FLAT(V_, U_, NT_)                                                                                          \
+#define LMI_FLAT(V_, U_, NT_, M_)                                                                                      \
   if (a.ev_start)                                                                                                      \
-    hipExtLaunchKernelGGL((gather_rows_flat_kernel<V_, U_, NT_>), dim3(grid * a.g.n), dim3(256), 0, st, a.ev_start,     \
-                          a.ev_stop, 0, a.g, a.src, upr, last_off, rpt, a.src_row_bytes, a.dst_row_bytes,              \
-                          a.row_counter, s->rows_seen_dev);                                                            \
+    hipExtLaunchKernelGGL((gather_rows_flat_kernel<V_, U_, NT_, M_>), dim3(grid * a.g.n), dim3(256), 0, st,             \
+                          a.ev_start, a.ev_stop, 0, a.g, a.src, (uint32_t)a.n_src, a.table, (uint32_t)a.n_table, upr,   \
+                          last_off, rpt, a.src_row_bytes, a.dst_row_bytes, a.row_counter, a.note_rows ? s->rows_seen_dev : nullptr); \
   else                                                                                                                 \
-    hipLaunchKernelGGL((gather_rows_flat_kernel<V_, U_, NT_>), dim3(grid * a.g.n), dim3(256), 0, st, a.g, a.src, upr,   \
-                       last_off, rpt, a.src_row_bytes, a.dst_row_bytes, a.row_counter, s->rows_seen_dev)
-#define LMI_FLAT_U(V_, NT_)                 \
-  if (U == 4) { LMI_FLAT(V_, 4, NT_); }     \
-  else if (U == 2) { LMI_FLAT(V_, 2, NT_); } \
-  else { LMI_FLAT(V_, 1, NT_); }
+    hipLaunchKernelGGL((gather_rows_flat_kernel<V_, U_, NT_, M_>), dim3(grid * a.g.n), dim3(256), 0, st, a.g, a.src,    \
+                       (uint32_t)a.n_src, a.table, (uint32_t)a.n_table, upr, last_off, rpt, a.src_row_bytes,           \
+                       a.dst_row_bytes, a.row_counter, a.note_rows ? s->rows_seen_dev : nullptr)
+#define LMI_FLAT_U(V_, NT_)                        \
+  if (a.table) { LMI_FLAT(V_, 2, NT_, true); }       \
+  else if (U == 4) { LMI_FLAT(V_, 4, NT_, false); } \
+  else if (U == 2) { LMI_FLAT(V_, 2, NT_, false); } \
+  else { LMI_FLAT(V_, 1, NT_, false); }
   if (aligned16 && nt) { LMI_FLAT_U(u32x4, true) }
   else if (aligned16) { LMI_FLAT_U(u32x4, false) }
   else if (nt) { LMI_FLAT_U(u32x4_a4, true) }
@@ -477,13 +498,16 @@ static int launch_move_rows_tiled(Server *s, hipStream_t st, const MoveArgs &a, 
   return LMI_OK;
 }
 
+// measurement knobs of the lane-group mover
+static bool lane_group_knobs(const Server *s, bool host_link) { return s->gather_vec != 0 || (s->gather_lpr != 0 && !host_link); }
+
 // Picks the widest vector that divides the row and all base addresses, and a
 // power-of-two lane group that covers one row when possible; rows such a group does not
 // fit exactly go to the tiled mover.
 static int launch_move_rows(Server *s, hipStream_t st, const MoveArgs &a, bool nt) {
   if (a.n_max <= 0 || a.row_bytes <= 0) return LMI_OK;
   if (a.g.n < 1 || a.g.n > LMI_MAX_GROUP) LMI_FAIL(LMI_ERR_ARG, "a row move serves 1..LMI_MAX_GROUP pipes");
-  uintptr_t align = (uintptr_t)a.src | (uintptr_t)a.src_row_bytes | (uintptr_t)a.dst_row_bytes | (uintptr_t)a.row_bytes;
+  uintptr_t align = (uintptr_t)a.src | (uintptr_t)a.table | (uintptr_t)a.src_row_bytes | (uintptr_t)a.dst_row_bytes | (uintptr_t)a.row_bytes;
   for (int k = 0; k < a.g.n; ++k) align |= (uintptr_t)a.g.p[k].dst;
   int vec = (align % 16 == 0) ? 16 : (align % 8 == 0) ? 8 : 4;
   if (align % 4 != 0) LMI_FAIL(LMI_ERR_ARG, "feature rows must be 4-byte aligned");
@@ -491,7 +515,7 @@ static int launch_move_rows(Server *s, hipStream_t st, const MoveArgs &a, bool n
     // a lane group fits exactly when the row is 8, 16, 32 or 64 aligned 16-byte chunks (128 .. 1024 bytes)
     const int64_t c16 = a.row_bytes / 16;
     const bool exact = vec == 16 && (c16 == 8 || c16 == 16 || c16 == 32 || c16 == 64);
-    const bool knobs = s->gather_vec != 0 || (s->gather_lpr != 0 && !a.host_link);  // measurement knobs of the lane-group mover
+    const bool knobs = lane_group_knobs(s, a.host_link != 0);
     // HBM gather (gather_flat): 0 or 3 the flat gather, 1 the LDS-tiled mover, 2 lane groups; host-link
     // gather (miss_flat): the LDS-tiled mover 0 when no lane group fits, 1 always, 2 never
     const int flat = a.host_link ? s->miss_flat : s->gather_flat;
@@ -1072,10 +1096,12 @@ static int launch_hits_int8(Server *s, const MoveGroup &g, hipStream_t st, int s
   return LMI_OK;
 }
 
-// HBM gather of the cache hits of rows [first, last) on stream `st`, for all n pipes in one launch.
-static int launch_hits(Server *s, Pipe *const *pp, int n, hipStream_t st, int seg, int seg_last) {
+// Gather of rows [first, last) on stream `st`, for all n pipes in one launch: the cache hits from HBM, and with
+// `misses` the other rows from the feature table in the same pass (only where gather_in_line allows it).
+static int launch_hits(Server *s, Pipe *const *pp, int n, hipStream_t st, int seg, int seg_last, bool misses = false) {
   LMI_TRY(lru_wait_copied(s, st));
   const int64_t n_max = s->node_cap[seg_last];
+  const bool have_cache = s->cache_kind != LMI_CACHE_NONE;
   MoveArgs m{};
   m.g.n = n;
   for (int k = 0; k < n; ++k) {
@@ -1084,11 +1110,18 @@ static int launch_hits(Server *s, Pipe *const *pp, int n, hipStream_t st, int se
     r.list = nullptr;  // rows [first, n) directly; cache_index < 0 (a miss) skips the row
     r.first_ptr = seg == 0 ? nullptr : &p.st->node_counter[9 + seg - 1];
     r.n_ptr = &p.st->node_counter[9 + seg_last];
-    r.src_index = p.cache_index;
+    r.src_index = have_cache ? p.cache_index : p.ids;
+    r.ids = p.ids;
     r.dst = (uint8_t *)p.features;
   }
   if (s->cache_kind == LMI_CACHE_INT8) return launch_hits_int8(s, m.g, st, seg_last);
-  m.src = s->cache_data;
+  m.src = have_cache ? s->cache_data : s->feat;
+  m.n_src = have_cache ? s->cache_rows : s->n_nodes;
+  if (misses && have_cache) {
+    m.table = s->feat;
+    m.n_table = s->n_nodes;
+  }
+  m.note_rows = true;
   m.src_row_bytes = m.dst_row_bytes = m.row_bytes = s->row_bytes;
   m.n_max = n_max;
   m.row_counter = s->prof_on ? s->d_prof_rows : nullptr;  // all rows of the segment: hits + misses
@@ -1123,18 +1156,53 @@ static int launch_misses(Server *s, Pipe *const *pp, int n, hipStream_t st, int 
   return launch_move_rows(s, st, m, s->gather_nt != 0);
 }
 
+// Every node has a slot: no batch has a miss.
+static bool no_miss_possible(const Server *s) {
+  return (s->cache_kind == LMI_CACHE_STATIC || s->cache_kind == LMI_CACHE_INT8) && s->cache_rows >= s->n_nodes;
+}
+
+// Hits and misses in one pass of the flat gather: full-width cache rows (an int8 hit and a miss are moved in
+// different ways) of at least 16 bytes, no measurement knob that asks for another mover.  A profiled batch keeps
+// two launches, so that each gather is timed by itself.
+static bool one_pass_gather(const Server *s) {
+  return s->cache_kind != LMI_CACHE_INT8 && s->row_bytes >= 16 && !lane_group_knobs(s, false) &&
+         (s->gather_flat == 0 || s->gather_flat == 3) && !s->prof_on;
+}
+
+// Whether the misses are gathered on the caller's stream like the hits.  A side stream for them costs a fork and a
+// join: 26 us on the device where a second launch on the same stream costs 5, and 11 us of the host's time for each
+// wait it queues.  It pays when it lets the misses of a batch overlap the sampling of the next one -- so not
+//  * when the table lies in HBM, or there is no cache, or no row can miss;
+//  * when what a batch can miss at all takes the link less time than the fork and join (1 MB: 20 us);
+//  * when the caller takes a batch in order, on the batch's own stream, before it issues the next (lmi_batch_wait
+//    on that stream, or reading the batch back): nothing is left to overlap.  The batch before tells.
+// ogbn-products-shaped, one batch of 800 seeds at a time with a wait on the same stream: 160 us with the side
+// stream, 122 us with everything on one and hits and misses in one launch (inference of 16 seeds: 70 and 36 us).
+bool gather_in_line(const Server *s, Pipe *const *pp, int n, int seg_last) {
+  if (s->split_miss == 0 || s->feat_loc != LMI_LOC_HOST || s->cache_kind == LMI_CACHE_NONE) return true;
+  if (s->prof_on) return false;
+  if (no_miss_possible(s)) return true;
+  if (s->split_miss != 1 || s->protect_hits) return false;
+  constexpr int64_t kFewBytes = 1 << 20;
+  if (n * s->node_cap[seg_last] * s->row_bytes <= kFewBytes) return true;
+  for (int k = 0; k < n; ++k)
+    if (!pp[k]->taken_in_order) return false;
+  return true;
+}
+
 // Gathers the rows [first, last) of a segment into each pipe's feature buffer:
 // cache hits from HBM, misses over the host link.  A wide host-link gather beside
 // the HBM gather cuts its bandwidth by more than half, so the misses of one batch
 // never share a stream with its hits, and run on a small grid (miss_blocks).  With
 // several pipes, the hits of all are one launch and so are the misses (group_miss).
 // Schedules (tuning key "split_miss"):
-//   0  both on the caller's stream, one after the other;
+//   0  both on the caller's stream, in one pass where one_pass_gather allows it;
 //   1  hits on the caller's stream, misses after them on the server's side stream,
 //      where they overlap the next batch's sampling;
 //   2  both on the side stream (a gather stage behind the sampling stage): the
 //      caller's stream is free for the next batch's sampling as soon as the lookup
 //      is done.
+// gather_in_line says when schedule 0 is taken whatever the knob says.
 // With 1 and 2 the caller's stream does not wait here: the next call on this pipe,
 // or lmi_batch_wait, joins.  The LRU cache joins at once (its insert copies the rows).
 int launch_misses_early(Server *s, Pipe *const *pp, int n, hipStream_t st, int seg, int seg_last) {
@@ -1150,17 +1218,20 @@ int launch_gather_group(Server *s, Pipe *const *pp, int n, hipStream_t st, int s
                         bool same_stream, int hit_seg_first) {
   const int hit_seg = hit_seg_first >= 0 ? hit_seg_first : seg;  // the hits of segments whose misses went ahead
   const bool have_cache = s->cache_kind != LMI_CACHE_NONE;
-  int mode = (s->feat_loc == LMI_LOC_HOST && have_cache && !same_stream) ? s->split_miss : 0;
+  const bool in_line = same_stream || gather_in_line(s, pp, n, seg_last);
+  int mode = in_line ? 0 : s->split_miss;
   // The gather kernels carry their own profiling events (prof_kernel_events); a bracket
   // left open by the sampling phase ends here.
   hipEvent_t closing = prof_phase(s, st, &s->prof_open, -1);
   if (mode == 0) {
-    for (int k = 0; k < n; ++k) {
-      pp[k]->tail_unjoined = true;  // everything is on the caller's stream
-      if (have_cache) LMI_TRY(launch_hits(s, pp + k, 1, st, seg, seg_last));
-      LMI_TRY(launch_misses(s, pp + k, 1, st, seg, seg_last));
-      if (lru_lists > 0) LMI_TRY(launch_lru_insert(s, *pp[k], st, lru_lists));
+    for (int k = 0; k < n; ++k) pp[k]->tail_unjoined = true;  // everything is on the caller's stream
+    if (one_pass_gather(s)) {
+      LMI_TRY(launch_hits(s, pp, n, st, seg, seg_last, true));
+    } else {
+      if (have_cache) LMI_TRY(launch_hits(s, pp, n, st, seg, seg_last));
+      if (!no_miss_possible(s)) LMI_TRY(launch_misses(s, pp, n, st, seg, seg_last));
     }
+    for (int k = 0; k < n && lru_lists > 0; ++k) LMI_TRY(launch_lru_insert(s, *pp[k], st, lru_lists));
     return LMI_OK;
   }
   hipEvent_t fork = closing;  // when mode 2 forks right here, the closing event doubles as the fork
@@ -1323,6 +1394,7 @@ int launch_lru_insert(Server *s, Pipe &p, hipStream_t st, int n_lists) {
   // keys and ticks are final: the next batch's lookup may start while the rows are still copied
   LMI_HIP(hipEventRecord(s->lru_ready, st));
   s->lru_pending = true;
+  s->lru_stream = st;
   // copy the granted rows from the output buffer (already gathered) into the cache
   for (int l = 0; l < n_lists; ++l) {
     MoveArgs m{};
@@ -1347,7 +1419,7 @@ int launch_lru_insert(Server *s, Pipe &p, hipStream_t st, int n_lists) {
 // The LRU state is batch-synchronous: a lookup sees the cache after the previous batch's
 // insertion.  Sampling does not touch the cache, so only the lookup has to wait.
 int lru_wait_ready(Server *s, hipStream_t st) {
-  if (s->cache_kind != LMI_CACHE_LRU || !s->lru_pending) return LMI_OK;
+  if (s->cache_kind != LMI_CACHE_LRU || !s->lru_pending || s->lru_stream == st) return LMI_OK;  // a stream orders itself
   if (hipEventQuery(s->lru_ready) == hipSuccess) {
     s->lru_pending = false;
     return LMI_OK;
@@ -1359,7 +1431,7 @@ int lru_wait_ready(Server *s, hipStream_t st) {
 
 // The rows the previous batch's insertion granted must be in the cache before a gather reads it.
 int lru_wait_copied(Server *s, hipStream_t st) {
-  if (s->cache_kind != LMI_CACHE_LRU || !s->lru_copy_pending) return LMI_OK;
+  if (s->cache_kind != LMI_CACHE_LRU || !s->lru_copy_pending || s->lru_stream == st) return LMI_OK;
   if (hipEventQuery(s->lru_copied) == hipSuccess) {
     s->lru_copy_pending = false;
     return LMI_OK;
@@ -1624,6 +1696,7 @@ int cache_build_static(Server *s, int64_t capacity_rows, int table_kind, bool in
     m.g.p[0].src_index = d_cached;
     m.g.p[0].dst = s->cache_data;
     m.src = s->feat;
+    m.n_src = N;
     m.src_row_bytes = m.dst_row_bytes = m.row_bytes = s->row_bytes;
     m.n_max = cap;
     LMI_TRY(launch_move_rows(s, 0, m, false));

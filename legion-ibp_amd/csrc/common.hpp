@@ -117,6 +117,8 @@ struct Pipe {
   hipStream_t last_stream = nullptr;
   bool tail_unjoined = false;
   hipEvent_t handover = nullptr;
+  bool taken_in_order = false;  // this batch's caller waited for the batch before on that batch's own stream, and only
+                                // then issued this one: its misses have nothing to overlap (gather_in_line)
   int32_t *seed_stage = nullptr;  // [batch_size] host seeds land here
   int32_t n_seeds = 0;
   int32_t hops_done = 0;
@@ -196,6 +198,7 @@ struct Server {
   bool lru_pending = false;        // an insertion may still be running
   hipEvent_t lru_copied = nullptr; // recorded when the granted rows are in the cache: the next HBM gather waits for it
   bool lru_copy_pending = false;
+  hipStream_t lru_stream = nullptr;  // the stream of the last insertion: it needs no event to be in order
   // sticky fault words in pinned + mapped host memory, written by kernels, never cleared by a batch:
   // [0] a seed id outside [0, n_nodes), [1] a look-back scan gave up
   volatile int32_t *fault_host = nullptr;
@@ -206,6 +209,8 @@ struct Server {
   int32_t *rows_seen_dev = nullptr;
   // pipes
   std::vector<Pipe> pipes;
+  int last_pipe = -1;          // the pipe a single batch was last issued on, and whether the caller has taken that batch
+  bool last_taken = false;     // on its own stream since (Pipe::taken_in_order)
   hipStream_t side = nullptr;  // server-owned second stream for gathers that must not hold up the caller's stream
   // tuning
   int gather_lpr = 0;     // lanes per row (0 = auto)
@@ -293,6 +298,8 @@ int launch_gather_seg(Server *s, Pipe &p, hipStream_t st, int seg, int seg_last,
 // same_stream: hits then misses on `st` whatever the schedule knob says (nothing is left pending).
 int launch_gather_group(Server *s, Pipe *const *pp, int n, hipStream_t st, int seg, int seg_last, int lru_lists,
                         bool same_stream = false, int hit_seg_first = -1);
+// whether the misses of these batches are gathered on the caller's stream
+bool gather_in_line(const Server *s, Pipe *const *pp, int n, int seg_last);
 // the host-link gather of segments [seg, seg_last] released now, ahead of the batch's later hops (split_lookup)
 int launch_misses_early(Server *s, Pipe *const *pp, int n, hipStream_t st, int seg, int seg_last);
 int launch_lru_insert(Server *s, Pipe &p, hipStream_t st, int n_lists);
