@@ -356,14 +356,6 @@ static int static_scratch_setup(int device) {
   return LMI_OK;
 }
 
-// The two 16-int headers live in the batch state; the caller of the static entry point owns
-// separate arrays for them.
-static __global__ void copy_headers_kernel(const DevState *st, int32_t *node_counter, int32_t *edge_counter) {
-  const int t = threadIdx.x;
-  if (t < 16) node_counter[t] = st->node_counter[t];
-  else if (t < 32) edge_counter[t - 16] = st->edge_counter[t - 16];
-}
-
 }  // namespace lmi
 
 using namespace lmi;
@@ -425,13 +417,13 @@ int lmi_server_create(const lmi_config *cfg, lmi_server **out) {
     rc = LMI_ERR_HIP;
   if (rc == LMI_OK) {  // sticky fault words: pinned host memory the kernels write and the host reads without a copy
     void *fh = nullptr, *fd = nullptr;
-    if (hipHostMalloc(&fh, 64, hipHostMallocMapped) != hipSuccess) rc = LMI_ERR_HIP;
+    if (hipHostMalloc(&fh, 128, hipHostMallocMapped) != hipSuccess) rc = LMI_ERR_HIP;
     if (rc == LMI_OK) {
-      memset(fh, 0, 64);
+      memset(fh, 0, 128);
       s->fault_host = (volatile int32_t *)fh;
       if (hipHostGetDevicePointer(&fd, fh, 0) != hipSuccess) rc = LMI_ERR_HIP;
       s->fault_dev = (int32_t *)fd;
-      s->rows_seen_host = s->fault_host + 8;  // the second half of the 64 bytes
+      s->rows_seen_host = s->fault_host + 8;  // LMI_MAX_GROUP words for whole batches, one for each segment
       s->rows_seen_dev = s->fault_dev ? s->fault_dev + 8 : nullptr;
     }
   }
@@ -765,9 +757,27 @@ static int batch_params(Server *s, Pipe &p, hipStream_t st, const int32_t *seeds
   bp->table_tag = max_epoch > 0 ? (int32_t)((uint32_t)p.epoch << id_bits) : 0;
   bp->table_mask = max_epoch > 0 ? (int32_t)(0xFFFFFFFFu << id_bits) : kUntaggedMask;
   bp->fault = s->fault_dev;
+  p.serial = p.serial == INT32_MAX ? 1 : p.serial + 1;
+  bp->serial = p.serial;
   bp->rng_seed = rng_seed ? rng_seed : s->cfg.seed + (uint64_t)(uint32_t)batch_counter;
   if (s->cache_kind == LMI_CACHE_LRU) ++s->lru_tick;
   bp->lru_tick = s->lru_tick;
+  return LMI_OK;
+}
+
+// All hops of a batch on each of n pipes, `early` and `late` the lookups that ride in the first hop and in the later
+// ones.  The last hop's fill is left to the launch that follows.  `own_begin`: the batch starts with a launch of its own
+// (a captured graph re-points that node; the static entry point wipes its table every time).  `misses_early`: the rows
+// on the first list are gathered over the host link from here on (split lookups).
+static int launch_sampling(Server *s, Pipe *const *pp, const BatchParams *bps, int n, hipStream_t st, bool own_begin,
+                           HopLookup early, HopLookup late, bool misses_early = false) {
+  bool begin = own_begin || !hop_sets_up(s);
+  for (int k = 0; k < n; ++k) begin = begin || bps[k].clear_table;
+  if (begin) LMI_TRY(launch_batch_generate(s, pp, bps, n, st, false));
+  for (int k = 0; k < s->cfg.hops; ++k) {
+    LMI_TRY(launch_hop(s, pp, n, st, k, true, true, k == 0 && !begin ? bps : nullptr, k == 0 ? early : late));
+    if (k == 0 && misses_early) LMI_TRY(launch_misses_early(s, pp, n, st, 0, 1));
+  }
   return LMI_OK;
 }
 
@@ -815,7 +825,8 @@ int lmi_op_cache_lookup(lmi_server *h, int pipe, void *stream, int segment) {
   LMI_TRY(lru_wait_ready(s, st));
   prof_phase(s, st, &s->prof_open, PROF_LOOKUP);
   Pipe *pp[1] = {&p};
-  LMI_TRY(launch_lookup(s, pp, 1, st, segment, segment));
+  const bool lists = s->cache_kind == LMI_CACHE_LRU || !gather_in_line(s, pp, 1, segment) || !one_pass_gather(s);
+  LMI_TRY(launch_lookup(s, pp, 1, st, segment, segment, lists));
   LMI_TRY(launch_gather_seg(s, p, st, segment, segment, 0));
   prof_phase(s, st, &s->prof_open, -1);
   return LMI_OK;
@@ -844,10 +855,8 @@ int lmi_presample(lmi_server *h, int pipe, void *stream, int mode, int32_t first
     LMI_TRY(batch_params(s, p, st, nullptr, 0, LMI_LOC_DEVICE, b, mode, 0, &bp));
     s->lru_tick = tick;  // presampling does not age the LRU cache
     Pipe *pp[1] = {&p};
-    LMI_TRY(launch_batch_generate(s, pp, &bp, 1, st, false));
-    for (int k = 0; k < s->cfg.hops; ++k) LMI_TRY(launch_hop(s, pp, 1, st, k, true, true));
-    LMI_TRY(launch_fill(s, pp, 1, st));
-    LMI_TRY(launch_hotness(s, p, st));
+    LMI_TRY(launch_sampling(s, pp, &bp, 1, st, false, HopLookup{}, HopLookup{}));
+    LMI_TRY(launch_hotness(s, p, st));  // finishes the last hop too
   }
   return LMI_OK;
 }
@@ -876,9 +885,11 @@ static int capture_batch_graph(Server *s, Pipe &p, hipStream_t st, const BatchPa
   s->prof_on = false;  // no event records inside the capture
   LMI_HIP(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
   Pipe *pp[1] = {&p};
-  int rc = launch_batch_generate(s, pp, &bp, 1, st, false);
-  for (int k = 0; rc == LMI_OK && k < s->cfg.hops; ++k) rc = launch_hop(s, pp, 1, st, k, true, true);
-  if (rc == LMI_OK) rc = launch_lookup(s, pp, 1, st, 0, s->cfg.hops);
+  // miss lists whatever the gather of the batch at hand will want: the graph serves the next batches too
+  const bool lru = s->cache_kind == LMI_CACHE_LRU;
+  const HopLookup look{lru ? LOOK_NOT : LOOK_LIST, 0};
+  int rc = launch_sampling(s, pp, &bp, 1, st, true, look, look);
+  if (rc == LMI_OK && lru) rc = launch_lookup(s, pp, 1, st, 0, s->cfg.hops);
   hipGraph_t g = nullptr;
   const hipError_t e = hipStreamEndCapture(st, &g);
   s->prof_on = prof;
@@ -907,6 +918,7 @@ static int capture_batch_graph(Server *s, Pipe &p, hipStream_t st, const BatchPa
 static int run_group(Server *s, Pipe *const *pp, const BatchParams *bps, int n, hipStream_t st) {
   for (int k = 0; k < n; ++k) pipe_begin(*pp[k], st);
   prof_phase(s, st, &s->prof_open, PROF_SAMPLE);
+  const bool lru = s->cache_kind == LMI_CACHE_LRU;
   bool split = false;
   if (s->use_graph && st != nullptr && n == 1) {  // the legacy default stream cannot be captured
     Pipe &p = *pp[0];
@@ -914,24 +926,23 @@ static int run_group(Server *s, Pipe *const *pp, const BatchParams *bps, int n, 
     if (!p.graph_exec) LMI_TRY(capture_batch_graph(s, p, st, bps[0]));
     LMI_TRY(graph_update_begin(s, p, bps[0]));
     LMI_HIP(hipGraphLaunch(p.graph_exec, st));
+    p.fill_pending = lru ? -1 : s->cfg.hops - 1;  // what the captured launches leave to the gather
   } else {
-    // split_lookup: the seeds and the first hop's nodes are looked up as soon as they are known and their
-    // misses start over the host link while the later hops are still being sampled
+    // the rows that miss are listed unless hits and misses are gathered in one pass
+    const bool in_line = gather_in_line(s, pp, n, s->cfg.hops);
+    const int mode = lru ? LOOK_NOT : in_line && one_pass_gather(s) ? LOOK_SLOTS : LOOK_LIST;
+    // split_lookup: the misses of the seeds and of the first hop's nodes start over the host link while the later hops
+    // are still being sampled
     split = s->split_lookup && s->cfg.hops >= 2 && s->feat_loc == LMI_LOC_HOST && s->split_miss == 1 &&
             (s->cache_kind == LMI_CACHE_STATIC || s->cache_kind == LMI_CACHE_INT8) &&
-            (s->split_lookup == 1 || (s->split_lookup == 2 && n > 1)) && !gather_in_line(s, pp, n, s->cfg.hops);
-    LMI_TRY(launch_batch_generate(s, pp, bps, n, st, false));
-    for (int k = 0; k < s->cfg.hops; ++k) {
-      LMI_TRY(launch_hop(s, pp, n, st, k, true, true));
-      if (split && k == 0) {
-        LMI_TRY(launch_lookup(s, pp, n, st, 0, 1));
-        LMI_TRY(launch_misses_early(s, pp, n, st, 0, 1));
-      }
+            (s->split_lookup == 1 || (s->split_lookup == 2 && n > 1)) && !in_line;
+    LMI_TRY(launch_sampling(s, pp, bps, n, st, false, HopLookup{mode, 0}, HopLookup{mode, split ? 2 : 0}, split));
+    if (lru) {
+      LMI_TRY(lru_wait_ready(s, st));  // sampling may overlap the previous batch's insertion, the lookup may not
+      LMI_TRY(launch_lookup(s, pp, n, st, 0, s->cfg.hops));
     }
-    LMI_TRY(lru_wait_ready(s, st));  // sampling may overlap the previous batch's insertion, the lookup may not
-    LMI_TRY(launch_lookup(s, pp, n, st, split ? 2 : 0, s->cfg.hops));
   }
-  LMI_TRY(launch_gather_group(s, pp, n, st, split ? 2 : 0, s->cfg.hops, s->cache_kind == LMI_CACHE_LRU ? 1 : 0, false, 0));
+  LMI_TRY(launch_gather_group(s, pp, n, st, split ? 2 : 0, s->cfg.hops, lru ? 1 : 0, false, 0));
   prof_phase(s, st, &s->prof_open, -1);
   return LMI_OK;
 }
@@ -1043,17 +1054,10 @@ int lmi_run_once_static(lmi_server *h, void *stream, const int32_t *seeds, int32
   const bool prof = s->prof_on;
   s->prof_on = false;  // profiling creates events: not here
   int rc = batch_params(s, p, st, seeds, n, LMI_LOC_DEVICE, 0, LMI_MODE_TRAIN, rng_seed, &bp);
-  if (rc == LMI_OK) rc = launch_batch_generate(s, pp, &bp, 1, st, false);
-  for (int k = 0; rc == LMI_OK && k < s->cfg.hops; ++k) rc = launch_hop(s, pp, 1, st, k, true, true);
-  if (rc == LMI_OK) rc = launch_lookup(s, pp, 1, st, 0, s->cfg.hops);
-  if (rc == LMI_OK) rc = launch_gather_group(s, pp, 1, st, 0, s->cfg.hops, 0, true);
-  if (rc == LMI_OK) {
-    hipLaunchKernelGGL(copy_headers_kernel, dim3(1), dim3(64), 0, st, p.st, out->node_counter, out->edge_counter);
-    if (hipGetLastError() != hipSuccess) {
-      set_error("launch of the header copy failed");
-      rc = LMI_ERR_HIP;
-    }
-  }
+  const HopLookup look{one_pass_gather(s) ? LOOK_SLOTS : LOOK_LIST, 0};
+  if (rc == LMI_OK) rc = launch_sampling(s, pp, &bp, 1, st, true, look, look);
+  const HeaderCopy headers{out->node_counter, out->edge_counter};
+  if (rc == LMI_OK) rc = launch_gather_group(s, pp, 1, st, 0, s->cfg.hops, 0, true, -1, &headers);
   s->prof_on = prof;
   return rc;
 }
@@ -1136,8 +1140,8 @@ int lmi_batch_counters(lmi_server *h, int pipe, void *stream, int32_t node_count
   LMI_HIP(hipMemcpy(&hs, s->pipes[pipe].st, sizeof(DevState), hipMemcpyDeviceToHost));
   if (node_counter) memcpy(node_counter, hs.node_counter, 64);
   if (edge_counter) memcpy(edge_counter, hs.edge_counter, 64);
-  if (hs.scan_fault) LMI_FAIL(LMI_ERR_HIP, "a device scan timed out waiting for an earlier tile");
-  if (hs.bad_id) LMI_FAIL(LMI_ERR_BAD_ID, "a seed id outside [0, %lld) was skipped", (long long)s->n_nodes);
+  if (hs.serial != 0 && hs.scan_fault == hs.serial) LMI_FAIL(LMI_ERR_HIP, "a device scan timed out waiting for an earlier tile");
+  if (hs.serial != 0 && hs.bad_id == hs.serial) LMI_FAIL(LMI_ERR_BAD_ID, "a seed id outside [0, %lld) was skipped", (long long)s->n_nodes);
   return LMI_OK;
 }
 

@@ -39,11 +39,38 @@ struct MoveRow {
   const int32_t *first_ptr, *n_ptr, *src_index, *dst_index;
   const int32_t *ids;  // gather_rows_flat_kernel<.., MISSES>: node id per row
   uint8_t *dst;
+  // the HBM gathers of a batch carry its last steps (MoveGroup::tail_blocks)
+  FillArgs fill;        // last hop's local ids (hop -1: already there)
+  HeaderCopy headers;   // where the batch's headers go besides its state (nodes null: nowhere)
 };
 struct MoveGroup {
   MoveRow p[LMI_MAX_GROUP];
   int n;
+  int tail_blocks;  // blocks [0, tail_blocks) of each pipe finish the batch, the rest gather
 };
+
+// The last steps of a batch in blocks of the gather: the fill is bound by random reads of the dedup table that leave
+// HBM's streams to the gather (four papers100M-shaped batches from a table in HBM: gather 152 us, with the fill 160).
+__device__ __forceinline__ void batch_tail(const MoveRow &r, int bx, int tail_blocks) {
+  if (bx == 0 && r.headers.nodes && threadIdx.x < 32) {
+    const int t = threadIdx.x & 15;
+    const DevState *st = r.fill.st;
+    if (threadIdx.x < 16) r.headers.nodes[t] = st->node_counter[t];
+    else r.headers.edges[t] = st->edge_counter[t];
+  }
+  fill_local_ids(r.fill, (int64_t)bx * blockDim.x + threadIdx.x, (int64_t)tail_blocks * blockDim.x);
+}
+
+// LMI_GRID_ROW for a kernel that carries batch_tail: those blocks leave, bx and gx count the others.
+#define LMI_GRID_ROW_TAIL(g)                                                          \
+  const GridRow lmi_gr_ = grid_row(blockIdx.x, (unsigned)(g).n);                      \
+  const int row = lmi_gr_.row;                                                        \
+  if (lmi_gr_.bx < (g).tail_blocks) {                                                 \
+    batch_tail((g).p[row], lmi_gr_.bx, (g).tail_blocks);                              \
+    return;                                                                           \
+  }                                                                                   \
+  const int bx = lmi_gr_.bx - (g).tail_blocks;                                        \
+  const int gx = (int)(gridDim.x / (unsigned)(g).n) - (g).tail_blocks
 
 template <typename V, int LPR, int U, bool NT, bool HOSTLINK>
 static __global__ __launch_bounds__(256) void move_rows_kernel(
@@ -261,7 +288,7 @@ static __global__ __launch_bounds__(256) void gather_rows_flat_kernel(MoveGroup 
                                                                       int rows_per_tile, int64_t src_pitch,
                                                                       int64_t dst_pitch, unsigned long long *row_counter,
                                                                       int32_t *rows_seen) {
-  LMI_GRID_ROW(g.n);
+  LMI_GRID_ROW_TAIL(g);
   const MoveRow &r = g.p[row];
   const int32_t *__restrict__ src_index = r.src_index;
   const int32_t *__restrict__ ids = r.ids;
@@ -327,15 +354,22 @@ static __global__ __launch_bounds__(256) void gather_rows_flat_kernel(MoveGroup 
 // its time.  The gather kernels leave the row count of every launch in pinned host memory
 // (rows_seen); the largest of the last launch, with an eighth on top, sizes the next grid.  The
 // kernels stride over their tiles by the grid, so a grid that turns out small is slower, not wrong.
-static int64_t hinted_rows(Server *s, int64_t n_max) {
+// Whole batches use the first LMI_MAX_GROUP words; a gather of one segment (operator by operator) has a word of its own,
+// or the seeds' 800 rows would size the grid of the last hop's 44 000 (284 instead of 190 us for the operators of a batch).
+static int64_t hinted_rows(Server *s, int64_t n_max, int word) {
   if (!s->rows_seen_host || !s->gather_adaptive) return n_max;
   int32_t seen = 0;
-  for (int k = 0; k < LMI_MAX_GROUP; ++k) {
-    const int32_t v = s->rows_seen_host[k];
+  const int words = word == 0 ? LMI_MAX_GROUP : 1;
+  for (int k = 0; k < words; ++k) {
+    const int32_t v = s->rows_seen_host[word + k];
     seen = v > seen ? v : seen;
   }
   if (seen <= 0) return n_max;  // nothing seen yet
   return std::min<int64_t>(n_max, (int64_t)seen + seen / 8 + 64);
+}
+
+static int rows_word(const Server *s, int seg, int seg_last) {
+  return seg_last == s->cfg.hops && (seg == 0 || seg != seg_last) ? 0 : LMI_MAX_GROUP + seg_last;
 }
 
 struct MoveArgs {
@@ -350,7 +384,7 @@ struct MoveArgs {
   int64_t n_src;                    // rows of src (flat gather: indexes at or beyond it move nothing)
   const uint8_t *table;             // flat gather: the feature table rows without a slot are read from, or null
   int64_t n_table;                  // node ids below this have a row there
-  bool note_rows;                   // flat gather: leave the row counts for later grids (a batch, not a cache being filled)
+  int note_rows;                    // flat gather: the word of rows_seen that receives the row counts (hinted_rows), or -1
   int64_t src_row_bytes, dst_row_bytes, row_bytes;  // row_bytes = bytes moved per row
   int64_t n_max;   // per pipe
 };
@@ -454,18 +488,18 @@ static int launch_gather_flat(Server *s, hipStream_t st, const MoveArgs &a, bool
   const int U = u_want >= 4 ? 4 : u_want >= 2 ? 2 : 1;
   int rpt = (int)std::max<int64_t>(2, std::min<int64_t>(64, 8192 / a.row_bytes));
   if (s->gather_tile_rows > 0) rpt = std::min(s->gather_tile_rows, 256);
-  const int64_t want = ceil_div(a.note_rows ? hinted_rows(s, a.n_max) : a.n_max, rpt);
+  const int64_t want = ceil_div(a.note_rows >= 0 ? hinted_rows(s, a.n_max, a.note_rows) : a.n_max, rpt);
   const int64_t cap = a.max_blocks > 0 ? a.max_blocks : s->gather_blocks > 0 ? s->gather_blocks : (int64_t)s->n_cu * 64;
-  const int grid = (int)std::max<int64_t>(1, std::min(want, cap));
+  const int grid = (int)std::max<int64_t>(1, std::min(want, cap)) + a.g.tail_blocks;
 #define LMI_FLAT(V_, U_, NT_, M_)                                                                                      \
   if (a.ev_start)                                                                                                      \
     hipExtLaunchKernelGGL((gather_rows_flat_kernel<V_, U_, NT_, M_>), dim3(grid * a.g.n), dim3(256), 0, st,             \
                           a.ev_start, a.ev_stop, 0, a.g, a.src, (uint32_t)a.n_src, a.table, (uint32_t)a.n_table, upr,   \
-                          last_off, rpt, a.src_row_bytes, a.dst_row_bytes, a.row_counter, a.note_rows ? s->rows_seen_dev : nullptr); \
+                          last_off, rpt, a.src_row_bytes, a.dst_row_bytes, a.row_counter, a.note_rows >= 0 ? s->rows_seen_dev + a.note_rows : nullptr); \
   else                                                                                                                 \
     hipLaunchKernelGGL((gather_rows_flat_kernel<V_, U_, NT_, M_>), dim3(grid * a.g.n), dim3(256), 0, st, a.g, a.src,    \
                        (uint32_t)a.n_src, a.table, (uint32_t)a.n_table, upr, last_off, rpt, a.src_row_bytes,           \
-                       a.dst_row_bytes, a.row_counter, a.note_rows ? s->rows_seen_dev : nullptr)
+                       a.dst_row_bytes, a.row_counter, a.note_rows >= 0 ? s->rows_seen_dev + a.note_rows : nullptr)
 #define LMI_FLAT_U(V_, NT_)                        \
   if (a.table) { LMI_FLAT(V_, 2, NT_, true); }       \
   else if (U == 4) { LMI_FLAT(V_, 4, NT_, false); } \
@@ -668,7 +702,7 @@ static __global__ __launch_bounds__(256) void gather_int8_tiled_kernel(MoveGroup
   __shared__ int s_row[TILE], s_slot[TILE];
   __shared__ float s_scale[TILE];
   __shared__ int s_cnt;
-  LMI_GRID_ROW(g.n);
+  LMI_GRID_ROW_TAIL(g);
   const int32_t *cache_index = g.p[row].src_index;
   OUT *out = reinterpret_cast<OUT *>(g.p[row].dst);
   const int n = *g.p[row].n_ptr;
@@ -780,17 +814,14 @@ static __global__ __launch_bounds__(256) void gather_int8_generic_kernel(MoveGro
 struct LookupArgs {
   const int32_t *ids;
   int64_t n_nodes;
-  int kind, table_kind;
-  const HashSlot *slots;
-  int log2cap;
-  const int32_t *slot_of;
-  const uint4 *rank_tab;
+  int kind;
+  SlotTable table;
   const int32_t *lru_keys;
   int32_t *lru_use;
   int64_t lru_sets;
   int lru_ways;
   int32_t *cache_index, *lru_fill;
-  int2 *miss_list;
+  int2 *miss_list;  // null: no list wanted
   DevState *st;
   int seg_first, seg_last, seg;
   const HashSlot *dedup;  // the batch's dedup table: value of a seed id = its first row
@@ -798,23 +829,6 @@ struct LookupArgs {
   int lookup_blocks;  // blocks [0, lookup_blocks) look rows up, the rest carry `fill`
   FillArgs fill;      // last step of the hop sampled just before (hop -1: none)
 };
-
-// Bitmap + rank table: the slot of a cached node is the number of cached nodes
-// with a smaller id = rank at the start of its 64-id word + set bits below it.
-__device__ __forceinline__ int32_t rank_find(const uint4 *tab, int32_t id) {
-  const uint4 e = tab[id >> 6];
-  const uint64_t bits = (uint64_t)e.x | ((uint64_t)e.y << 32);
-  const int b = id & 63;
-  if (!((bits >> b) & 1ull)) return -1;
-  return (int32_t)e.z + __popcll(bits & ((1ull << b) - 1ull));
-}
-
-__device__ __forceinline__ int32_t static_find(int table_kind, const HashSlot *slots, int log2cap,
-                                               const int32_t *slot_of, const uint4 *rank_tab, int32_t id) {
-  if (table_kind == LMI_TABLE_RANK) return rank_find(rank_tab, id);
-  if (table_kind == LMI_TABLE_DIRECT) return slot_of[id];
-  return table_find(slots, log2cap, id);
-}
 
 // id -> slot for rows [first, last) of the batch -> cache_index[].  Rows that
 // miss are appended to the segment's miss list as (row, id) pairs: ballot +
@@ -877,12 +891,13 @@ static __global__ __launch_bounds__(kLookupBlock) void lookup_kernel(LookupGroup
                               table_find(a.dedup, a.dedup_log2cap, id, a.st->table_tag, a.st->table_mask) != i;
           a.lru_fill[i] = repeat ? -2 : -1;
         } else if (a.kind != LMI_CACHE_NONE) {
-          slot = static_find(a.table_kind, a.slots, a.log2cap, a.slot_of, a.rank_tab, id);
+          slot = static_find(a.table, id);
         }
         miss = slot < 0;
       }
       a.cache_index[i] = slot;
     }
+    if (!a.miss_list) continue;
     const uint64_t mm = __ballot(miss);
     if (lane == 0) wave_cnt[wid] = __popcll(mm);
     __syncthreads();
@@ -902,9 +917,7 @@ static __global__ __launch_bounds__(kLookupBlock) void lookup_kernel(LookupGroup
   }
 }
 
-static inline int64_t seg_list_base(const Server *s, int seg) { return seg == 0 ? 0 : s->node_cap[seg - 1]; }
-
-int launch_lookup(Server *s, Pipe *const *pp, int n, hipStream_t st, int seg_first, int seg_last) {
+int launch_lookup(Server *s, Pipe *const *pp, int n, hipStream_t st, int seg_first, int seg_last, bool with_list) {
   LookupGroup g{};
   g.n = n;
   const int64_t n_max = s->node_cap[seg_last];
@@ -918,17 +931,13 @@ int launch_lookup(Server *s, Pipe *const *pp, int n, hipStream_t st, int seg_fir
     a.ids = p.ids;
     a.n_nodes = s->n_nodes;
     a.kind = s->cache_kind;
-    a.table_kind = s->table_kind;
-    a.slots = s->id_table.slots;
-    a.log2cap = s->id_table.log2cap;
-    a.slot_of = s->slot_of;
-    a.rank_tab = s->rank_tab;
+    a.table = slot_table(s);
     a.lru_keys = s->lru_keys;
     a.lru_use = s->lru_use;
     a.lru_sets = s->lru_sets;
     a.lru_ways = s->lru_ways;
     a.cache_index = p.cache_index;
-    a.miss_list = p.miss_list + seg_list_base(s, seg_first);
+    a.miss_list = with_list ? p.miss_list + miss_list_base(s, seg_first) : nullptr;
     a.lru_fill = p.lru_fill;
     a.dedup = p.dedup.slots;
     a.dedup_log2cap = p.dedup.log2cap;
@@ -1008,7 +1017,7 @@ int pipes_join(Pipe *const *pp, int n, hipStream_t st) {
 }
 
 // int8 rows: dequantised inside the gather.
-static int launch_hits_int8(Server *s, const MoveGroup &g, hipStream_t st, int seg_last) {
+static int launch_hits_int8(Server *s, const MoveGroup &g, hipStream_t st, int seg, int seg_last) {
   const int64_t n_max = s->node_cap[seg_last];
   const int dim = s->cfg.feat_dim;
   const int64_t want = ceil_div(n_max, 4);
@@ -1032,17 +1041,17 @@ static int launch_hits_int8(Server *s, const MoveGroup &g, hipStream_t st, int s
     // 768-element fp16 rows, share of HBM peak: 8 rows per tile 45 %, 16 51 %, 32 54 %, 64 52 %
     const int tile_rows = s->gather_tile_rows > 0 ? std::min(64, s->gather_tile_rows) : 32;
     // sized by the rows the last launches held (hinted_rows): a block without a tile is not free
-    const int64_t want_f = ceil_div(hinted_rows(s, n_max), tile_rows);
+    const int64_t want_f = ceil_div(hinted_rows(s, n_max, rows_word(s, seg, seg_last)), tile_rows);
     const int64_t cap_f = s->gather_blocks > 0 ? s->gather_blocks
                           : s->gather_adaptive ? (int64_t)s->n_cu * 64 : auto_gather_blocks(s, want_f);
-    const int grid_f = g.n * (int)std::max<int64_t>(1, std::min<int64_t>(want_f, cap_f));
+    const int grid_f = g.n * ((int)std::max<int64_t>(1, std::min<int64_t>(want_f, cap_f)) + g.tail_blocks);
 #define LMI_INT8_FLAT(KERN)                                                                                   \
   if (e0)                                                                                                     \
     hipExtLaunchKernelGGL((KERN), dim3(grid_f), dim3(256), 0, st, e0, e1, 0, g, q, s->cache_scale, dim,        \
-                          tile_rows, rc, s->rows_seen_dev);                                                   \
+                          tile_rows, rc, s->rows_seen_dev + rows_word(s, seg, seg_last));                      \
   else                                                                                                        \
     hipLaunchKernelGGL((KERN), dim3(grid_f), dim3(256), 0, st, g, q, s->cache_scale, dim, tile_rows, rc,       \
-                       s->rows_seen_dev)
+                       s->rows_seen_dev + rows_word(s, seg, seg_last))
 #define LMI_INT8_FLAT_U(OUT_, EPL_)                                    \
   if (s->gather_unroll >= 4) {                                         \
     LMI_INT8_FLAT((gather_int8_tiled_kernel<OUT_, EPL_, 4>));           \
@@ -1096,10 +1105,45 @@ static int launch_hits_int8(Server *s, const MoveGroup &g, hipStream_t st, int s
   return LMI_OK;
 }
 
+// Hands the batches' last steps to a launch over `g`.
+static void tail_args(Server *s, Pipe *const *pp, int n, const HeaderCopy *headers, MoveGroup *g) {
+  const int pending = pp[0]->fill_pending;  // the pipes are in step
+  if (pending < 0 && !headers) return;
+  g->tail_blocks = pending >= 0 ? fill_blocks(s->edge_cap[pending], 256) : 1;
+  for (int k = 0; k < n; ++k) {
+    g->p[k].fill = fill_args(*pp[k], pending);
+    if (headers) g->p[k].headers = *headers;
+    pp[k]->fill_pending = -1;
+  }
+}
+
+static __global__ __launch_bounds__(256) void batch_tail_kernel(MoveGroup g) {
+  LMI_GRID_ROW(g.n);
+  batch_tail(g.p[row], bx, g.tail_blocks);
+}
+
+// ... or to a launch of their own, if anything is left.
+static int launch_batch_tail(Server *s, Pipe *const *pp, int n, hipStream_t st, const HeaderCopy *headers) {
+  MoveGroup g{};
+  g.n = n;
+  tail_args(s, pp, n, headers, &g);
+  if (g.tail_blocks == 0) return LMI_OK;
+  hipLaunchKernelGGL(batch_tail_kernel, dim3(g.tail_blocks * n), dim3(256), 0, st, g);
+  LMI_HIP(hipGetLastError());
+  return LMI_OK;
+}
+
 // Gather of rows [first, last) on stream `st`, for all n pipes in one launch: the cache hits from HBM, and with
 // `misses` the other rows from the feature table in the same pass (only where gather_in_line allows it).
-static int launch_hits(Server *s, Pipe *const *pp, int n, hipStream_t st, int seg, int seg_last, bool misses = false) {
+static int launch_hits(Server *s, Pipe *const *pp, int n, hipStream_t st, int seg, int seg_last, bool misses = false,
+                       const HeaderCopy *headers = nullptr) {
   LMI_TRY(lru_wait_copied(s, st));
+  // what is left of the batch rides in the flat and the tiled int8 gather; a profiled gather is timed by itself
+  const bool carries = !s->prof_on && (s->cache_kind == LMI_CACHE_INT8
+                                           ? s->cfg.feat_dim % 16 == 0 && s->gather_flat != 2
+                                           : s->row_bytes >= 16 && !lane_group_knobs(s, false) &&
+                                                 (s->gather_flat == 0 || s->gather_flat == 3));
+  if (!carries) LMI_TRY(launch_batch_tail(s, pp, n, st, headers));
   const int64_t n_max = s->node_cap[seg_last];
   const bool have_cache = s->cache_kind != LMI_CACHE_NONE;
   MoveArgs m{};
@@ -1113,15 +1157,17 @@ static int launch_hits(Server *s, Pipe *const *pp, int n, hipStream_t st, int se
     r.src_index = have_cache ? p.cache_index : p.ids;
     r.ids = p.ids;
     r.dst = (uint8_t *)p.features;
+    r.fill.hop = -1;
   }
-  if (s->cache_kind == LMI_CACHE_INT8) return launch_hits_int8(s, m.g, st, seg_last);
+  if (carries) tail_args(s, pp, n, headers, &m.g);
+  if (s->cache_kind == LMI_CACHE_INT8) return launch_hits_int8(s, m.g, st, seg, seg_last);
   m.src = have_cache ? s->cache_data : s->feat;
   m.n_src = have_cache ? s->cache_rows : s->n_nodes;
   if (misses && have_cache) {
     m.table = s->feat;
     m.n_table = s->n_nodes;
   }
-  m.note_rows = true;
+  m.note_rows = rows_word(s, seg, seg_last);
   m.src_row_bytes = m.dst_row_bytes = m.row_bytes = s->row_bytes;
   m.n_max = n_max;
   m.row_counter = s->prof_on ? s->d_prof_rows : nullptr;  // all rows of the segment: hits + misses
@@ -1137,7 +1183,7 @@ static int launch_misses(Server *s, Pipe *const *pp, int n, hipStream_t st, int 
   m.g.n = n;
   for (int k = 0; k < n; ++k) {
     MoveRow &r = m.g.p[k];
-    r.list = pp[k]->miss_list + seg_list_base(s, seg);
+    r.list = pp[k]->miss_list + miss_list_base(s, seg);
     r.n_ptr = &pp[k]->st->n_miss[seg];
     r.dst = (uint8_t *)pp[k]->features;
   }
@@ -1164,7 +1210,7 @@ static bool no_miss_possible(const Server *s) {
 // Hits and misses in one pass of the flat gather: full-width cache rows (an int8 hit and a miss are moved in
 // different ways) of at least 16 bytes, no measurement knob that asks for another mover.  A profiled batch keeps
 // two launches, so that each gather is timed by itself.
-static bool one_pass_gather(const Server *s) {
+bool one_pass_gather(const Server *s) {
   return s->cache_kind != LMI_CACHE_INT8 && s->row_bytes >= 16 && !lane_group_knobs(s, false) &&
          (s->gather_flat == 0 || s->gather_flat == 3) && !s->prof_on;
 }
@@ -1215,28 +1261,31 @@ int launch_misses_early(Server *s, Pipe *const *pp, int n, hipStream_t st, int s
 }
 
 int launch_gather_group(Server *s, Pipe *const *pp, int n, hipStream_t st, int seg, int seg_last, int lru_lists,
-                        bool same_stream, int hit_seg_first) {
+                        bool same_stream, int hit_seg_first, const HeaderCopy *headers) {
   const int hit_seg = hit_seg_first >= 0 ? hit_seg_first : seg;  // the hits of segments whose misses went ahead
   const bool have_cache = s->cache_kind != LMI_CACHE_NONE;
   const bool in_line = same_stream || gather_in_line(s, pp, n, seg_last);
   int mode = in_line ? 0 : s->split_miss;
   // The gather kernels carry their own profiling events (prof_kernel_events); a bracket
   // left open by the sampling phase ends here.
-  hipEvent_t closing = prof_phase(s, st, &s->prof_open, -1);
+  prof_phase(s, st, &s->prof_open, -1);
   if (mode == 0) {
     for (int k = 0; k < n; ++k) pp[k]->tail_unjoined = true;  // everything is on the caller's stream
     if (one_pass_gather(s)) {
-      LMI_TRY(launch_hits(s, pp, n, st, seg, seg_last, true));
+      LMI_TRY(launch_hits(s, pp, n, st, seg, seg_last, true, headers));
     } else {
-      if (have_cache) LMI_TRY(launch_hits(s, pp, n, st, seg, seg_last));
+      if (have_cache) LMI_TRY(launch_hits(s, pp, n, st, seg, seg_last, false, headers));
+      else LMI_TRY(launch_batch_tail(s, pp, n, st, headers));
       if (!no_miss_possible(s)) LMI_TRY(launch_misses(s, pp, n, st, seg, seg_last));
     }
     for (int k = 0; k < n && lru_lists > 0; ++k) LMI_TRY(launch_lru_insert(s, *pp[k], st, lru_lists));
     return LMI_OK;
   }
-  hipEvent_t fork = closing;  // when mode 2 forks right here, the closing event doubles as the fork
-  if (mode == 2)
+  hipEvent_t fork = nullptr;
+  if (mode == 2) {
+    LMI_TRY(launch_batch_tail(s, pp, n, st, nullptr));
     for (int k = 0; k < n; ++k) pp[k]->tail_unjoined = false;  // both gathers run behind the fork
+  }
   if (mode == 1) {
     // Host-link reads in flight halve the HBM gather's bandwidth: optionally hold the hits back
     // until the side stream has drained the host-link gathers issued before (other pipes').
@@ -1256,7 +1305,6 @@ int launch_gather_group(Server *s, Pipe *const *pp, int n, hipStream_t st, int s
     // behind a late fork the join event covers the whole batch; ahead of an early one the HBM gather stays
     // on the caller's stream alone
     for (int k = 0; k < n; ++k) pp[k]->tail_unjoined = early;
-    fork = nullptr;
     if (early) {
       fork = pp[0]->fork;
       LMI_HIP(hipEventRecord(fork, st));
@@ -1377,7 +1425,7 @@ int launch_lru_insert(Server *s, Pipe &p, hipStream_t st, int n_lists) {
   if (s->cache_kind != LMI_CACHE_LRU) return LMI_OK;
   LruArgs a{};
   a.ids = p.ids;
-  for (int l = 0; l < n_lists; ++l) a.miss_list[l] = p.miss_list + seg_list_base(s, l);
+  for (int l = 0; l < n_lists; ++l) a.miss_list[l] = p.miss_list + miss_list_base(s, l);
   a.st = p.st;
   a.n_lists = n_lists;
   a.keys = s->lru_keys;
@@ -1400,7 +1448,7 @@ int launch_lru_insert(Server *s, Pipe &p, hipStream_t st, int n_lists) {
     MoveArgs m{};
     m.g.n = 1;
     MoveRow &r = m.g.p[0];
-    r.list = p.miss_list + seg_list_base(s, l);
+    r.list = p.miss_list + miss_list_base(s, l);
     r.n_ptr = &p.st->n_miss[l];
     r.src_index = nullptr;
     m.src_from_list = 0;
@@ -1449,10 +1497,16 @@ __device__ __forceinline__ int64_t rank_key(const int64_t *indptr, const uint32_
 
 // Presampling hotness (reference: HotnessMeasure, cache/cache_impl.cuh:190-198): one
 // count per appearance of a node among a batch's sampled ids.
+// Extra blocks finish a hop left pending.
 static __global__ __launch_bounds__(256) void hotness_kernel(const int32_t *ids, const DevState *st, int64_t n_nodes,
-                                                             uint32_t *hot) {
+                                                             uint32_t *hot, FillArgs fill, int fill_grid) {
+  const int bx = (int)blockIdx.x - fill_grid, gx = (int)gridDim.x - fill_grid;
+  if (bx < 0) {
+    fill_local_ids(fill, (int64_t)blockIdx.x * blockDim.x + threadIdx.x, (int64_t)fill_grid * blockDim.x);
+    return;
+  }
   const int n = st->node_counter[7];
-  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
+  for (int i = bx * blockDim.x + threadIdx.x; i < n; i += gx * blockDim.x) {
     const int32_t v = ids[i];
     if (v >= 0 && v < n_nodes) atomicAdd(&hot[v], 1u);
   }
@@ -1464,7 +1518,10 @@ int launch_hotness(Server *s, Pipe &p, hipStream_t st) {
     LMI_HIP(hipMemsetAsync(s->hot, 0, (size_t)s->n_nodes * 4, st));
   }
   const int grid = (int)std::max<int64_t>(1, std::min<int64_t>(ceil_div(s->max_nodes, 256), (int64_t)s->n_cu * 4));
-  hipLaunchKernelGGL(hotness_kernel, dim3(grid), dim3(256), 0, st, p.ids, p.st, s->n_nodes, s->hot);
+  const int pending = p.fill_pending, extra = pending >= 0 ? fill_blocks(s->edge_cap[pending], 256) : 0;
+  hipLaunchKernelGGL(hotness_kernel, dim3(grid + extra), dim3(256), 0, st, p.ids, p.st, s->n_nodes, s->hot,
+                     fill_args(p, pending), extra);
+  p.fill_pending = -1;
   LMI_HIP(hipGetLastError());
   return LMI_OK;
 }
@@ -1697,6 +1754,7 @@ int cache_build_static(Server *s, int64_t capacity_rows, int table_kind, bool in
     m.g.p[0].dst = s->cache_data;
     m.src = s->feat;
     m.n_src = N;
+    m.note_rows = -1;
     m.src_row_bytes = m.dst_row_bytes = m.row_bytes = s->row_bytes;
     m.n_max = cap;
     LMI_TRY(launch_move_rows(s, 0, m, false));
@@ -1736,10 +1794,9 @@ int cache_build_lru(Server *s, int64_t n_sets, int32_t ways) {
   return LMI_OK;
 }
 
-static __global__ void dump_static_kernel(int table_kind, const HashSlot *slots, int log2cap, const int32_t *slot_of,
-                                          const uint4 *rank_tab, int64_t n, int32_t *out) {
+static __global__ void dump_static_kernel(SlotTable table, int64_t n, int32_t *out) {
   for (int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; v < n; v += (int64_t)gridDim.x * blockDim.x)
-    out[v] = static_find(table_kind, slots, log2cap, slot_of, rank_tab, (int32_t)v);
+    out[v] = static_find(table, (int32_t)v);
 }
 
 int cache_dump(Server *s, int32_t *slot_of, int64_t n, int32_t *aux) {
@@ -1760,8 +1817,7 @@ int cache_dump(Server *s, int32_t *slot_of, int64_t n, int32_t *aux) {
   if (n != s->n_nodes) LMI_FAIL(LMI_ERR_ARG, "dump needs n == n_nodes");
   int32_t *d = nullptr;
   LMI_HIP(hipMalloc(&d, n * 4));
-  hipLaunchKernelGGL(dump_static_kernel, dim3(s->n_cu * 4), dim3(256), 0, 0, s->table_kind, s->id_table.slots,
-                     s->id_table.log2cap, s->slot_of, s->rank_tab, n, d);
+  hipLaunchKernelGGL(dump_static_kernel, dim3(s->n_cu * 4), dim3(256), 0, 0, slot_table(s), n, d);
   LMI_HIP(hipMemcpy(slot_of, d, n * 4, hipMemcpyDeviceToHost));
   (void)hipFree(d);
   return LMI_OK;

@@ -50,10 +50,12 @@ struct DevState {
   // One miss list per lookup segment (0 = seeds or the whole
   // batch, k = nodes added by hop k); zeroed at batch start.
   int32_t n_miss[LMI_MAX_HOPS + 1];
+  // Conditions: raised when equal to `serial`, the batch's number (a batch that starts while its own kernels already
+  // raise conditions cannot clear them first; a number of an earlier batch means nothing).
   int32_t scan_fault;  // a look-back scan gave up waiting (never expected; reported as an error)
-  int32_t reserved[LMI_MAX_HOPS];
-  int32_t bad_id;      // set when a seed id is outside [0, n_nodes)
-  int32_t scan_total;  // total of the last device scan
+  int32_t bad_id;      // a seed id is outside [0, n_nodes)
+  int32_t serial;
+  int32_t reserved;
   // per-batch parameters, written by the first kernel of a batch so that every
   // later kernel (and a replayed HIP graph) reads them from HBM
   uint32_t rng_lo, rng_hi;   // 64-bit Philox key of this batch
@@ -92,6 +94,7 @@ struct Pipe {
   Table dedup;                 // global id -> local id (per batch)
   int32_t *eslot[2] = {nullptr, nullptr};  // [max_edges_hop] table slot of each edge's source; hops alternate
                                            // so that a hop's slots survive into the next hop's first kernel
+  int32_t serial = 0;          // number of the last batch, never 0 once there was one
   int32_t epoch = 0;           // dedup-table epoch of the last batch
   int id_bits = 0;             // key bits below the epoch tag when that batch ran
   bool table_dirty = true;     // the table must be wiped before its next use
@@ -134,7 +137,7 @@ struct BatchParams {
   int32_t lru_tick;
   int32_t table_tag, table_mask;  // see table_insert_min
   int32_t clear_table;            // 1: the epochs ran out (or the table is new): wipe it first
-  int32_t pad;
+  int32_t serial;                 // number of the batch among its pipe's (DevState::serial)
   uint64_t rng_seed;
   const int32_t *seeds;
   const int32_t *labels;
@@ -204,13 +207,14 @@ struct Server {
   volatile int32_t *fault_host = nullptr;
   int32_t *fault_dev = nullptr;  // the same words as the device addresses them
   bool fault_told[2] = {false, false};  // lmi_batch_wait has reported the condition once already
-  // row counts the gather kernels leave behind, one word per pipe of a launch, in the same pinned allocation
+  // row counts the gather kernels leave behind, one word per pipe of a launch (and one per segment gathered by itself),
+  // in the same pinned allocation
   volatile int32_t *rows_seen_host = nullptr;
   int32_t *rows_seen_dev = nullptr;
   // pipes
   std::vector<Pipe> pipes;
   int last_pipe = -1;          // the pipe a single batch was last issued on, and whether the caller has taken that batch
-  bool last_taken = false;     // on its own stream since (Pipe::taken_in_order)
+  bool last_taken = true;      // on its own stream since (Pipe::taken_in_order); before the first batch nothing is in flight
   hipStream_t side = nullptr;  // server-owned second stream for gathers that must not hold up the caller's stream
   // tuning
   int gather_lpr = 0;     // lanes per row (0 = auto)
@@ -273,8 +277,21 @@ int graph_update_begin(Server *s, Pipe &p, const BatchParams &bp);
 // extra blocks; otherwise a kernel of its own finishes the hop.
 // The launchers below take n pipes that are in step (same stage of their batches) and serve
 // them with the same launches, their blocks interleaved over blockIdx.x (LMI_GRID_ROW).
-int launch_hop(Server *s, Pipe *const *pp, int n, hipStream_t st, int hop, bool stage_seeds, bool defer_fill);
+// begin != null: no batch_begin_kernel ran, the first hop takes the batches' parameters from here and sets up the state.
+// look: the cache lookup of the nodes a hop adds (hop 0: of the seeds too) rides in its flag scan.
+struct HopLookup {
+  int mode = 0;      // LOOK_*
+  int miss_seg = 0;  // LOOK_LIST: the miss list that receives them
+};
+enum { LOOK_NOT = 0, LOOK_SLOTS = 1, LOOK_LIST = 2 };  // not at all; cache_index only; cache_index and the miss list
+int launch_hop(Server *s, Pipe *const *pp, int n, hipStream_t st, int hop, bool stage_seeds, bool defer_fill,
+               const BatchParams *begin = nullptr, HopLookup look = HopLookup{});
+bool hop_sets_up(const Server *s);  // whether launch_hop can take `begin`
 int launch_fill(Server *s, Pipe *const *pp, int n, hipStream_t st);  // finishes a hop left pending, if any
+struct SlotTable;
+SlotTable slot_table(const Server *s);
+// where the miss list of lookup segment `seg` starts in Pipe::miss_list
+inline int64_t miss_list_base(const Server *s, int seg) { return seg == 0 ? 0 : s->node_cap[seg - 1]; }
 struct FillArgs;
 FillArgs fill_args(const Pipe &p, int hop);
 int fill_blocks(int64_t e_max, int block);  // grid share of a fill over at most e_max edges
@@ -286,9 +303,10 @@ enum { SCAN_EPI_NONE = 0, SCAN_EPI_HOP_EDGES = 1, SCAN_EPI_HOP_NODES = 2 };
 int cache_build_static(Server *s, int64_t capacity_rows, int table_kind, bool int8);
 int cache_build_lru(Server *s, int64_t n_sets, int32_t ways);
 void cache_free(Server *s);
-// Extra blocks of the lookup finish a hop left pending (launch_hop, defer_fill).  (Finishing
+// The lookup as a kernel of its own: operator by operator, and for the LRU cache, whose lookup has to wait for the
+// insertion of the batch before.  Extra blocks of it finish a hop left pending (launch_hop, defer_fill).  (Finishing
 // it on the side stream instead, ahead of the host-link gather, measured 2 % slower.)
-int launch_lookup(Server *s, Pipe *const *pp, int n, hipStream_t st, int seg_first, int seg_last);
+int launch_lookup(Server *s, Pipe *const *pp, int n, hipStream_t st, int seg_first, int seg_last, bool with_list = true);
 int launch_hotness(Server *s, Pipe &p, hipStream_t st);
 // lru_lists > 0: the LRU insertion of that many miss lists follows the gather on the stream the
 // misses were gathered on (the side stream when it is in use), and the caller's stream does not wait.
@@ -296,10 +314,16 @@ int launch_gather_seg(Server *s, Pipe &p, hipStream_t st, int seg, int seg_last,
 // The same for n pipes in step: the HBM gathers one after another, one fork, then the
 // host-link gathers one after another on the side stream.
 // same_stream: hits then misses on `st` whatever the schedule knob says (nothing is left pending).
+// headers: where the caller of the static entry point wants the two 16-int headers (one pipe), or null.
+struct HeaderCopy {
+  int32_t *nodes, *edges;
+};
 int launch_gather_group(Server *s, Pipe *const *pp, int n, hipStream_t st, int seg, int seg_last, int lru_lists,
-                        bool same_stream = false, int hit_seg_first = -1);
-// whether the misses of these batches are gathered on the caller's stream
+                        bool same_stream = false, int hit_seg_first = -1, const HeaderCopy *headers = nullptr);
+// whether the misses of these batches are gathered on the caller's stream, and whether in the same pass as the hits
+// (no miss list is needed then)
 bool gather_in_line(const Server *s, Pipe *const *pp, int n, int seg_last);
+bool one_pass_gather(const Server *s);
 // the host-link gather of segments [seg, seg_last] released now, ahead of the batch's later hops (split_lookup)
 int launch_misses_early(Server *s, Pipe *const *pp, int n, hipStream_t st, int seg, int seg_last);
 int launch_lru_insert(Server *s, Pipe &p, hipStream_t st, int n_lists);

@@ -40,10 +40,15 @@ __device__ __forceinline__ uint32_t sample_draw(uint64_t seed, uint32_t hop, uin
 // lmi_batch_counters) and in the server's sticky fault word, which lives in pinned host
 // memory and is never cleared by a later batch, so the host sees it without reading the
 // device (lmi_server_status).
-__device__ __forceinline__ void raise_fault(DevState *st, int which) {
-  if (which == kFaultBadId) st->bad_id = 1; else st->scan_fault = 1;
-  if (st->fault) __hip_atomic_store(&st->fault[which], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+struct FaultTo {    // where a condition of this batch is recorded
+  int32_t serial;   // number of the batch
+  int32_t *sticky;  // the server's words, or null
+};
+__device__ __forceinline__ void raise_fault(DevState *st, int which, FaultTo to) {
+  if (which == kFaultBadId) st->bad_id = to.serial; else st->scan_fault = to.serial;
+  if (to.sticky) __hip_atomic_store(&to.sticky[which], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
+__device__ __forceinline__ FaultTo fault_to(const DevState *st) { return FaultTo{st->serial, st->fault}; }
 
 // -------------------------------------------------------------- hash table
 __device__ __forceinline__ uint32_t hash_id(int32_t key, int log2cap) {
@@ -105,6 +110,31 @@ __device__ __forceinline__ int32_t table_find(const HashSlot *slots, int log2cap
   }
 }
 
+// Bitmap + rank table: the slot of a cached node is the number of cached nodes
+// with a smaller id = rank at the start of its 64-id word + set bits below it.
+__device__ __forceinline__ int32_t rank_find(const uint4 *tab, int32_t id) {
+  const uint4 e = tab[id >> 6];
+  const uint64_t bits = (uint64_t)e.x | ((uint64_t)e.y << 32);
+  const int b = id & 63;
+  if (!((bits >> b) & 1ull)) return -1;
+  return (int32_t)e.z + __popcll(bits & ((1ull << b) - 1ull));
+}
+
+// The id -> slot table of the static / int8 caches.
+struct SlotTable {
+  int kind;  // LMI_TABLE_*, or -1: no cache
+  const HashSlot *slots;
+  int log2cap;
+  const int32_t *slot_of;
+  const uint4 *rank_tab;
+};
+__device__ __forceinline__ int32_t static_find(const SlotTable &t, int32_t id) {
+  if (t.kind < 0) return -1;
+  if (t.kind == LMI_TABLE_RANK) return rank_find(t.rank_tab, id);
+  if (t.kind == LMI_TABLE_DIRECT) return t.slot_of[id];
+  return table_find(t.slots, t.log2cap, id);
+}
+
 // Last step of a hop: the local id of every edge source is the value its table slot
 // holds once the hop's first occurrences have published theirs.  Strided over the
 // `n_threads` threads that take part, `tid` being this thread's place among them.
@@ -113,7 +143,7 @@ struct FillArgs {
   const HashSlot *slots;
   const int32_t *eslot;  // table slot per edge of hop `hop` (| kKnownRepeat)
   int32_t *agg_src_off;
-  int hop;               // -1: nothing to fill
+  int hop = -1;          // -1: nothing to fill
 };
 
 __device__ __forceinline__ void fill_local_ids(const FillArgs &f, int64_t tid, int64_t n_threads) {

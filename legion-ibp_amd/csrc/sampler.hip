@@ -30,25 +30,34 @@
 
 namespace lmi {
 
-struct HopArgs {
+struct HopShared {  // what the pipes of a launch have in common
   // graph
   const int64_t *indptr;
   const int32_t *indices;
   int64_t n_nodes;
-  int fanout, hop;
-  // pipe
+  int fanout, hop, hops;
+  int log2cap;      // dedup tables
+  int max_tiles;
+  int stage_seeds;  // hop 0 only: the seeds have not been staged by batch_generate_kernel yet
+  int begin;        // hop 0 only: no batch_begin_kernel ran, the parameters are in HopArgs::bp and the state is set up here
+  int tile_blocks;  // hop_count_sample: blocks [0, tile_blocks) own node tiles, the rest fill; hop_flag_scan: own edge
+                    // tiles, the rest look the seeds up
+  // cache lookup of the nodes the hop adds (hop_flag_scan)
+  int look_mode, miss_seg;
+  SlotTable cache;
+};
+struct HopArgs {
   DevState *st;
   int32_t *ids, *labels;
   int32_t *row_ptr;  // block CSR row pointers of this hop
-  int32_t *agg_src_ids, *agg_src_off, *agg_dst_off;
+  int32_t *agg_src_ids, *agg_dst_off;
   HashSlot *slots;
-  int log2cap;
   int32_t *eslot;   // table slot per edge of this hop (| kKnownRepeat)
   ScanChain chain_nodes, chain_edges;
-  int max_tiles;
-  int stage_seeds;  // hop 0 only: the seeds have not been staged by batch_generate_kernel yet
-  int tile_blocks;  // hop_count_sample: blocks [0, tile_blocks) own node tiles, the rest fill
   FillArgs fill;    // the previous hop's last step, carried by hop_count_sample (hop -1: none)
+  BatchParams bp;   // HopShared::begin
+  int32_t *cache_index;
+  int2 *miss_list;
 };
 
 // Several mini-batches (pipes) can share every launch of the sampling phase: block b
@@ -56,9 +65,11 @@ struct HopArgs {
 // in the same launch costs far less than a second launch.
 constexpr int kMaxGroup = LMI_MAX_GROUP;
 struct HopGroup {
+  HopShared c;
   HopArgs p[kMaxGroup];
   int n;
 };
+static_assert(sizeof(HopGroup) <= 4096, "a kernel's arguments");
 struct FillGroup {
   FillArgs p[kMaxGroup];
   int n;
@@ -75,8 +86,34 @@ struct BeginGroup {
 };
 
 // ------------------------------------------------------------ batch start
+// The state of a batch that starts: headers, counts, and the parameters where later kernels read them.
+// scan_fault and bad_id stay as they are: they hold a batch's number, not a flag, and other blocks of the same launch may
+// be raising them.
+__device__ __forceinline__ void state_begin(DevState *st, const BatchParams &bp, int hops) {
+#pragma unroll
+  for (int i = 0; i < 16; ++i) st->node_counter[i] = st->edge_counter[i] = 0;
+#pragma unroll
+  for (int i = 0; i <= LMI_MAX_HOPS; ++i) st->n_miss[i] = 0;
+  st->node_counter[8] = hops;
+  st->node_counter[9] = bp.n_seeds;
+  st->node_counter[1] = st->node_counter[3] = st->node_counter[5] = bp.n_seeds;
+  st->node_counter[7] = bp.n_seeds;
+  st->serial = bp.serial;
+  st->rng_lo = (uint32_t)bp.rng_seed;
+  st->rng_hi = (uint32_t)(bp.rng_seed >> 32);
+  st->lru_tick = bp.lru_tick;
+  st->n_seeds = bp.n_seeds;
+  st->table_tag = bp.table_tag;
+  st->table_mask = bp.table_mask;
+  st->seeds = bp.seeds;
+  st->labels_in = bp.labels;
+  st->fault = bp.fault;
+}
+
 // Clears the dedup table (key = -1, value = INT_MAX), resets the pipe state and
-// the scan chains, and stores the per-batch parameters where later kernels read them.
+// the scan chains, and stores the per-batch parameters where later kernels read them.  Most batches do without this
+// launch (2-9 us): their table needs no wiping, the last flag scan of the batch before left chain_nodes clean, every
+// hop's first kernel resets chain_edges, and the first hop's first kernel can set up the state (HopShared::begin).
 static __global__ __launch_bounds__(256) void batch_begin_kernel(BeginGroup g, int64_t n_slots, int hops,
                                                                  int max_tiles) {
   LMI_GRID_ROW(g.n);
@@ -95,21 +132,8 @@ static __global__ __launch_bounds__(256) void batch_begin_kernel(BeginGroup g, i
   scan_chain_reset(chain_nodes, max_tiles, tid, stride);
   scan_chain_reset(chain_edges, max_tiles, tid, stride);
   if (tid == 0) {
-    int32_t *w = reinterpret_cast<int32_t *>(st);
-    for (int i = 0; i < (int)(sizeof(DevState) / 4); ++i) w[i] = 0;
-    st->node_counter[8] = hops;
-    st->node_counter[9] = bp.n_seeds;
-    st->node_counter[1] = st->node_counter[3] = st->node_counter[5] = bp.n_seeds;
-    st->node_counter[7] = bp.n_seeds;
-    st->rng_lo = (uint32_t)bp.rng_seed;
-    st->rng_hi = (uint32_t)(bp.rng_seed >> 32);
-    st->lru_tick = bp.lru_tick;
-    st->n_seeds = bp.n_seeds;
-    st->table_tag = bp.table_tag;
-    st->table_mask = bp.table_mask;
-    st->seeds = bp.seeds;
-    st->labels_in = bp.labels;
-    st->fault = bp.fault;
+    state_begin(st, bp, hops);
+    st->scan_fault = st->bad_id = 0;
   }
 }
 
@@ -123,7 +147,7 @@ static __global__ __launch_bounds__(256) void batch_generate_kernel(int64_t n_no
   ids[i] = id;
   labels[i] = st->labels_in ? st->labels_in[i] : -1;
   if (id < 0 || id >= n_nodes) {
-    raise_fault(st, kFaultBadId);
+    raise_fault(st, kFaultBadId, fault_to(st));
     return;
   }
   table_insert_min(slots, log2cap, id, i, st->table_tag, st->table_mask);
@@ -142,12 +166,13 @@ static __global__ __launch_bounds__(kScanBlock) void hop_count_scan_kernel(HopGr
   __shared__ int lds[kScanBlock / kWave + 1];
   __shared__ int s_prefix;
   DevState *st = a.st;
-  const int n = st->node_counter[9 + a.hop];
+  const FaultTo fault = fault_to(st);
+  const int n = st->node_counter[9 + g.c.hop];
   const int n_tiles = (n + TILE - 1) / TILE;
   if (n_tiles == 0) {
     if (bx == 0 && threadIdx.x == 0) {
       a.row_ptr[0] = 0;
-      scan_epilogue(SCAN_EPI_HOP_EDGES, st, a.hop, 0);
+      scan_epilogue(SCAN_EPI_HOP_EDGES, st, g.c.hop, 0);
     }
     return;
   }
@@ -161,15 +186,15 @@ static __global__ __launch_bounds__(kScanBlock) void hop_count_scan_kernel(HopGr
       const int i = base + j;
       id[j] = -1;
       if (i < n) {
-        if (a.stage_seeds) {
+        if (g.c.stage_seeds) {
           id[j] = st->seeds[i];
           a.ids[i] = id[j];
           a.labels[i] = st->labels_in ? st->labels_in[i] : -1;
         } else {
           id[j] = a.ids[i];
         }
-        if (id[j] < 0 || id[j] >= a.n_nodes) {
-          if (a.stage_seeds) raise_fault(st, kFaultBadId);
+        if (id[j] < 0 || id[j] >= g.c.n_nodes) {
+          if (g.c.stage_seeds) raise_fault(st, kFaultBadId, fault);
           id[j] = -1;
         }
       }
@@ -180,25 +205,25 @@ static __global__ __launch_bounds__(kScanBlock) void hop_count_scan_kernel(HopGr
     for (int j = 0; j < ITEMS; ++j) {
       lo[j] = hi[j] = 0;
       if (id[j] >= 0) {
-        lo[j] = a.indptr[id[j]];
-        hi[j] = a.indptr[id[j] + 1];
+        lo[j] = g.c.indptr[id[j]];
+        hi[j] = g.c.indptr[id[j] + 1];
       }
     }
-    if (a.stage_seeds) {
+    if (g.c.stage_seeds) {
 #pragma unroll
       for (int j = 0; j < ITEMS; ++j)
-        if (id[j] >= 0) table_insert_min(a.slots, a.log2cap, id[j], base + j, st->table_tag, st->table_mask);
+        if (id[j] >= 0) table_insert_min(a.slots, g.c.log2cap, id[j], base + j, st->table_tag, st->table_mask);
     }
     int v[ITEMS], sum = 0;
 #pragma unroll
     for (int j = 0; j < ITEMS; ++j) {
       const int64_t deg = hi[j] - lo[j];
-      v[j] = (int)(deg < (int64_t)a.fanout ? deg : (int64_t)a.fanout);
+      v[j] = (int)(deg < (int64_t)g.c.fanout ? deg : (int64_t)g.c.fanout);
       sum += v[j];
     }
     int total;
     const int ex = block_exclusive_scan<kScanBlock>(sum, lds, total);
-    const int prefix = scan_tile_prefix(a.chain_nodes, tile, total, &s_prefix, st);
+    const int prefix = scan_tile_prefix(a.chain_nodes, tile, total, &s_prefix, st, fault);
     if (prefix == kScanFaultPrefix) return;  // the whole block: no offset, no writes
     int run = prefix + ex;
 #pragma unroll
@@ -208,7 +233,7 @@ static __global__ __launch_bounds__(kScanBlock) void hop_count_scan_kernel(HopGr
     }
     if (tile == n_tiles - 1 && threadIdx.x == 0) {
       a.row_ptr[n] = prefix + total;
-      scan_epilogue(SCAN_EPI_HOP_EDGES, st, a.hop, prefix + total);
+      scan_epilogue(SCAN_EPI_HOP_EDGES, st, g.c.hop, prefix + total);
     }
   }
 }
@@ -225,20 +250,20 @@ static __global__ __launch_bounds__(256) void hop_sample_kernel(HopGroup g) {
   const HopArgs &a = g.p[row];  // this block's pipe (mini-batch)
   const DevState *st = a.st;
   const int64_t flat = (int64_t)bx * blockDim.x + threadIdx.x;
-  scan_chain_reset(a.chain_edges, a.max_tiles, flat, (int64_t)gx * blockDim.x);
+  scan_chain_reset(a.chain_edges, g.c.max_tiles, flat, (int64_t)gx * blockDim.x);
   const uint64_t seed = (uint64_t)st->rng_lo | ((uint64_t)st->rng_hi << 32);
   const int32_t tag = st->table_tag, tag_mask = st->table_mask;
-  const int n_prev = st->node_counter[9 + a.hop];
-  const int eoff = st->edge_counter[12 + a.hop + 1];
-  const int fanout = a.fanout;
+  const int n_prev = st->node_counter[9 + g.c.hop];
+  const int eoff = st->edge_counter[12 + g.c.hop + 1];
+  const int fanout = g.c.fanout;
   const int lane = threadIdx.x & (G - 1);
   const int group = (int)(flat / G);
   const int n_groups = gx * blockDim.x / G;
   for (int i = group; i < n_prev; i += n_groups) {
     const int32_t v = a.ids[i];
-    if (v < 0 || v >= a.n_nodes) continue;
-    const int64_t beg = a.indptr[v];
-    const int64_t deg = a.indptr[v + 1] - beg;
+    if (v < 0 || v >= g.c.n_nodes) continue;
+    const int64_t beg = g.c.indptr[v];
+    const int64_t deg = g.c.indptr[v + 1] - beg;
     const int base = a.row_ptr[i];
     int64_t pick = lane;
     int count;
@@ -248,7 +273,7 @@ static __global__ __launch_bounds__(256) void hop_sample_kernel(HopGroup g) {
       count = fanout;
       const uint32_t j = (uint32_t)(deg - fanout) + (uint32_t)lane;
       uint32_t t = 0xFFFFFFFFu;
-      if (lane < fanout) t = __umulhi(sample_draw(seed, (uint32_t)a.hop, (uint32_t)v, (uint32_t)lane), j + 1u);
+      if (lane < fanout) t = __umulhi(sample_draw(seed, (uint32_t)g.c.hop, (uint32_t)v, (uint32_t)lane), j + 1u);
       bool dup = false;
       for (int q = 0; q + 1 < fanout; ++q) {
         const uint32_t mine = dup ? j : t;
@@ -258,11 +283,11 @@ static __global__ __launch_bounds__(256) void hop_sample_kernel(HopGroup g) {
       pick = dup ? j : t;
     }
     if (lane < count) {
-      const int32_t nbr = a.indices[beg + pick];
+      const int32_t nbr = g.c.indices[beg + pick];
       const int e = base + lane;
       a.agg_src_ids[eoff + e] = nbr;
       a.agg_dst_off[eoff + e] = i;
-      a.eslot[e] = (int)table_insert_min(a.slots, a.log2cap, nbr, n_prev + e, tag, tag_mask);
+      a.eslot[e] = (int)table_insert_min(a.slots, g.c.log2cap, nbr, n_prev + e, tag, tag_mask);
     }
   }
 }
@@ -281,11 +306,11 @@ static __global__ __launch_bounds__(256) void hop_sample_lds_kernel(HopGroup g) 
   __shared__ int32_t lds_slot[TAB];
   const DevState *st = a.st;
   const int64_t flat = (int64_t)bx * blockDim.x + threadIdx.x;
-  scan_chain_reset(a.chain_edges, a.max_tiles, flat, (int64_t)gx * blockDim.x);
+  scan_chain_reset(a.chain_edges, g.c.max_tiles, flat, (int64_t)gx * blockDim.x);
   const uint64_t seed = (uint64_t)st->rng_lo | ((uint64_t)st->rng_hi << 32);
-  const int n_prev = st->node_counter[9 + a.hop];
-  const int eoff = st->edge_counter[12 + a.hop + 1];
-  const int fanout = a.fanout;
+  const int n_prev = st->node_counter[9 + g.c.hop];
+  const int eoff = st->edge_counter[12 + g.c.hop + 1];
+  const int fanout = g.c.fanout;
   const int lane = threadIdx.x & (G - 1);
   const int group = (int)(flat / G);
   const int n_groups = gx * blockDim.x / G;
@@ -303,9 +328,9 @@ static __global__ __launch_bounds__(256) void hop_sample_lds_kernel(HopGroup g) 
     int e = 0, h = 0;
     if (i < n_prev) {
       const int32_t v = a.ids[i];
-      if (v >= 0 && v < a.n_nodes) {
-        const int64_t beg = a.indptr[v];
-        const int64_t deg = a.indptr[v + 1] - beg;
+      if (v >= 0 && v < g.c.n_nodes) {
+        const int64_t beg = g.c.indptr[v];
+        const int64_t deg = g.c.indptr[v + 1] - beg;
         const int base = a.row_ptr[i];
         int64_t pick = lane;
         int count;
@@ -315,7 +340,7 @@ static __global__ __launch_bounds__(256) void hop_sample_lds_kernel(HopGroup g) 
           count = fanout;
           const uint32_t j = (uint32_t)(deg - fanout) + (uint32_t)lane;
           uint32_t t = 0xFFFFFFFFu;
-          if (lane < fanout) t = __umulhi(sample_draw(seed, (uint32_t)a.hop, (uint32_t)v, (uint32_t)lane), j + 1u);
+          if (lane < fanout) t = __umulhi(sample_draw(seed, (uint32_t)g.c.hop, (uint32_t)v, (uint32_t)lane), j + 1u);
           bool dup = false;
           for (int q = 0; q + 1 < fanout; ++q) {
             const uint32_t mine = dup ? j : t;
@@ -326,7 +351,7 @@ static __global__ __launch_bounds__(256) void hop_sample_lds_kernel(HopGroup g) 
         }
         if (lane < count) {
           active = true;
-          nbr = a.indices[beg + pick];
+          nbr = g.c.indices[beg + pick];
           e = base + lane;
           a.agg_src_ids[eoff + e] = nbr;
           a.agg_dst_off[eoff + e] = i;
@@ -342,7 +367,7 @@ static __global__ __launch_bounds__(256) void hop_sample_lds_kernel(HopGroup g) 
     }
     __syncthreads();
     if (active && lds_min[h] == e)
-      lds_slot[h] = (int)table_insert_min(a.slots, a.log2cap, nbr, n_prev + e, st->table_tag, st->table_mask);
+      lds_slot[h] = (int)table_insert_min(a.slots, g.c.log2cap, nbr, n_prev + e, st->table_tag, st->table_mask);
     __syncthreads();
     // an edge that lost inside the block is a repeat whatever the table said to the winner
     if (active) a.eslot[e] = (lds_min[h] == e) ? lds_slot[h] : (lds_slot[h] | (int32_t)kKnownRepeat);
@@ -367,55 +392,64 @@ static __global__ __launch_bounds__(256) void hop_count_sample_kernel(HopGroup g
   __shared__ int s_prefix;
   DevState *st = a.st;
   const int64_t flat = (int64_t)bx * blockDim.x + threadIdx.x;
-  scan_chain_reset(a.chain_edges, a.max_tiles, flat, (int64_t)gx * blockDim.x);
-  if (bx >= a.tile_blocks) {  // extra blocks: the previous hop's local ids
-    fill_local_ids(a.fill, (int64_t)(bx - a.tile_blocks) * blockDim.x + threadIdx.x,
-                   (int64_t)(gx - a.tile_blocks) * blockDim.x);
+  scan_chain_reset(a.chain_edges, g.c.max_tiles, flat, (int64_t)gx * blockDim.x);
+  if (bx >= g.c.tile_blocks) {  // extra blocks: the previous hop's local ids
+    fill_local_ids(a.fill, (int64_t)(bx - g.c.tile_blocks) * blockDim.x + threadIdx.x,
+                   (int64_t)(gx - g.c.tile_blocks) * blockDim.x);
     return;
   }
-  const int n_prev = st->node_counter[9 + a.hop];
+  // a batch that starts here takes its parameters from the arguments (nobody in this launch may read the state that one
+  // of its threads sets up), any other from the state
+  const bool begin = g.c.begin != 0;
+  const BatchParams &bp = a.bp;
+  const FaultTo fault = begin ? FaultTo{bp.serial, bp.fault} : fault_to(st);
+  const int n_prev = begin ? bp.n_seeds : st->node_counter[9 + g.c.hop];
   const int n_tiles = (n_prev + NPB - 1) / NPB;
   if (n_tiles == 0) {
     if (bx == 0 && threadIdx.x == 0) {
+      if (begin) state_begin(st, bp, g.c.hops);
       a.row_ptr[0] = 0;
-      scan_epilogue(SCAN_EPI_HOP_EDGES, st, a.hop, 0);
+      scan_epilogue(SCAN_EPI_HOP_EDGES, st, g.c.hop, 0);
     }
     return;
   }
   const int tile = bx;
   if (tile >= n_tiles) return;
-  // ---- counts, tile scan (wavefront 0)
   const int t = threadIdx.x;
+  if (begin && tile == n_tiles - 1 && t == 0) state_begin(st, bp, g.c.hops);  // the thread that updates the headers below
+  const int32_t tag = begin ? bp.table_tag : st->table_tag, tag_mask = begin ? bp.table_mask : st->table_mask;
+  // ---- counts, tile scan (wavefront 0)
   const int my = tile * NPB + t;
   int cnt = 0, ex = 0, total = 0;
   int32_t id = -1;
   int64_t lo = 0, hi = 0;
   if (t < kWave) {
     if (t < NPB && my < n_prev) {
-      if (a.stage_seeds) {
-        id = st->seeds[my];
+      if (g.c.stage_seeds) {
+        const int32_t *labels = begin ? bp.labels : st->labels_in;
+        id = (begin ? bp.seeds : st->seeds)[my];
         a.ids[my] = id;
-        a.labels[my] = st->labels_in ? st->labels_in[my] : -1;
+        a.labels[my] = labels ? labels[my] : -1;
       } else {
         id = a.ids[my];
       }
-      if (id < 0 || id >= a.n_nodes) {
-        if (a.stage_seeds) raise_fault(st, kFaultBadId);
+      if (id < 0 || id >= g.c.n_nodes) {
+        if (g.c.stage_seeds) raise_fault(st, kFaultBadId, fault);
         id = -1;
       }
     }
     if (id >= 0) {
-      lo = a.indptr[id];
-      hi = a.indptr[id + 1];
-      if (a.stage_seeds) table_insert_min(a.slots, a.log2cap, id, my, st->table_tag, st->table_mask);
+      lo = g.c.indptr[id];
+      hi = g.c.indptr[id + 1];
+      if (g.c.stage_seeds) table_insert_min(a.slots, g.c.log2cap, id, my, tag, tag_mask);
     }
     const int64_t deg = hi - lo;
-    cnt = (int)(deg < (int64_t)a.fanout ? deg : (int64_t)a.fanout);
+    cnt = (int)(deg < (int64_t)g.c.fanout ? deg : (int64_t)g.c.fanout);
     const int inc = wave_inclusive_scan(cnt);
     ex = inc - cnt;
     total = __shfl(inc, kWave - 1, kWave);
   }
-  const int prefix = scan_tile_prefix(a.chain_nodes, tile, total, &s_prefix, st);
+  const int prefix = scan_tile_prefix(a.chain_nodes, tile, total, &s_prefix, st, fault);
   if (prefix == kScanFaultPrefix) return;  // the whole block: no offset, no writes
   if (t < NPB) {
     s_id[t] = id;
@@ -426,14 +460,13 @@ static __global__ __launch_bounds__(256) void hop_count_sample_kernel(HopGroup g
   }
   if (tile == n_tiles - 1 && t == 0) {
     a.row_ptr[n_prev] = prefix + total;
-    scan_epilogue(SCAN_EPI_HOP_EDGES, st, a.hop, prefix + total);
+    scan_epilogue(SCAN_EPI_HOP_EDGES, st, g.c.hop, prefix + total);
   }
   __syncthreads();
   // ---- sampling: the edge offset of the hop is fixed by the hops before it
-  const uint64_t seed = (uint64_t)st->rng_lo | ((uint64_t)st->rng_hi << 32);
-  const int32_t tag = st->table_tag, tag_mask = st->table_mask;
-  const int eoff = (a.hop == 0) ? 0 : st->edge_counter[12 + a.hop] + st->edge_counter[9 + a.hop];
-  const int fanout = a.fanout;
+  const uint64_t seed = begin ? bp.rng_seed : (uint64_t)st->rng_lo | ((uint64_t)st->rng_hi << 32);
+  const int eoff = (g.c.hop == 0) ? 0 : st->edge_counter[12 + g.c.hop] + st->edge_counter[9 + g.c.hop];
+  const int fanout = g.c.fanout;
   const int lane = t & (G - 1);
   for (int q = t / G; q < NPB; q += 256 / G) {
     const int i = tile * NPB + q;
@@ -450,7 +483,7 @@ static __global__ __launch_bounds__(256) void hop_count_sample_kernel(HopGroup g
       count = fanout;
       const uint32_t j = (uint32_t)(deg - fanout) + (uint32_t)lane;
       uint32_t d = 0xFFFFFFFFu;
-      if (lane < fanout) d = __umulhi(sample_draw(seed, (uint32_t)a.hop, (uint32_t)v, (uint32_t)lane), j + 1u);
+      if (lane < fanout) d = __umulhi(sample_draw(seed, (uint32_t)g.c.hop, (uint32_t)v, (uint32_t)lane), j + 1u);
       bool dup = false;
       for (int r = 0; r + 1 < fanout; ++r) {
         const uint32_t mine = dup ? j : d;
@@ -460,11 +493,11 @@ static __global__ __launch_bounds__(256) void hop_count_sample_kernel(HopGroup g
       pick = dup ? j : d;
     }
     if (lane < count) {
-      const int32_t nbr = a.indices[beg + pick];
+      const int32_t nbr = g.c.indices[beg + pick];
       const int e = base + lane;
       a.agg_src_ids[eoff + e] = nbr;
       a.agg_dst_off[eoff + e] = i;
-      a.eslot[e] = (int)table_insert_min(a.slots, a.log2cap, nbr, n_prev + e, tag, tag_mask);
+      a.eslot[e] = (int)table_insert_min(a.slots, g.c.log2cap, nbr, n_prev + e, tag, tag_mask);
     }
   }
 }
@@ -484,17 +517,27 @@ static __global__ __launch_bounds__(kScanBlock) void hop_flag_scan_kernel(HopGro
   __shared__ int s_prefix;
   DevState *st = a.st;
   const int64_t flat = (int64_t)bx * blockDim.x + threadIdx.x;
-  scan_chain_reset(a.chain_nodes, a.max_tiles, flat, (int64_t)gx * blockDim.x);  // for the next hop
-  const int n_prev = st->node_counter[9 + a.hop];
-  const int n = st->edge_counter[9 + a.hop + 1];
-  const int eoff = st->edge_counter[12 + a.hop + 1];
-  const int n_tiles = (n + TILE - 1) / TILE;
-  if (n_tiles == 0) {
-    if (bx == 0 && threadIdx.x == 0) scan_epilogue(SCAN_EPI_HOP_NODES, st, a.hop, 0);
-    return;
-  }
-  const int tile = bx;
-  if (tile < n_tiles) {
+  scan_chain_reset(a.chain_nodes, g.c.max_tiles, flat, (int64_t)gx * blockDim.x);  // for the next hop
+  int32_t local[ITEMS], node[ITEMS], slot_of[ITEMS];
+  bool look[ITEMS];  // a row to look up
+#pragma unroll
+  for (int j = 0; j < ITEMS; ++j) local[j] = node[j] = -1, look[j] = false;
+  if (bx >= g.c.tile_blocks) {  // extra blocks: the seeds' lookup (ids[] holds them since the hop's first kernel)
+    const int i = (bx - g.c.tile_blocks) * kScanBlock + (int)threadIdx.x;
+    if (i < st->n_seeds) {
+      node[0] = a.ids[i];
+      local[0] = i;
+      look[0] = true;
+    }
+  } else {
+    const FaultTo fault = fault_to(st);
+    const int n_prev = st->node_counter[9 + g.c.hop];
+    const int n = st->edge_counter[9 + g.c.hop + 1];
+    const int eoff = st->edge_counter[12 + g.c.hop + 1];
+    const int n_tiles = (n + TILE - 1) / TILE;
+    if (n_tiles == 0 && bx == 0 && threadIdx.x == 0) scan_epilogue(SCAN_EPI_HOP_NODES, st, g.c.hop, 0);
+    const int tile = bx;
+    if (tile >= n_tiles) return;
     const int base = tile * TILE + threadIdx.x * ITEMS;
     int v[ITEMS], slot[ITEMS], sum = 0;
 #pragma unroll
@@ -512,19 +555,51 @@ static __global__ __launch_bounds__(kScanBlock) void hop_flag_scan_kernel(HopGro
     }
     int total;
     const int ex = block_exclusive_scan<kScanBlock>(sum, lds, total);
-    const int prefix = scan_tile_prefix(a.chain_edges, tile, total, &s_prefix, st);
+    const int prefix = scan_tile_prefix(a.chain_edges, tile, total, &s_prefix, st, fault);
     if (prefix == kScanFaultPrefix) return;  // the whole block: no ranks, no writes
-    int run = prefix + ex;
+    int run = n_prev + prefix + ex;
 #pragma unroll
     for (int j = 0; j < ITEMS; ++j) {
-      if (v[j]) {
-        const int local = n_prev + run;
-        a.ids[local] = a.agg_src_ids[eoff + base + j];
-        a.slots[slot[j]].val = local;
-      }
+      look[j] = v[j] != 0;
+      local[j] = run;
+      node[j] = look[j] ? a.agg_src_ids[eoff + base + j] : -1;
       run += v[j];
     }
-    if (tile == n_tiles - 1 && threadIdx.x == 0) scan_epilogue(SCAN_EPI_HOP_NODES, st, a.hop, prefix + total);
+#pragma unroll
+    for (int j = 0; j < ITEMS; ++j)
+      if (look[j]) {
+        a.ids[local[j]] = node[j];
+        a.slots[slot[j]].val = local[j];
+      }
+    if (tile == n_tiles - 1 && threadIdx.x == 0) scan_epilogue(SCAN_EPI_HOP_NODES, st, g.c.hop, prefix + total);
+  }
+  // ---- cache lookup of the rows the block holds.  In this kernel because the id is in a register here and the random
+  // read of the cache's table hides behind the other tiles' look-back: as a kernel of its own the lookup was a launch
+  // and a pass over the ids: 30 us, its part of the last fill included, for a group of four papers100M-shaped
+  // batches, whose flag scans did not get slower (31 + 12 us).
+  if (g.c.look_mode == LOOK_NOT) return;
+  int misses = 0;
+#pragma unroll
+  for (int j = 0; j < ITEMS; ++j) {
+    slot_of[j] = -1;
+    if (look[j] && node[j] >= 0 && node[j] < g.c.n_nodes) slot_of[j] = static_find(g.c.cache, node[j]);
+  }
+#pragma unroll
+  for (int j = 0; j < ITEMS; ++j) {
+    if (look[j]) a.cache_index[local[j]] = slot_of[j];
+    look[j] = look[j] && slot_of[j] < 0 && node[j] >= 0 && node[j] < g.c.n_nodes;  // from here on: a miss
+    misses += look[j] ? 1 : 0;
+  }
+  if (g.c.look_mode == LOOK_LIST) {  // one atomic per block: one per wavefront on the same counter costs 24 ns each
+    int total;
+    int at = block_exclusive_scan<kScanBlock>(misses, lds, total);
+    if (total == 0) return;
+    if (threadIdx.x == 0) s_prefix = atomicAdd(&st->n_miss[g.c.miss_seg], total);
+    __syncthreads();
+    at += s_prefix;
+#pragma unroll
+    for (int j = 0; j < ITEMS; ++j)
+      if (look[j]) a.miss_list[at++] = make_int2(local[j], node[j]);
   }
 }
 
@@ -536,6 +611,11 @@ static __global__ __launch_bounds__(256) void hop_fill_kernel(FillGroup g) {
 }
 
 // ---------------------------------------------------------------- launchers
+SlotTable slot_table(const Server *s) {
+  return SlotTable{s->cache_kind == LMI_CACHE_NONE ? -1 : s->table_kind, s->id_table.slots, s->id_table.log2cap, s->slot_of,
+                   s->rank_tab};
+}
+
 static ScanChain chain_of(const Pipe &p, int which) { return ScanChain{p.chain_status[which]}; }
 
 static int begin_grid(const Pipe &p) {
@@ -571,6 +651,7 @@ int launch_batch_generate(Server *s, Pipe *const *pp, const BatchParams *bps, in
   for (int k = 0; k < n; ++k) {
     pp[k]->n_seeds = bps[k].n_seeds;
     pp[k]->hops_done = 0;
+    pp[k]->fill_pending = -1;
   }
   return LMI_OK;
 }
@@ -598,35 +679,50 @@ int graph_update_begin(Server *s, Pipe &p, const BatchParams &bp) {
 
 // One hop for each of the n pipes, all in the same launches (the pipes are in step: same hop,
 // same pending fill).
-int launch_hop(Server *s, Pipe *const *pp, int n, hipStream_t st, int hop, bool stage_seeds, bool defer_fill) {
+bool hop_sets_up(const Server *s) { return s->fuse_count && !s->lds_dedup; }
+
+int launch_hop(Server *s, Pipe *const *pp, int n, hipStream_t st, int hop, bool stage_seeds, bool defer_fill,
+               const BatchParams *begin, HopLookup look) {
   const int f = s->cfg.fanout[hop];
   const int64_t n_max = s->node_cap[hop], e_max = s->edge_cap[hop];
   Pipe &p0 = *pp[0];
   HopGroup g{};
   g.n = n;
+  g.c.indptr = s->indptr;
+  g.c.indices = s->indices;
+  g.c.n_nodes = s->n_nodes;
+  g.c.fanout = f;
+  g.c.hop = hop;
+  g.c.hops = s->cfg.hops;
+  g.c.log2cap = p0.dedup.log2cap;
+  g.c.max_tiles = p0.max_tiles;
+  g.c.stage_seeds = (hop == 0 && stage_seeds) ? 1 : 0;
+  g.c.begin = begin ? 1 : 0;
+  g.c.look_mode = look.mode;
+  g.c.miss_seg = look.miss_seg;
+  g.c.cache = slot_table(s);
   for (int k = 0; k < n; ++k) {
     Pipe &p = *pp[k];
     HopArgs &a = g.p[k];
-    a.indptr = s->indptr;
-    a.indices = s->indices;
-    a.n_nodes = s->n_nodes;
-    a.fanout = f;
-    a.hop = hop;
     a.st = p.st;
     a.ids = p.ids;
     a.labels = p.labels;
     a.row_ptr = p.blk_indptr[hop];
     a.agg_src_ids = p.agg_src_ids;
-    a.agg_src_off = p.agg_src_off;
     a.agg_dst_off = p.agg_dst_off;
     a.slots = p.dedup.slots;
-    a.log2cap = p.dedup.log2cap;
     a.eslot = p.eslot[hop & 1];
     a.chain_nodes = chain_of(p, 0);
     a.chain_edges = chain_of(p, 1);
-    a.max_tiles = p.max_tiles;
-    a.stage_seeds = (hop == 0 && stage_seeds) ? 1 : 0;
     a.fill.hop = -1;
+    a.cache_index = p.cache_index;
+    a.miss_list = p.miss_list + miss_list_base(s, look.miss_seg);
+    if (begin) {
+      a.bp = begin[k];
+      p.n_seeds = begin[k].n_seeds;
+      p.hops_done = 0;
+      p.fill_pending = -1;
+    }
   }
   int G = 4;
   while (G < f) G <<= 1;
@@ -639,8 +735,8 @@ int launch_hop(Server *s, Pipe *const *pp, int n, hipStream_t st, int hop, bool 
     const int tile_blocks = (int)ceil_div(std::max<int64_t>(n_max, 1), npb);
     int grid = tile_blocks;
     if (p0.fill_pending >= 0) grid += fill_blocks(s->edge_cap[p0.fill_pending], 256);
+    g.c.tile_blocks = tile_blocks;
     for (int k = 0; k < n; ++k) {
-      g.p[k].tile_blocks = tile_blocks;
       if (pp[k]->fill_pending >= 0) g.p[k].fill = fill_args(*pp[k], pp[k]->fill_pending);
       pp[k]->fill_pending = -1;
     }
@@ -690,12 +786,16 @@ int launch_hop(Server *s, Pipe *const *pp, int n, hipStream_t st, int hop, bool 
     }
   }
   const int64_t em = std::max<int64_t>(e_max, 1);
-  if (em <= 1024 * 1024)
-    hipLaunchKernelGGL(hop_flag_scan_kernel<2>, dim3(((int)ceil_div(em, kScanBlock * 2)) * n), dim3(kScanBlock), 0, st, g);
-  else if (em <= 2560 * 1024)
-    hipLaunchKernelGGL(hop_flag_scan_kernel<4>, dim3(((int)ceil_div(em, kScanBlock * 4)) * n), dim3(kScanBlock), 0, st, g);
-  else
-    hipLaunchKernelGGL(hop_flag_scan_kernel<8>, dim3(((int)ceil_div(em, kScanBlock * 8)) * n), dim3(kScanBlock), 0, st, g);
+  const int seed_blocks = (hop == 0 && look.mode != LOOK_NOT) ? (int)ceil_div(s->cfg.batch_size, kScanBlock) : 0;
+#define LMI_FLAG(I_)                                                                                                 \
+  {                                                                                                                  \
+    g.c.tile_blocks = (int)ceil_div(em, kScanBlock * I_);                                                            \
+    hipLaunchKernelGGL(hop_flag_scan_kernel<I_>, dim3((g.c.tile_blocks + seed_blocks) * n), dim3(kScanBlock), 0, st, g); \
+  }
+  if (em <= 1024 * 1024) LMI_FLAG(2)
+  else if (em <= 2560 * 1024) LMI_FLAG(4)
+  else LMI_FLAG(8)
+#undef LMI_FLAG
   LMI_HIP(hipGetLastError());
   for (int k = 0; k < n; ++k) {
     pp[k]->fill_pending = hop;

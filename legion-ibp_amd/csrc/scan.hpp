@@ -147,7 +147,7 @@ __device__ __forceinline__ void scan_publish(ScanChain c, int tile, unsigned lon
 // Wavefront 0 looks back 64 tiles per step (lookback_window).  lds_prefix is one shared int.
 // Contains __syncthreads.
 __device__ __forceinline__ int scan_tile_prefix(ScanChain c, int tile, int aggregate, int *lds_prefix,
-                                                DevState *st) {
+                                                DevState *st, FaultTo fault) {
   if (threadIdx.x < kWave) {
     const int lane = threadIdx.x;
     int prefix = 0;
@@ -159,7 +159,7 @@ __device__ __forceinline__ int scan_tile_prefix(ScanChain c, int tile, int aggre
       int spins = 0;
       // after a first fault every later tile gives up almost at once, so a broken chain drains
       // in milliseconds
-      const bool broken = st->scan_fault != 0;
+      const bool broken = st->scan_fault == fault.serial;
       const long long t0 = wall_clock64();
       while (true) {
         const int j = base - lane;
@@ -171,7 +171,7 @@ __device__ __forceinline__ int scan_tile_prefix(ScanChain c, int tile, int aggre
           ++spins;
           const bool out_of_time = broken ? spins >= 64 : ((spins & 1023) == 0 && wall_clock64() - t0 > kScanWaitTicks);
           if (!out_of_time) continue;
-          if (lane == 0) raise_fault(st, kFaultScan);  // never expected; bounded so that the grid always drains
+          if (lane == 0) raise_fault(st, kFaultScan, fault);  // never expected; bounded so that the grid always drains
           prefix = kScanFaultPrefix;
           break;
         }

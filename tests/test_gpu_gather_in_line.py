@@ -3,7 +3,8 @@
 import numpy as np
 import pytest
 
-from test_gpu_parity import assert_batch_equal, make_features, random_graph
+from conftest import random_graph
+from test_gpu_parity import assert_batch_equal, make_features
 
 pytestmark = pytest.mark.gpu
 
