@@ -17,8 +17,10 @@ __device__ __forceinline__ Philox4 philox4x32_10(uint32_t c0, uint32_t c1, uint3
                                                  uint32_t k0, uint32_t k1) {
 #pragma unroll
   for (int r = 0; r < 10; ++r) {
-    const uint32_t hi0 = __umulhi(0xD2511F53u, c0), lo0 = 0xD2511F53u * c0;
-    const uint32_t hi1 = __umulhi(0xCD9E8D57u, c2), lo1 = 0xCD9E8D57u * c2;
+    // one 32 x 32 -> 64 product each (v_mad_u64_u32) instead of a high and a low one
+    const uint64_t p0 = (uint64_t)0xD2511F53u * c0, p1 = (uint64_t)0xCD9E8D57u * c2;
+    const uint32_t hi0 = (uint32_t)(p0 >> 32), lo0 = (uint32_t)p0;
+    const uint32_t hi1 = (uint32_t)(p1 >> 32), lo1 = (uint32_t)p1;
     c0 = hi1 ^ c1 ^ k0;
     c1 = lo1;
     c2 = hi0 ^ c3 ^ k1;
@@ -33,6 +35,57 @@ __device__ __forceinline__ Philox4 philox4x32_10(uint32_t c0, uint32_t c1, uint3
 __device__ __forceinline__ uint32_t sample_draw(uint64_t seed, uint32_t hop, uint32_t node,
                                                 uint32_t slot) {
   return philox4x32_10(node, hop, slot, 0u, (uint32_t)seed, (uint32_t)(seed >> 32)).x;
+}
+
+// What lane R of each lane group of G lanes holds, in every lane of the group, R a constant (G <= 16) or the same in the
+// whole wavefront: moves between registers, where a shuffle goes through the LDS unit and its latency.
+template <int G, int R>
+__device__ __forceinline__ uint32_t group_lane(uint32_t v) {
+  static_assert(G == 4 || G == 8 || G == 16, "lane groups inside a row of 16 lanes");
+  if constexpr (G == 4) {
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, R * 0x55, 0xf, 0xf, true);  // quad_perm R,R,R,R
+  } else {
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x150 + R, 0xf, 0xf, true);  // row_newbcast
+    if constexpr (G == 16) return lo;
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x150 + ((R + 8) & 15), 0xf, 0xf, true);
+    return (threadIdx.x & 8) ? hi : lo;
+  }
+}
+template <int G>
+__device__ __forceinline__ uint32_t group_lane(uint32_t v, int r) {
+  static_assert(G == 32 || G == 64, "lane groups of several rows");
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)v, r);
+  if constexpr (G == 64) return lo;
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)v, r + 32);
+  return (threadIdx.x & 32) ? hi : lo;
+}
+
+// Floyd's rule within a lane group: lane s drew t out of [0, j], j = deg - fanout + s; its pick is t unless an earlier
+// lane picked that already, and j then.  All lanes of the group call; lanes from `fanout` on hold t = 0xFFFFFFFF.
+// One step per lane, each waiting for the one before: through shuffles a step took the LDS unit's latency (24 of them
+// for a fanout of 25).
+template <int G, int R>
+__device__ __forceinline__ void floyd_step(uint32_t t, uint32_t j, int lane, int fanout, bool &dup) {
+  if constexpr (R + 1 < G) {
+    if (R + 1 < fanout) {
+      const uint32_t p = group_lane<G, R>(dup ? j : t);
+      dup = dup || (lane > R && t == p);
+      floyd_step<G, R + 1>(t, j, lane, fanout, dup);
+    }
+  }
+}
+template <int G>
+__device__ __forceinline__ uint32_t floyd_pick(uint32_t t, uint32_t j, int lane, int fanout) {
+  bool dup = false;
+  if constexpr (G <= 16) {
+    floyd_step<G, 0>(t, j, lane, fanout, dup);
+  } else {
+    for (int r = 0; r + 1 < fanout; ++r) {
+      const uint32_t p = group_lane<G>(dup ? j : t, r);
+      dup = dup || (lane > r && t == p);
+    }
+  }
+  return dup ? j : t;
 }
 
 // ------------------------------------------------------------------ faults

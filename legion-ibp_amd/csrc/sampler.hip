@@ -86,30 +86,6 @@ struct BeginGroup {
 };
 
 // ------------------------------------------------------------ batch start
-// The state of a batch that starts: headers, counts, and the parameters where later kernels read them.
-// scan_fault and bad_id stay as they are: they hold a batch's number, not a flag, and other blocks of the same launch may
-// be raising them.
-__device__ __forceinline__ void state_begin(DevState *st, const BatchParams &bp, int hops) {
-#pragma unroll
-  for (int i = 0; i < 16; ++i) st->node_counter[i] = st->edge_counter[i] = 0;
-#pragma unroll
-  for (int i = 0; i <= LMI_MAX_HOPS; ++i) st->n_miss[i] = 0;
-  st->node_counter[8] = hops;
-  st->node_counter[9] = bp.n_seeds;
-  st->node_counter[1] = st->node_counter[3] = st->node_counter[5] = bp.n_seeds;
-  st->node_counter[7] = bp.n_seeds;
-  st->serial = bp.serial;
-  st->rng_lo = (uint32_t)bp.rng_seed;
-  st->rng_hi = (uint32_t)(bp.rng_seed >> 32);
-  st->lru_tick = bp.lru_tick;
-  st->n_seeds = bp.n_seeds;
-  st->table_tag = bp.table_tag;
-  st->table_mask = bp.table_mask;
-  st->seeds = bp.seeds;
-  st->labels_in = bp.labels;
-  st->fault = bp.fault;
-}
-
 // Clears the dedup table (key = -1, value = INT_MAX), resets the pipe state and
 // the scan chains, and stores the per-batch parameters where later kernels read them.  Most batches do without this
 // launch (2-9 us): their table needs no wiping, the last flag scan of the batch before left chain_nodes clean, every
@@ -274,13 +250,7 @@ static __global__ __launch_bounds__(256) void hop_sample_kernel(HopGroup g) {
       const uint32_t j = (uint32_t)(deg - fanout) + (uint32_t)lane;
       uint32_t t = 0xFFFFFFFFu;
       if (lane < fanout) t = __umulhi(sample_draw(seed, (uint32_t)g.c.hop, (uint32_t)v, (uint32_t)lane), j + 1u);
-      bool dup = false;
-      for (int q = 0; q + 1 < fanout; ++q) {
-        const uint32_t mine = dup ? j : t;
-        const uint32_t p = __shfl(mine, q, G);
-        if (lane > q && t == p) dup = true;
-      }
-      pick = dup ? j : t;
+      pick = floyd_pick<G>(t, j, lane, fanout);
     }
     if (lane < count) {
       const int32_t nbr = g.c.indices[beg + pick];
@@ -341,13 +311,7 @@ static __global__ __launch_bounds__(256) void hop_sample_lds_kernel(HopGroup g) 
           const uint32_t j = (uint32_t)(deg - fanout) + (uint32_t)lane;
           uint32_t t = 0xFFFFFFFFu;
           if (lane < fanout) t = __umulhi(sample_draw(seed, (uint32_t)g.c.hop, (uint32_t)v, (uint32_t)lane), j + 1u);
-          bool dup = false;
-          for (int q = 0; q + 1 < fanout; ++q) {
-            const uint32_t mine = dup ? j : t;
-            const uint32_t p = __shfl(mine, q, G);
-            if (lane > q && t == p) dup = true;
-          }
-          pick = dup ? j : t;
+          pick = floyd_pick<G>(t, j, lane, fanout);
         }
         if (lane < count) {
           active = true;
@@ -484,13 +448,7 @@ static __global__ __launch_bounds__(256) void hop_count_sample_kernel(HopGroup g
       const uint32_t j = (uint32_t)(deg - fanout) + (uint32_t)lane;
       uint32_t d = 0xFFFFFFFFu;
       if (lane < fanout) d = __umulhi(sample_draw(seed, (uint32_t)g.c.hop, (uint32_t)v, (uint32_t)lane), j + 1u);
-      bool dup = false;
-      for (int r = 0; r + 1 < fanout; ++r) {
-        const uint32_t mine = dup ? j : d;
-        const uint32_t p = __shfl(mine, r, G);
-        if (lane > r && d == p) dup = true;
-      }
-      pick = dup ? j : d;
+      pick = floyd_pick<G>(d, j, lane, fanout);
     }
     if (lane < count) {
       const int32_t nbr = g.c.indices[beg + pick];

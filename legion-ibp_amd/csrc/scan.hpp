@@ -38,6 +38,30 @@ __device__ __forceinline__ void tile_reduce_store(int v, int32_t *tile_sums, int
   __syncthreads();
 }
 
+// The state of a batch that starts: headers, counts, and the parameters where later kernels read them.
+// scan_fault and bad_id stay as they are: they hold a batch's number, not a flag, and other blocks of the same launch may
+// be raising them.
+__device__ __forceinline__ void state_begin(DevState *st, const BatchParams &bp, int hops) {
+#pragma unroll
+  for (int i = 0; i < 16; ++i) st->node_counter[i] = st->edge_counter[i] = 0;
+#pragma unroll
+  for (int i = 0; i <= LMI_MAX_HOPS; ++i) st->n_miss[i] = 0;
+  st->node_counter[8] = hops;
+  st->node_counter[9] = bp.n_seeds;
+  st->node_counter[1] = st->node_counter[3] = st->node_counter[5] = bp.n_seeds;
+  st->node_counter[7] = bp.n_seeds;
+  st->serial = bp.serial;
+  st->rng_lo = (uint32_t)bp.rng_seed;
+  st->rng_hi = (uint32_t)(bp.rng_seed >> 32);
+  st->lru_tick = bp.lru_tick;
+  st->n_seeds = bp.n_seeds;
+  st->table_tag = bp.table_tag;
+  st->table_mask = bp.table_mask;
+  st->seeds = bp.seeds;
+  st->labels_in = bp.labels;
+  st->fault = bp.fault;
+}
+
 // Header updates that ride on the scan total (thread 0 of the single block).
 // Reference semantics: counter_update, engine/operator_impl.cu:58-91.
 __device__ __forceinline__ void scan_epilogue(int epilogue, DevState *st, int hop, int total) {
