@@ -771,6 +771,7 @@ static int batch_params(Server *s, Pipe &p, hipStream_t st, const int32_t *seeds
 // on the first list are gathered over the host link from here on (split lookups).
 static int launch_sampling(Server *s, Pipe *const *pp, const BatchParams *bps, int n, hipStream_t st, bool own_begin,
                            HopLookup early, HopLookup late, bool misses_early = false) {
+  if (!own_begin && !misses_early && small_batch(s)) return launch_small(s, pp, bps, n, st, early);
   bool begin = own_begin || !hop_sets_up(s);
   for (int k = 0; k < n; ++k) begin = begin || bps[k].clear_table;
   if (begin) LMI_TRY(launch_batch_generate(s, pp, bps, n, st, false));
@@ -1055,7 +1056,7 @@ int lmi_run_once_static(lmi_server *h, void *stream, const int32_t *seeds, int32
   s->prof_on = false;  // profiling creates events: not here
   int rc = batch_params(s, p, st, seeds, n, LMI_LOC_DEVICE, 0, LMI_MODE_TRAIN, rng_seed, &bp);
   const HopLookup look{one_pass_gather(s) ? LOOK_SLOTS : LOOK_LIST, 0};
-  if (rc == LMI_OK) rc = launch_sampling(s, pp, &bp, 1, st, true, look, look);
+  if (rc == LMI_OK) rc = small_batch(s) ? launch_small(s, pp, &bp, 1, st, look) : launch_sampling(s, pp, &bp, 1, st, true, look, look);
   const HeaderCopy headers{out->node_counter, out->edge_counter};
   if (rc == LMI_OK) rc = launch_gather_group(s, pp, 1, st, 0, s->cfg.hops, 0, true, -1, &headers);
   s->prof_on = prof;
@@ -1230,6 +1231,7 @@ int lmi_tune(lmi_server *h, const char *key, int64_t value) {
     for (auto &p : s->pipes) p.table_dirty = true;
   }
   else if (!strcmp(key, "profile_every")) s->prof_every = (int)std::max<int64_t>(1, value);
+  else if (!strcmp(key, "small_edges")) s->small_edges = value;
   else if (!strcmp(key, "fuse_small_max")) s->fuse_small_max = value;
   else if (!strcmp(key, "split_miss")) s->split_miss = (int)value;
   else if (!strcmp(key, "use_graph")) s->use_graph = (int)value;

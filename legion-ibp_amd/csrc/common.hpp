@@ -234,6 +234,8 @@ struct Server {
   int64_t table_epochs = int64_t(1) << 30;  // batches a dedup table serves between wipes, less one (also
                                             // bounded by the key bits the node ids leave free)
   int fuse_count = 1;     // 1: row counts, their scan and the sampling of a hop share one launch
+  int64_t small_edges = 7000;  // batches whose largest hop is expected to hold at most this many edges are sampled by one
+                               // workgroup (small_batch)
   int lds_dedup = 0;      // 1: hop_sample stages its probes through an LDS hash table
   int split_miss = 1;     // gather schedule, see launch_gather_group
   int use_graph = 0;      // 1: lmi_run_once replays a captured HIP graph of the sampling kernels (measured
@@ -286,6 +288,9 @@ struct HopLookup {
 enum { LOOK_NOT = 0, LOOK_SLOTS = 1, LOOK_LIST = 2 };  // not at all; cache_index only; cache_index and the miss list
 int launch_hop(Server *s, Pipe *const *pp, int n, hipStream_t st, int hop, bool stage_seeds, bool defer_fill,
                const BatchParams *begin = nullptr, HopLookup look = HopLookup{});
+// small.hip: the sampling phase of small batches, lookup included, in one launch of one workgroup per batch
+bool small_batch(const Server *s);
+int launch_small(Server *s, Pipe *const *pp, const BatchParams *bps, int n, hipStream_t st, HopLookup look);
 bool hop_sets_up(const Server *s);  // whether launch_hop can take `begin`
 int launch_fill(Server *s, Pipe *const *pp, int n, hipStream_t st);  // finishes a hop left pending, if any
 struct SlotTable;

@@ -1,0 +1,357 @@
+// The whole sampling phase of a small batch in one workgroup.
+//
+// A small batch is bound by latency: in the general path every hop is two launches whose blocks pass counts through
+// HBM (look-back) and deduplicate through atomics on a table in HBM, four launches of 5-10 us each for 16 seeds that
+// touch 500 nodes.  One workgroup of 1024 threads has all of it within a barrier's reach instead: the dedup table, the
+// slots of a hop's edges and the nodes being sampled lie in LDS, the scans are block scans, and one launch per group of
+// batches (a workgroup each) does the seeds, every hop, the relabelling, the cache lookup and the headers.  What is left
+// of HBM is the chain seed -> row pointers -> neighbours -> row pointers ... that no kernel can shorten.
+// us per batch, gather included, on the general path and here: 16 seeds, fanouts 10,5 (445 edges in the last hop): 33 / 18;
+// 64 seeds of a Cora-shaped graph, 25,10 (3 680 edges): 36 / 27; 64 seeds, 10,5 (2 332): 38 / 25, six of them in a
+// group 39 / 25; three hops 5,4,3 (3 918): 52 / 41; 128 seeds of the Cora-shaped graph (6 979): 38 / 37.  1024 threads,
+// because draws and probes fill the CU's four SIMDs: with 512 the second of these takes 33, with 256 50.
+// Outputs are those of the general path, bit for bit (same draws, same candidates in the dedup table, same ranks).
+#include <algorithm>
+
+#include "scan.hpp"
+
+namespace lmi {
+
+constexpr int kSmallBlock = 1024;
+constexpr int kSmallItems = 4;  // edges per thread and step of the flag scan
+constexpr int kSmallNodes = 2;  // nodes in flight per lane group
+constexpr int64_t kSmallLds = 160 * 1024;
+
+struct SmallPipe {
+  DevState *st;
+  int32_t *ids, *labels;
+  int32_t *row_ptr[LMI_MAX_HOPS];
+  int32_t *agg_src_ids, *agg_src_off, *agg_dst_off;
+  int32_t *cache_index;
+  int2 *miss_list;
+  BatchParams bp;
+};
+struct SmallGroup {
+  const int64_t *indptr;
+  const int32_t *indices;
+  int64_t n_nodes;
+  int fanout[LMI_MAX_HOPS];
+  int hops;
+  int log2t;      // LDS dedup table
+  int look_mode;
+  SlotTable cache;
+  SmallPipe p[LMI_MAX_GROUP];
+};
+static_assert(sizeof(SmallGroup) <= 4096, "a kernel's arguments");
+
+// The block's LDS, carved by hand: its sizes follow the batch.
+struct SmallLds {
+  int64_t *beg, *deg;  // [kSmallBlock] rows of the nodes being sampled; those of the first kSmallBlock nodes stay for the
+                       // next hop, which then starts without a read
+  int32_t *key, *val;  // dedup table: id, lowest candidate (later: local id)
+  int *base, *node;    // [kSmallBlock] place of the node's first edge, its id
+  int *scan;           // block scans (kSmallScan ints); the last two count misses and the nodes placed in `order`
+  uint16_t *order;     // [kSmallBlock] the nodes being sampled, those that draw first
+  uint16_t *eslot;     // table slot of each edge of the hop
+};
+constexpr int kSmallScan = 32;
+__host__ __device__ inline int64_t small_lds_bytes(int log2t, int64_t edges) {
+  return (int64_t(8) << log2t) + kSmallBlock * 26 + kSmallScan * 4 + 2 * ((edges + 7) / 8 * 8);
+}
+
+// Slot of `id`, its value lowered to at most `cand`.  The table is no larger than the distinct ids a valid graph can
+// give a batch need; neighbour ids outside the graph could fill it, so the probe is bounded and reports them.
+__device__ __forceinline__ int small_insert(const SmallLds &l, int log2t, int32_t id, int cand, bool *full) {
+  const int mask = (1 << log2t) - 1;
+  int h = (int)hash_id(id, log2t);
+  for (int probes = 0; probes <= mask; ++probes) {
+    int32_t k = l.key[h];
+    if (k == kEmptyKey) k = atomicCAS(&l.key[h], kEmptyKey, id);
+    if (k == kEmptyKey || k == id) {
+      atomicMin(&l.val[h], cand);
+      return h;
+    }
+    h = (h + 1) & mask;
+  }
+  *full = true;
+  return 0;
+}
+
+// Samples the n_here staged nodes, a lane group per node and kSmallNodes nodes in flight, so that their neighbour reads
+// overlap.  The nodes come in the order of SmallLds::order, those that draw first: a wavefront computes draws for all its
+// groups if one of them needs any, and draws are what one CU is slow at.  (64 seeds of a Cora-shaped graph, where a
+// quarter of the nodes draw: 30.4 us in plain order, 27.0 in this one, gather and launches included.)
+template <int G>
+__device__ __forceinline__ void small_sample(const SmallLds &l, const SmallGroup &g, const SmallPipe &a, int hop, int n_here,
+                                             int c0, int n_known, int eoff, bool *full) {
+  const int lane = threadIdx.x & (G - 1), per_pass = kSmallBlock / G, fanout = g.fanout[hop];
+  for (int k0 = threadIdx.x / G; k0 < n_here; k0 += per_pass * kSmallNodes) {
+    int32_t nbr[kSmallNodes];
+    int at[kSmallNodes];  // the node, or -1 in a lane without an edge
+#pragma unroll
+    for (int u = 0; u < kSmallNodes; ++u) {
+      at[u] = -1;
+      nbr[u] = -1;
+      if (k0 + u * per_pass >= n_here) continue;
+      const int q = n_here > per_pass ? l.order[k0 + u * per_pass] : k0;
+      const int64_t deg = l.deg[q];
+      uint32_t pick = (uint32_t)lane;
+      if (deg > (int64_t)fanout) {
+        const uint32_t j = (uint32_t)(deg - fanout) + (uint32_t)lane;
+        uint32_t d = 0xFFFFFFFFu;
+        if (lane < fanout)
+          d = __umulhi(sample_draw(a.bp.rng_seed, (uint32_t)hop, (uint32_t)l.node[q], (uint32_t)lane), j + 1u);
+        bool dup = false;  // Floyd's rule (floyd_pick); a loop, for code that runs once per batch is paid for by its length
+#pragma unroll 1
+        for (int r = 0; r + 1 < fanout; ++r) {
+          const uint32_t p = __shfl(dup ? j : d, r, G);
+          dup = dup || (lane > r && d == p);
+        }
+        pick = dup ? j : d;
+      }
+      if ((int64_t)lane < deg && lane < fanout) {
+        at[u] = q;
+        nbr[u] = g.indices[l.beg[q] + pick];
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < kSmallNodes; ++u) {
+      if (at[u] < 0) continue;
+      const int e = l.base[at[u]] + lane;
+      a.agg_src_ids[eoff + e] = nbr[u];
+      a.agg_dst_off[eoff + e] = c0 + at[u];
+      l.eslot[e] = (uint16_t)small_insert(l, g.log2t, nbr[u], n_known + e, full);
+    }
+  }
+}
+
+static __global__ __launch_bounds__(kSmallBlock) void batch_small_kernel(SmallGroup g) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  const SmallPipe &a = g.p[blockIdx.x];
+  const BatchParams &bp = a.bp;
+  const int t = threadIdx.x, T = 1 << g.log2t;
+  SmallLds l;
+  l.beg = reinterpret_cast<int64_t *>(smem);
+  l.deg = l.beg + kSmallBlock;
+  l.key = reinterpret_cast<int32_t *>(l.deg + kSmallBlock);
+  l.val = l.key + T;
+  l.base = reinterpret_cast<int *>(l.val + T);
+  l.node = l.base + kSmallBlock;
+  l.scan = l.node + kSmallBlock;
+  l.order = reinterpret_cast<uint16_t *>(l.scan + kSmallScan);
+  l.eslot = l.order + kSmallBlock;
+  int *n_miss = l.scan + kSmallScan - 1, *n_draw = l.scan + kSmallScan - 2;
+  const FaultTo fault{bp.serial, bp.fault};
+  for (int i = t; i < T; i += kSmallBlock) {
+    l.key[i] = kEmptyKey;
+    l.val[i] = kIntMax;
+  }
+  if (t == 0) {
+    *n_miss = *n_draw = 0;
+    state_begin(a.st, bp, g.hops);
+  }
+  __syncthreads();
+  bool full = false;
+  // Rows [first, last) of the batch by a thread each: the cache lookup, the miss list (its order is arbitrary) and, where
+  // the next hop will sample them from LDS, their row pointers, all in flight together.  Hop -1: the seeds.
+  const auto rows = [&](int hop, int first, int last) {
+    const bool stay = hop + 1 < g.hops;
+    for (int i0 = first; i0 < last; i0 += kSmallBlock) {
+      const int i = i0 + t;
+      bool miss = false;
+      int32_t id = -1;
+      if (i < last) {
+        id = hop < 0 ? bp.seeds[i] : i < kSmallBlock ? l.node[i] : a.ids[i];
+        const bool good = id >= 0 && id < g.n_nodes;
+        int64_t lo = 0, hi = 0;
+        if (stay && i < kSmallBlock && good) {
+          lo = g.indptr[id];
+          hi = g.indptr[id + 1];
+        }
+        int32_t slot = -1;
+        if (g.look_mode != LOOK_NOT && good) slot = static_find(g.cache, id);
+        if (hop < 0) {
+          a.ids[i] = id;
+          a.labels[i] = bp.labels ? bp.labels[i] : -1;
+          if (i < kSmallBlock) l.node[i] = id;
+          if (good) small_insert(l, g.log2t, id, i, &full);
+          else raise_fault(a.st, kFaultBadId, fault);
+        }
+        if (stay && i < kSmallBlock) {
+          l.beg[i] = lo;
+          l.deg[i] = hi - lo;
+        }
+        if (g.look_mode != LOOK_NOT) a.cache_index[i] = slot;
+        miss = good && slot < 0;
+      }
+      if (g.look_mode == LOOK_LIST) {
+        const uint64_t m = __ballot(miss);
+        int at = 0;
+        if ((t & (kWave - 1)) == 0 && m) at = atomicAdd(n_miss, __popcll(m));
+        at = __shfl(at, 0, kWave) + __popcll(m & lanemask_lt());
+        if (miss) a.miss_list[at] = make_int2(i, id);
+      }
+    }
+  };
+  rows(-1, 0, bp.n_seeds);
+  __syncthreads();
+  int n_known = bp.n_seeds, eoff = 0;
+  for (int hop = 0; hop < g.hops; ++hop) {
+    const int fanout = g.fanout[hop];
+    int G = 4;
+    while (G < fanout) G <<= 1;
+    int32_t *row_ptr = a.row_ptr[hop];
+    // ---- sampling, kSmallBlock nodes at a time: all nodes known so far, in order
+    int n_edges = 0;
+    const bool here = n_known <= kSmallBlock;  // all their rows are in LDS
+    for (int c0 = 0; c0 < n_known; c0 += kSmallBlock) {
+      const int my = c0 + t;
+      int64_t deg = 0;
+      if (here) {
+        if (my < n_known) deg = l.deg[t];
+      } else {
+        int32_t id = -1;
+        int64_t lo = 0, hi = 0;
+        if (my < n_known) id = a.ids[my];
+        if (id >= 0 && id < g.n_nodes) {
+          lo = g.indptr[id];
+          hi = g.indptr[id + 1];
+        }
+        l.beg[t] = lo;
+        l.deg[t] = deg = hi - lo;
+        l.node[t] = id;
+      }
+      int total;
+      const int base = n_edges + block_exclusive_scan<kSmallBlock>(
+                                     (int)(deg < (int64_t)fanout ? deg : (int64_t)fanout), l.scan, total);
+      if (my < n_known) row_ptr[my] = base;
+      l.base[t] = base;
+      // places in the order: nodes that draw from the front, the others from the back
+      const int n_here = n_known - c0 < kSmallBlock ? n_known - c0 : kSmallBlock;
+      const bool draws = deg > (int64_t)fanout;
+      const uint64_t m = __ballot(draws), m2 = __ballot(!draws && my < n_known);
+      int ahead = 0;
+      if ((t & (kWave - 1)) == 0) ahead = atomicAdd(n_draw, __popcll(m) | (__popcll(m2) << 16));
+      ahead = __shfl(ahead, 0, kWave);
+      if (draws) l.order[(ahead & 0xffff) + __popcll(m & lanemask_lt())] = (uint16_t)t;
+      else if (my < n_known) l.order[n_here - 1 - (ahead >> 16) - __popcll(m2 & lanemask_lt())] = (uint16_t)t;
+      __syncthreads();
+      if (t == 0) *n_draw = 0;  // for the next nodes, some barriers away
+      switch (G) {
+        case 4: small_sample<4>(l, g, a, hop, n_here, c0, n_known, eoff, &full); break;
+        case 8: small_sample<8>(l, g, a, hop, n_here, c0, n_known, eoff, &full); break;
+        case 16: small_sample<16>(l, g, a, hop, n_here, c0, n_known, eoff, &full); break;
+        case 32: small_sample<32>(l, g, a, hop, n_here, c0, n_known, eoff, &full); break;
+        default: small_sample<64>(l, g, a, hop, n_here, c0, n_known, eoff, &full); break;
+      }
+      n_edges += total;
+      __syncthreads();  // the next nodes overwrite these; the table is complete behind the last ones
+    }
+    if (t == 0) {
+      row_ptr[n_known] = n_edges;
+      scan_epilogue(SCAN_EPI_HOP_EDGES, a.st, hop, n_edges);
+    }
+    // ---- first occurrences: ranks in edge order, ids, local ids.  An edge is one iff the value of its slot names the
+    // edge (a published local id never does: it is at most the candidate it replaces, see hop_flag_scan_kernel).
+    int n_new = 0;
+    for (int e0 = 0; e0 < n_edges; e0 += kSmallBlock * kSmallItems) {
+      const int e = e0 + t * kSmallItems;
+      int slot[kSmallItems], first[kSmallItems], sum = 0;
+#pragma unroll
+      for (int u = 0; u < kSmallItems; ++u) {
+        slot[u] = e + u < n_edges ? (int)l.eslot[e + u] : 0;
+        first[u] = e + u < n_edges && l.val[slot[u]] == n_known + e + u ? 1 : 0;
+        sum += first[u];
+      }
+      int total;
+      int at = n_known + n_new + block_exclusive_scan<kSmallBlock>(sum, l.scan, total);
+      n_new += total;
+#pragma unroll
+      for (int u = 0; u < kSmallItems; ++u)
+        if (first[u]) {
+          const int32_t id = l.key[slot[u]];
+          l.val[slot[u]] = at;
+          a.ids[at] = id;
+          if (at < kSmallBlock) l.node[at] = id;
+          ++at;
+        }
+    }
+    __syncthreads();
+    // ---- local ids of the edges' sources, lookup of the new rows
+    for (int e = t; e < n_edges; e += kSmallBlock) a.agg_src_off[eoff + e] = l.val[l.eslot[e]];
+    rows(hop, n_known, n_known + n_new);
+    if (t == 0) scan_epilogue(SCAN_EPI_HOP_NODES, a.st, hop, n_new);
+    n_known += n_new;
+    eoff += n_edges;
+    __syncthreads();  // the next hop overwrites the edges' slots, and reads what was written here
+  }
+  if (full) raise_fault(a.st, kFaultBadId, fault);
+  if (t == 0) a.st->n_miss[0] = *n_miss;
+}
+
+// Distinct ids bound the table: a batch's worst case or, in a small graph, its nodes.  Load at most 0.95 in a worst case
+// that real batches, which fill a quarter of it, do not come near.
+static int small_log2t(const Server *s) {
+  const int64_t distinct = std::min(s->max_nodes, s->n_nodes);
+  int lg = 6;
+  while ((int64_t(1) << lg) * 95 < 100 * distinct) ++lg;
+  return lg;
+}
+
+// Edges of the largest hop as the graph's mean degree has it (a quarter more for the degrees of neighbours).
+static double small_expected_edges(const Server *s) {
+  const double mean = 1.25 * (double)s->n_edges / (double)s->n_nodes;
+  double nodes = s->cfg.batch_size, most = 0;
+  for (int k = 0; k < s->cfg.hops; ++k) {
+    const double e = nodes * std::min<double>(mean, s->cfg.fanout[k]);
+    most = std::max(most, e);
+    nodes += e;
+  }
+  return most;
+}
+
+// Which batches: those whose largest hop is expected to hold at most small_edges edges (where one workgroup, on one CU,
+// is still faster than launches over the whole device), and whose table and edges fit the LDS of a CU in the worst
+// case.  Not with the LRU cache: its lookup waits for the insertion before and asks the dedup table in HBM for repeated
+// seeds.
+bool small_batch(const Server *s) {
+  const int lg = small_log2t(s);
+  return s->cache_kind != LMI_CACHE_LRU && lg <= 15 && small_lds_bytes(lg, s->max_edges_hop) <= kSmallLds &&
+         small_expected_edges(s) <= (double)s->small_edges && !s->lds_dedup && s->fuse_count;
+}
+
+int launch_small(Server *s, Pipe *const *pp, const BatchParams *bps, int n, hipStream_t st, HopLookup look) {
+  SmallGroup g{};
+  g.indptr = s->indptr;
+  g.indices = s->indices;
+  g.n_nodes = s->n_nodes;
+  g.hops = s->cfg.hops;
+  for (int k = 0; k < s->cfg.hops; ++k) g.fanout[k] = s->cfg.fanout[k];
+  g.log2t = small_log2t(s);
+  g.look_mode = look.mode;
+  g.cache = slot_table(s);
+  for (int k = 0; k < n; ++k) {
+    Pipe &p = *pp[k];
+    SmallPipe &a = g.p[k];
+    a.st = p.st;
+    a.ids = p.ids;
+    a.labels = p.labels;
+    for (int h = 0; h < LMI_MAX_HOPS; ++h) a.row_ptr[h] = p.blk_indptr[h];
+    a.agg_src_ids = p.agg_src_ids;
+    a.agg_src_off = p.agg_src_off;
+    a.agg_dst_off = p.agg_dst_off;
+    a.cache_index = p.cache_index;
+    a.miss_list = p.miss_list;
+    a.bp = bps[k];
+    p.n_seeds = bps[k].n_seeds;
+    p.hops_done = s->cfg.hops;
+    p.fill_pending = -1;
+    if (bps[k].clear_table) p.table_dirty = true;  // this batch leaves the table in HBM as it is
+  }
+  hipLaunchKernelGGL(batch_small_kernel, dim3(n), dim3(kSmallBlock), (size_t)small_lds_bytes(g.log2t, s->max_edges_hop),
+                     st, g);
+  LMI_HIP(hipGetLastError());
+  return LMI_OK;
+}
+
+}  // namespace lmi
