@@ -9,7 +9,7 @@
 //   cache/cache.cu:559-656              FillUp: choose rows, copy them, build the map
 //   comp_cache/static_cache_kernel.cuh:6-29,185-266   set = id mod n_sets, ways contiguous
 // What differs on purpose: hot set = top rows by (out-degree desc, id asc) found
-// with a threshold search and two scans (no sort, no presampling); our own
+// with a histogram of the keys and two scans (no sort, no presampling); our own
 // open-addressing table (or a direct map) instead of the vendored cuckoo table;
 // a batch-synchronous LRU (the reference's LRU source is absent); int8 + per-row
 // scale instead of the un-vendored lossless codec; one lane moves 16 bytes and
@@ -590,8 +590,14 @@ __device__ __forceinline__ float load_elem(const uint8_t *row, int i, int dtype)
 }
 
 // One wavefront per row: absmax over the row, scale = absmax / 127,
-// q = clamp(rint(x / scale), -127, 127).  Build-time only, so the source row
-// (usually in pinned host memory) is read twice rather than staged.
+// q = clamp(rint(x / scale), -127, 127).  The row usually lies in pinned host memory, whose link bounds the build: rows
+// of up to 64 * KEEP elements stay in registers between the two passes over them, longer ones (KEEP 0) are read twice.
+__device__ __forceinline__ int8_t quantize_elem(float x, float absmax, float sc) {
+  float v = (absmax == 0.0f) ? 0.0f : rintf(x / sc);
+  v = fminf(127.0f, fmaxf(-127.0f, v));
+  return (int8_t)v;
+}
+template <int KEEP>
 static __global__ __launch_bounds__(256) void quantize_rows_kernel(
     const int32_t *row_ids, int64_t n_rows, const uint8_t *feat, int dim, int dtype, int64_t row_bytes,
     int8_t *q, float *scale) {
@@ -600,16 +606,26 @@ static __global__ __launch_bounds__(256) void quantize_rows_kernel(
   const int64_t n_waves = (int64_t)gridDim.x * blockDim.x / kWave;
   for (int64_t r = wave; r < n_rows; r += n_waves) {
     const uint8_t *row = feat + (int64_t)row_ids[r] * row_bytes;
+    float x[KEEP > 0 ? KEEP : 1];
     float a = 0.0f;
-    for (int i = lane; i < dim; i += kWave) a = fmaxf(a, fabsf(load_elem(row, i, dtype)));
+    if constexpr (KEEP > 0) {
+#pragma unroll
+      for (int k = 0; k < KEEP; ++k) x[k] = lane + k * kWave < dim ? load_elem(row, lane + k * kWave, dtype) : 0.0f;
+#pragma unroll
+      for (int k = 0; k < KEEP; ++k) a = fmaxf(a, fabsf(x[k]));
+    } else {
+      for (int i = lane; i < dim; i += kWave) a = fmaxf(a, fabsf(load_elem(row, i, dtype)));
+    }
 #pragma unroll
     for (int d = kWave / 2; d > 0; d >>= 1) a = fmaxf(a, __shfl_xor(a, d, kWave));
     const float sc = a / 127.0f;
     if (lane == 0) scale[r] = sc;
-    for (int i = lane; i < dim; i += kWave) {
-      float v = (a == 0.0f) ? 0.0f : rintf(load_elem(row, i, dtype) / sc);
-      v = fminf(127.0f, fmaxf(-127.0f, v));
-      q[r * dim + i] = (int8_t)v;
+    if constexpr (KEEP > 0) {
+#pragma unroll
+      for (int k = 0; k < KEEP; ++k)
+        if (lane + k * kWave < dim) q[r * dim + lane + k * kWave] = quantize_elem(x[k], a, sc);
+    } else {
+      for (int i = lane; i < dim; i += kWave) q[r * dim + i] = quantize_elem(load_elem(row, i, dtype), a, sc);
     }
   }
 }
@@ -1526,26 +1542,24 @@ int launch_hotness(Server *s, Pipe &p, hipStream_t st) {
   return LMI_OK;
 }
 
-static __global__ __launch_bounds__(256) void degree_stats_kernel(const int64_t *indptr, const uint32_t *hot,
-                                                                  int64_t n, int64_t thr,
-                                                                  unsigned long long *count_ge,
-                                                                  unsigned long long *max_deg) {
-  unsigned long long c = 0, m = 0;
+// Histogram of the ranking keys in [lo, hi): bin (key - lo) >> shift, or with shift < 0 the key's bit length.  A block
+// counts in LDS and adds its bins once: one same-address atomic per wavefront, as a count of the keys above a bound
+// needs, took 190 us for 2.4 M nodes, this 12.
+constexpr int kRankBins = 4096;
+static __global__ __launch_bounds__(1024) void rank_histogram_kernel(const int64_t *indptr, const uint32_t *hot, int64_t n,
+                                                                     int64_t lo, int64_t hi, int shift,
+                                                                     unsigned long long *bins) {
+  __shared__ unsigned int s_bin[kRankBins];
+  for (int b = threadIdx.x; b < kRankBins; b += blockDim.x) s_bin[b] = 0;
+  __syncthreads();
   for (int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; v < n; v += (int64_t)gridDim.x * blockDim.x) {
-    const unsigned long long d = (unsigned long long)rank_key(indptr, hot, v);
-    c += (d >= (unsigned long long)thr) ? 1 : 0;
-    m = d > m ? d : m;
+    const int64_t key = rank_key(indptr, hot, v);
+    if (key < lo || key >= hi) continue;
+    atomicAdd(&s_bin[shift < 0 ? (key == 0 ? 0 : 64 - __clzll(key)) : (int)((key - lo) >> shift)], 1u);
   }
-#pragma unroll
-  for (int d = kWave / 2; d > 0; d >>= 1) {
-    c += __shfl_down(c, d, kWave);
-    const unsigned long long o = __shfl_down(m, d, kWave);
-    m = o > m ? o : m;
-  }
-  if ((threadIdx.x & (kWave - 1)) == 0) {
-    if (c) atomicAdd(count_ge, c);
-    atomicMax(max_deg, m);
-  }
+  __syncthreads();
+  for (int b = threadIdx.x; b < kRankBins; b += blockDim.x)
+    if (s_bin[b]) atomicAdd(&bins[b], (unsigned long long)s_bin[b]);
 }
 
 // mode 0: cnt[v] = (deg == thr);  mode 1: cnt[v] = member flag using tie ranks.
@@ -1622,34 +1636,75 @@ int launch_table_clear(Table &t, hipStream_t st) {
   return LMI_OK;
 }
 
-void cache_free(Server *s) {
+// No cache any more, and no batch in flight that still reads it; its buffers stay for the build that follows.
+static void cache_drop(Server *s) {
   (void)hipDeviceSynchronize();  // batches in flight (side stream included) still read the old cache
   s->lru_pending = s->lru_copy_pending = false;
-  if (s->cache_data) (void)hipFree(s->cache_data);
-  if (s->cache_scale) (void)hipFree(s->cache_scale);
-  if (s->id_table.slots) (void)hipFree(s->id_table.slots);
-  if (s->slot_of) (void)hipFree(s->slot_of);
-  if (s->rank_tab) (void)hipFree(s->rank_tab);
   if (s->lru_keys) (void)hipFree(s->lru_keys);  // one allocation: lru_use points into it
   if (s->lru_head) (void)hipFree(s->lru_head);
-  s->cache_data = nullptr;
-  s->cache_scale = nullptr;
-  s->id_table = Table{};
-  s->slot_of = nullptr;
-  s->rank_tab = nullptr;
   s->lru_keys = s->lru_use = s->lru_head = nullptr;
   s->cache_kind = LMI_CACHE_NONE;
   s->cache_rows = 0;
 }
 
-static int count_ge(const Server *s, int64_t thr, unsigned long long *d_pair, int64_t *count, int64_t *max_deg) {
-  LMI_HIP(hipMemset(d_pair, 0, 16));
-  hipLaunchKernelGGL(degree_stats_kernel, dim3(s->n_cu * 8), dim3(256), 0, 0, s->indptr,
-                     s->policy == LMI_POLICY_PRESAMPLED ? s->hot : nullptr, s->n_nodes, thr, d_pair, d_pair + 1);
-  unsigned long long h[2];
-  LMI_HIP(hipMemcpy(h, d_pair, 16, hipMemcpyDeviceToHost));
-  *count = (int64_t)h[0];
-  if (max_deg) *max_deg = (int64_t)h[1];
+void cache_free(Server *s) {
+  cache_drop(s);
+  if (s->cache_data) (void)hipFree(s->cache_data);
+  if (s->cache_scale) (void)hipFree(s->cache_scale);
+  if (s->id_table.slots) (void)hipFree(s->id_table.slots);
+  if (s->slot_of) (void)hipFree(s->slot_of);
+  if (s->rank_tab) (void)hipFree(s->rank_tab);
+  s->cache_data = nullptr;
+  s->cache_scale = nullptr;
+  s->id_table = Table{};
+  s->slot_of = nullptr;
+  s->rank_tab = nullptr;
+  if (s->build_scratch) (void)hipFree(s->build_scratch);
+  s->build_scratch = nullptr;
+  s->build_scratch_bytes = 0;
+  for (size_t &b : s->cache_buf) b = 0;
+}
+
+// The largest key `thr` that at least `cap` nodes (1 <= cap <= nodes) reach, and how many lie above it: the octave of
+// keys first, then 4096 bins at a time of what is left (two passes for keys below 8192).
+static int rank_threshold(const Server *s, int64_t cap, unsigned long long *d_bins, int64_t *thr, int64_t *above) {
+  std::vector<unsigned long long> bins(kRankBins);
+  int64_t lo = 0, size = INT64_MAX;
+  int shift = -1;
+  *above = 0;
+  while (true) {
+    LMI_HIP(hipMemsetAsync(d_bins, 0, kRankBins * 8, 0));
+    hipLaunchKernelGGL(rank_histogram_kernel, dim3(s->n_cu), dim3(1024), 0, 0, s->indptr,
+                       s->policy == LMI_POLICY_PRESAMPLED ? s->hot : nullptr, s->n_nodes, lo,
+                       size == INT64_MAX ? size : lo + size, shift, d_bins);
+    LMI_HIP(hipGetLastError());
+    LMI_HIP(hipMemcpy(bins.data(), d_bins, kRankBins * 8, hipMemcpyDeviceToHost));
+    int b = kRankBins - 1;
+    for (; b > 0 && *above + (int64_t)bins[b] < cap; --b) *above += (int64_t)bins[b];
+    if (shift < 0) {
+      lo = b == 0 ? 0 : int64_t(1) << (b - 1);  // bit length b: keys [2^(b-1), 2^b)
+      size = b == 0 ? 1 : lo;
+    } else {
+      lo += (int64_t)b << shift;
+      size = int64_t(1) << shift;
+    }
+    if (size == 1) break;
+    shift = 0;
+    while ((size >> shift) > kRankBins) ++shift;
+  }
+  *thr = lo;
+  return LMI_OK;
+}
+
+// A buffer of the cache: kept when it has the size already (a cache that is built again), else allocated.
+static int cache_buffer(void **p, size_t *have, size_t want) {
+  if (*p && *have == want) return LMI_OK;
+  if (*p) (void)hipFree(*p);
+  *p = nullptr;
+  *have = 0;
+  if (want == 0) return LMI_OK;
+  LMI_HIP(hipMalloc(p, want));
+  *have = want;
   return LMI_OK;
 }
 
@@ -1661,53 +1716,66 @@ int cache_build_static(Server *s, int64_t capacity_rows, int table_kind, bool in
   if (table_kind != LMI_TABLE_HASH && table_kind != LMI_TABLE_DIRECT && table_kind != LMI_TABLE_RANK)
     LMI_FAIL(LMI_ERR_ARG, "bad table kind");
   if (s->n_nodes >= (int64_t(1) << 31) - kScanTile) LMI_FAIL(LMI_ERR_CAPACITY, "too many nodes");
-  cache_free(s);
+  cache_drop(s);
   const int64_t N = s->n_nodes;
   const int64_t cap = std::max<int64_t>(0, std::min(capacity_rows, N));
   s->table_kind = table_kind;
   s->cache_row_bytes = int8 ? s->cfg.feat_dim : s->row_bytes;
-  if (cap == 0) LMI_FAIL(LMI_ERR_ARG, "cache capacity must be at least one row");
-  if (s->policy == LMI_POLICY_PRESAMPLED && !s->hot)
-    LMI_FAIL(LMI_ERR_STATE, "the presampled policy needs lmi_presample (or presampling operators) first");
-  const uint32_t *hot_key = s->policy == LMI_POLICY_PRESAMPLED ? s->hot : nullptr;
+  const bool presampled = s->policy == LMI_POLICY_PRESAMPLED;
+  int lg = 4;
+  while ((int64_t(1) << lg) < 2 * cap) ++lg;
+  if (cap == 0 || (presampled && !s->hot) || (table_kind == LMI_TABLE_HASH && lg > 31)) {
+    cache_free(s);
+    if (cap == 0) LMI_FAIL(LMI_ERR_ARG, "cache capacity must be at least one row");
+    if (presampled && !s->hot)
+      LMI_FAIL(LMI_ERR_STATE, "the presampled policy needs lmi_presample (or presampling operators) first");
+    LMI_FAIL(LMI_ERR_CAPACITY, "cache too large for the hash table");
+  }
+  const uint32_t *hot_key = presampled ? s->hot : nullptr;
+  // What the cache before had in another size goes first, so that the two never lie in memory together.  (Taking
+  // 40 MB of scratch anew costs a build 0.5 ms.)
+  const size_t want[kCacheBufs] = {(size_t)cap * s->cache_row_bytes, int8 ? (size_t)cap * 4 : 0,
+                                   table_kind == LMI_TABLE_HASH ? size_t(8) << lg : 0,
+                                   table_kind == LMI_TABLE_DIRECT ? (size_t)N * 4 : 0,
+                                   table_kind == LMI_TABLE_RANK ? (size_t)ceil_div(N, 64) * 16 : 0};
+  void **const buf[kCacheBufs] = {(void **)&s->cache_data, (void **)&s->cache_scale, (void **)&s->id_table.slots,
+                                  (void **)&s->slot_of, (void **)&s->rank_tab};
+  for (int k = 0; k < kCacheBufs; ++k)
+    if (s->cache_buf[k] != want[k]) LMI_TRY(cache_buffer(buf[k], &s->cache_buf[k], 0));
 
-  // build-time scratch, released on every return path
+  // build-time scratch in one allocation: released on every return path, or kept for the next build when it is small
   struct Scratch {
-    std::vector<void *> ptrs;
+    Server *s;
+    uint8_t *base = nullptr;
+    size_t bytes = 0;
     ~Scratch() {
-      for (void *q : ptrs) (void)hipFree(q);
+      if (s->build_scratch_bytes > kKeepBuildScratch) {
+        (void)hipFree(s->build_scratch);
+        s->build_scratch = nullptr;
+        s->build_scratch_bytes = 0;
+      }
     }
-    hipError_t get(void **p, size_t bytes) {
-      const hipError_t e = hipMalloc(p, bytes ? bytes : 1);
-      if (e == hipSuccess) ptrs.push_back(*p);
-      return e;
+    size_t take(size_t n) {
+      const size_t at = bytes;
+      bytes += (n + 255) / 256 * 256;
+      return at;
     }
-  } scratch;
-  unsigned long long *d_pair = nullptr;
-  int32_t *d_cnt = nullptr, *d_tie = nullptr, *d_slot = nullptr, *d_tiles = nullptr, *d_n = nullptr,
-          *d_cached = nullptr;
-  LMI_HIP(scratch.get((void **)&d_pair, 16));
-  LMI_HIP(scratch.get((void **)&d_cnt, (N + 1) * 4));
-  LMI_HIP(scratch.get((void **)&d_tie, (N + 1) * 4));
-  LMI_HIP(scratch.get((void **)&d_slot, (N + 1) * 4));
-  LMI_HIP(scratch.get((void **)&d_tiles, (ceil_div(N, kScanTile) + 1) * 4));
-  LMI_HIP(scratch.get((void **)&d_n, 8));
-  LMI_HIP(scratch.get((void **)&d_cached, cap * 4));
+  } scratch{s};
+  const size_t o_bins = scratch.take(kRankBins * 8), o_cnt = scratch.take((N + 1) * 4), o_tie = scratch.take((N + 1) * 4),
+               o_slot = scratch.take((N + 1) * 4), o_tiles = scratch.take((ceil_div(N, kScanTile) + 1) * 4),
+               o_n = scratch.take(8), o_cached = scratch.take(cap * 4);
+  LMI_TRY(cache_buffer(&s->build_scratch, &s->build_scratch_bytes, scratch.bytes));
+  scratch.base = (uint8_t *)s->build_scratch;
+  unsigned long long *d_bins = (unsigned long long *)(scratch.base + o_bins);
+  int32_t *d_cnt = (int32_t *)(scratch.base + o_cnt), *d_tie = (int32_t *)(scratch.base + o_tie),
+          *d_slot = (int32_t *)(scratch.base + o_slot), *d_tiles = (int32_t *)(scratch.base + o_tiles),
+          *d_n = (int32_t *)(scratch.base + o_n), *d_cached = (int32_t *)(scratch.base + o_cached);
   const int32_t n32[2] = {(int32_t)N, 0};
   LMI_HIP(hipMemcpy(d_n, n32, 8, hipMemcpyHostToDevice));
 
-  // threshold degree: largest d with count(deg >= d) >= cap
-  int64_t cnt = 0, max_deg = 0;
-  LMI_TRY(count_ge(s, 0, d_pair, &cnt, &max_deg));
-  int64_t lo = 0, hi = max_deg + 1;
-  while (hi - lo > 1) {
-    const int64_t mid = lo + (hi - lo) / 2;
-    LMI_TRY(count_ge(s, mid, d_pair, &cnt, nullptr));
-    if (cnt >= cap) lo = mid; else hi = mid;
-  }
-  const int64_t thr = lo;
-  LMI_TRY(count_ge(s, thr + 1, d_pair, &cnt, nullptr));
-  const int64_t ties_taken = cap - cnt;
+  int64_t thr = 0, above = 0;
+  LMI_TRY(rank_threshold(s, cap, d_bins, &thr, &above));
+  const int64_t ties_taken = cap - above;
 
   const int grid = scan_grid(N);
   hipLaunchKernelGGL(member_flag_kernel, dim3(grid), dim3(kScanBlock), 0, 0, s->indptr, hot_key, d_n, thr, 0, nullptr,
@@ -1720,17 +1788,11 @@ int cache_build_static(Server *s, int64_t capacity_rows, int table_kind, bool in
   LMI_HIP(hipMemcpy(&total, d_n + 1, 4, hipMemcpyDeviceToHost));
   if (total != cap) LMI_FAIL(LMI_ERR_HIP, "static cache selection picked %d rows, expected %lld", total, (long long)cap);
 
+  for (int k = 0; k < kCacheBufs; ++k) LMI_TRY(cache_buffer(buf[k], &s->cache_buf[k], want[k]));
   if (table_kind == LMI_TABLE_HASH) {
-    int lg = 4;
-    while ((int64_t(1) << lg) < 2 * cap) ++lg;
-    if (lg > 31) LMI_FAIL(LMI_ERR_CAPACITY, "cache too large for the hash table");
     s->id_table.log2cap = lg;
-    LMI_HIP(hipMalloc(&s->id_table.slots, size_t(8) << lg));
     LMI_TRY(launch_table_clear(s->id_table, 0));
-  } else if (table_kind == LMI_TABLE_DIRECT) {
-    LMI_HIP(hipMalloc(&s->slot_of, N * 4));
-  } else {
-    LMI_HIP(hipMalloc(&s->rank_tab, (size_t)ceil_div(N, 64) * 16));
+  } else if (table_kind == LMI_TABLE_RANK) {
     hipLaunchKernelGGL(publish_rank_kernel, dim3(s->n_cu * 8), dim3(256), 0, 0, d_cnt, d_slot, N, s->rank_tab);
   }
   hipLaunchKernelGGL(publish_slots_kernel, dim3(s->n_cu * 8), dim3(256), 0, 0, d_cnt, d_slot, N, table_kind,
@@ -1738,13 +1800,17 @@ int cache_build_static(Server *s, int64_t capacity_rows, int table_kind, bool in
   LMI_HIP(hipGetLastError());
 
   // rows
-  LMI_HIP(hipMalloc(&s->cache_data, (size_t)cap * s->cache_row_bytes));
   int32_t cap32[2] = {(int32_t)cap, 0};
   LMI_HIP(hipMemcpy(d_n, cap32, 8, hipMemcpyHostToDevice));
   if (int8) {
-    LMI_HIP(hipMalloc(&s->cache_scale, (size_t)cap * 4));
-    hipLaunchKernelGGL(quantize_rows_kernel, dim3(s->n_cu * 8), dim3(256), 0, 0, d_cached, cap, s->feat,
-                       s->cfg.feat_dim, s->cfg.feat_dtype, s->row_bytes, (int8_t *)s->cache_data, s->cache_scale);
+#define LMI_QUANT(KEEP_)                                                                                              \
+  hipLaunchKernelGGL(quantize_rows_kernel<KEEP_>, dim3(s->n_cu * 8), dim3(256), 0, 0, d_cached, cap, s->feat,          \
+                     s->cfg.feat_dim, s->cfg.feat_dtype, s->row_bytes, (int8_t *)s->cache_data, s->cache_scale)
+    if (s->cfg.feat_dim <= 4 * kWave) LMI_QUANT(4);
+    else if (s->cfg.feat_dim <= 12 * kWave) LMI_QUANT(12);
+    else if (s->cfg.feat_dim <= 24 * kWave) LMI_QUANT(24);
+    else LMI_QUANT(0);
+#undef LMI_QUANT
     LMI_HIP(hipGetLastError());
   } else {
     MoveArgs m{};
@@ -1780,7 +1846,7 @@ int cache_build_lru(Server *s, int64_t n_sets, int32_t ways) {
   LMI_HIP(hipMalloc(&s->lru_keys, rows * 8));  // per set: `ways` keys, then `ways` ticks
   s->lru_use = s->lru_keys + ways;
   LMI_HIP(hipMalloc(&s->lru_head, n_sets * 4));
-  LMI_HIP(hipMalloc(&s->cache_data, (size_t)rows * s->row_bytes));
+  LMI_TRY(cache_buffer((void **)&s->cache_data, &s->cache_buf[0], (size_t)rows * s->row_bytes));
   const int g = 2048;
   hipLaunchKernelGGL(lru_init_kernel, dim3(g), dim3(256), 0, 0, s->lru_keys, rows * 2, ways);
   hipLaunchKernelGGL(fill_i32_kernel, dim3(g), dim3(256), 0, 0, s->lru_head, n_sets, -1);

@@ -149,6 +149,8 @@ struct EventPair {  // device time between two recorded events, attributed to `k
   int kind;
 };
 
+constexpr size_t kKeepBuildScratch = size_t(64) << 20;
+constexpr int kCacheBufs = 5;  // Server::cache_buf
 struct Server {
   lmi_config cfg{};
   int64_t max_nodes = 0, max_edges = 0, max_edges_hop = 0;
@@ -179,6 +181,9 @@ struct Server {
   Table id_table;                    // hash id -> slot
   int32_t *slot_of = nullptr;        // direct id -> slot
   uint4 *rank_tab = nullptr;         // per 64 ids: {bits lo, bits hi, rank of first id, 0}
+  size_t cache_buf[kCacheBufs] = {};  // bytes held by cache_data, cache_scale, id_table, slot_of and rank_tab
+  void *build_scratch = nullptr;   // of the last static / int8 build, kept up to kKeepBuildScratch bytes
+  size_t build_scratch_bytes = 0;
   int64_t lru_sets = 0;
   int32_t lru_ways = 0;
   int32_t lru_tick = 0;
