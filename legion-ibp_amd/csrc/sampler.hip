@@ -199,6 +199,7 @@ static __global__ __launch_bounds__(kScanBlock) void hop_count_scan_kernel(HopGr
     }
     int total;
     const int ex = block_exclusive_scan<kScanBlock>(sum, lds, total);
+    if (threadIdx.x == 0) scan_tile_announce(a.chain_nodes, tile, total);
     const int prefix = scan_tile_prefix(a.chain_nodes, tile, total, &s_prefix, st, fault);
     if (prefix == kScanFaultPrefix) return;  // the whole block: no offset, no writes
     int run = prefix + ex;
@@ -413,49 +414,59 @@ static __global__ __launch_bounds__(256) void hop_count_sample_kernel(HopGroup g
     ex = inc - cnt;
     total = __shfl(inc, kWave - 1, kWave);
   }
-  const int prefix = scan_tile_prefix(a.chain_nodes, tile, total, &s_prefix, st, fault);
-  if (prefix == kScanFaultPrefix) return;  // the whole block: no offset, no writes
+  if (t == 0) scan_tile_announce(a.chain_nodes, tile, total);
   if (t < NPB) {
     s_id[t] = id;
     s_beg[t] = lo;
     s_deg[t] = hi - lo;
-    s_row[t] = prefix + ex;
-    if (my < n_prev) a.row_ptr[my] = prefix + ex;
-  }
-  if (tile == n_tiles - 1 && t == 0) {
-    a.row_ptr[n_prev] = prefix + total;
-    scan_epilogue(SCAN_EPI_HOP_EDGES, st, g.c.hop, prefix + total);
+    s_row[t] = ex;
   }
   __syncthreads();
-  // ---- sampling: the edge offset of the hop is fixed by the hops before it
+  // ---- sampling.  What is drawn depends on no other tile: the draws are made and the neighbour reads of up to PASSES
+  // nodes per lane group are issued before the look-back, which hides behind them; only where the edges go needs it.
   const uint64_t seed = begin ? bp.rng_seed : (uint64_t)st->rng_lo | ((uint64_t)st->rng_hi << 32);
+  // the edge offset of the hop is fixed by the hops before it
   const int eoff = (g.c.hop == 0) ? 0 : st->edge_counter[12 + g.c.hop] + st->edge_counter[9 + g.c.hop];
   const int fanout = g.c.fanout;
   const int lane = t & (G - 1);
-  for (int q = t / G; q < NPB; q += 256 / G) {
-    const int i = tile * NPB + q;
-    if (i >= n_prev) break;
-    const int32_t v = s_id[q];
-    if (v < 0) continue;
-    const int64_t beg = s_beg[q], deg = s_deg[q];
-    const int base = s_row[q];
-    int64_t pick = lane;
-    int count;
-    if (deg <= (int64_t)fanout) {
-      count = (int)deg;
-    } else {
-      count = fanout;
-      const uint32_t j = (uint32_t)(deg - fanout) + (uint32_t)lane;
-      uint32_t d = 0xFFFFFFFFu;
-      if (lane < fanout) d = __umulhi(sample_draw(seed, (uint32_t)g.c.hop, (uint32_t)v, (uint32_t)lane), j + 1u);
-      pick = floyd_pick<G>(d, j, lane, fanout);
+  constexpr int PER_PASS = 256 / G, PASSES = NPB / PER_PASS < 4 ? NPB / PER_PASS : 4;
+  int prefix = 0;
+  for (int q0 = t / G; q0 < NPB; q0 += PER_PASS * PASSES) {
+    int32_t nbr[PASSES];
+    bool on[PASSES];
+#pragma unroll
+    for (int u = 0; u < PASSES; ++u) {
+      const int q = q0 + u * PER_PASS;
+      const int32_t v = s_id[q];  // -1 behind the last node
+      const int64_t beg = s_beg[q], deg = s_deg[q];
+      int64_t pick = lane;
+      nbr[u] = -1;
+      on[u] = v >= 0 && lane < fanout && (int64_t)lane < deg;
+      if (deg > (int64_t)fanout) {
+        const uint32_t j = (uint32_t)(deg - fanout) + (uint32_t)lane;
+        uint32_t d = 0xFFFFFFFFu;
+        if (lane < fanout) d = __umulhi(sample_draw(seed, (uint32_t)g.c.hop, (uint32_t)v, (uint32_t)lane), j + 1u);
+        pick = floyd_pick<G>(d, j, lane, fanout);
+      }
+      if (on[u]) nbr[u] = g.c.indices[beg + pick];
     }
-    if (lane < count) {
-      const int32_t nbr = g.c.indices[beg + pick];
-      const int e = base + lane;
-      a.agg_src_ids[eoff + e] = nbr;
-      a.agg_dst_off[eoff + e] = i;
-      a.eslot[e] = (int)table_insert_min(a.slots, g.c.log2cap, nbr, n_prev + e, tag, tag_mask);
+    if (q0 == t / G) {  // the first time round, all threads alike
+      prefix = scan_tile_prefix(a.chain_nodes, tile, total, &s_prefix, st, fault);
+      if (prefix == kScanFaultPrefix) return;  // the whole block: no offset, no writes
+      if (t < NPB && my < n_prev) a.row_ptr[my] = prefix + ex;
+      if (tile == n_tiles - 1 && t == 0) {
+        a.row_ptr[n_prev] = prefix + total;
+        scan_epilogue(SCAN_EPI_HOP_EDGES, st, g.c.hop, prefix + total);
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < PASSES; ++u) {
+      if (!on[u]) continue;
+      const int q = q0 + u * PER_PASS;
+      const int e = prefix + s_row[q] + lane;
+      a.agg_src_ids[eoff + e] = nbr[u];
+      a.agg_dst_off[eoff + e] = tile * NPB + q;
+      a.eslot[e] = (int)table_insert_min(a.slots, g.c.log2cap, nbr[u], n_prev + e, tag, tag_mask);
     }
   }
 }
@@ -479,13 +490,15 @@ static __global__ __launch_bounds__(kScanBlock) void hop_flag_scan_kernel(HopGro
   int32_t local[ITEMS], node[ITEMS], slot_of[ITEMS];
   bool look[ITEMS];  // a row to look up
 #pragma unroll
-  for (int j = 0; j < ITEMS; ++j) local[j] = node[j] = -1, look[j] = false;
+  for (int j = 0; j < ITEMS; ++j) local[j] = node[j] = slot_of[j] = -1, look[j] = false;
+  const int look_mode = g.c.look_mode;
   if (bx >= g.c.tile_blocks) {  // extra blocks: the seeds' lookup (ids[] holds them since the hop's first kernel)
     const int i = (bx - g.c.tile_blocks) * kScanBlock + (int)threadIdx.x;
     if (i < st->n_seeds) {
       node[0] = a.ids[i];
       local[0] = i;
       look[0] = true;
+      if (look_mode != LOOK_NOT && node[0] >= 0 && node[0] < g.c.n_nodes) slot_of[0] = static_find(g.c.cache, node[0]);
     }
   } else {
     const FaultTo fault = fault_to(st);
@@ -498,6 +511,7 @@ static __global__ __launch_bounds__(kScanBlock) void hop_flag_scan_kernel(HopGro
     if (tile >= n_tiles) return;
     const int base = tile * TILE + threadIdx.x * ITEMS;
     int v[ITEMS], slot[ITEMS], sum = 0;
+    // the source ids beside the slots, and the lookups ahead of the look-back: two reads less in a row
 #pragma unroll
     for (int j = 0; j < ITEMS; ++j) {
       const int e = base + j;
@@ -506,21 +520,29 @@ static __global__ __launch_bounds__(kScanBlock) void hop_flag_scan_kernel(HopGro
       if (e < n) {
         const int32_t es = a.eslot[e];  // sign bit = kKnownRepeat: no need to look
         slot[j] = es & (int32_t)~kKnownRepeat;
-        if (es >= 0) flag = (a.slots[slot[j]].val == n_prev + e) ? 1 : 0;
+        if (es >= 0) {
+          node[j] = a.agg_src_ids[eoff + e];
+          flag = (a.slots[slot[j]].val == n_prev + e) ? 1 : 0;
+        }
       }
       v[j] = flag;
       sum += flag;
     }
     int total;
     const int ex = block_exclusive_scan<kScanBlock>(sum, lds, total);
+    if (threadIdx.x == 0) scan_tile_announce(a.chain_edges, tile, total);
+#pragma unroll
+    for (int j = 0; j < ITEMS; ++j) {
+      look[j] = v[j] != 0;
+      if (look_mode != LOOK_NOT && look[j] && node[j] >= 0 && node[j] < g.c.n_nodes)
+        slot_of[j] = static_find(g.c.cache, node[j]);
+    }
     const int prefix = scan_tile_prefix(a.chain_edges, tile, total, &s_prefix, st, fault);
     if (prefix == kScanFaultPrefix) return;  // the whole block: no ranks, no writes
     int run = n_prev + prefix + ex;
 #pragma unroll
     for (int j = 0; j < ITEMS; ++j) {
-      look[j] = v[j] != 0;
       local[j] = run;
-      node[j] = look[j] ? a.agg_src_ids[eoff + base + j] : -1;
       run += v[j];
     }
 #pragma unroll
@@ -535,20 +557,15 @@ static __global__ __launch_bounds__(kScanBlock) void hop_flag_scan_kernel(HopGro
   // read of the cache's table hides behind the other tiles' look-back: as a kernel of its own the lookup was a launch
   // and a pass over the ids: 30 us, its part of the last fill included, for a group of four papers100M-shaped
   // batches, whose flag scans did not get slower (31 + 12 us).
-  if (g.c.look_mode == LOOK_NOT) return;
+  if (look_mode == LOOK_NOT) return;
   int misses = 0;
-#pragma unroll
-  for (int j = 0; j < ITEMS; ++j) {
-    slot_of[j] = -1;
-    if (look[j] && node[j] >= 0 && node[j] < g.c.n_nodes) slot_of[j] = static_find(g.c.cache, node[j]);
-  }
 #pragma unroll
   for (int j = 0; j < ITEMS; ++j) {
     if (look[j]) a.cache_index[local[j]] = slot_of[j];
     look[j] = look[j] && slot_of[j] < 0 && node[j] >= 0 && node[j] < g.c.n_nodes;  // from here on: a miss
     misses += look[j] ? 1 : 0;
   }
-  if (g.c.look_mode == LOOK_LIST) {  // one atomic per block: one per wavefront on the same counter costs 24 ns each
+  if (look_mode == LOOK_LIST) {  // one atomic per block: one per wavefront on the same counter costs 24 ns each
     int total;
     int at = block_exclusive_scan<kScanBlock>(misses, lds, total);
     if (total == 0) return;

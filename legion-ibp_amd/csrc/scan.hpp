@@ -165,9 +165,14 @@ __device__ __forceinline__ void scan_publish(ScanChain c, int tile, unsigned lon
   __hip_atomic_store(&c.status[tile], word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Publishes this tile's aggregate and returns the exclusive prefix of the tile
-// (sum of all earlier tiles) to every thread of the block, or kScanFaultPrefix to every
-// thread when the wait ran out: the tile then has no valid offset and must write nothing.
+// Publishes this tile's aggregate; one thread of the block calls, as early as the sum is known.
+__device__ __forceinline__ void scan_tile_announce(ScanChain c, int tile, int aggregate) {
+  scan_publish(c, tile, (tile == 0 ? kScanInclusive : kScanAggregate) | (unsigned int)aggregate);
+}
+
+// Returns the exclusive prefix (sum of all earlier tiles) of a tile that was announced to every
+// thread of the block, or kScanFaultPrefix to every thread when the wait ran out: the tile then
+// has no valid offset and must write nothing.
 // Wavefront 0 looks back 64 tiles per step (lookback_window).  lds_prefix is one shared int.
 // Contains __syncthreads.
 __device__ __forceinline__ int scan_tile_prefix(ScanChain c, int tile, int aggregate, int *lds_prefix,
@@ -175,10 +180,7 @@ __device__ __forceinline__ int scan_tile_prefix(ScanChain c, int tile, int aggre
   if (threadIdx.x < kWave) {
     const int lane = threadIdx.x;
     int prefix = 0;
-    if (tile == 0) {
-      if (lane == 0) scan_publish(c, 0, kScanInclusive | (unsigned int)aggregate);
-    } else {
-      if (lane == 0) scan_publish(c, tile, kScanAggregate | (unsigned int)aggregate);
+    if (tile > 0) {
       int base = tile - 1;
       int spins = 0;
       // after a first fault every later tile gives up almost at once, so a broken chain drains
