@@ -394,7 +394,7 @@ static void launch_move_vlu(hipStream_t st, const MoveArgs &a, int grid, bool nt
   const int chunks = (int)(a.row_bytes / sizeof(V));
   // with profiling on, the launch carries its own start / stop events
 #define LMI_MOVE(NT_, HL_)                                                                                      \
-  if (a.ev_start)                                                                                               \
+  if (a.ev_start || a.ev_stop)                                                                                  \
     hipExtLaunchKernelGGL((move_rows_kernel<V, LPR, U, NT_, HL_>), dim3(grid * a.g.n), dim3(256), 0, st,         \
                           a.ev_start, a.ev_stop, 0, a.g, a.src_from_list, a.src, chunks, a.src_row_bytes,        \
                           a.dst_row_bytes, a.row_counter);                                                       \
@@ -442,7 +442,7 @@ static int64_t auto_gather_blocks(const Server *s, int64_t want) {
 template <typename V16, int TILE, int U>
 static void launch_tiled_vtu(hipStream_t st, const MoveArgs &a, int grid, bool nt, int cpr, int tail, int tile_rows) {
 #define LMI_TILED(NT_, HL_)                                                                                         \
-  if (a.ev_start)                                                                                                   \
+  if (a.ev_start || a.ev_stop)                                                                                      \
     hipExtLaunchKernelGGL((move_rows_tiled_kernel<V16, TILE, U, NT_, HL_>), dim3(grid * a.g.n), dim3(256), 0, st,    \
                           a.ev_start, a.ev_stop, 0, a.g, a.src_from_list, a.src, cpr, tail, tile_rows,              \
                           a.src_row_bytes, a.dst_row_bytes, a.row_counter);                                          \
@@ -832,10 +832,7 @@ struct LookupArgs {
   int64_t n_nodes;
   int kind;
   SlotTable table;
-  const int32_t *lru_keys;
-  int32_t *lru_use;
-  int64_t lru_sets;
-  int lru_ways;
+  LruSets lru;
   int32_t *cache_index, *lru_fill;
   int2 *miss_list;  // null: no list wanted
   DevState *st;
@@ -881,27 +878,7 @@ static __global__ __launch_bounds__(kLookupBlock) void lookup_kernel(LookupGroup
       int slot = -1;
       if (id >= 0 && id < a.n_nodes) {
         if (a.kind == LMI_CACHE_LRU) {
-          // a set's record is its keys followed by its ticks (one 64-byte line for 8 ways), so the
-          // tick of a hit is written into the line its key was just read from
-          const int set = (int)((uint32_t)id % (uint32_t)a.lru_sets);
-          const int64_t rec = (int64_t)set * 2 * a.lru_ways;
-          int way = -1;
-          if ((a.lru_ways & 3) == 0) {  // a set's keys start on a 16-byte boundary: four ways per load
-            for (int w = 0; w < a.lru_ways; w += 4) {
-              const int4 k = *reinterpret_cast<const int4 *>(a.lru_keys + rec + w);
-              if (k.x == id) way = w;
-              if (k.y == id) way = w + 1;
-              if (k.z == id) way = w + 2;
-              if (k.w == id) way = w + 3;
-            }
-          } else {
-            for (int w = 0; w < a.lru_ways; ++w)
-              if (a.lru_keys[rec + w] == id) way = w;
-          }
-          if (way >= 0) {
-            slot = set * a.lru_ways + way;  // sets * ways < 2^31
-            a.lru_use[rec + way] = a.st->lru_tick;
-          }
+          slot = lru_find(a.lru, id, a.st->lru_tick);
           // a repeated seed keeps both rows, but the id is offered for insertion once, by its first row
           const bool repeat = i < a.st->n_seeds &&
                               table_find(a.dedup, a.dedup_log2cap, id, a.st->table_tag, a.st->table_mask) != i;
@@ -948,10 +925,7 @@ int launch_lookup(Server *s, Pipe *const *pp, int n, hipStream_t st, int seg_fir
     a.n_nodes = s->n_nodes;
     a.kind = s->cache_kind;
     a.table = slot_table(s);
-    a.lru_keys = s->lru_keys;
-    a.lru_use = s->lru_use;
-    a.lru_sets = s->lru_sets;
-    a.lru_ways = s->lru_ways;
+    a.lru = lru_sets(s);
     a.cache_index = p.cache_index;
     a.miss_list = with_list ? p.miss_list + miss_list_base(s, seg_first) : nullptr;
     a.lru_fill = p.lru_fill;
@@ -1380,14 +1354,15 @@ struct LruArgs {
   int ways;
 };
 
-static __global__ __launch_bounds__(256) void lru_chain_kernel(LruArgs a) {
+// Not needed where the lookup has chained the misses already (LOOK_LRU).
+static __global__ __launch_bounds__(256) void lru_chain_kernel(LruArgs a, LruSets t) {
   for (int l = 0; l < a.n_lists; ++l) {
     const int n = a.st->n_miss[l];
     for (int j = blockIdx.x * blockDim.x + threadIdx.x; j < n; j += gridDim.x * blockDim.x) {
       const int2 pr = a.miss_list[l][j];  // (row, id)
       const int i = pr.x;
       if (a.fill[i] != -1) continue;  // the later row of a repeated seed
-      a.next[i] = atomicExch(&a.head[(uint32_t)pr.y % (uint32_t)a.sets], i);
+      lru_chain(t, a.next, i, pr.y);
     }
   }
 }
@@ -1452,11 +1427,12 @@ int launch_lru_insert(Server *s, Pipe &p, hipStream_t st, int n_lists) {
   a.sets = s->lru_sets;
   a.ways = s->lru_ways;
   const int grid = (int)std::max<int64_t>(1, std::min<int64_t>(ceil_div(s->max_nodes, 256), (int64_t)s->n_cu * 4));
-  hipLaunchKernelGGL(lru_chain_kernel, dim3(grid), dim3(256), 0, st, a);
-  hipLaunchKernelGGL(lru_place_kernel, dim3(grid), dim3(256), 0, st, a);
-  LMI_HIP(hipGetLastError());
+  if (!p.lru_chained) hipLaunchKernelGGL(lru_chain_kernel, dim3(grid), dim3(256), 0, st, a, lru_sets(s));
+  p.lru_chained = false;
+  // The events are the kernels' own completions: recorded behind them they were packets of their own and cost 6 us each.
   // keys and ticks are final: the next batch's lookup may start while the rows are still copied
-  LMI_HIP(hipEventRecord(s->lru_ready, st));
+  hipExtLaunchKernelGGL(lru_place_kernel, dim3(grid), dim3(256), 0, st, nullptr, s->lru_ready, 0, a);
+  LMI_HIP(hipGetLastError());
   s->lru_pending = true;
   s->lru_stream = st;
   // copy the granted rows from the output buffer (already gathered) into the cache
@@ -1473,9 +1449,9 @@ int launch_lru_insert(Server *s, Pipe &p, hipStream_t st, int n_lists) {
     r.dst = s->cache_data;
     m.src_row_bytes = m.dst_row_bytes = m.row_bytes = s->row_bytes;
     m.n_max = s->node_cap[s->cfg.hops];
+    if (l == n_lists - 1) m.ev_stop = s->lru_copied;
     LMI_TRY(launch_move_rows(s, st, m, false));
   }
-  LMI_HIP(hipEventRecord(s->lru_copied, st));
   s->lru_copy_pending = true;
   return LMI_OK;
 }

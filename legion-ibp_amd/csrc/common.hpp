@@ -110,6 +110,7 @@ struct Pipe {
   // first pipe of the group its misses were gathered with (one record and one wait per group: a
   // wait on another queue's event costs a stream about 10 us, fired or not).
   hipEvent_t join_of = nullptr;
+  bool lru_chained = false;    // the lookup has put this batch's misses on the lists of their sets
   bool side_pending = false;   // the side stream may still owe this pipe's miss rows (join_of not yet seen complete)
   bool join_waited = false;    // a wait for join_of has been queued on join_waiter: that stream needs no second one,
   hipStream_t join_waiter = nullptr;  // any other stream still does
@@ -290,7 +291,9 @@ struct HopLookup {
   int mode = 0;      // LOOK_*
   int miss_seg = 0;  // LOOK_LIST: the miss list that receives them
 };
-enum { LOOK_NOT = 0, LOOK_SLOTS = 1, LOOK_LIST = 2 };  // not at all; cache_index only; cache_index and the miss list
+// not at all; cache_index only; cache_index and the miss list; the same in the LRU cache, whose hits are marked and whose
+// misses go on the lists of their sets
+enum { LOOK_NOT = 0, LOOK_SLOTS = 1, LOOK_LIST = 2, LOOK_LRU = 3 };
 int launch_hop(Server *s, Pipe *const *pp, int n, hipStream_t st, int hop, bool stage_seeds, bool defer_fill,
                const BatchParams *begin = nullptr, HopLookup look = HopLookup{});
 // small.hip: the sampling phase of small batches, lookup included, in one launch of one workgroup per batch
@@ -300,6 +303,8 @@ bool hop_sets_up(const Server *s);  // whether launch_hop can take `begin`
 int launch_fill(Server *s, Pipe *const *pp, int n, hipStream_t st);  // finishes a hop left pending, if any
 struct SlotTable;
 SlotTable slot_table(const Server *s);
+struct LruSets;
+LruSets lru_sets(const Server *s);
 // where the miss list of lookup segment `seg` starts in Pipe::miss_list
 inline int64_t miss_list_base(const Server *s, int seg) { return seg == 0 ? 0 : s->node_cap[seg - 1]; }
 struct FillArgs;
@@ -313,8 +318,8 @@ enum { SCAN_EPI_NONE = 0, SCAN_EPI_HOP_EDGES = 1, SCAN_EPI_HOP_NODES = 2 };
 int cache_build_static(Server *s, int64_t capacity_rows, int table_kind, bool int8);
 int cache_build_lru(Server *s, int64_t n_sets, int32_t ways);
 void cache_free(Server *s);
-// The lookup as a kernel of its own: operator by operator, and for the LRU cache, whose lookup has to wait for the
-// insertion of the batch before.  Extra blocks of it finish a hop left pending (launch_hop, defer_fill).  (Finishing
+// The lookup as a kernel of its own: operator by operator, and for the LRU cache where its lookup has to wait for the
+// insertion of the batch before on another stream.  Extra blocks of it finish a hop left pending (launch_hop, defer_fill).  (Finishing
 // it on the side stream instead, ahead of the host-link gather, measured 2 % slower.)
 int launch_lookup(Server *s, Pipe *const *pp, int n, hipStream_t st, int seg_first, int seg_last, bool with_list = true);
 int launch_hotness(Server *s, Pipe &p, hipStream_t st);

@@ -188,6 +188,41 @@ __device__ __forceinline__ int32_t static_find(const SlotTable &t, int32_t id) {
   return table_find(t.slots, t.log2cap, id);
 }
 
+// The dynamic cache.  A set's record is its keys followed by its ticks (one 64-byte line for 8 ways), so the tick of a
+// hit is written into the line its key was just read from.
+struct LruSets {
+  const int32_t *keys;  // first record
+  int32_t *use;         // its ticks
+  int32_t *head;        // first row of each set's list of misses, -1: none
+  int64_t sets;
+  int ways;
+};
+// Slot of `id` or -1; a hit is marked as used at `tick`.
+__device__ __forceinline__ int32_t lru_find(const LruSets &t, int32_t id, int32_t tick) {
+  const int set = (int)((uint32_t)id % (uint32_t)t.sets);
+  const int64_t rec = (int64_t)set * 2 * t.ways;
+  int way = -1;
+  if ((t.ways & 3) == 0) {  // a set's keys start on a 16-byte boundary: four ways per load
+    for (int w = 0; w < t.ways; w += 4) {
+      const int4 k = *reinterpret_cast<const int4 *>(t.keys + rec + w);
+      if (k.x == id) way = w;
+      if (k.y == id) way = w + 1;
+      if (k.z == id) way = w + 2;
+      if (k.w == id) way = w + 3;
+    }
+  } else {
+    for (int w = 0; w < t.ways; ++w)
+      if (t.keys[rec + w] == id) way = w;
+  }
+  if (way < 0) return -1;
+  t.use[rec + way] = tick;
+  return set * t.ways + way;  // sets * ways < 2^31
+}
+// Puts a miss on its set's list.
+__device__ __forceinline__ void lru_chain(const LruSets &t, int32_t *next, int row, int32_t id) {
+  next[row] = atomicExch(&t.head[(uint32_t)id % (uint32_t)t.sets], row);
+}
+
 // Last step of a hop: the local id of every edge source is the value its table slot
 // holds once the hop's first occurrences have published theirs.  Strided over the
 // `n_threads` threads that take part, `tid` being this thread's place among them.

@@ -45,6 +45,7 @@ struct HopShared {  // what the pipes of a launch have in common
   // cache lookup of the nodes the hop adds (hop_flag_scan)
   int look_mode, miss_seg;
   SlotTable cache;
+  LruSets lru;  // LOOK_LRU
 };
 struct HopArgs {
   DevState *st;
@@ -58,6 +59,7 @@ struct HopArgs {
   BatchParams bp;   // HopShared::begin
   int32_t *cache_index;
   int2 *miss_list;
+  int32_t *lru_fill, *lru_next;
 };
 
 // Several mini-batches (pipes) can share every launch of the sampling phase: block b
@@ -477,6 +479,9 @@ static __global__ __launch_bounds__(256) void hop_count_sample_kernel(HopGroup g
 // node's place after the n_prev known nodes: the edge appends the node to ids[] and
 // publishes the local id in the table.  Publishing while other tiles still read is safe: a
 // later edge of the same node compares the value with its own, larger, index either way.
+__device__ __forceinline__ int32_t hop_lookup(const HopGroup &g, const HopArgs &a, int32_t id) {
+  return g.c.look_mode == LOOK_LRU ? lru_find(g.c.lru, id, a.st->lru_tick) : static_find(g.c.cache, id);
+}
 template <int ITEMS>
 static __global__ __launch_bounds__(kScanBlock) void hop_flag_scan_kernel(HopGroup g) {
   LMI_GRID_ROW(g.n);
@@ -498,7 +503,7 @@ static __global__ __launch_bounds__(kScanBlock) void hop_flag_scan_kernel(HopGro
       node[0] = a.ids[i];
       local[0] = i;
       look[0] = true;
-      if (look_mode != LOOK_NOT && node[0] >= 0 && node[0] < g.c.n_nodes) slot_of[0] = static_find(g.c.cache, node[0]);
+      if (look_mode != LOOK_NOT && node[0] >= 0 && node[0] < g.c.n_nodes) slot_of[0] = hop_lookup(g, a, node[0]);
     }
   } else {
     const FaultTo fault = fault_to(st);
@@ -535,7 +540,7 @@ static __global__ __launch_bounds__(kScanBlock) void hop_flag_scan_kernel(HopGro
     for (int j = 0; j < ITEMS; ++j) {
       look[j] = v[j] != 0;
       if (look_mode != LOOK_NOT && look[j] && node[j] >= 0 && node[j] < g.c.n_nodes)
-        slot_of[j] = static_find(g.c.cache, node[j]);
+        slot_of[j] = hop_lookup(g, a, node[j]);
     }
     const int prefix = scan_tile_prefix(a.chain_edges, tile, total, &s_prefix, st, fault);
     if (prefix == kScanFaultPrefix) return;  // the whole block: no ranks, no writes
@@ -565,7 +570,18 @@ static __global__ __launch_bounds__(kScanBlock) void hop_flag_scan_kernel(HopGro
     look[j] = look[j] && slot_of[j] < 0 && node[j] >= 0 && node[j] < g.c.n_nodes;  // from here on: a miss
     misses += look[j] ? 1 : 0;
   }
-  if (look_mode == LOOK_LIST) {  // one atomic per block: one per wavefront on the same counter costs 24 ns each
+  if (look_mode == LOOK_LRU) {
+#pragma unroll
+    for (int j = 0; j < ITEMS; ++j) {
+      if (!look[j]) continue;
+      // a repeated seed keeps both rows, but the id is offered for insertion once, by its first row
+      const bool repeat = bx >= g.c.tile_blocks &&
+                          table_find(a.slots, g.c.log2cap, node[j], st->table_tag, st->table_mask) != local[j];
+      a.lru_fill[local[j]] = repeat ? -2 : -1;
+      if (!repeat) lru_chain(g.c.lru, a.lru_next, local[j], node[j]);
+    }
+  }
+  if (look_mode >= LOOK_LIST) {  // one atomic per block: one per wavefront on the same counter costs 24 ns each
     int total;
     int at = block_exclusive_scan<kScanBlock>(misses, lds, total);
     if (total == 0) return;
@@ -590,6 +606,8 @@ SlotTable slot_table(const Server *s) {
   return SlotTable{s->cache_kind == LMI_CACHE_NONE ? -1 : s->table_kind, s->id_table.slots, s->id_table.log2cap, s->slot_of,
                    s->rank_tab};
 }
+
+LruSets lru_sets(const Server *s) { return LruSets{s->lru_keys, s->lru_use, s->lru_head, s->lru_sets, s->lru_ways}; }
 
 static ScanChain chain_of(const Pipe &p, int which) { return ScanChain{p.chain_status[which]}; }
 
@@ -676,6 +694,7 @@ int launch_hop(Server *s, Pipe *const *pp, int n, hipStream_t st, int hop, bool 
   g.c.look_mode = look.mode;
   g.c.miss_seg = look.miss_seg;
   g.c.cache = slot_table(s);
+  g.c.lru = lru_sets(s);
   for (int k = 0; k < n; ++k) {
     Pipe &p = *pp[k];
     HopArgs &a = g.p[k];
@@ -692,6 +711,9 @@ int launch_hop(Server *s, Pipe *const *pp, int n, hipStream_t st, int hop, bool 
     a.fill.hop = -1;
     a.cache_index = p.cache_index;
     a.miss_list = p.miss_list + miss_list_base(s, look.miss_seg);
+    a.lru_fill = p.lru_fill;
+    a.lru_next = p.lru_next;
+    if (look.mode == LOOK_LRU) p.lru_chained = true;
     if (begin) {
       a.bp = begin[k];
       p.n_seeds = begin[k].n_seeds;

@@ -1,0 +1,50 @@
+"""The LRU cache where its lookup rides in the flag scans (batches taken in order on one stream), beside its lookup as a
+launch of its own (batches in flight, another stream, profiled): every mixture leaves the oracle's cache."""
+import numpy as np
+import pytest
+
+from conftest import random_graph
+from test_gpu_parity import assert_batch_equal, make_features
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("ways", [3, 8])
+@pytest.mark.parametrize("fanout", [[12, 6], [5, 4, 3]])
+def test_lookups_in_flag_scans_and_alone_mixed(lmi, oracle, ways, fanout):
+    rng = np.random.default_rng(ways)
+    n_nodes, batch, dim, sets = 20_000, 400, 100, 150
+    indptr, indices = random_graph(rng, n_nodes, 12, hubs=3, hub_deg=900)
+    feats = make_features(lmi, rng, n_nodes, dim)
+    host_rows = feats.array.view(np.uint8).reshape(n_nodes, dim * 4)
+    srv = lmi.Server(batch, fanout, dim, pipes=2, seed=3)
+    streams = [lmi.stream_create(), lmi.stream_create()]
+    cache = oracle.Lru(sets, ways, dim * 4)
+    try:
+        srv.load_graph(indptr, indices)
+        srv.attach_features(feats)
+        srv.build_lru_cache(sets, ways)
+        for it in range(12):
+            seeds = rng.integers(0, n_nodes, batch if it % 3 else 65).astype(np.int32)   # repeated ones among them
+            seeds[1] = seeds[0]
+            stream, pipe = streams[it // 5 % 2], it % 2
+            if it == 7:
+                srv.profile_enable(1)
+            if it == 9:
+                srv.profile_enable(0)
+            srv.run_once(seeds, rng_seed=it + 1, pipe=pipe, stream=stream)
+            o = oracle.sample_batch(indptr, indices, seeds, fanout, it + 1)
+            hit = cache.access(o.ids, host_rows)[0]
+            if it in (3, 4):
+                continue   # not taken before the next batch is issued
+            g = srv.fetch(pipe=pipe, stream=stream)
+            assert_batch_equal(g, o)
+            np.testing.assert_array_equal(g.cache_index, hit)
+            assert g.features.tobytes() == feats.array[o.ids].tobytes()
+        keys, use = srv.cache_dump(sets * ways, with_aux=True)
+        want = cache.state()
+        np.testing.assert_array_equal(keys.ravel(), want[0].ravel())
+        np.testing.assert_array_equal(use.ravel(), want[1].ravel())
+    finally:
+        srv.close()
+        feats.free()
