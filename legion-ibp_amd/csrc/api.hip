@@ -827,8 +827,12 @@ int lmi_op_cache_lookup(lmi_server *h, int pipe, void *stream, int segment) {
   prof_phase(s, st, &s->prof_open, PROF_LOOKUP);
   Pipe *pp[1] = {&p};
   const bool lists = s->cache_kind == LMI_CACHE_LRU || !gather_in_line(s, pp, 1, segment) || !one_pass_gather(s);
-  LMI_TRY(launch_lookup(s, pp, 1, st, segment, segment, lists));
-  LMI_TRY(launch_gather_seg(s, p, st, segment, segment, 0));
+  if (!lists && lookup_rides_in_gather(s)) {
+    LMI_TRY(launch_lookup_gather(s, p, st, segment));
+  } else {
+    LMI_TRY(launch_lookup(s, pp, 1, st, segment, segment, lists));
+    LMI_TRY(launch_gather_seg(s, p, st, segment, segment, 0));
+  }
   prof_phase(s, st, &s->prof_open, -1);
   return LMI_OK;
 }

@@ -38,6 +38,7 @@ struct MoveRow {
   const int2 *list;
   const int32_t *first_ptr, *n_ptr, *src_index, *dst_index;
   const int32_t *ids;  // gather_rows_flat_kernel<.., MISSES>: node id per row
+  int32_t *look_index; // gather_rows_flat_kernel<.., LOOK>: receives the slot per row
   uint8_t *dst;
   // the HBM gathers of a batch carry its last steps (MoveGroup::tail_blocks)
   FillArgs fill;        // last hop's local ids (hop -1: already there)
@@ -279,15 +280,19 @@ static __global__ __launch_bounds__(256) void move_rows_tiled_kernel(
 // MISSES: a row without a slot is read from the feature table by its node id in the same pass (gather_in_line says
 // when).  The table may lie behind the host link: the wavefronts that hold such rows then wait for the link, which
 // bounds the launch, while the hits of all others stream past.
+// LOOK: the slots are not known yet: a block looks its tile's rows up first, a thread each, and hands the slots to the
+// others through LDS.  One read in a row more per tile instead of a launch and a pass over the ids.
 // rows_seen (pinned host memory, or null): the launch leaves each pipe's row count there for the host
 // to size later grids by (see launch_gather_flat).
-template <typename V16, int U, bool NT, bool MISSES>
+constexpr int kFlatTileMax = 256;  // rows per tile
+template <typename V16, int U, bool NT, bool MISSES, bool LOOK>
 static __global__ __launch_bounds__(256) void gather_rows_flat_kernel(MoveGroup g, const uint8_t *__restrict__ src,
                                                                       uint32_t n_src, const uint8_t *__restrict__ table,
                                                                       uint32_t n_table, int upr, int last_off,
                                                                       int rows_per_tile, int64_t src_pitch,
                                                                       int64_t dst_pitch, unsigned long long *row_counter,
-                                                                      int32_t *rows_seen) {
+                                                                      int32_t *rows_seen, SlotTable look) {
+  __shared__ int s_slot[LOOK ? kFlatTileMax : 1];
   LMI_GRID_ROW_TAIL(g);
   const MoveRow &r = g.p[row];
   const int32_t *__restrict__ src_index = r.src_index;
@@ -306,6 +311,16 @@ static __global__ __launch_bounds__(256) void gather_rows_flat_kernel(MoveGroup 
     const int row0 = first + tile * rows_per_tile;
     const int nr = n - row0 < rows_per_tile ? n - row0 : rows_per_tile;
     const int lim = nr * upr;
+    if constexpr (LOOK) {
+      __syncthreads();  // the tile before is done with its slots
+      if ((int)threadIdx.x < nr) {
+        const int32_t node = ids[row0 + threadIdx.x];
+        const int32_t found = (uint32_t)node < n_table ? static_find(look, node) : -1;
+        s_slot[threadIdx.x] = found;
+        r.look_index[row0 + threadIdx.x] = found;
+      }
+      __syncthreads();
+    }
     int rr = r0, uu = u0;
     for (int f0 = threadIdx.x; f0 < lim; f0 += 256 * U) {
       int slot[U], id[U], off[U];
@@ -316,7 +331,7 @@ static __global__ __launch_bounds__(256) void gather_rows_flat_kernel(MoveGroup 
         const int i = row0 + rr;
         slot[k] = id[k] = -1;
         if (f0 + 256 * k < lim) {
-          slot[k] = src_index[i];
+          slot[k] = LOOK ? s_slot[rr] : src_index[i];
           if (MISSES) id[k] = ids[i];  // beside the slot, not behind it: a miss waits for one read, not for two
         }
         off[k] = (uu == upr - 1) ? last_off : 16 * uu;
@@ -384,6 +399,7 @@ struct MoveArgs {
   int64_t n_src;                    // rows of src (flat gather: indexes at or beyond it move nothing)
   const uint8_t *table;             // flat gather: the feature table rows without a slot are read from, or null
   int64_t n_table;                  // node ids below this have a row there
+  int look;                         // flat gather with a table: look the slots up on the way
   int note_rows;                    // flat gather: the word of rows_seen that receives the row counts (hinted_rows), or -1
   int64_t src_row_bytes, dst_row_bytes, row_bytes;  // row_bytes = bytes moved per row
   int64_t n_max;   // per pipe
@@ -487,24 +503,26 @@ static int launch_gather_flat(Server *s, hipStream_t st, const MoveArgs &a, bool
   const int u_want = s->gather_unroll > 0 ? s->gather_unroll : 2;
   const int U = u_want >= 4 ? 4 : u_want >= 2 ? 2 : 1;
   int rpt = (int)std::max<int64_t>(2, std::min<int64_t>(64, 8192 / a.row_bytes));
-  if (s->gather_tile_rows > 0) rpt = std::min(s->gather_tile_rows, 256);
+  if (s->gather_tile_rows > 0) rpt = std::min(s->gather_tile_rows, kFlatTileMax);
   const int64_t want = ceil_div(a.note_rows >= 0 ? hinted_rows(s, a.n_max, a.note_rows) : a.n_max, rpt);
   const int64_t cap = a.max_blocks > 0 ? a.max_blocks : s->gather_blocks > 0 ? s->gather_blocks : (int64_t)s->n_cu * 64;
   const int grid = (int)std::max<int64_t>(1, std::min(want, cap)) + a.g.tail_blocks;
-#define LMI_FLAT(V_, U_, NT_, M_)                                                                                      \
+  const SlotTable look = slot_table(s);
+#define LMI_FLAT(V_, U_, NT_, M_, L_)                                                                                      \
   if (a.ev_start)                                                                                                      \
-    hipExtLaunchKernelGGL((gather_rows_flat_kernel<V_, U_, NT_, M_>), dim3(grid * a.g.n), dim3(256), 0, st,             \
+    hipExtLaunchKernelGGL((gather_rows_flat_kernel<V_, U_, NT_, M_, L_>), dim3(grid * a.g.n), dim3(256), 0, st,             \
                           a.ev_start, a.ev_stop, 0, a.g, a.src, (uint32_t)a.n_src, a.table, (uint32_t)a.n_table, upr,   \
-                          last_off, rpt, a.src_row_bytes, a.dst_row_bytes, a.row_counter, a.note_rows >= 0 ? s->rows_seen_dev + a.note_rows : nullptr); \
+                          last_off, rpt, a.src_row_bytes, a.dst_row_bytes, a.row_counter, a.note_rows >= 0 ? s->rows_seen_dev + a.note_rows : nullptr, look); \
   else                                                                                                                 \
-    hipLaunchKernelGGL((gather_rows_flat_kernel<V_, U_, NT_, M_>), dim3(grid * a.g.n), dim3(256), 0, st, a.g, a.src,    \
+    hipLaunchKernelGGL((gather_rows_flat_kernel<V_, U_, NT_, M_, L_>), dim3(grid * a.g.n), dim3(256), 0, st, a.g, a.src,    \
                        (uint32_t)a.n_src, a.table, (uint32_t)a.n_table, upr, last_off, rpt, a.src_row_bytes,           \
-                       a.dst_row_bytes, a.row_counter, a.note_rows >= 0 ? s->rows_seen_dev + a.note_rows : nullptr)
+                       a.dst_row_bytes, a.row_counter, a.note_rows >= 0 ? s->rows_seen_dev + a.note_rows : nullptr, look)
 #define LMI_FLAT_U(V_, NT_)                        \
-  if (a.table) { LMI_FLAT(V_, 2, NT_, true); }       \
-  else if (U == 4) { LMI_FLAT(V_, 4, NT_, false); } \
-  else if (U == 2) { LMI_FLAT(V_, 2, NT_, false); } \
-  else { LMI_FLAT(V_, 1, NT_, false); }
+  if (a.look) { LMI_FLAT(V_, 2, NT_, true, true); }         \
+  else if (a.table) { LMI_FLAT(V_, 2, NT_, true, false); }  \
+  else if (U == 4) { LMI_FLAT(V_, 4, NT_, false, false); } \
+  else if (U == 2) { LMI_FLAT(V_, 2, NT_, false, false); } \
+  else { LMI_FLAT(V_, 1, NT_, false, false); }
   if (aligned16 && nt) { LMI_FLAT_U(u32x4, true) }
   else if (aligned16) { LMI_FLAT_U(u32x4, false) }
   else if (nt) { LMI_FLAT_U(u32x4_a4, true) }
@@ -1126,7 +1144,7 @@ static int launch_batch_tail(Server *s, Pipe *const *pp, int n, hipStream_t st, 
 // Gather of rows [first, last) on stream `st`, for all n pipes in one launch: the cache hits from HBM, and with
 // `misses` the other rows from the feature table in the same pass (only where gather_in_line allows it).
 static int launch_hits(Server *s, Pipe *const *pp, int n, hipStream_t st, int seg, int seg_last, bool misses = false,
-                       const HeaderCopy *headers = nullptr) {
+                       const HeaderCopy *headers = nullptr, bool look = false) {
   LMI_TRY(lru_wait_copied(s, st));
   // what is left of the batch rides in the flat and the tiled int8 gather; a profiled gather is timed by itself
   const bool carries = !s->prof_on && (s->cache_kind == LMI_CACHE_INT8
@@ -1146,6 +1164,7 @@ static int launch_hits(Server *s, Pipe *const *pp, int n, hipStream_t st, int se
     r.n_ptr = &p.st->node_counter[9 + seg_last];
     r.src_index = have_cache ? p.cache_index : p.ids;
     r.ids = p.ids;
+    r.look_index = p.cache_index;
     r.dst = (uint8_t *)p.features;
     r.fill.hop = -1;
   }
@@ -1156,6 +1175,7 @@ static int launch_hits(Server *s, Pipe *const *pp, int n, hipStream_t st, int se
   if (misses && have_cache) {
     m.table = s->feat;
     m.n_table = s->n_nodes;
+    m.look = look ? 1 : 0;
   }
   m.note_rows = rows_word(s, seg, seg_last);
   m.src_row_bytes = m.dst_row_bytes = m.row_bytes = s->row_bytes;
@@ -1224,6 +1244,16 @@ bool gather_in_line(const Server *s, Pipe *const *pp, int n, int seg_last) {
   for (int k = 0; k < n; ++k)
     if (!pp[k]->taken_in_order) return false;
   return true;
+}
+
+// Lookup and gather of one segment in one launch (operator by operator; gather_in_line and one_pass_gather hold): a static
+// cache with full-width rows.  The operators of a products-shaped batch: 126 us with
+// three lookup launches (and one more at the start of the batch), 109 without.
+bool lookup_rides_in_gather(const Server *s) { return s->cache_kind == LMI_CACHE_STATIC; }
+int launch_lookup_gather(Server *s, Pipe &p, hipStream_t st, int seg) {
+  Pipe *pp[1] = {&p};
+  p.tail_unjoined = true;  // everything is on the caller's stream
+  return launch_hits(s, pp, 1, st, seg, seg, true, nullptr, true);
 }
 
 // Gathers the rows [first, last) of a segment into each pipe's feature buffer:

@@ -325,6 +325,8 @@ int launch_lookup(Server *s, Pipe *const *pp, int n, hipStream_t st, int seg_fir
 int launch_hotness(Server *s, Pipe &p, hipStream_t st);
 // lru_lists > 0: the LRU insertion of that many miss lists follows the gather on the stream the
 // misses were gathered on (the side stream when it is in use), and the caller's stream does not wait.
+bool lookup_rides_in_gather(const Server *s);
+int launch_lookup_gather(Server *s, Pipe &p, hipStream_t st, int seg);
 int launch_gather_seg(Server *s, Pipe &p, hipStream_t st, int seg, int seg_last, int lru_lists);
 // The same for n pipes in step: the HBM gathers one after another, one fork, then the
 // host-link gathers one after another on the side stream.
