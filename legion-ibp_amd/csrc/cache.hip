@@ -1397,48 +1397,85 @@ static __global__ __launch_bounds__(256) void lru_chain_kernel(LruArgs a, LruSet
   }
 }
 
+// Serves the set of the miss `pr` (row, id) if its row is at the head of the set's list; granted(row, slot) for every row
+// that gets a way.
+template <typename F>
+__device__ __forceinline__ void lru_place(const LruArgs &a, int2 pr, int tick, F granted) {
+  const int i = pr.x;
+  const int64_t set = (uint32_t)pr.y % (uint32_t)a.sets;  // sets < 2^31
+  if (a.head[set] != i) return;  // some other row's thread serves this set
+  const int64_t base = set * a.ways;     // the set's first slot (row of the cache)
+  const int64_t rec = set * 2 * a.ways;  // the set's record: keys, then ticks
+  int last = -1;  // the row placed last; the next one is the smallest row above it
+  for (int placed = 0; placed < a.ways; ++placed) {
+    int row = kIntMax;
+    for (int r = i; r != -1; r = a.next[r])
+      if (r > last && r < row) row = r;
+    if (row == kIntMax) break;  // everybody is placed
+    int best = -1, best_use = kIntMax;
+    if ((a.ways & 3) == 0) {  // four ways per load, same order of preference (lowest way wins a tie)
+      for (int w = 0; w < a.ways; w += 4) {
+        const int4 u = *reinterpret_cast<const int4 *>(a.use + rec + w);
+        if (u.x < tick && u.x < best_use) best = w, best_use = u.x;
+        if (u.y < tick && u.y < best_use) best = w + 1, best_use = u.y;
+        if (u.z < tick && u.z < best_use) best = w + 2, best_use = u.z;
+        if (u.w < tick && u.w < best_use) best = w + 3, best_use = u.w;
+      }
+    } else {
+      for (int w = 0; w < a.ways; ++w) {
+        const int u = a.use[rec + w];
+        if (u < tick && u < best_use) best = w, best_use = u;
+      }
+    }
+    if (best < 0) break;  // every way was touched in this batch
+    a.keys[rec + best] = a.ids[row];
+    a.use[rec + best] = tick;
+    a.fill[row] = (int)(base + best);
+    granted(row, (int)(base + best));
+    last = row;
+  }
+  for (int r = i; r != -1; r = a.next[r])
+    if (a.fill[r] == -1) a.fill[r] = -2;  // no way left for these
+  a.head[set] = -1;  // ready for the next batch
+}
+
 static __global__ __launch_bounds__(256) void lru_place_kernel(LruArgs a) {
   const int tick = a.st->lru_tick;
   for (int l = 0; l < a.n_lists; ++l) {
     const int n = a.st->n_miss[l];
-    for (int j = blockIdx.x * blockDim.x + threadIdx.x; j < n; j += gridDim.x * blockDim.x) {
-      const int2 pr = a.miss_list[l][j];  // (row, id)
-      const int i = pr.x;
-      const int64_t set = (uint32_t)pr.y % (uint32_t)a.sets;  // sets < 2^31
-      if (a.head[set] != i) continue;  // some other row's thread serves this set
-      const int64_t base = set * a.ways;     // the set's first slot (row of the cache)
-      const int64_t rec = set * 2 * a.ways;  // the set's record: keys, then ticks
-      int last = -1;  // the row placed last; the next one is the smallest row above it
-      for (int placed = 0; placed < a.ways; ++placed) {
-        int row = kIntMax;
-        for (int r = i; r != -1; r = a.next[r])
-          if (r > last && r < row) row = r;
-        if (row == kIntMax) break;  // everybody is placed
-        int best = -1, best_use = kIntMax;
-        if ((a.ways & 3) == 0) {  // four ways per load, same order of preference (lowest way wins a tie)
-          for (int w = 0; w < a.ways; w += 4) {
-            const int4 u = *reinterpret_cast<const int4 *>(a.use + rec + w);
-            if (u.x < tick && u.x < best_use) best = w, best_use = u.x;
-            if (u.y < tick && u.y < best_use) best = w + 1, best_use = u.y;
-            if (u.z < tick && u.z < best_use) best = w + 2, best_use = u.z;
-            if (u.w < tick && u.w < best_use) best = w + 3, best_use = u.w;
-          }
-        } else {
-          for (int w = 0; w < a.ways; ++w) {
-            const int u = a.use[rec + w];
-            if (u < tick && u < best_use) best = w, best_use = u;
-          }
-        }
-        if (best < 0) break;  // every way was touched in this batch
-        a.keys[rec + best] = a.ids[row];
-        a.use[rec + best] = tick;
-        a.fill[row] = (int)(base + best);
-        last = row;
-      }
-      for (int r = i; r != -1; r = a.next[r])
-        if (a.fill[r] == -1) a.fill[r] = -2;  // no way left for these
-      a.head[set] = -1;  // ready for the next batch
+    for (int j = blockIdx.x * blockDim.x + threadIdx.x; j < n; j += gridDim.x * blockDim.x)
+      lru_place(a, a.miss_list[l][j], tick, [](int, int) {});
+  }
+}
+
+// Placement and copy in one launch, for an insertion whose end nobody waits for half-way (on the caller's stream): the
+// first kLruTile threads of a block each serve a miss, the block copies the rows they granted (at most 64 ways each).  A
+// tile this small makes some hundred blocks of a few thousand misses, whose serial walks overlap.  Rows of 16 bytes and
+// more, as in gather_rows_flat_kernel.
+constexpr int kLruTile = 32;
+static __global__ __launch_bounds__(256) void lru_place_copy_kernel(LruArgs a, const uint8_t *rows, uint8_t *cache,
+                                                                    int64_t row_bytes) {
+  __shared__ int2 s_row[kLruTile * 64];
+  __shared__ int s_n;
+  const int tick = a.st->lru_tick;
+  const int upr = (int)((row_bytes + 15) / 16);
+  const int n = a.st->n_miss[0];
+  for (int j0 = blockIdx.x * kLruTile; j0 < n; j0 += gridDim.x * kLruTile) {
+    if (threadIdx.x == 0) s_n = 0;
+    __syncthreads();
+    if ((int)threadIdx.x < kLruTile && j0 + (int)threadIdx.x < n)
+      lru_place(a, a.miss_list[0][j0 + threadIdx.x], tick,
+                [&](int row, int slot) { s_row[atomicAdd(&s_n, 1)] = make_int2(row, slot); });
+    __syncthreads();
+    const int units = s_n * upr;
+    for (int f = threadIdx.x; f < units; f += 256) {
+      const int2 r = s_row[f / upr];
+      const int u = f % upr;
+      const int64_t off = u == upr - 1 ? row_bytes - 16 : 16 * u;
+      *reinterpret_cast<u32x4_a4 *>(cache + r.y * row_bytes + off) =
+          *reinterpret_cast<const u32x4_a4 *>(rows + r.x * row_bytes + off);
     }
+    __syncthreads();
   }
 }
 
@@ -1459,6 +1496,17 @@ int launch_lru_insert(Server *s, Pipe &p, hipStream_t st, int n_lists) {
   const int grid = (int)std::max<int64_t>(1, std::min<int64_t>(ceil_div(s->max_nodes, 256), (int64_t)s->n_cu * 4));
   if (!p.lru_chained) hipLaunchKernelGGL(lru_chain_kernel, dim3(grid), dim3(256), 0, st, a, lru_sets(s));
   p.lru_chained = false;
+  if (n_lists == 1 && st != s->side && s->row_bytes >= 16) {
+    const int tiles = (int)std::max<int64_t>(1, std::min<int64_t>(ceil_div(s->max_nodes, kLruTile), (int64_t)s->n_cu * 8));
+    hipExtLaunchKernelGGL(lru_place_copy_kernel, dim3(tiles), dim3(256), 0, st, nullptr, s->lru_ready, 0, a,
+                          (const uint8_t *)p.features, s->cache_data, s->row_bytes);
+    LMI_HIP(hipGetLastError());
+    s->lru_pending = s->lru_copy_pending = true;
+    s->lru_done = s->lru_ready;
+    s->lru_stream = st;
+    return LMI_OK;
+  }
+  s->lru_done = s->lru_copied;
   // The events are the kernels' own completions: recorded behind them they were packets of their own and cost 6 us each.
   // keys and ticks are final: the next batch's lookup may start while the rows are still copied
   hipExtLaunchKernelGGL(lru_place_kernel, dim3(grid), dim3(256), 0, st, nullptr, s->lru_ready, 0, a);
@@ -1502,12 +1550,12 @@ int lru_wait_ready(Server *s, hipStream_t st) {
 // The rows the previous batch's insertion granted must be in the cache before a gather reads it.
 int lru_wait_copied(Server *s, hipStream_t st) {
   if (s->cache_kind != LMI_CACHE_LRU || !s->lru_copy_pending || s->lru_stream == st) return LMI_OK;
-  if (hipEventQuery(s->lru_copied) == hipSuccess) {
+  if (hipEventQuery(s->lru_done) == hipSuccess) {
     s->lru_copy_pending = false;
     return LMI_OK;
   }
   (void)hipGetLastError();
-  LMI_HIP(hipStreamWaitEvent(st, s->lru_copied, 0));
+  LMI_HIP(hipStreamWaitEvent(st, s->lru_done, 0));
   return LMI_OK;
 }
 
@@ -1887,11 +1935,14 @@ int cache_dump(Server *s, int32_t *slot_of, int64_t n, int32_t *aux) {
     return LMI_OK;
   }
   if (n != s->n_nodes) LMI_FAIL(LMI_ERR_ARG, "dump needs n == n_nodes");
-  int32_t *d = nullptr;
-  LMI_HIP(hipMalloc(&d, n * 4));
+  // through the scratch of the build where that was kept
+  const bool kept = s->build_scratch_bytes >= (size_t)n * 4;
+  int32_t *d = (int32_t *)s->build_scratch;
+  if (!kept) LMI_HIP(hipMalloc(&d, n * 4));
   hipLaunchKernelGGL(dump_static_kernel, dim3(s->n_cu * 4), dim3(256), 0, 0, slot_table(s), n, d);
-  LMI_HIP(hipMemcpy(slot_of, d, n * 4, hipMemcpyDeviceToHost));
-  (void)hipFree(d);
+  const hipError_t e = hipMemcpy(slot_of, d, n * 4, hipMemcpyDeviceToHost);
+  if (!kept) (void)hipFree(d);
+  LMI_HIP(e);
   return LMI_OK;
 }
 

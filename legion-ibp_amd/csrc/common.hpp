@@ -207,6 +207,7 @@ struct Server {
   bool lru_pending = false;        // an insertion may still be running
   hipEvent_t lru_copied = nullptr; // recorded when the granted rows are in the cache: the next HBM gather waits for it
   bool lru_copy_pending = false;
+  hipEvent_t lru_done = nullptr;   // the one of the two that the last insertion's rows are behind
   hipStream_t lru_stream = nullptr;  // the stream of the last insertion: it needs no event to be in order
   // sticky fault words in pinned + mapped host memory, written by kernels, never cleared by a batch:
   // [0] a seed id outside [0, n_nodes), [1] a look-back scan gave up
