@@ -391,7 +391,7 @@ def gather_variants(lmi, srv, info, w):
     for mb in (8, 16, 64, 256):
         srv.tune("miss_blocks", mb)
         run("host-link gather on %3d blocks" % mb)
-    srv.tune("miss_blocks", int(own.get("miss_blocks", 32)))
+    srv.tune("miss_blocks", int(own.get("miss_blocks", -1)))
     srv.tune("split_miss", 0)
     run("host-link gather on the caller's stream (no overlap)")
     srv.tune("split_miss", 1)
@@ -595,13 +595,13 @@ def main():
     if args.issue != "runner" and args.runner_steps > 0:
         lmi.check(lmi.lib().lmi_device_sync())
         if "miss_blocks" not in dict(kv.split("=") for kv in args.tune):
-            srv.tune("miss_blocks", 32)   # the runner of the host shim sets no knobs: the library's own host-link grid
+            srv.tune("miss_blocks", -1)   # the runner of the host shim sets no knobs: the library's own host-link grid
         r0 = time.perf_counter()
         runner_steps(done, args.runner_steps)
         lmi.check(lmi.lib().lmi_device_sync())
         r1 = time.perf_counter()
         srv.status()
-        srv.tune("miss_blocks", int(tunes.get("miss_blocks", 32)))
+        srv.tune("miss_blocks", int(tunes.get("miss_blocks", -1)))
         runner = dict(batches_s=round(args.runner_steps / (r1 - r0), 2), steps=args.runner_steps,
                       what="one lmi_run_once per batch on 2 pipes, the library's default host-link grid; before batch i+1 "
                            "is issued the host waits for batch i-1 to be complete (GPURunner::RunOnce with the hand-off "

@@ -1202,7 +1202,8 @@ static int launch_misses(Server *s, Pipe *const *pp, int n, hipStream_t st, int 
   m.src_row_bytes = m.dst_row_bytes = m.row_bytes = s->row_bytes;
   m.n_max = s->node_cap[seg_last];
   if (s->feat_loc == LMI_LOC_HOST) {
-    const int blocks = blocks_override > 0 ? blocks_override : s->miss_blocks > 0 ? s->miss_blocks : s->n_cu;
+    const int usual = s->miss_blocks >= 0 ? s->miss_blocks : n >= 4 ? 40 : 32;
+    const int blocks = blocks_override > 0 ? blocks_override : usual > 0 ? usual : s->n_cu;
     m.max_blocks = std::max(1, (blocks + n - 1) / n);  // per pipe
     m.unroll = s->miss_unroll;
     m.host_link = 1;

@@ -248,8 +248,11 @@ struct Server {
   int use_graph = 0;      // 1: lmi_run_once replays a captured HIP graph of the sampling kernels (measured
                           // 2-3 % slower than plain launches here: the host enqueues a batch in 85 us,
                           // well inside its 205 us of device time, and a graph's end costs 9 us)
-  int miss_blocks = 32;   // grid of the host-link gather: enough reads in flight to fill the link, few enough
-                          // not to crowd HBM traffic out of the memory pipeline
+  int miss_blocks = -1;   // grid of the host-link gather: enough reads in flight to fill the link, few enough
+                          // not to crowd HBM traffic out of the memory pipeline.  -1: 32, and 40 for groups of four and
+                          // more batches, which wait for the link (us per group on 32 / 40 / 48 / 64 blocks: six
+                          // papers100M-shaped batches 504 / 497 / 498 / 532, four MAG240M-shaped int8 328 / 317 / 316 /
+                          // 323, two products-shaped 147 / 156 / 161 / 176); 0: one per CU
   int miss_unroll = 1;    // rows in flight per lane in the host-link gather
   // profiling
   bool prof_on = false;                 // the batch being issued is profiled (events + device row counters)
