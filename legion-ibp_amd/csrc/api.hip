@@ -166,8 +166,10 @@ static int pipe_alloc(Server *s, Pipe &p) {
   LMI_TRY(dmalloc(&p.eslot[0], s->max_edges_hop));
   LMI_TRY(dmalloc(&p.eslot[1], s->max_edges_hop));
   p.max_tiles = scan_max_tiles(s);
-  LMI_TRY(dmalloc(&p.chain_status[0], p.max_tiles));
-  LMI_TRY(dmalloc(&p.chain_status[1], p.max_tiles));
+  for (auto &chain : p.chain_status) {
+    LMI_TRY(dmalloc(&chain, p.max_tiles));
+    LMI_HIP(hipMemset(chain, 0, (size_t)p.max_tiles * sizeof(*chain)));  // no tile has announced a sum
+  }
   LMI_TRY(dmalloc(&p.miss_list, s->max_nodes));
   LMI_TRY(dmalloc(&p.lru_fill, s->max_nodes));
   LMI_TRY(dmalloc(&p.lru_next, s->max_nodes));
@@ -176,6 +178,7 @@ static int pipe_alloc(Server *s, Pipe &p) {
   LMI_HIP(hipEventCreateWithFlags(&p.fork_early, hipEventDisableTiming));
   LMI_HIP(hipEventCreateWithFlags(&p.join, hipEventDisableTiming));
   LMI_HIP(hipEventCreateWithFlags(&p.handover, hipEventDisableTiming));
+  LMI_HIP(hipStreamSynchronize(nullptr));  // the fills above: a caller's stream does not wait for the null stream
   return LMI_OK;
 }
 
@@ -716,7 +719,15 @@ static int ready(Server *s) {
   return LMI_OK;
 }
 
-// Resolves where this batch's seeds live and the per-batch scalars.
+// Bits of a dedup-table key that a node id takes.
+static int table_id_bits(const Server *s) {
+  int id_bits = 1;
+  while (id_bits < 31 && (int64_t(1) << id_bits) < s->n_nodes) ++id_bits;
+  return id_bits;
+}
+
+// Resolves where this batch's seeds live and the per-batch scalars.  Leaves the pipe and the server as they are: the call
+// may still be refused for another batch of its group (batch_taken settles what changes).
 static int batch_params(Server *s, Pipe &p, hipStream_t st, const int32_t *seeds, int32_t n, int seeds_location,
                         int32_t batch_counter, int mode, uint64_t rng_seed, BatchParams *bp) {
   LMI_TRY(ready(s));
@@ -742,27 +753,34 @@ static int batch_params(Server *s, Pipe &p, hipStream_t st, const int32_t *seeds
   bp->n_seeds = n;
   // dedup-table epoch: keys carry it in the bits above the widest node id, so the table is
   // wiped only when the epochs run out (or it is new, or the id width changed)
-  int id_bits = 1;
-  while (id_bits < 31 && (int64_t(1) << id_bits) < s->n_nodes) ++id_bits;
+  const int id_bits = table_id_bits(s);
   const int32_t max_epoch = (int32_t)std::min<int64_t>((int64_t(1) << (31 - id_bits)) - 1, s->table_epochs);  // 0: wipe every batch
-  if (p.table_dirty || p.epoch >= max_epoch || p.id_bits != id_bits) {
-    p.epoch = 0;
-    bp->clear_table = 1;
-  } else {
-    ++p.epoch;
-    bp->clear_table = 0;
-  }
-  p.table_dirty = false;
-  p.id_bits = id_bits;
-  bp->table_tag = max_epoch > 0 ? (int32_t)((uint32_t)p.epoch << id_bits) : 0;
+  bp->clear_table = p.table_dirty || p.epoch >= max_epoch || p.id_bits != id_bits ? 1 : 0;
+  const int32_t epoch = bp->clear_table ? 0 : p.epoch + 1;
+  bp->table_tag = max_epoch > 0 ? (int32_t)((uint32_t)epoch << id_bits) : 0;
   bp->table_mask = max_epoch > 0 ? (int32_t)(0xFFFFFFFFu << id_bits) : kUntaggedMask;
   bp->fault = s->fault_dev;
-  p.serial = p.serial == INT32_MAX ? 1 : p.serial + 1;
-  bp->serial = p.serial;
+  bp->serial = p.serial == INT32_MAX ? 1 : p.serial + 1;
   bp->rng_seed = rng_seed ? rng_seed : s->cfg.seed + (uint64_t)(uint32_t)batch_counter;
-  if (s->cache_kind == LMI_CACHE_LRU) ++s->lru_tick;
-  bp->lru_tick = s->lru_tick;
+  bp->lru_tick = s->lru_tick + (s->cache_kind == LMI_CACHE_LRU ? 1 : 0);
   return LMI_OK;
+}
+
+// The batches of a call that nothing refuses any more: their pipes move on to them.
+static void batch_taken(Server *s, Pipe *const *pp, const BatchParams *bps, int n) {
+  for (int k = 0; k < n; ++k) {
+    Pipe &p = *pp[k];
+    p.epoch = bps[k].clear_table ? 0 : p.epoch + 1;
+    p.id_bits = table_id_bits(s);
+    p.table_dirty = false;
+    p.serial = bps[k].serial;
+    s->lru_tick = bps[k].lru_tick;
+  }
+}
+// A launch of theirs failed: what it left in the tables and in the scan words is wiped before their next use.
+static int batch_failed(Pipe *const *pp, int n, int rc) {
+  for (int k = 0; k < n && rc != LMI_OK; ++k) pp[k]->table_dirty = true;
+  return rc;
 }
 
 // All hops of a batch on each of n pipes, `early` and `late` the lookups that ride in the first hop and in the later
@@ -790,12 +808,13 @@ int lmi_op_batch_generate(lmi_server *h, int pipe, void *stream, const int32_t *
   hipStream_t st = (hipStream_t)stream;
   BatchParams bp{};
   prof_batch(s);
-  single_issued(s, pipe);
   LMI_TRY(pipe_join(p, st));
   pipe_begin(p, st);
   LMI_TRY(batch_params(s, p, st, seeds, n, seeds_location, batch_counter, mode, rng_seed, &bp));
+  single_issued(s, pipe);
   Pipe *pp[1] = {&p};
-  return launch_batch_generate(s, pp, &bp, 1, st, true);
+  batch_taken(s, pp, &bp, 1);
+  return batch_failed(pp, 1, launch_batch_generate(s, pp, &bp, 1, st, true));
 }
 
 int lmi_op_random_sample(lmi_server *h, int pipe, void *stream, int hop) {
@@ -856,11 +875,12 @@ int lmi_presample(lmi_server *h, int pipe, void *stream, int mode, int32_t first
     BatchParams bp{};
     LMI_TRY(pipe_join(p, st));
     pipe_begin(p, st);
-    const int tick = s->lru_tick;
     LMI_TRY(batch_params(s, p, st, nullptr, 0, LMI_LOC_DEVICE, b, mode, 0, &bp));
-    s->lru_tick = tick;  // presampling does not age the LRU cache
     Pipe *pp[1] = {&p};
-    LMI_TRY(launch_sampling(s, pp, &bp, 1, st, false, HopLookup{}, HopLookup{}));
+    const int tick = s->lru_tick;
+    batch_taken(s, pp, &bp, 1);
+    s->lru_tick = tick;  // presampling does not age the LRU cache
+    LMI_TRY(batch_failed(pp, 1, launch_sampling(s, pp, &bp, 1, st, false, HopLookup{}, HopLookup{})));
     LMI_TRY(launch_hotness(s, p, st));  // finishes the last hop too
   }
   return LMI_OK;
@@ -920,7 +940,7 @@ static int capture_batch_graph(Server *s, Pipe &p, hipStream_t st, const BatchPa
 
 // One batch on each of n pipes, served by the same launches.
 // The caller has ordered `st` behind the pipes' previous batches (pipes_join) before it staged the seeds.
-static int run_group(Server *s, Pipe *const *pp, const BatchParams *bps, int n, hipStream_t st) {
+static int run_group_launches(Server *s, Pipe *const *pp, const BatchParams *bps, int n, hipStream_t st) {
   for (int k = 0; k < n; ++k) pipe_begin(*pp[k], st);
   prof_phase(s, st, &s->prof_open, PROF_SAMPLE);
   const bool lru = s->cache_kind == LMI_CACHE_LRU;
@@ -954,6 +974,10 @@ static int run_group(Server *s, Pipe *const *pp, const BatchParams *bps, int n, 
   prof_phase(s, st, &s->prof_open, -1);
   return LMI_OK;
 }
+static int run_group(Server *s, Pipe *const *pp, const BatchParams *bps, int n, hipStream_t st) {
+  batch_taken(s, pp, bps, n);
+  return batch_failed(pp, n, run_group_launches(s, pp, bps, n, st));
+}
 
 int lmi_run_once(lmi_server *h, int pipe, void *stream, const int32_t *seeds, int32_t n, int seeds_location,
                  int32_t batch_counter, int mode, uint64_t rng_seed) {
@@ -964,11 +988,11 @@ int lmi_run_once(lmi_server *h, int pipe, void *stream, const int32_t *seeds, in
   hipStream_t st = (hipStream_t)stream;
   BatchParams bp{};
   prof_batch(s);
-  single_issued(s, pipe);
   // a pipe's previous batch may still be gathering misses, or sit on another stream: only behind it may
   // this batch's first command, the copy of host seeds into the pipe's staging buffer, be queued
   LMI_TRY(pipes_join(pp, 1, st));
   LMI_TRY(batch_params(s, *pp[0], st, seeds, n, seeds_location, batch_counter, mode, rng_seed, &bp));
+  single_issued(s, pipe);
   return run_group(s, pp, &bp, 1, st);
 }
 
@@ -991,13 +1015,13 @@ int lmi_run_group(lmi_server *h, int n_batches, const int32_t *pipes, void *stre
     pp[k] = &s->pipes[pipes[k]];
   }
   prof_batch(s, n_batches);
-  s->last_pipe = -1;  // a group is prefetched: its misses overlap the next group's sampling
-  s->last_taken = false;
-  for (int k = 0; k < n_batches; ++k) pp[k]->taken_in_order = false;
   LMI_TRY(pipes_join(pp, n_batches, st));  // before the seeds are staged: see lmi_run_once
   for (int k = 0; k < n_batches; ++k)
     LMI_TRY(batch_params(s, *pp[k], st, seeds ? seeds[k] : nullptr, (seeds && n_seeds) ? n_seeds[k] : 0, seeds_location,
                          batch_counters[k], mode, rng_seeds ? rng_seeds[k] : 0, &bps[k]));
+  s->last_pipe = -1;  // a group is prefetched: its misses overlap the next group's sampling
+  s->last_taken = false;
+  for (int k = 0; k < n_batches; ++k) pp[k]->taken_in_order = false;
   return run_group(s, pp, bps, n_batches, st);
 }
 
