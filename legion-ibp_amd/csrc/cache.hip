@@ -509,7 +509,7 @@ static int launch_gather_flat(Server *s, hipStream_t st, const MoveArgs &a, bool
   const int grid = (int)std::max<int64_t>(1, std::min(want, cap)) + a.g.tail_blocks;
   const SlotTable look = slot_table(s);
 #define LMI_FLAT(V_, U_, NT_, M_, L_)                                                                                      \
-  if (a.ev_start)                                                                                                      \
+  if (a.ev_start || a.ev_stop)                                                                                         \
     hipExtLaunchKernelGGL((gather_rows_flat_kernel<V_, U_, NT_, M_, L_>), dim3(grid * a.g.n), dim3(256), 0, st,             \
                           a.ev_start, a.ev_stop, 0, a.g, a.src, (uint32_t)a.n_src, a.table, (uint32_t)a.n_table, upr,   \
                           last_off, rpt, a.src_row_bytes, a.dst_row_bytes, a.row_counter, a.note_rows >= 0 ? s->rows_seen_dev + a.note_rows : nullptr, look); \
@@ -967,14 +967,24 @@ int launch_lookup(Server *s, Pipe *const *pp, int n, hipStream_t st, int seg_fir
 // wait on another queue's event holds a stream up for about 10 us even when the event fired long
 // ago, so that wait is only queued when the host cannot already see the event as complete.  Work
 // of the batch that `join_of` does not cover sits on the caller's stream that carried the batch:
-// the same stream orders itself, another one is put behind an event recorded there now (at that
-// stream's present tail, which is at or behind the batch's last kernel).
+// the same stream orders itself.  Another one waits for the batch's own end where that was marked
+// (tail_event), so that it does not wait for batches queued behind it and does not need that stream
+// any more; else, as between operators, for an event recorded there now (at that stream's present
+// tail, which is at or behind the batch's last kernel).
 int pipe_handover(Pipe &p, hipStream_t st) {
-  if (p.tail_unjoined && p.last_stream != st && p.handover) {
+  if (!p.tail_unjoined || p.last_stream == st || !p.handover) return LMI_OK;
+  if (p.tail_event) {
+    if (hipEventQuery(p.tail_event) == hipSuccess) {
+      p.tail_unjoined = false;
+      return LMI_OK;
+    }
+    (void)hipGetLastError();
+    LMI_HIP(hipStreamWaitEvent(st, p.tail_event, 0));
+  } else {
     LMI_HIP(hipEventRecord(p.handover, p.last_stream));
     LMI_HIP(hipStreamWaitEvent(st, p.handover, 0));
-    p.last_stream = st;  // `st` now carries the order
   }
+  p.last_stream = st;  // `st` now carries the order
   return LMI_OK;
 }
 
@@ -1025,7 +1035,7 @@ int pipes_join(Pipe *const *pp, int n, hipStream_t st) {
 }
 
 // int8 rows: dequantised inside the gather.
-static int launch_hits_int8(Server *s, const MoveGroup &g, hipStream_t st, int seg, int seg_last) {
+static int launch_hits_int8(Server *s, const MoveGroup &g, hipStream_t st, int seg, int seg_last, hipEvent_t end) {
   const int64_t n_max = s->node_cap[seg_last];
   const int dim = s->cfg.feat_dim;
   const int64_t want = ceil_div(n_max, 4);
@@ -1035,8 +1045,9 @@ static int launch_hits_int8(Server *s, const MoveGroup &g, hipStream_t st, int s
   unsigned long long *rc = s->prof_on ? s->d_prof_rows : nullptr;
   hipEvent_t e0, e1;
   prof_kernel_events(s, PROF_GATHER_HIT, &e0, &e1);
+  if (end) e1 = end;
 #define LMI_INT8(KERN)                                                                                   \
-  if (e0)                                                                                                \
+  if (e0 || e1)                                                                                          \
     hipExtLaunchKernelGGL((KERN), dim3(grid), dim3(256), 0, st, e0, e1, 0, g, q, s->cache_scale, dim, rc); \
   else                                                                                                   \
     hipLaunchKernelGGL((KERN), dim3(grid), dim3(256), 0, st, g, q, s->cache_scale, dim, rc)
@@ -1054,7 +1065,7 @@ static int launch_hits_int8(Server *s, const MoveGroup &g, hipStream_t st, int s
                           : s->gather_adaptive ? (int64_t)s->n_cu * 64 : auto_gather_blocks(s, want_f);
     const int grid_f = g.n * ((int)std::max<int64_t>(1, std::min<int64_t>(want_f, cap_f)) + g.tail_blocks);
 #define LMI_INT8_FLAT(KERN)                                                                                   \
-  if (e0)                                                                                                     \
+  if (e0 || e1)                                                                                               \
     hipExtLaunchKernelGGL((KERN), dim3(grid_f), dim3(256), 0, st, e0, e1, 0, g, q, s->cache_scale, dim,        \
                           tile_rows, rc, s->rows_seen_dev + rows_word(s, seg, seg_last));                      \
   else                                                                                                        \
@@ -1142,9 +1153,10 @@ static int launch_batch_tail(Server *s, Pipe *const *pp, int n, hipStream_t st, 
 }
 
 // Gather of rows [first, last) on stream `st`, for all n pipes in one launch: the cache hits from HBM, and with
-// `misses` the other rows from the feature table in the same pass (only where gather_in_line allows it).
+// `misses` the other rows from the feature table in the same pass (only where gather_in_line allows it).  end: an event
+// that marks the end of the launch (not with a profiled gather, which carries events of its own).
 static int launch_hits(Server *s, Pipe *const *pp, int n, hipStream_t st, int seg, int seg_last, bool misses = false,
-                       const HeaderCopy *headers = nullptr, bool look = false) {
+                       const HeaderCopy *headers = nullptr, bool look = false, hipEvent_t end = nullptr) {
   LMI_TRY(lru_wait_copied(s, st));
   // what is left of the batch rides in the flat and the tiled int8 gather; a profiled gather is timed by itself
   const bool carries = !s->prof_on && (s->cache_kind == LMI_CACHE_INT8
@@ -1169,7 +1181,7 @@ static int launch_hits(Server *s, Pipe *const *pp, int n, hipStream_t st, int se
     r.fill.hop = -1;
   }
   if (carries) tail_args(s, pp, n, headers, &m.g);
-  if (s->cache_kind == LMI_CACHE_INT8) return launch_hits_int8(s, m.g, st, seg, seg_last);
+  if (s->cache_kind == LMI_CACHE_INT8) return launch_hits_int8(s, m.g, st, seg, seg_last, end);
   m.src = have_cache ? s->cache_data : s->feat;
   m.n_src = have_cache ? s->cache_rows : s->n_nodes;
   if (misses && have_cache) {
@@ -1182,13 +1194,15 @@ static int launch_hits(Server *s, Pipe *const *pp, int n, hipStream_t st, int se
   m.n_max = n_max;
   m.row_counter = s->prof_on ? s->d_prof_rows : nullptr;  // all rows of the segment: hits + misses
   prof_kernel_events(s, PROF_GATHER_HIT, &m.ev_start, &m.ev_stop);
+  if (end) m.ev_stop = end;
   return launch_move_rows(s, st, m, s->gather_nt != 0);
 }
 
 // Gather of the rows on the segment's miss list from the feature table, on a
 // small grid when the table sits behind the host link (few bytes in flight fill it).
 // One launch for all n pipes; the small grid is then shared between them.
-static int launch_misses(Server *s, Pipe *const *pp, int n, hipStream_t st, int seg, int seg_last, int blocks_override = 0) {
+static int launch_misses(Server *s, Pipe *const *pp, int n, hipStream_t st, int seg, int seg_last, int blocks_override = 0,
+                         hipEvent_t end = nullptr) {
   MoveArgs m{};
   m.g.n = n;
   for (int k = 0; k < n; ++k) {
@@ -1210,6 +1224,7 @@ static int launch_misses(Server *s, Pipe *const *pp, int n, hipStream_t st, int 
   }
   m.row_counter = s->prof_on ? s->d_prof_rows + 1 : nullptr;  // misses
   prof_kernel_events(s, PROF_GATHER_MISS, &m.ev_start, &m.ev_stop);
+  if (end) m.ev_stop = end;
   return launch_move_rows(s, st, m, s->gather_nt != 0);
 }
 
@@ -1291,15 +1306,24 @@ int launch_gather_group(Server *s, Pipe *const *pp, int n, hipStream_t st, int s
   // left open by the sampling phase ends here.
   prof_phase(s, st, &s->prof_open, -1);
   if (mode == 0) {
-    for (int k = 0; k < n; ++k) pp[k]->tail_unjoined = true;  // everything is on the caller's stream
-    if (one_pass_gather(s)) {
-      LMI_TRY(launch_hits(s, pp, n, st, seg, seg_last, true, headers));
-    } else {
-      if (have_cache) LMI_TRY(launch_hits(s, pp, n, st, seg, seg_last, false, headers));
-      else LMI_TRY(launch_batch_tail(s, pp, n, st, headers));
-      if (!no_miss_possible(s)) LMI_TRY(launch_misses(s, pp, n, st, seg, seg_last));
+    // The batch ends on the caller's stream.  Its last kernel carries the event that says so (for the first pipe's event
+    // all pipes of a group): recorded behind it the event would be a packet of its own, and recorded when another stream
+    // asks it would stand for whatever is queued by then.  Not for a segment: its batch goes on.
+    const bool whole = hit_seg == 0 && seg_last == s->cfg.hops;
+    const hipEvent_t end = whole && !s->prof_on ? pp[0]->handover : nullptr;
+    const bool last_hits = lru_lists == 0 && (one_pass_gather(s) || no_miss_possible(s));
+    for (int k = 0; k < n; ++k) {
+      pp[k]->tail_unjoined = true;
+      pp[k]->tail_event = end;
     }
-    for (int k = 0; k < n && lru_lists > 0; ++k) LMI_TRY(launch_lru_insert(s, *pp[k], st, lru_lists));
+    if (one_pass_gather(s)) {
+      LMI_TRY(launch_hits(s, pp, n, st, seg, seg_last, true, headers, false, last_hits ? end : nullptr));
+    } else {
+      if (have_cache) LMI_TRY(launch_hits(s, pp, n, st, seg, seg_last, false, headers, false, last_hits ? end : nullptr));
+      else LMI_TRY(launch_batch_tail(s, pp, n, st, headers));
+      if (!no_miss_possible(s)) LMI_TRY(launch_misses(s, pp, n, st, seg, seg_last, 0, lru_lists == 0 ? end : nullptr));
+    }
+    for (int k = 0; k < n && lru_lists > 0; ++k) LMI_TRY(launch_lru_insert(s, *pp[k], st, lru_lists, end));
     return LMI_OK;
   }
   hipEvent_t fork = nullptr;
@@ -1480,7 +1504,7 @@ static __global__ __launch_bounds__(256) void lru_place_copy_kernel(LruArgs a, c
   }
 }
 
-int launch_lru_insert(Server *s, Pipe &p, hipStream_t st, int n_lists) {
+int launch_lru_insert(Server *s, Pipe &p, hipStream_t st, int n_lists, hipEvent_t end) {
   if (s->cache_kind != LMI_CACHE_LRU) return LMI_OK;
   LruArgs a{};
   a.ids = p.ids;
@@ -1499,15 +1523,16 @@ int launch_lru_insert(Server *s, Pipe &p, hipStream_t st, int n_lists) {
   p.lru_chained = false;
   if (n_lists == 1 && st != s->side && s->row_bytes >= 16) {
     const int tiles = (int)std::max<int64_t>(1, std::min<int64_t>(ceil_div(s->max_nodes, kLruTile), (int64_t)s->n_cu * 8));
-    hipExtLaunchKernelGGL(lru_place_copy_kernel, dim3(tiles), dim3(256), 0, st, nullptr, s->lru_ready, 0, a,
+    s->lru_keyed = s->lru_done = end ? end : s->lru_ready;
+    hipExtLaunchKernelGGL(lru_place_copy_kernel, dim3(tiles), dim3(256), 0, st, nullptr, s->lru_done, 0, a,
                           (const uint8_t *)p.features, s->cache_data, s->row_bytes);
     LMI_HIP(hipGetLastError());
     s->lru_pending = s->lru_copy_pending = true;
-    s->lru_done = s->lru_ready;
     s->lru_stream = st;
     return LMI_OK;
   }
-  s->lru_done = s->lru_copied;
+  s->lru_keyed = s->lru_ready;
+  s->lru_done = end ? end : s->lru_copied;
   // The events are the kernels' own completions: recorded behind them they were packets of their own and cost 6 us each.
   // keys and ticks are final: the next batch's lookup may start while the rows are still copied
   hipExtLaunchKernelGGL(lru_place_kernel, dim3(grid), dim3(256), 0, st, nullptr, s->lru_ready, 0, a);
@@ -1528,7 +1553,7 @@ int launch_lru_insert(Server *s, Pipe &p, hipStream_t st, int n_lists) {
     r.dst = s->cache_data;
     m.src_row_bytes = m.dst_row_bytes = m.row_bytes = s->row_bytes;
     m.n_max = s->node_cap[s->cfg.hops];
-    if (l == n_lists - 1) m.ev_stop = s->lru_copied;
+    if (l == n_lists - 1) m.ev_stop = s->lru_done;
     LMI_TRY(launch_move_rows(s, st, m, false));
   }
   s->lru_copy_pending = true;
@@ -1539,12 +1564,12 @@ int launch_lru_insert(Server *s, Pipe &p, hipStream_t st, int n_lists) {
 // insertion.  Sampling does not touch the cache, so only the lookup has to wait.
 int lru_wait_ready(Server *s, hipStream_t st) {
   if (s->cache_kind != LMI_CACHE_LRU || !s->lru_pending || s->lru_stream == st) return LMI_OK;  // a stream orders itself
-  if (hipEventQuery(s->lru_ready) == hipSuccess) {
+  if (hipEventQuery(s->lru_keyed) == hipSuccess) {
     s->lru_pending = false;
     return LMI_OK;
   }
   (void)hipGetLastError();  // "not ready" is an answer, not a failure
-  LMI_HIP(hipStreamWaitEvent(st, s->lru_ready, 0));
+  LMI_HIP(hipStreamWaitEvent(st, s->lru_keyed, 0));
   return LMI_OK;
 }
 

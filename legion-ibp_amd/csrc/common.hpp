@@ -117,10 +117,13 @@ struct Pipe {
   // The caller's stream that carried the pipe's last batch, and whether that stream still holds work
   // of the batch that `join_of` does not cover (everything when no side stream is used; the HBM
   // gather when the side stream was released ahead of it).  A later call that uses the pipe from
-  // ANOTHER stream is then ordered behind `last_stream` through `handover` (pipe_join).
+  // ANOTHER stream is then ordered behind that work (pipe_handover): through `tail_event`, the
+  // completion of the batch's last kernel, where the batch ran on that stream to its end, else
+  // through `handover`, recorded on `last_stream` by then.
   hipStream_t last_stream = nullptr;
   bool tail_unjoined = false;
   hipEvent_t handover = nullptr;
+  hipEvent_t tail_event = nullptr;  // the pipe's own `handover`, or that of the first pipe of its group
   bool taken_in_order = false;  // this batch's caller waited for the batch before on that batch's own stream, and only
                                 // then issued this one: its misses have nothing to overlap (gather_in_line)
   int32_t *seed_stage = nullptr;  // [batch_size] host seeds land here
@@ -207,7 +210,8 @@ struct Server {
   bool lru_pending = false;        // an insertion may still be running
   hipEvent_t lru_copied = nullptr; // recorded when the granted rows are in the cache: the next HBM gather waits for it
   bool lru_copy_pending = false;
-  hipEvent_t lru_done = nullptr;   // the one of the two that the last insertion's rows are behind
+  hipEvent_t lru_keyed = nullptr;  // the event of the last insertion that its keys and ticks are behind: lru_ready, or its
+  hipEvent_t lru_done = nullptr;   // batch's tail_event; and the one that its rows are behind: lru_copied, or the same
   hipStream_t lru_stream = nullptr;  // the stream of the last insertion: it needs no event to be in order
   // sticky fault words in pinned + mapped host memory, written by kernels, never cleared by a batch:
   // [0] a seed id outside [0, n_nodes), [1] a look-back scan gave up
@@ -347,7 +351,8 @@ bool gather_in_line(const Server *s, Pipe *const *pp, int n, int seg_last);
 bool one_pass_gather(const Server *s);
 // the host-link gather of segments [seg, seg_last] released now, ahead of the batch's later hops (split_lookup)
 int launch_misses_early(Server *s, Pipe *const *pp, int n, hipStream_t st, int seg, int seg_last);
-int launch_lru_insert(Server *s, Pipe &p, hipStream_t st, int n_lists);
+// end: an event that marks the end of the insertion, or null
+int launch_lru_insert(Server *s, Pipe &p, hipStream_t st, int n_lists, hipEvent_t end = nullptr);
 int lru_wait_ready(Server *s, hipStream_t st);
 int lru_wait_copied(Server *s, hipStream_t st);  // orders `st` behind the last LRU insertion
 int pipe_join(Pipe &p, hipStream_t st);  // make `st` wait for the pipe's last batch, wherever it ran
@@ -356,6 +361,7 @@ int pipe_handover(Pipe &p, hipStream_t st);  // only for what another caller's s
 inline void pipe_begin(Pipe &p, hipStream_t st) {
   p.last_stream = st;
   p.tail_unjoined = true;
+  p.tail_event = nullptr;
 }
 // the same for n pipes, each distinct event waited on once
 int pipes_join(Pipe *const *pp, int n, hipStream_t st);
