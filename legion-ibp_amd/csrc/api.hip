@@ -957,7 +957,8 @@ static int run_group_launches(Server *s, Pipe *const *pp, const BatchParams *bps
   } else {
     // the rows that miss are listed unless hits and misses are gathered in one pass
     const bool in_line = gather_in_line(s, pp, n, s->cfg.hops);
-    // The LRU lookup rides in the flag scans too where the insertion before it is on this stream: a launch for the lookup
+    // The LRU lookup rides in the flag scans too where the insertion before it is on this stream (for all its handle tells:
+    // the wait is queued all the same): a launch for the lookup
     // and one for the lists of misses less (four batches of 1 024 seeds and three hops: 396 us before, 386 with it).
     const bool lru_rides = lru && in_line && (!s->lru_pending || s->lru_stream == st);
     const int mode = lru ? (lru_rides ? LOOK_LRU : LOOK_NOT) : in_line && one_pass_gather(s) ? LOOK_SLOTS : LOOK_LIST;
@@ -966,6 +967,7 @@ static int run_group_launches(Server *s, Pipe *const *pp, const BatchParams *bps
     split = s->split_lookup && s->cfg.hops >= 2 && s->feat_loc == LMI_LOC_HOST && s->split_miss == 1 &&
             (s->cache_kind == LMI_CACHE_STATIC || s->cache_kind == LMI_CACHE_INT8) &&
             (s->split_lookup == 1 || (s->split_lookup == 2 && n > 1)) && !in_line;
+    if (lru_rides) LMI_TRY(lru_wait_ready(s, st));
     LMI_TRY(launch_sampling(s, pp, bps, n, st, false, HopLookup{mode, 0}, HopLookup{mode, split ? 2 : 0}, split));
     if (lru && !lru_rides) {
       LMI_TRY(lru_wait_ready(s, st));  // sampling may overlap the previous batch's insertion, the lookup may not

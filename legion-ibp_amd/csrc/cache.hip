@@ -1561,9 +1561,11 @@ int launch_lru_insert(Server *s, Pipe &p, hipStream_t st, int n_lists, hipEvent_
 }
 
 // The LRU state is batch-synchronous: a lookup sees the cache after the previous batch's
-// insertion.  Sampling does not touch the cache, so only the lookup has to wait.
+// insertion.  Sampling does not touch the cache, so only the lookup has to wait.  The event is asked for also where the
+// insertion ran on a stream of the same handle: that stream may be gone and the handle another stream's by now, and on
+// the stream itself the wait costs nothing.
 int lru_wait_ready(Server *s, hipStream_t st) {
-  if (s->cache_kind != LMI_CACHE_LRU || !s->lru_pending || s->lru_stream == st) return LMI_OK;  // a stream orders itself
+  if (s->cache_kind != LMI_CACHE_LRU || !s->lru_pending) return LMI_OK;
   if (hipEventQuery(s->lru_keyed) == hipSuccess) {
     s->lru_pending = false;
     return LMI_OK;
@@ -1575,7 +1577,7 @@ int lru_wait_ready(Server *s, hipStream_t st) {
 
 // The rows the previous batch's insertion granted must be in the cache before a gather reads it.
 int lru_wait_copied(Server *s, hipStream_t st) {
-  if (s->cache_kind != LMI_CACHE_LRU || !s->lru_copy_pending || s->lru_stream == st) return LMI_OK;
+  if (s->cache_kind != LMI_CACHE_LRU || !s->lru_copy_pending) return LMI_OK;
   if (hipEventQuery(s->lru_done) == hipSuccess) {
     s->lru_copy_pending = false;
     return LMI_OK;

@@ -212,7 +212,7 @@ struct Server {
   bool lru_copy_pending = false;
   hipEvent_t lru_keyed = nullptr;  // the event of the last insertion that its keys and ticks are behind: lru_ready, or its
   hipEvent_t lru_done = nullptr;   // batch's tail_event; and the one that its rows are behind: lru_copied, or the same
-  hipStream_t lru_stream = nullptr;  // the stream of the last insertion: it needs no event to be in order
+  hipStream_t lru_stream = nullptr;  // the stream of the last insertion, to tell whether waiting for it holds anything up
   // sticky fault words in pinned + mapped host memory, written by kernels, never cleared by a batch:
   // [0] a seed id outside [0, n_nodes), [1] a look-back scan gave up
   volatile int32_t *fault_host = nullptr;

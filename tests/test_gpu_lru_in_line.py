@@ -48,3 +48,39 @@ def test_lookups_in_flag_scans_and_alone_mixed(lmi, oracle, ways, fanout):
     finally:
         srv.close()
         feats.free()
+
+
+def test_streams_that_come_and_go_between_batches(lmi, oracle):
+    """Streams destroyed behind their batch, unsynchronised: a new one may get the same handle."""
+    rng = np.random.default_rng(5)
+    n_nodes, batch, dim, sets, ways, fanout = 20_000, 500, 100, 300, 8, [12, 6]
+    indptr, indices = random_graph(rng, n_nodes, 12, hubs=3, hub_deg=900)
+    feats = make_features(lmi, rng, n_nodes, dim)
+    host_rows = feats.array.view(np.uint8).reshape(n_nodes, dim * 4)
+    srv = lmi.Server(batch, fanout, dim, pipes=4, seed=3)
+    cache = oracle.Lru(sets, ways, dim * 4)
+    try:
+        srv.load_graph(indptr, indices)
+        srv.attach_features(feats)
+        srv.build_lru_cache(sets, ways)
+        for it in range(24):
+            seeds = rng.choice(n_nodes, batch, replace=False).astype(np.int32)
+            stream = lmi.stream_create()
+            srv.run_once(seeds, rng_seed=it + 1, pipe=it % 4, stream=stream)
+            srv.batch_wait(it % 4, stream)
+            o = oracle.sample_batch(indptr, indices, seeds, fanout, it + 1)
+            hit = cache.access(o.ids, host_rows)[0]
+            if it % 4 == 3:
+                g = srv.fetch(pipe=it % 4, stream=stream)
+                assert_batch_equal(g, o)
+                np.testing.assert_array_equal(g.cache_index, hit)
+                assert g.features.tobytes() == feats.array[o.ids].tobytes()
+            lmi.check(lmi.lib().lmi_stream_destroy(stream))
+        lmi.check(lmi.lib().lmi_device_sync())
+        keys, use = srv.cache_dump(sets * ways, with_aux=True)
+        want = cache.state()
+        np.testing.assert_array_equal(keys.ravel(), want[0].ravel())
+        np.testing.assert_array_equal(use.ravel(), want[1].ravel())
+    finally:
+        srv.close()
+        feats.free()
