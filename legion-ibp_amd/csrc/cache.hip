@@ -855,11 +855,19 @@ struct LookupArgs {
   int2 *miss_list;  // null: no list wanted
   DevState *st;
   int seg_first, seg_last, seg;
-  const HashSlot *dedup;  // the batch's dedup table: value of a seed id = its first row
+  const HashSlot *dedup;  // the batch's dedup table: value of a seed id = its first row; null: it was in LDS and is gone
   int dedup_log2cap;
   int lookup_blocks;  // blocks [0, lookup_blocks) look rows up, the rest carry `fill`
   FillArgs fill;      // last step of the hop sampled just before (hop -1: none)
 };
+
+// Whether seed row i repeats an earlier one, by looking (a batch small enough for LDS has few seeds).
+__device__ __forceinline__ bool seed_repeats(const int32_t *ids, int i) {
+  const int32_t id = ids[i];
+  for (int j = 0; j < i; ++j)
+    if (ids[j] == id) return true;
+  return false;
+}
 
 // id -> slot for rows [first, last) of the batch -> cache_index[].  Rows that
 // miss are appended to the segment's miss list as (row, id) pairs: ballot +
@@ -898,8 +906,9 @@ static __global__ __launch_bounds__(kLookupBlock) void lookup_kernel(LookupGroup
         if (a.kind == LMI_CACHE_LRU) {
           slot = lru_find(a.lru, id, a.st->lru_tick);
           // a repeated seed keeps both rows, but the id is offered for insertion once, by its first row
-          const bool repeat = i < a.st->n_seeds &&
-                              table_find(a.dedup, a.dedup_log2cap, id, a.st->table_tag, a.st->table_mask) != i;
+          const bool repeat =
+              i < a.st->n_seeds &&
+              (a.dedup ? table_find(a.dedup, a.dedup_log2cap, id, a.st->table_tag, a.st->table_mask) != i : seed_repeats(a.ids, i));
           a.lru_fill[i] = repeat ? -2 : -1;
         } else if (a.kind != LMI_CACHE_NONE) {
           slot = static_find(a.table, id);
@@ -947,7 +956,7 @@ int launch_lookup(Server *s, Pipe *const *pp, int n, hipStream_t st, int seg_fir
     a.cache_index = p.cache_index;
     a.miss_list = with_list ? p.miss_list + miss_list_base(s, seg_first) : nullptr;
     a.lru_fill = p.lru_fill;
-    a.dedup = p.dedup.slots;
+    a.dedup = p.table_in_lds ? nullptr : p.dedup.slots;
     a.dedup_log2cap = p.dedup.log2cap;
     a.st = p.st;
     a.seg_first = seg_first;

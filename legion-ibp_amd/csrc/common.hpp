@@ -98,6 +98,7 @@ struct Pipe {
   int32_t epoch = 0;           // dedup-table epoch of the last batch
   int id_bits = 0;             // key bits below the epoch tag when that batch ran
   bool table_dirty = true;     // the table must be wiped before its next use
+  bool table_in_lds = false;   // the batch was sampled by one workgroup: `dedup` knows nothing of it, and may never have been wiped
   int fill_pending = -1;       // hop whose edge sources still wait for their local ids (launch_fill)
   unsigned long long *chain_status[2] = {nullptr, nullptr};  // look-back scan state: [0] node scans, [1] edge scans
   int32_t max_tiles = 0;

@@ -658,6 +658,7 @@ int launch_batch_generate(Server *s, Pipe *const *pp, const BatchParams *bps, in
     pp[k]->n_seeds = bps[k].n_seeds;
     pp[k]->hops_done = 0;
     pp[k]->fill_pending = -1;
+    pp[k]->table_in_lds = false;
   }
   return LMI_OK;
 }
@@ -732,6 +733,7 @@ int launch_hop(Server *s, Pipe *const *pp, int n, hipStream_t st, int hop, bool 
       p.n_seeds = begin[k].n_seeds;
       p.hops_done = 0;
       p.fill_pending = -1;
+      p.table_in_lds = false;
     }
   }
   int G = 4;

@@ -346,6 +346,7 @@ int launch_small(Server *s, Pipe *const *pp, const BatchParams *bps, int n, hipS
     p.n_seeds = bps[k].n_seeds;
     p.hops_done = s->cfg.hops;
     p.fill_pending = -1;
+    p.table_in_lds = true;
     if (bps[k].clear_table) p.table_dirty = true;  // this batch leaves the table in HBM as it is
   }
   hipLaunchKernelGGL(batch_small_kernel, dim3(n), dim3(kSmallBlock), (size_t)small_lds_bytes(g.log2t, s->max_edges_hop),

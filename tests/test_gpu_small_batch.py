@@ -96,3 +96,40 @@ def test_conditions_presampling_and_a_table_that_was_never_wiped(lmi, oracle):
     finally:
         srv.close()
         feats.free()
+
+
+def test_segments_looked_up_in_another_cache_than_they_were_sampled_beside(lmi, oracle):
+    """A batch sampled by one workgroup leaves no dedup table in memory; a lookup in a dynamic cache built afterwards, which
+    offers a repeated seed once, does not need it."""
+    rng = np.random.default_rng(4)
+    n_nodes, batch, dim, fanout, sets, ways = 20_000, 65, 16, [10, 5], 40, 8
+    indptr, indices = random_graph(rng, n_nodes, 9)
+    feats = make_features(lmi, rng, n_nodes, dim)
+    srv = lmi.Server(batch, fanout, dim, pipes=2, seed=9)
+    try:
+        srv.load_graph(indptr, indices)
+        srv.attach_features(feats)
+        srv.build_lru_cache(sets, ways)
+        for it in range(3):   # the clock of the cache moves on
+            srv.run_once(rng.integers(0, n_nodes, batch).astype(np.int32), rng_seed=it + 1)
+        srv.build_static_cache(n_nodes // 4)
+        seeds = rng.integers(0, n_nodes, batch).astype(np.int32)
+        seeds[[5, 40, 64]] = seeds[3]
+        srv.run_once(seeds, rng_seed=7, pipe=1)
+        o = oracle.sample_batch(indptr, indices, seeds, fanout, 7)
+        assert_batch_equal(srv.fetch(pipe=1), o)
+        srv.build_lru_cache(sets, ways)
+        cache = oracle.Lru(sets, ways, dim * 4)
+        hit = cache.access(o.ids, feats.array.view(np.uint8).reshape(n_nodes, dim * 4))[0]
+        for segment in range(3):
+            srv.op_cache_lookup(segment, pipe=1)
+        srv.op_io_complete(pipe=1)
+        g = srv.fetch(pipe=1)
+        np.testing.assert_array_equal(g.cache_index, hit)
+        assert g.features.tobytes() == feats.array[o.ids].tobytes()
+        keys = srv.cache_dump(sets * ways)
+        assert (keys >= 0).any()
+        np.testing.assert_array_equal(keys.ravel(), cache.state()[0].ravel())
+    finally:
+        srv.close()
+        feats.free()
