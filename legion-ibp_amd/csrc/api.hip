@@ -180,7 +180,8 @@ static int pipe_alloc(Server *s, Pipe &p) {
   // Orders streams of this device among each other: with its system-scope fence, which only the host and other devices
   // need and a stream they synchronise has, a batch of 16 seeds took 21.9 us instead of 20.1.
   LMI_HIP(hipEventCreateWithFlags(&p.handover, hipEventDisableTiming | hipEventDisableSystemFence));
-  LMI_HIP(hipStreamSynchronize(nullptr));  // the fills above: a caller's stream does not wait for the null stream
+  LMI_HIP(hipEventRecord(p.handover, nullptr));  // what an event's first use costs (15 us) is paid here
+  LMI_HIP(hipStreamSynchronize(nullptr));        // the fills above: a caller's stream does not wait for the null stream
   return LMI_OK;
 }
 
