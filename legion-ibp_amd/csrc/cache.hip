@@ -1168,6 +1168,7 @@ static int launch_hits(Server *s, Pipe *const *pp, int n, hipStream_t st, int se
                        const HeaderCopy *headers = nullptr, bool look = false, hipEvent_t end = nullptr) {
   LMI_TRY(lru_wait_copied(s, st));
   // what is left of the batch rides in the flat and the tiled int8 gather; a profiled gather is timed by itself
+  // (launch_gather_group)
   const bool carries = !s->prof_on && (s->cache_kind == LMI_CACHE_INT8
                                            ? s->cfg.feat_dim % 16 == 0 && s->gather_flat != 2
                                            : s->row_bytes >= 16 && !lane_group_knobs(s, false) &&
@@ -1261,7 +1262,6 @@ bool one_pass_gather(const Server *s) {
 // stream, 122 us with everything on one and hits and misses in one launch (inference of 16 seeds: 70 and 36 us).
 bool gather_in_line(const Server *s, Pipe *const *pp, int n, int seg_last) {
   if (s->split_miss == 0 || s->feat_loc != LMI_LOC_HOST || s->cache_kind == LMI_CACHE_NONE) return true;
-  if (s->prof_on) return false;
   if (no_miss_possible(s)) return true;
   if (s->split_miss != 1 || s->protect_hits) return false;
   constexpr int64_t kFewBytes = 1 << 20;
@@ -1312,7 +1312,8 @@ int launch_gather_group(Server *s, Pipe *const *pp, int n, hipStream_t st, int s
   const bool in_line = same_stream || gather_in_line(s, pp, n, seg_last);
   int mode = in_line ? 0 : s->split_miss;
   // The gather kernels carry their own profiling events (prof_kernel_events); a bracket
-  // left open by the sampling phase ends here.
+  // left open by the sampling phase ends here, with the last hop's fill.
+  if (s->prof_on) LMI_TRY(launch_batch_tail(s, pp, n, st, headers));
   prof_phase(s, st, &s->prof_open, -1);
   if (mode == 0) {
     // The batch ends on the caller's stream.  Its last kernel carries the event that says so (for the first pipe's event
