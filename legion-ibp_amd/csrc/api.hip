@@ -181,7 +181,14 @@ static int pipe_alloc(Server *s, Pipe &p) {
   // need and a stream they synchronise has, a batch of 16 seeds took 21.9 us instead of 20.1.
   LMI_HIP(hipEventCreateWithFlags(&p.handover, hipEventDisableTiming | hipEventDisableSystemFence));
   LMI_HIP(hipEventRecord(p.handover, nullptr));  // what an event's first use costs (15 us) is paid here
-  LMI_HIP(hipStreamSynchronize(nullptr));        // the fills above: a caller's stream does not wait for the null stream
+  return LMI_OK;
+}
+
+// All pipes from `have` on.  Their fills are complete before a caller's stream, which does not wait for the null stream,
+// can use them.
+static int pipes_alloc(Server *s, size_t have) {
+  for (size_t k = have; k < s->pipes.size(); ++k) LMI_TRY(pipe_alloc(s, s->pipes[k]));
+  LMI_HIP(hipStreamSynchronize(nullptr));
   return LMI_OK;
 }
 
@@ -411,9 +418,7 @@ int lmi_server_create(const lmi_config *cfg, lmi_server **out) {
   hipDeviceProp_t prop;
   if (hipGetDeviceProperties(&prop, cfg->device_id) == hipSuccess) s->n_cu = prop.multiProcessorCount;
   s->pipes.resize(cfg->pipes);
-  int rc = LMI_OK;
-  for (auto &p : s->pipes)
-    if ((rc = pipe_alloc(s, p)) != LMI_OK) break;
+  int rc = pipes_alloc(s, 0);
   if (rc == LMI_OK && hipMalloc(&s->d_scalar, 64) != hipSuccess) rc = LMI_ERR_HIP;
   if (rc == LMI_OK && hipStreamCreateWithFlags(&s->side, hipStreamNonBlocking) != hipSuccess) rc = LMI_ERR_HIP;
   if (rc == LMI_OK && hipEventCreateWithFlags(&s->lru_ready, hipEventDisableTiming) != hipSuccess) rc = LMI_ERR_HIP;
@@ -449,8 +454,7 @@ int lmi_server_pipes(lmi_server *h, int32_t pipes) {
   if ((size_t)pipes <= have) return LMI_OK;  // never shrinks: callers may hold views of the existing sets
   LMI_HIP(hipSetDevice(s->cfg.device_id));
   s->pipes.resize((size_t)pipes);  // moves the host-side records only; device buffers stay where they are
-  int rc = LMI_OK;
-  for (size_t k = have; k < s->pipes.size() && rc == LMI_OK; ++k) rc = pipe_alloc(s, s->pipes[k]);
+  const int rc = pipes_alloc(s, have);
   if (rc != LMI_OK) {
     for (size_t k = have; k < s->pipes.size(); ++k) pipe_free(s->pipes[k]);
     s->pipes.resize(have);

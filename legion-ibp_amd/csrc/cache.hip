@@ -1161,6 +1161,9 @@ static int launch_batch_tail(Server *s, Pipe *const *pp, int n, hipStream_t st, 
   return LMI_OK;
 }
 
+// No cache and the table behind the host link: every row of a batch comes over the link.
+static bool all_rows_over_link(const Server *s) { return s->cache_kind == LMI_CACHE_NONE && s->feat_loc == LMI_LOC_HOST; }
+
 // Gather of rows [first, last) on stream `st`, for all n pipes in one launch: the cache hits from HBM, and with
 // `misses` the other rows from the feature table in the same pass (only where gather_in_line allows it).  end: an event
 // that marks the end of the launch (not with a profiled gather, which carries events of its own).
@@ -1199,6 +1202,13 @@ static int launch_hits(Server *s, Pipe *const *pp, int n, hipStream_t st, int se
     m.n_table = s->n_nodes;
     m.look = look ? 1 : 0;
   }
+  if (all_rows_over_link(s)) {
+    // A grid that fills the link, not the device: more reads in flight cost the link a tenth (3 400 rows of 4 096 bytes,
+    // us on the whole grid 309, 256 blocks 278, 128 273, 96 273, 64 278, 48 285; 24 000 rows of 256 bytes 182, 171, 168,
+    // 169, 168, 173; four batches of 24 000 rows of 3 072 bytes, on all of the blocks, 5 558, 5 396, 5 604, 5 548, 5 434, 5 508).
+    const int blocks = s->miss_blocks > 0 ? s->miss_blocks : s->miss_blocks == 0 ? s->n_cu : 96;
+    m.max_blocks = std::max(1, (blocks + n - 1) / n);  // per pipe
+  }
   m.note_rows = rows_word(s, seg, seg_last);
   m.src_row_bytes = m.dst_row_bytes = m.row_bytes = s->row_bytes;
   m.n_max = n_max;
@@ -1226,7 +1236,8 @@ static int launch_misses(Server *s, Pipe *const *pp, int n, hipStream_t st, int 
   m.src_row_bytes = m.dst_row_bytes = m.row_bytes = s->row_bytes;
   m.n_max = s->node_cap[seg_last];
   if (s->feat_loc == LMI_LOC_HOST) {
-    const int usual = s->miss_blocks >= 0 ? s->miss_blocks : n >= 4 ? 40 : 32;
+    // (listed rows without a cache: nothing runs beside them)
+    const int usual = s->miss_blocks >= 0 ? s->miss_blocks : all_rows_over_link(s) ? 64 : n >= 4 ? 40 : 32;
     const int blocks = blocks_override > 0 ? blocks_override : usual > 0 ? usual : s->n_cu;
     m.max_blocks = std::max(1, (blocks + n - 1) / n);  // per pipe
     m.unroll = s->miss_unroll;
@@ -1245,10 +1256,12 @@ static bool no_miss_possible(const Server *s) {
 
 // Hits and misses in one pass of the flat gather: full-width cache rows (an int8 hit and a miss are moved in
 // different ways) of at least 16 bytes, no measurement knob that asks for another mover.  A profiled batch keeps
-// two launches, so that each gather is timed by itself.
+// two launches, so that each gather is timed by itself.  Where all rows come over the link, rows of more than a block's
+// 256 lanes of 16 bytes are listed and left to the LDS-tiled mover, which keeps whole rows in flight (us of a batch of
+// 24 000 rows in one pass / listed: 4 096 bytes 1 829 / 1 855, 5 732 bytes 2 760 / 2 626, 8 192 bytes 3 717 / 3 606).
 bool one_pass_gather(const Server *s) {
   return s->cache_kind != LMI_CACHE_INT8 && s->row_bytes >= 16 && !lane_group_knobs(s, false) &&
-         (s->gather_flat == 0 || s->gather_flat == 3) && !s->prof_on;
+         (s->gather_flat == 0 || s->gather_flat == 3) && !s->prof_on && !(all_rows_over_link(s) && s->row_bytes > 4096);
 }
 
 // Whether the misses are gathered on the caller's stream like the hits.  A side stream for them costs a fork and a

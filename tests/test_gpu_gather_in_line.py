@@ -11,8 +11,8 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("cached", ["nothing", "some", "all"])
 @pytest.mark.parametrize("where", ["host", "device"])
-@pytest.mark.parametrize("dim,dtype", [(4, np.float32), (5, np.float32), (66, np.float16), (100, np.float32),
-                                       (256, np.float32), (1433, np.float32)])
+@pytest.mark.parametrize("dim,dtype", [(4, np.float32), (5, np.float32), (66, np.float16), (100, np.float32), (1024, np.float32),
+                                       (256, np.float32), (1025, np.float32), (1433, np.float32)])
 def test_hits_and_misses_in_one_pass(lmi, oracle, dim, dtype, where, cached):
     rng = np.random.default_rng(dim)
     n_nodes, batch, fanout = 20_000, 400, [12, 6]     # the worst case of a batch is above 1 MB for every row size but 16 B
