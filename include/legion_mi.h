@@ -302,6 +302,17 @@ int lmi_steps_per_epoch(lmi_server *s, int mode, int32_t *steps);
  * for the same batches.  lmi_tune("profile_every", n) profiles one batch in n. */
 int lmi_profile_enable(lmi_server *s, int level);
 int lmi_profile_read(lmi_server *s, lmi_profile *out, int reset);  /* synchronises the device */
+/* Batches (or segments, operator by operator) that took each of the launches the library chooses by size, cache and call
+ * order, since the server was created: what a test of such a launch asks, so that it cannot pass beside it. */
+typedef struct lmi_routes {
+  int64_t small_batches;     /* sampled whole by one workgroup */
+  int64_t scan_lookups;      /* looked up in the flag scans: static, int8 or no cache */
+  int64_t lru_scan_lookups;  /* looked up in the flag scans: LRU cache */
+  int64_t gather_lookups;    /* segments looked up in their gather */
+  int64_t one_pass_gathers;  /* hits and misses in one launch on the caller's stream */
+  int64_t lru_place_copies;  /* LRU insertions in one launch */
+} lmi_routes;
+int lmi_routes_get(lmi_server *s, lmi_routes *out);
 /* Tuning knobs by name (e.g. "gather_lanes_per_row", "gather_unroll", "lds_dedup"). */
 int lmi_tune(lmi_server *s, const char *key, int64_t value);
 /* Plain device copy of `bytes` bytes, repeated; returns mean ms per copy

@@ -1244,6 +1244,13 @@ int lmi_profile_read(lmi_server *h, lmi_profile *out, int reset) {
   return LMI_OK;
 }
 
+int lmi_routes_get(lmi_server *h, lmi_routes *out) {
+  Server *s = reinterpret_cast<Server *>(h);
+  if (!s || !out) LMI_FAIL(LMI_ERR_ARG, "null argument");
+  *out = s->routes;
+  return LMI_OK;
+}
+
 int lmi_tune(lmi_server *h, const char *key, int64_t value) {
   Server *s = reinterpret_cast<Server *>(h);
   if (!s || !key) LMI_FAIL(LMI_ERR_ARG, "null argument");

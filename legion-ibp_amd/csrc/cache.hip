@@ -1291,6 +1291,7 @@ bool lookup_rides_in_gather(const Server *s) { return s->cache_kind == LMI_CACHE
 int launch_lookup_gather(Server *s, Pipe &p, hipStream_t st, int seg) {
   Pipe *pp[1] = {&p};
   p.tail_unjoined = true;  // everything is on the caller's stream
+  ++s->routes.gather_lookups;
   return launch_hits(s, pp, 1, st, seg, seg, true, nullptr, true);
 }
 
@@ -1340,6 +1341,7 @@ int launch_gather_group(Server *s, Pipe *const *pp, int n, hipStream_t st, int s
       pp[k]->tail_event = end;
     }
     if (one_pass_gather(s)) {
+      s->routes.one_pass_gathers += n;
       LMI_TRY(launch_hits(s, pp, n, st, seg, seg_last, true, headers, false, last_hits ? end : nullptr));
     } else {
       if (have_cache) LMI_TRY(launch_hits(s, pp, n, st, seg, seg_last, false, headers, false, last_hits ? end : nullptr));
@@ -1550,6 +1552,7 @@ int launch_lru_insert(Server *s, Pipe &p, hipStream_t st, int n_lists, hipEvent_
     hipExtLaunchKernelGGL(lru_place_copy_kernel, dim3(tiles), dim3(256), 0, st, nullptr, s->lru_done, 0, a,
                           (const uint8_t *)p.features, s->cache_data, s->row_bytes);
     LMI_HIP(hipGetLastError());
+    ++s->routes.lru_place_copies;
     s->lru_pending = s->lru_copy_pending = true;
     s->lru_stream = st;
     return LMI_OK;

@@ -5,6 +5,7 @@
 #include <hip/hip_fp16.h>
 #include <stdint.h>
 
+#include <atomic>
 #include <string>
 #include <vector>
 
@@ -225,8 +226,11 @@ struct Server {
   int32_t *rows_seen_dev = nullptr;
   // pipes
   std::vector<Pipe> pipes;
-  int last_pipe = -1;          // the pipe a single batch was last issued on, and whether the caller has taken that batch
-  bool last_taken = true;      // on its own stream since (Pipe::taken_in_order); before the first batch nothing is in flight
+  // the pipe a single batch was last issued on, and whether the caller has taken that batch on its own stream since
+  // (Pipe::taken_in_order); before the first batch nothing is in flight.  Another thread may take a batch meanwhile.
+  std::atomic<int> last_pipe{-1};
+  std::atomic<bool> last_taken{true};
+  lmi_routes routes{};
   hipStream_t side = nullptr;  // server-owned second stream for gathers that must not hold up the caller's stream
   // tuning
   int gather_lpr = 0;     // lanes per row (0 = auto)

@@ -809,6 +809,7 @@ int launch_hop(Server *s, Pipe *const *pp, int n, hipStream_t st, int hop, bool 
   else LMI_FLAG(8)
 #undef LMI_FLAG
   LMI_HIP(hipGetLastError());
+  if (hop == 0 && look.mode != LOOK_NOT) (look.mode == LOOK_LRU ? s->routes.lru_scan_lookups : s->routes.scan_lookups) += n;
   for (int k = 0; k < n; ++k) {
     pp[k]->fill_pending = hop;
     pp[k]->hops_done = hop + 1;

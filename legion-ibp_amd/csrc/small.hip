@@ -352,6 +352,7 @@ int launch_small(Server *s, Pipe *const *pp, const BatchParams *bps, int n, hipS
   hipLaunchKernelGGL(batch_small_kernel, dim3(n), dim3(kSmallBlock), (size_t)small_lds_bytes(g.log2t, s->max_edges_hop),
                      st, g);
   LMI_HIP(hipGetLastError());
+  s->routes.small_batches += n;
   return LMI_OK;
 }
 
