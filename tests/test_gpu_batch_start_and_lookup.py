@@ -44,6 +44,8 @@ def test_seed_counts_at_block_edges(lmi, oracle, table, lists):
             np.testing.assert_array_equal(g.cache_index, slot[o.ids])
             assert g.features.tobytes() == feats.array[o.ids].tobytes()
         assert bad is not None
+        routes = srv.routes()
+        assert routes["scan_lookups"] == (14 if lists else 7) and routes["small_batches"] == 0
         with pytest.raises(lmi.LegionError):
             srv.status(clear=True)
         srv.status()

@@ -54,6 +54,8 @@ def test_hits_and_misses_in_one_pass(lmi, oracle, dim, dtype, where, cached):
             assert g.features.tobytes() == feats.array[o.ids].tobytes()
             if cached == "some":
                 np.testing.assert_array_equal(g.cache_index, oracle.static_cache_build(indptr, n_nodes // 5)[o.ids])
+        listed = cached == "nothing" and where == "host" and feats.array.strides[0] > 4096
+        assert srv.routes()["one_pass_gathers"] == (0 if listed else 4)
     finally:
         srv.close()
         feats.free()

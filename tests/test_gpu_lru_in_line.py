@@ -45,6 +45,8 @@ def test_lookups_in_flag_scans_and_alone_mixed(lmi, oracle, ways, fanout):
         want = cache.state()
         np.testing.assert_array_equal(keys.ravel(), want[0].ravel())
         np.testing.assert_array_equal(use.ravel(), want[1].ravel())
+        routes = srv.routes()   # some ways each
+        assert 0 < routes["lru_scan_lookups"] < 12 and 0 < routes["lru_place_copies"] < 12
     finally:
         srv.close()
         feats.free()
@@ -81,6 +83,51 @@ def test_streams_that_come_and_go_between_batches(lmi, oracle):
         want = cache.state()
         np.testing.assert_array_equal(keys.ravel(), want[0].ravel())
         np.testing.assert_array_equal(use.ravel(), want[1].ravel())
+    finally:
+        srv.close()
+        feats.free()
+
+
+@pytest.mark.parametrize("dim,dtype,sets,ways", [
+    (2, np.float32, 150, 8),        # 8 bytes: less than a unit, placed and copied apart
+    (4, np.float32, 150, 3),        # one unit
+    (5, np.float32, 150, 8),        # 20 bytes: units that overlap, at 4-byte alignment
+    (66, np.float16, 150, 8),       # 132
+    (1433, np.float32, 40, 8),      # 5 732
+    (33, np.float32, 6, 64),        # 132, and a tile of 32 misses that grants up to 64 ways each
+])
+def test_rows_of_every_size_reach_the_cache(lmi, oracle, dim, dtype, sets, ways):
+    """Rows copied into the cache are read back as hits by later batches of the same nodes."""
+    rng = np.random.default_rng(dim + ways)
+    n_nodes, batch, fanout = 5_000, 200, [6, 4]
+    indptr, indices = random_graph(rng, n_nodes, 12)
+    feats = make_features(lmi, rng, n_nodes, dim, dtype)
+    host_rows = feats.array.view(np.uint8).reshape(n_nodes, -1)
+    srv = lmi.Server(batch, fanout, dim, feat_dtype=lmi.F16 if dtype == np.float16 else lmi.F32, pipes=2, seed=3)
+    stream = lmi.stream_create()
+    cache = oracle.Lru(sets, ways, host_rows.shape[1])
+    try:
+        srv.load_graph(indptr, indices)
+        srv.attach_features(feats)
+        srv.build_lru_cache(sets, ways)
+        hits = 0
+        for it in range(6):
+            seeds = rng.integers(0, 400, batch).astype(np.int32)   # the same few hundred nodes, repeated ones among them
+            srv.run_once(seeds, rng_seed=it // 2 + 1, pipe=it % 2, stream=stream)
+            o = oracle.sample_batch(indptr, indices, seeds, fanout, it // 2 + 1)
+            slots = cache.access(o.ids, host_rows)[0]
+            hits += int((slots >= 0).sum())
+            g = srv.fetch(pipe=it % 2, stream=stream)
+            assert_batch_equal(g, o)
+            np.testing.assert_array_equal(g.cache_index, slots)
+            assert g.features.tobytes() == feats.array[o.ids].tobytes()
+        assert hits > 100
+        keys, use = srv.cache_dump(sets * ways, with_aux=True)
+        want = cache.state()
+        np.testing.assert_array_equal(keys.ravel(), want[0].ravel())
+        np.testing.assert_array_equal(use.ravel(), want[1].ravel())
+        routes = srv.routes()
+        assert routes["lru_scan_lookups"] == 6 and routes["lru_place_copies"] == (6 if host_rows.shape[1] >= 16 else 0)
     finally:
         srv.close()
         feats.free()

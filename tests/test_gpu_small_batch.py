@@ -40,10 +40,12 @@ def test_small_batches_match_the_oracle_and_the_general_path(lmi, oracle, shape,
             got = []
             for edges in (1 << 20, 0):
                 srv.tune("small_edges", edges)
+                before = srv.routes()["small_batches"]
                 srv.run_once(seeds, rng_seed=it + 1, pipe=2, stream=stream)
                 got.append(srv.fetch(pipe=2, stream=stream))
                 srv.run_group([0, 1], [0, 0], seeds=[seeds, seeds[:n // 2]], rng_seeds=[it + 1, it + 2], stream=stream)
                 got += [srv.fetch(pipe=0, stream=stream), srv.fetch(pipe=1, stream=stream)]
+                assert srv.routes()["small_batches"] - before == (3 if edges else 0)
             for k, (a, b) in enumerate(zip(got[:3], got[3:])):
                 mine, key = (seeds[:n // 2], it + 2) if k == 2 else (seeds, it + 1)
                 assert_batch_equal(a, oracle.sample_batch(indptr, indices, mine, fanout, key))
@@ -77,6 +79,7 @@ def test_conditions_presampling_and_a_table_that_was_never_wiped(lmi, oracle):
             o = oracle.sample_batch(indptr, indices, train[b * batch:(b + 1) * batch], fanout, 9 + b)
             np.add.at(want, o.ids, 1)
         np.testing.assert_array_equal(hot, want)
+        assert srv.routes()["small_batches"] == 4
         seeds = train[:batch].copy()
         # pipe 1: a small batch first, then the general kernels on the table that it did not touch
         srv.run_once(seeds, rng_seed=5, pipe=1)
@@ -118,6 +121,7 @@ def test_segments_looked_up_in_another_cache_than_they_were_sampled_beside(lmi, 
         srv.run_once(seeds, rng_seed=7, pipe=1)
         o = oracle.sample_batch(indptr, indices, seeds, fanout, 7)
         assert_batch_equal(srv.fetch(pipe=1), o)
+        assert srv.routes()["small_batches"] == 1   # not with the dynamic cache
         srv.build_lru_cache(sets, ways)
         cache = oracle.Lru(sets, ways, dim * 4)
         hit = cache.access(o.ids, feats.array.view(np.uint8).reshape(n_nodes, dim * 4))[0]

@@ -238,14 +238,15 @@ def hip_runtime():
     return hip
 
 
-def test_static_entry_point_replayed_from_a_captured_graph(lmi, oracle):
+@pytest.mark.parametrize("batch,fanout", [(256, [25, 10]), (32, [10, 5])])   # the second in one workgroup
+def test_static_entry_point_replayed_from_a_captured_graph(lmi, oracle, batch, fanout):
     """The callers the entry point is for: its launches captured once in a HIP graph and replayed
     with other seeds in the same buffer; eager batches and synchronisations between the replays,
     every replay checked.  Captured in the global mode, in which an allocation by the capturing
     thread is an error."""
     hip = hip_runtime()
     rng = np.random.default_rng(23)
-    n_nodes, dim, batch, fanout = 30_000, 128, 256, [25, 10]
+    n_nodes, dim = 30_000, 128
     indptr, indices = random_graph(rng, n_nodes, 14, hubs=8, hub_deg=3000)
     feats = lmi.HostBuffer((n_nodes, dim), np.float32)
     feats.array[...] = rng.standard_normal((n_nodes, dim)).astype(np.float32)
@@ -278,6 +279,7 @@ def test_static_entry_point_replayed_from_a_captured_graph(lmi, oracle):
             o = oracle.sample_batch(indptr, indices, seeds, fanout, 77)
             assert np.array_equal(got.ids, o.ids) and np.array_equal(got.agg_src_off, o.agg_src_off)
         srv.status()
+        assert srv.routes()["small_batches"] == (1 + 4 if batch == 32 else 0)   # the captured call, the eager batches
     finally:
         if graph_exec.value:
             hip.hipGraphExecDestroy(graph_exec)
