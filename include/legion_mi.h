@@ -223,8 +223,10 @@ int lmi_op_io_complete(lmi_server *s, int pipe, void *stream);
 /* Runner::RunOnce (engine/server.cu:330-400): the whole operator chain with one
  * gather over all rows.  With lmi_tune("use_graph", 1) and a non-default stream the
  * sampling part replays a HIP graph captured on first use instead of launching its
- * kernels one by one.  Returns with the host-link part of the gather
- * possibly still running on the server's side stream: see lmi_batch_wait. */
+ * kernels one by one.  Returns with the host-link part of the gather possibly still
+ * running on the server's side stream (see lmi_batch_wait), unless it has nothing to
+ * overlap: a caller who takes each batch on the batch's own stream (lmi_batch_wait or
+ * lmi_batch_counters there) before issuing the next has all of it on that stream. */
 int lmi_run_once(lmi_server *s, int pipe, void *stream, const int32_t *seeds, int32_t n,
                  int seeds_location, int32_t batch_counter, int mode, uint64_t rng_seed);
 
@@ -299,7 +301,9 @@ int lmi_steps_per_epoch(lmi_server *s, int mode, int32_t *steps);
 /* level 0: off; 1: HIP events bracket the sampling phase and the lookup of a batch and each
  * gather kernel carries a start / stop event pair of its own; 2: only the gather kernels
  * are timed, nothing is queued between kernels.  Rows per gather are counted on the device
- * for the same batches.  lmi_tune("profile_every", n) profiles one batch in n. */
+ * for the same batches.  lmi_tune("profile_every", n) profiles one batch in n.  A profiled batch
+ * gathers its hits and its misses in two launches, each timed, also where an unprofiled one would
+ * gather them in one pass, and finishes its last hop with the sampling. */
 int lmi_profile_enable(lmi_server *s, int level);
 int lmi_profile_read(lmi_server *s, lmi_profile *out, int reset);  /* synchronises the device */
 /* Batches (or segments, operator by operator) that took each of the launches the library chooses by size, cache and call

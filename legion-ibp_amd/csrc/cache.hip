@@ -1264,7 +1264,8 @@ bool one_pass_gather(const Server *s) {
          (s->gather_flat == 0 || s->gather_flat == 3) && !s->prof_on && !(all_rows_over_link(s) && s->row_bytes > 4096);
 }
 
-// Whether the misses are gathered on the caller's stream like the hits.  A side stream for them costs a fork and a
+// Whether the misses are gathered on the caller's stream like the hits (profiled batches too, in two launches).  A side
+// stream for them costs a fork and a
 // join: 26 us on the device where a second launch on the same stream costs 5, and 11 us of the host's time for each
 // wait it queues.  It pays when it lets the misses of a batch overlap the sampling of the next one -- so not
 //  * when the table lies in HBM, or there is no cache, or no row can miss;
@@ -1295,21 +1296,7 @@ int launch_lookup_gather(Server *s, Pipe &p, hipStream_t st, int seg) {
   return launch_hits(s, pp, 1, st, seg, seg, true, nullptr, true);
 }
 
-// Gathers the rows [first, last) of a segment into each pipe's feature buffer:
-// cache hits from HBM, misses over the host link.  A wide host-link gather beside
-// the HBM gather cuts its bandwidth by more than half, so the misses of one batch
-// never share a stream with its hits, and run on a small grid (miss_blocks).  With
-// several pipes, the hits of all are one launch and so are the misses (group_miss).
-// Schedules (tuning key "split_miss"):
-//   0  both on the caller's stream, in one pass where one_pass_gather allows it;
-//   1  hits on the caller's stream, misses after them on the server's side stream,
-//      where they overlap the next batch's sampling;
-//   2  both on the side stream (a gather stage behind the sampling stage): the
-//      caller's stream is free for the next batch's sampling as soon as the lookup
-//      is done.
-// gather_in_line says when schedule 0 is taken whatever the knob says.
-// With 1 and 2 the caller's stream does not wait here: the next call on this pipe,
-// or lmi_batch_wait, joins.  The LRU cache joins at once (its insert copies the rows).
+// The host-link gather of segments [seg, seg_last], released ahead of the batch's later hops.
 int launch_misses_early(Server *s, Pipe *const *pp, int n, hipStream_t st, int seg, int seg_last) {
   hipEvent_t fork = pp[0]->fork_early;
   LMI_HIP(hipEventRecord(fork, st));
@@ -1319,6 +1306,22 @@ int launch_misses_early(Server *s, Pipe *const *pp, int n, hipStream_t st, int s
   return LMI_OK;  // the join event that launch_gather_group records behind the batch's last misses covers these
 }
 
+// Gathers the rows [first, last) of a segment into each pipe's feature buffer:
+// cache hits from HBM, misses from the feature table, over the host link where it lies
+// in host memory.  With several pipes, the hits of all are one launch and so are the
+// misses (group_miss).  Schedules (tuning key "split_miss"):
+//   0  both on the caller's stream, in one pass where one_pass_gather allows it;
+//   1  hits on the caller's stream, misses on the server's side stream, where they
+//      overlap the next batch's sampling.  A wide host-link gather beside HBM gathers
+//      cuts their bandwidth by more than half: it runs on a small grid (miss_blocks);
+//   2  both on the side stream (a gather stage behind the sampling stage): the
+//      caller's stream is free for the next batch's sampling as soon as the lookup
+//      is done.
+// gather_in_line says when schedule 0 is taken whatever the knob says: nothing is left
+// then for a side stream to overlap, and a wide grid has no neighbour to slow.
+// With 1 and 2 the caller's stream does not wait here: the next call on this pipe,
+// or lmi_batch_wait, joins.  A segment of an LRU batch joins at once (a later call
+// inserts the gathered rows).
 int launch_gather_group(Server *s, Pipe *const *pp, int n, hipStream_t st, int seg, int seg_last, int lru_lists,
                         bool same_stream, int hit_seg_first, const HeaderCopy *headers) {
   const int hit_seg = hit_seg_first >= 0 ? hit_seg_first : seg;  // the hits of segments whose misses went ahead

@@ -293,13 +293,7 @@ void prof_kernel_events(Server *s, int kind, hipEvent_t *start, hipEvent_t *stop
 // stage_seeds: also run the seed-staging kernel now (otherwise hop 0 stages them itself)
 int launch_batch_generate(Server *s, Pipe *const *pp, const BatchParams *bps, int n, hipStream_t st, bool stage_seeds);
 int graph_update_begin(Server *s, Pipe &p, const BatchParams &bp);
-// defer_fill: leave the last step of the hop (local ids of the edge sources) to the next
-// kernel of the batch -- the next hop's first kernel or the lookup -- which carries it in
-// extra blocks; otherwise a kernel of its own finishes the hop.
-// The launchers below take n pipes that are in step (same stage of their batches) and serve
-// them with the same launches, their blocks interleaved over blockIdx.x (LMI_GRID_ROW).
-// begin != null: no batch_begin_kernel ran, the first hop takes the batches' parameters from here and sets up the state.
-// look: the cache lookup of the nodes a hop adds (hop 0: of the seeds too) rides in its flag scan.
+// The cache lookup of the nodes a hop adds (hop 0: of the seeds too), in its flag scan.
 struct HopLookup {
   int mode = 0;      // LOOK_*
   int miss_seg = 0;  // LOOK_LIST: the miss list that receives them
@@ -307,6 +301,12 @@ struct HopLookup {
 // not at all; cache_index only; cache_index and the miss list; the same in the LRU cache, whose hits are marked and whose
 // misses go on the lists of their sets
 enum { LOOK_NOT = 0, LOOK_SLOTS = 1, LOOK_LIST = 2, LOOK_LRU = 3 };
+// The launchers below take n pipes that are in step (same stage of their batches) and serve
+// them with the same launches, their blocks interleaved over blockIdx.x (LMI_GRID_ROW).
+// defer_fill: leave the last step of the hop (local ids of the edge sources) to the next
+// kernel of the batch -- the next hop's first kernel, the gather, or a lookup of its own --
+// which carries it in extra blocks; otherwise a kernel of its own finishes the hop.
+// begin != null: no batch_begin_kernel ran, the first hop takes the batches' parameters from here and sets up the state.
 int launch_hop(Server *s, Pipe *const *pp, int n, hipStream_t st, int hop, bool stage_seeds, bool defer_fill,
                const BatchParams *begin = nullptr, HopLookup look = HopLookup{});
 // small.hip: the sampling phase of small batches, lookup included, in one launch of one workgroup per batch
@@ -332,18 +332,17 @@ int cache_build_static(Server *s, int64_t capacity_rows, int table_kind, bool in
 int cache_build_lru(Server *s, int64_t n_sets, int32_t ways);
 void cache_free(Server *s);
 // The lookup as a kernel of its own: operator by operator, and for the LRU cache where its lookup has to wait for the
-// insertion of the batch before on another stream.  Extra blocks of it finish a hop left pending (launch_hop, defer_fill).  (Finishing
-// it on the side stream instead, ahead of the host-link gather, measured 2 % slower.)
+// insertion of the batch before on another stream.  Extra blocks of it finish a hop left pending (launch_hop, defer_fill).
 int launch_lookup(Server *s, Pipe *const *pp, int n, hipStream_t st, int seg_first, int seg_last, bool with_list = true);
 int launch_hotness(Server *s, Pipe &p, hipStream_t st);
-// lru_lists > 0: the LRU insertion of that many miss lists follows the gather on the stream the
-// misses were gathered on (the side stream when it is in use), and the caller's stream does not wait.
 bool lookup_rides_in_gather(const Server *s);
 int launch_lookup_gather(Server *s, Pipe &p, hipStream_t st, int seg);
+// Gather of a segment.  lru_lists > 0: the LRU insertion of that many miss lists follows the gather on the stream the
+// misses were gathered on (the side stream when it is in use), and the caller's stream does not wait.
 int launch_gather_seg(Server *s, Pipe &p, hipStream_t st, int seg, int seg_last, int lru_lists);
-// The same for n pipes in step: the HBM gathers one after another, one fork, then the
-// host-link gathers one after another on the side stream.
-// same_stream: hits then misses on `st` whatever the schedule knob says (nothing is left pending).
+// The same for n pipes in step, their HBM gathers in one launch and their host-link gathers in another
+// (group_miss), or all rows in one where the gather is in line (gather_in_line, one_pass_gather).
+// same_stream: everything on `st` whatever the schedule knob says (nothing is left pending).
 // headers: where the caller of the static entry point wants the two 16-int headers (one pipe), or null.
 struct HeaderCopy {
   int32_t *nodes, *edges;

@@ -20,10 +20,12 @@
 //                       two kernels, hop_count_scan + hop_sample.)
 //   2. hop_flag_scan    first-occurrence flags -> ranks (single-pass scan); first
 //                       occurrences append their node to ids[] and publish its local id
-//                       in the table; new node count
+//                       in the table; new node count.  The cache lookup of the appended
+//                       nodes (hop 0: of the seeds too) rides along.
 //   3. fill             local id of every edge source = its table slot's value.  Inside a
 //                       batch this rides in extra blocks of the next kernel (the next
-//                       hop's step 1, or the cache lookup); hop_fill_kernel does it alone.
+//                       hop's step 1, or the gather); hop_fill_kernel does it alone.
+// Batches expected to be small go through one workgroup instead (small.hip).
 #include <algorithm>
 
 #include "scan.hpp"
@@ -684,10 +686,11 @@ int graph_update_begin(Server *s, Pipe &p, const BatchParams &bp) {
   return LMI_OK;
 }
 
-// One hop for each of the n pipes, all in the same launches (the pipes are in step: same hop,
-// same pending fill).
+// Only the fused first kernel of a hop can set the batch up.
 bool hop_sets_up(const Server *s) { return s->fuse_count && !s->lds_dedup; }
 
+// One hop for each of the n pipes, all in the same launches (the pipes are in step: same hop,
+// same pending fill).
 int launch_hop(Server *s, Pipe *const *pp, int n, hipStream_t st, int hop, bool stage_seeds, bool defer_fill,
                const BatchParams *begin, HopLookup look) {
   const int f = s->cfg.fanout[hop];

@@ -6,9 +6,9 @@
 // slots of a hop's edges and the nodes being sampled lie in LDS, the scans are block scans, and one launch per group of
 // batches (a workgroup each) does the seeds, every hop, the relabelling, the cache lookup and the headers.  What is left
 // of HBM is the chain seed -> row pointers -> neighbours -> row pointers ... that no kernel can shorten.
-// us per batch, gather included, on the general path and here: 16 seeds, fanouts 10,5 (445 edges in the last hop): 33 / 18;
-// 64 seeds of a Cora-shaped graph, 25,10 (3 680 edges): 36 / 27; 64 seeds, 10,5 (2 332): 38 / 25, six of them in a
-// group 39 / 25; three hops 5,4,3 (3 918): 52 / 41; 128 seeds of the Cora-shaped graph (6 979): 38 / 37.  1024 threads,
+// us per batch, gather included, on the general path and here: 16 seeds, fanouts 10,5 (445 edges in the last hop): 35 / 20;
+// 64 seeds of a Cora-shaped graph, 25,10 (3 680 edges): 37 / 28; 64 seeds, 10,5 (2 332): 38 / 26, six of them in a
+// group 39 / 27; three hops 5,4,3 (3 918): 54 / 42; 128 seeds of the Cora-shaped graph (6 979): 38 / 38.  1024 threads,
 // because draws and probes fill the CU's four SIMDs: with 512 the second of these takes 33, with 256 50.
 // Outputs are those of the general path, bit for bit (same draws, same candidates in the dedup table, same ranks).
 #include <algorithm>
@@ -80,7 +80,7 @@ __device__ __forceinline__ int small_insert(const SmallLds &l, int log2t, int32_
 // Samples the n_here staged nodes, a lane group per node and kSmallNodes nodes in flight, so that their neighbour reads
 // overlap.  The nodes come in the order of SmallLds::order, those that draw first: a wavefront computes draws for all its
 // groups if one of them needs any, and draws are what one CU is slow at.  (64 seeds of a Cora-shaped graph, where a
-// quarter of the nodes draw: 30.4 us in plain order, 27.0 in this one, gather and launches included.)
+// quarter of the nodes draw: 30.4 us in plain order, 27.0 in this one, gather and launches included, both in one run.)
 template <int G>
 __device__ __forceinline__ void small_sample(const SmallLds &l, const SmallGroup &g, const SmallPipe &a, int hop, int n_here,
                                              int c0, int n_known, int eoff, bool *full) {
