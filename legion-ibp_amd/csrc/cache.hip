@@ -1332,12 +1332,12 @@ int launch_gather_group(Server *s, Pipe *const *pp, int n, hipStream_t st, int s
   // left open by the sampling phase ends here, with the last hop's fill.
   if (s->prof_on) LMI_TRY(launch_batch_tail(s, pp, n, st, headers));
   prof_phase(s, st, &s->prof_open, -1);
+  // What a batch leaves on the caller's stream ends with a kernel of its gather, which carries an event that says so (the
+  // first pipe's for all pipes of a group): recorded behind it the event would be a packet of its own, and recorded when
+  // another stream asks it would stand for whatever is queued by then.  Not for a segment: its batch goes on.
+  const bool whole = hit_seg == 0 && seg_last == s->cfg.hops;
+  const hipEvent_t end = whole && !s->prof_on ? pp[0]->handover : nullptr;
   if (mode == 0) {
-    // The batch ends on the caller's stream.  Its last kernel carries the event that says so (for the first pipe's event
-    // all pipes of a group): recorded behind it the event would be a packet of its own, and recorded when another stream
-    // asks it would stand for whatever is queued by then.  Not for a segment: its batch goes on.
-    const bool whole = hit_seg == 0 && seg_last == s->cfg.hops;
-    const hipEvent_t end = whole && !s->prof_on ? pp[0]->handover : nullptr;
     const bool last_hits = lru_lists == 0 && (one_pass_gather(s) || no_miss_possible(s));
     for (int k = 0; k < n; ++k) {
       pp[k]->tail_unjoined = true;
@@ -1377,12 +1377,16 @@ int launch_gather_group(Server *s, Pipe *const *pp, int n, hipStream_t st, int s
                        (lru_lists == 0 && (s->early_fork == 1 || (s->early_fork == 2 && n > 1)));
     // behind a late fork the join event covers the whole batch; ahead of an early one the HBM gather stays
     // on the caller's stream alone
-    for (int k = 0; k < n; ++k) pp[k]->tail_unjoined = early;
+    for (int k = 0; k < n; ++k) {
+      pp[k]->tail_unjoined = early;
+      pp[k]->tail_event = early ? end : nullptr;
+    }
     if (early) {
       fork = pp[0]->fork;
       LMI_HIP(hipEventRecord(fork, st));
     }
-    LMI_TRY(launch_hits(s, pp, n, st, hit_seg, seg_last));  // one launch for the group
+    // one launch for the group
+    LMI_TRY(launch_hits(s, pp, n, st, hit_seg, seg_last, false, nullptr, false, early ? end : nullptr));
   }
   if (!fork) {  // one fork for the whole group
     fork = pp[0]->fork;

@@ -120,8 +120,8 @@ struct Pipe {
   // of the batch that `join_of` does not cover (everything when no side stream is used; the HBM
   // gather when the side stream was released ahead of it).  A later call that uses the pipe from
   // ANOTHER stream is then ordered behind that work (pipe_handover): through `tail_event`, the
-  // completion of the batch's last kernel, where the batch ran on that stream to its end, else
-  // through `handover`, recorded on `last_stream` by then.
+  // completion of its last kernel, or, between operators and for a profiled batch, through
+  // `handover`, recorded on `last_stream` by then.
   hipStream_t last_stream = nullptr;
   bool tail_unjoined = false;
   hipEvent_t handover = nullptr;

@@ -23,6 +23,8 @@ def make_server(lmi, cache, batch, n_nodes, dim, rng):
         srv.build_int8_cache(n_nodes, lmi.TABLE_HASH)
     elif cache == "lru":
         srv.build_lru_cache(n_nodes // 8, 8)
+    elif cache == "groups":
+        srv.build_static_cache(n_nodes // 2, lmi.TABLE_RANK)
     if cache == "in line":
         srv.tune("split_miss", 0)
     return srv, indptr, indices, feats
@@ -56,8 +58,9 @@ def test_taking_a_batch_does_not_wait_for_the_next_ones(lmi, oracle, cache, grou
         feats.free()
 
 
-@pytest.mark.parametrize("cache", ["static", "int8", "lru", "none", "in line"])
+@pytest.mark.parametrize("cache", ["static", "int8", "lru", "none", "in line", "groups"])
 def test_a_pipe_whose_stream_is_gone(lmi, oracle, cache):
+    """groups: their misses are gathered on the side stream, released ahead of the HBM gather."""
     rng = np.random.default_rng(2)
     n_nodes, batch, dim = 20_000, 300, 16
     srv, indptr, indices, feats = make_server(lmi, cache, batch, n_nodes, dim, rng)
@@ -67,7 +70,11 @@ def test_a_pipe_whose_stream_is_gone(lmi, oracle, cache):
         for it in range(12):
             stream, others = lmi.stream_create(), [lmi.stream_create() for _ in range(it % 3)]
             seeds = rng.choice(n_nodes, batch, replace=False).astype(np.int32)
-            srv.run_once(seeds, rng_seed=it + 1, pipe=it % 2, stream=stream)
+            if cache == "groups":
+                srv.run_group([it % 2, 2], [0, 0], seeds=[seeds, seeds], rng_seeds=[it + 1, 99], stream=stream)
+            else:
+                srv.run_once(seeds, rng_seed=it + 1, pipe=it % 2, stream=stream)
+            srv.batch_wait(it % 2, stream)
             o = oracle.sample_batch(indptr, indices, seeds, [12, 8], it + 1)
             hit = lru.access(o.ids, host_rows)[0] if cache == "lru" else None
             lmi.check(lmi.lib().lmi_stream_sync(stream))
