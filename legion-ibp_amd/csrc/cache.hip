@@ -983,12 +983,13 @@ int launch_lookup(Server *s, Pipe *const *pp, int n, hipStream_t st, int seg_fir
 int pipe_handover(Pipe &p, hipStream_t st) {
   if (!p.tail_unjoined || p.last_stream == st || !p.handover) return LMI_OK;
   if (p.tail_event) {
-    if (hipEventQuery(p.tail_event) == hipSuccess) {
-      p.tail_unjoined = false;
-      return LMI_OK;
+    const bool done = hipEventQuery(p.tail_event) == hipSuccess;
+    if (!done) {
+      (void)hipGetLastError();  // "not ready" is an answer, not a failure
+      LMI_HIP(hipStreamWaitEvent(st, p.tail_event, 0));
     }
-    (void)hipGetLastError();
-    LMI_HIP(hipStreamWaitEvent(st, p.tail_event, 0));
+    if (p.tail_follow) p.tail_event = nullptr;
+    else if (done) p.tail_unjoined = false;
   } else {
     LMI_HIP(hipEventRecord(p.handover, p.last_stream));
     LMI_HIP(hipStreamWaitEvent(st, p.handover, 0));
@@ -1337,6 +1338,15 @@ int launch_gather_group(Server *s, Pipe *const *pp, int n, hipStream_t st, int s
   // another stream asks it would stand for whatever is queued by then.  Not for a segment: its batch goes on.
   const bool whole = hit_seg == 0 && seg_last == s->cfg.hops;
   const hipEvent_t end = whole && !s->prof_on ? pp[0]->handover : nullptr;
+  // LRU batches are host-link-bound (a fifth of their rows miss): their host-link gather starts
+  // beside the HBM gather instead of behind it.  The insertion that follows it on the side stream
+  // only overwrites ways this batch's lookup did not touch, so the hits never read a row it writes.
+  const bool early = (lru_lists > 0 && s->lru_early_miss) ||
+                     (lru_lists == 0 && (s->early_fork == 1 || (s->early_fork == 2 && n > 1)));
+  // Behind a side stream's join event nobody follows the stream that takes a batch, so neither where the gather is in
+  // line only because that side stream would have nothing to overlap.
+  const bool sided = s->feat_loc == LMI_LOC_HOST && have_cache && (s->split_miss == 2 || (s->split_miss == 1 && !early));
+  for (int k = 0; k < n; ++k) pp[k]->tail_follow = !sided;
   if (mode == 0) {
     const bool last_hits = lru_lists == 0 && (one_pass_gather(s) || no_miss_possible(s));
     for (int k = 0; k < n; ++k) {
@@ -1370,11 +1380,6 @@ int launch_gather_group(Server *s, Pipe *const *pp, int n, hipStream_t st, int s
         s->side_busy = false;
       }
     }
-    // LRU batches are host-link-bound (a fifth of their rows miss): their host-link gather starts
-    // beside the HBM gather instead of behind it.  The insertion that follows it on the side stream
-    // only overwrites ways this batch's lookup did not touch, so the hits never read a row it writes.
-    const bool early = (lru_lists > 0 && s->lru_early_miss) ||
-                       (lru_lists == 0 && (s->early_fork == 1 || (s->early_fork == 2 && n > 1)));
     // behind a late fork the join event covers the whole batch; ahead of an early one the HBM gather stays
     // on the caller's stream alone
     for (int k = 0; k < n; ++k) {

@@ -126,6 +126,8 @@ struct Pipe {
   bool tail_unjoined = false;
   hipEvent_t handover = nullptr;
   hipEvent_t tail_event = nullptr;  // the pipe's own `handover`, or that of the first pipe of its group
+  bool tail_follow = false;  // whoever takes the batch on another stream may count on the pipe's next batch to wait for
+                             // what is queued there by then (the reads of the outputs): that stream is `last_stream` then
   bool taken_in_order = false;  // this batch's caller waited for the batch before on that batch's own stream, and only
                                 // then issued this one: its misses have nothing to overlap (gather_in_line)
   int32_t *seed_stage = nullptr;  // [batch_size] host seeds land here
