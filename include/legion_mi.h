@@ -150,6 +150,9 @@ int lmi_copy_device(void *dev_dst, const void *dev_src, size_t bytes, void *stre
 int lmi_ipc_export(const void *dev_ptr, void *handle, int64_t *offset, int64_t *alloc_bytes);
 int lmi_ipc_open(const void *handle, void **dev_base);
 int lmi_ipc_close(void *dev_base);
+/* A stream that carried batches may be destroyed once they have been waited for (lmi_batch_wait, lmi_stream_sync).  One that
+ * carried operators one by one, presampling or a profiled batch, or that took a batch of another stream, must exist until the
+ * pipe has been used from another stream. */
 int lmi_stream_create(void **stream);
 int lmi_stream_destroy(void *stream);
 int lmi_stream_sync(void *stream);
