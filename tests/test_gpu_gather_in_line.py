@@ -61,3 +61,42 @@ def test_hits_and_misses_in_one_pass(lmi, oracle, dim, dtype, where, cached):
         feats.free()
         if table:
             lmi.check(lmi.lib().lmi_device_free(table))
+
+
+@pytest.mark.parametrize("dim", [1024, 1025])
+@pytest.mark.parametrize("blocks", [-1, 1, 300])
+def test_segments_and_groups_without_a_cache(lmi, oracle, dim, blocks):
+    """All rows over the host link: rows of up to 4 096 bytes in one pass, longer ones listed, on any grid."""
+    rng = np.random.default_rng(dim)
+    n_nodes, batch, fanout = 5_000, 100, [6, 4]
+    indptr, indices = random_graph(rng, n_nodes, 12)
+    feats = make_features(lmi, rng, n_nodes, dim)
+    srv = lmi.Server(batch, fanout, dim, pipes=3, seed=3)
+    stream = lmi.stream_create()
+
+    def check(pipe, seeds, key):
+        g = srv.fetch(pipe=pipe, stream=stream)
+        assert_batch_equal(g, oracle.sample_batch(indptr, indices, seeds, fanout, key))
+        assert g.features.tobytes() == feats.array[g.ids].tobytes()
+        assert (g.cache_index == -1).all()
+
+    try:
+        srv.load_graph(indptr, indices)
+        srv.attach_features(feats)
+        srv.tune("miss_blocks", blocks)
+        for it, n in enumerate([batch, 1, 64]):
+            seeds = rng.integers(0, n_nodes, n).astype(np.int32)
+            srv.op_batch_generate(seeds, rng_seed=it + 1, pipe=0, stream=stream)
+            srv.op_cache_lookup(0, pipe=0, stream=stream)
+            for hop in range(2):
+                srv.op_random_sample(hop, pipe=0, stream=stream)
+                srv.op_cache_lookup(hop + 1, pipe=0, stream=stream)
+            srv.op_io_complete(pipe=0, stream=stream)
+            check(0, seeds, it + 1)
+            srv.run_group([0, 1, 2], [0, 0, 0], seeds=[seeds, seeds[:n // 2], seeds[::-1]], rng_seeds=[7, 8, 9], stream=stream)
+            check(0, seeds, 7)
+            check(1, seeds[:n // 2], 8)
+            check(2, np.ascontiguousarray(seeds[::-1]), 9)
+    finally:
+        srv.close()
+        feats.free()

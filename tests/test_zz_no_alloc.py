@@ -88,6 +88,8 @@ def assert_same(a, b):
     ("int8", 768, np.float16, [25, 15], 64),
     ("static", 100, np.float32, [5, 4, 3], 700),
     ("none", 64, np.float32, [64, 2], 128),
+    ("none", 1100, np.float32, [6, 4], 200),   # rows that are listed before they are moved
+    ("none", 1100, np.float32, [6, 4], 20),    # the same behind one workgroup
 ])
 def test_static_entry_point_matches_run_once_twice_in_a_row(lmi, oracle, cache, dim, dtype, fanout, batch):
     rng = np.random.default_rng(11)
