@@ -313,8 +313,8 @@ int lmi_profile_read(lmi_server *s, lmi_profile *out, int reset);  /* synchronis
  * order, since the server was created: what a test of such a launch asks, so that it cannot pass beside it. */
 typedef struct lmi_routes {
   int64_t small_batches;     /* sampled whole by one workgroup */
-  int64_t scan_lookups;      /* looked up in the flag scans: static, int8 or no cache */
-  int64_t lru_scan_lookups;  /* looked up in the flag scans: LRU cache */
+  int64_t scan_lookups;      /* looked up by the hops' kernels: static, int8 or no cache */
+  int64_t lru_scan_lookups;  /* looked up by the hops' kernels: LRU cache */
   int64_t gather_lookups;    /* segments looked up in their gather */
   int64_t one_pass_gathers;  /* hits and misses in one launch on the caller's stream */
   int64_t lru_place_copies;  /* LRU insertions in one launch */

@@ -9,7 +9,7 @@
 
 #include <hip/hip_ext.h>
 
-#include "common.hpp"
+#include "scan.hpp"
 
 namespace lmi {
 
@@ -115,8 +115,7 @@ static int dmalloc(T **p, int64_t count) {
 static void pipe_free(Pipe &p) {
   void *ptrs[] = {p.ids, p.features, p.labels, p.agg_src_ids, p.agg_src_off, p.agg_dst_off, p.blk_indptr[0],
                   p.blk_indptr[1], p.blk_indptr[2], p.cache_index, p.st, p.dedup.slots, p.eslot[0], p.eslot[1],
-                  p.miss_list, p.lru_fill, p.lru_next, p.seed_stage,
-                  p.chain_status[0], p.chain_status[1]};
+                  p.miss_list, p.lru_fill, p.lru_next, p.seed_stage, p.scan_words};
   for (void *q : ptrs)
     if (q) (void)hipFree(q);
   if (p.graph_exec) (void)hipGraphExecDestroy(p.graph_exec);
@@ -146,7 +145,7 @@ static int32_t scan_max_tiles(const Server *s) {
     while (G < s->cfg.fanout[k]) G <<= 1;
     tiles = std::max(tiles, ceil_div(s->node_cap[k], (int64_t)std::min(64, 256 / G)));  // smallest tile
   }
-  return (int32_t)tiles + 1;
+  return (int32_t)(tiles + ceil_div(s->cfg.batch_size, kScanBlock)) + 1;  // the first hop's seed tiles
 }
 
 static int pipe_alloc(Server *s, Pipe &p) {
@@ -166,10 +165,8 @@ static int pipe_alloc(Server *s, Pipe &p) {
   LMI_TRY(dmalloc(&p.eslot[0], s->max_edges_hop));
   LMI_TRY(dmalloc(&p.eslot[1], s->max_edges_hop));
   p.max_tiles = scan_max_tiles(s);
-  for (auto &chain : p.chain_status) {
-    LMI_TRY(dmalloc(&chain, p.max_tiles));
-    LMI_HIP(hipMemset(chain, 0, (size_t)p.max_tiles * sizeof(*chain)));  // no tile has announced a sum
-  }
+  LMI_TRY(dmalloc(&p.scan_words, (int64_t)kScanChains * p.max_tiles));
+  LMI_HIP(hipMemset(p.scan_words, 0, (size_t)kScanChains * p.max_tiles * 8));  // no batch's stamp
   LMI_TRY(dmalloc(&p.miss_list, s->max_nodes));
   LMI_TRY(dmalloc(&p.lru_fill, s->max_nodes));
   LMI_TRY(dmalloc(&p.lru_next, s->max_nodes));
@@ -338,13 +335,12 @@ constexpr size_t kOffState = 0;
 constexpr size_t kOffTable = 256;
 constexpr size_t kOffEslot0 = kOffTable + (size_t(8) << kStaticLog2Cap);
 constexpr size_t kOffEslot1 = kOffEslot0 + size_t(4) * LMI_STATIC_MAX_HOP_EDGES;
-constexpr size_t kOffChain0 = kOffEslot1 + size_t(4) * LMI_STATIC_MAX_HOP_EDGES;
-constexpr size_t kOffChain1 = kOffChain0 + size_t(8) * kStaticMaxTiles;
-constexpr size_t kOffMiss = kOffChain1 + size_t(8) * kStaticMaxTiles;
+constexpr size_t kOffScan = kOffEslot1 + size_t(4) * LMI_STATIC_MAX_HOP_EDGES;
+constexpr size_t kOffMiss = kOffScan + size_t(8) * kScanChains * kStaticMaxTiles;
 constexpr size_t kStaticUsed = kOffMiss + size_t(8) * LMI_STATIC_MAX_NODES;
 static_assert(sizeof(DevState) <= 256, "the batch state has a 256-byte slot at the head of the scratch");
 static_assert(kStaticUsed <= LMI_STATIC_SCRATCH_BYTES, "the scratch array is too small for its pieces");
-static_assert(kOffEslot0 % 256 == 0 && kOffChain0 % 256 == 0 && kOffChain1 % 256 == 0 && kOffMiss % 256 == 0,
+static_assert(kOffEslot0 % 256 == 0 && kOffScan % 256 == 0 && kOffMiss % 256 == 0,
               "every piece starts on a 256-byte boundary");
 
 static __device__ __align__(256) unsigned char scratch[LMI_STATIC_SCRATCH_BYTES];
@@ -436,6 +432,8 @@ int lmi_server_create(const lmi_config *cfg, lmi_server **out) {
       s->fault_dev = (int32_t *)fd;
       s->rows_seen_host = s->fault_host + 8;  // LMI_MAX_GROUP words for whole batches, one for each segment
       s->rows_seen_dev = s->fault_dev ? s->fault_dev + 8 : nullptr;
+      s->nodes_seen_host = s->fault_host + 24;  // LMI_MAX_HOPS words
+      s->nodes_seen_dev = s->fault_dev ? s->fault_dev + 24 : nullptr;
     }
   }
   if (rc != LMI_OK) {
@@ -762,12 +760,12 @@ static int batch_params(Server *s, Pipe &p, hipStream_t st, const int32_t *seeds
   // wiped only when the epochs run out (or it is new, or the id width changed)
   const int id_bits = table_id_bits(s);
   const int32_t max_epoch = (int32_t)std::min<int64_t>((int64_t(1) << (31 - id_bits)) - 1, s->table_epochs);  // 0: wipe every batch
-  bp->clear_table = p.table_dirty || p.epoch >= max_epoch || p.id_bits != id_bits ? 1 : 0;
+  bp->clear_table = p.table_dirty || p.epoch >= max_epoch || p.id_bits != id_bits || p.serial == kMaxSerial ? 1 : 0;
   const int32_t epoch = bp->clear_table ? 0 : p.epoch + 1;
   bp->table_tag = max_epoch > 0 ? (int32_t)((uint32_t)epoch << id_bits) : 0;
   bp->table_mask = max_epoch > 0 ? (int32_t)(0xFFFFFFFFu << id_bits) : kUntaggedMask;
   bp->fault = s->fault_dev;
-  bp->serial = p.serial == INT32_MAX ? 1 : p.serial + 1;
+  bp->serial = p.serial == kMaxSerial ? 1 : p.serial + 1;
   bp->rng_seed = rng_seed ? rng_seed : s->cfg.seed + (uint64_t)(uint32_t)batch_counter;
   bp->lru_tick = s->lru_tick + (s->cache_kind == LMI_CACHE_LRU ? 1 : 0);
   return LMI_OK;
@@ -962,7 +960,7 @@ static int run_group_launches(Server *s, Pipe *const *pp, const BatchParams *bps
   } else {
     // the rows that miss are listed unless hits and misses are gathered in one pass
     const bool in_line = gather_in_line(s, pp, n, s->cfg.hops);
-    // The LRU lookup rides in the flag scans too where the insertion before it is on this stream (for all its handle tells:
+    // The LRU lookup rides in the hops' kernels too where the insertion before it is on this stream (for all its handle tells:
     // the wait is queued all the same): a launch for the lookup
     // and one for the lists of misses less (four batches of 1 024 seeds and three hops: 396 us before, 386 with it).
     const bool lru_rides = lru && in_line && (!s->lru_pending || s->lru_stream == st);
@@ -1083,8 +1081,7 @@ int lmi_run_once_static(lmi_server *h, void *stream, const int32_t *seeds, int32
   p.dedup.log2cap = lg;
   p.eslot[0] = reinterpret_cast<int32_t *>(ptr + kOffEslot0);
   p.eslot[1] = reinterpret_cast<int32_t *>(ptr + kOffEslot1);
-  p.chain_status[0] = reinterpret_cast<unsigned long long *>(ptr + kOffChain0);
-  p.chain_status[1] = reinterpret_cast<unsigned long long *>(ptr + kOffChain1);
+  p.scan_words = reinterpret_cast<unsigned long long *>(ptr + kOffScan);
   p.max_tiles = tiles;
   p.miss_list = reinterpret_cast<int2 *>(ptr + kOffMiss);
   p.fill_pending = -1;
@@ -1279,7 +1276,7 @@ int lmi_tune(lmi_server *h, const char *key, int64_t value) {
   }
   else if (!strcmp(key, "profile_every")) s->prof_every = (int)std::max<int64_t>(1, value);
   else if (!strcmp(key, "small_edges")) s->small_edges = value;
-  else if (!strcmp(key, "fuse_small_max")) s->fuse_small_max = value;
+  else if (!strcmp(key, "fuse_small_max")) (void)value;  // accepted as before; tiles are chosen by hop_shape
   else if (!strcmp(key, "split_miss")) s->split_miss = (int)value;
   else if (!strcmp(key, "use_graph")) s->use_graph = (int)value;
   else if (!strcmp(key, "miss_blocks")) s->miss_blocks = (int)value;

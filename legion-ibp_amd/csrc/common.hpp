@@ -5,6 +5,7 @@
 #include <hip/hip_fp16.h>
 #include <stdint.h>
 
+#include <algorithm>
 #include <atomic>
 #include <string>
 #include <vector>
@@ -17,6 +18,7 @@ constexpr int kWave = 64;
 constexpr int32_t kEmptyKey = -1;
 constexpr int32_t kUntaggedMask = (int32_t)0x80000000u;  // tag mask of an untagged table: only key -1 is free
 constexpr int32_t kIntMax = 0x7fffffff;
+constexpr int32_t kMaxSerial = (1 << 28) - 1;  // batch numbers of a pipe run from 1 to this, then the scan words are zeroed
 
 // ---------------------------------------------------------------- errors
 void set_error(const char *fmt, ...);
@@ -98,10 +100,10 @@ struct Pipe {
   int32_t serial = 0;          // number of the last batch, never 0 once there was one
   int32_t epoch = 0;           // dedup-table epoch of the last batch
   int id_bits = 0;             // key bits below the epoch tag when that batch ran
-  bool table_dirty = true;     // the table must be wiped before its next use
+  bool table_dirty = true;     // the table (and the scan words) must be wiped before its next use
   bool table_in_lds = false;   // the batch was sampled by one workgroup: `dedup` knows nothing of it, and may never have been wiped
   int fill_pending = -1;       // hop whose edge sources still wait for their local ids (launch_fill)
-  unsigned long long *chain_status[2] = {nullptr, nullptr};  // look-back scan state: [0] node scans, [1] edge scans
+  unsigned long long *scan_words = nullptr;  // look-back scan state: kScanChains chains
   int32_t max_tiles = 0;
   int2 *miss_list = nullptr;   // [max_nodes] (row, id) pairs of cache misses
   int32_t *lru_fill = nullptr;                        // [max_nodes] slot granted to a miss
@@ -226,6 +228,9 @@ struct Server {
   // in the same pinned allocation
   volatile int32_t *rows_seen_host = nullptr;
   int32_t *rows_seen_dev = nullptr;
+  // nodes that a batch knew before each hop, left there by the hops' kernels
+  volatile int32_t *nodes_seen_host = nullptr;
+  int32_t *nodes_seen_dev = nullptr;
   // pipes
   std::vector<Pipe> pipes;
   // the pipe a single batch was last issued on, and whether the caller has taken that batch on its own stream since
@@ -248,7 +253,6 @@ struct Server {
                           // mover; 2 power-of-two lane groups, tiled only when no lane group fits the row
   int miss_flat = 0;      // the same choice for the host-link gather
   int int8_epl = 0;       // tiled int8 gather: elements per lane (0 = one 16-byte store per lane: 8 fp16 or 4 fp32)
-  int64_t fuse_small_max = 32768;  // hops of at most this many nodes use the small tile of hop_tile_nodes
   int64_t table_epochs = int64_t(1) << 30;  // batches a dedup table serves between wipes, less one (also
                                             // bounded by the key bits the node ids leave free)
   int fuse_count = 1;     // 1: row counts, their scan and the sampling of a hop share one launch
@@ -295,7 +299,7 @@ void prof_kernel_events(Server *s, int kind, hipEvent_t *start, hipEvent_t *stop
 // stage_seeds: also run the seed-staging kernel now (otherwise hop 0 stages them itself)
 int launch_batch_generate(Server *s, Pipe *const *pp, const BatchParams *bps, int n, hipStream_t st, bool stage_seeds);
 int graph_update_begin(Server *s, Pipe &p, const BatchParams &bp);
-// The cache lookup of the nodes a hop adds (hop 0: of the seeds too), in its flag scan.
+// The cache lookup of the nodes a hop adds (hop 0: of the seeds too), in its kernel.
 struct HopLookup {
   int mode = 0;      // LOOK_*
   int miss_seg = 0;  // LOOK_LIST: the miss list that receives them
@@ -375,12 +379,10 @@ int cache_dump(Server *s, int32_t *slot_of, int64_t n, int32_t *aux);
 
 inline int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
-// Nodes per block of the fused count-and-sample kernel for a hop of at most n_max nodes
-// sampled G lanes per node: a small hop takes one node per lane group (more, smaller tiles
-// keep every CU busy), a large one a full wavefront of nodes.
-inline int hop_tile_nodes(int64_t n_max, int G, int64_t small_max = 32768) {
-  const int per_pass = 256 / G;
-  return (n_max <= small_max && per_pass < 64) ? per_pass : 64;
-}
+// Tile of hop_kernel: threads, and nodes per lane group.
+struct HopShape {
+  int block, passes;
+};
+HopShape hop_shape(const Server *s, int n, int hop, int n_seeds, int G);
 
 }  // namespace lmi

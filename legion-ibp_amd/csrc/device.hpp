@@ -129,17 +129,17 @@ __device__ __forceinline__ uint32_t table_insert_min(HashSlot *slots, int log2ca
   const uint32_t mask = (1u << log2cap) - 1u;
   const int32_t stored = key | tag;
   uint32_t h = hash_id(key, log2cap);
+  const unsigned long long mine = (unsigned long long)(uint32_t)stored | ((unsigned long long)(uint32_t)cand << 32);
   while (true) {
     unsigned long long *word = reinterpret_cast<unsigned long long *>(&slots[h]);
-    const unsigned long long raw = *reinterpret_cast<const volatile unsigned long long *>(word);
-    const int32_t k = (int32_t)(uint32_t)raw, v = (int32_t)(uint32_t)(raw >> 32);
-    if ((k & tag_mask) != tag) {  // free: claim it with key and value together
-      const unsigned long long mine = (unsigned long long)(uint32_t)stored | ((unsigned long long)(uint32_t)cand << 32);
-      if (atomicCAS(word, raw, mine) == raw) return h;
-      continue;  // somebody else took it: look at what it holds now
+    unsigned long long raw = __hip_atomic_load(word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    while (((int32_t)(uint32_t)raw & tag_mask) != tag) {  // free: claim it with key and value together
+      const unsigned long long was = atomicCAS(word, raw, mine);
+      if (was == raw) return h;
+      raw = was;  // somebody else took it: this is what it holds now
     }
-    if (k == stored) {
-      if (v > cand) {
+    if ((int32_t)(uint32_t)raw == stored) {
+      if ((int32_t)(uint32_t)(raw >> 32) > cand) {
         atomicMin(&slots[h].val, cand);
         return h;
       }
@@ -149,14 +149,23 @@ __device__ __forceinline__ uint32_t table_insert_min(HashSlot *slots, int log2ca
   }
 }
 
-// Read-only probe: value or -1.
+// Read-only probe: value or -1.  FRESH: other tiles of the same launch insert too, possibly on another die, whose L2 this
+// one does not see.
+template <bool FRESH = false>
 __device__ __forceinline__ int32_t table_find(const HashSlot *slots, int log2cap, int32_t key, int32_t tag = 0,
                                               int32_t tag_mask = kUntaggedMask) {
   const uint32_t mask = (1u << log2cap) - 1u;
   const int32_t stored = key | tag;
   uint32_t h = hash_id(key, log2cap);
   while (true) {
-    const int2 kv = *reinterpret_cast<const int2 *>(&slots[h]);
+    int2 kv;
+    if constexpr (FRESH) {
+      const unsigned long long raw = __hip_atomic_load(reinterpret_cast<const unsigned long long *>(&slots[h]),
+                                                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      kv = make_int2((int32_t)(uint32_t)raw, (int32_t)(uint32_t)(raw >> 32));
+    } else {
+      kv = *reinterpret_cast<const int2 *>(&slots[h]);
+    }
     if (kv.x == stored) return kv.y;
     if ((kv.x & tag_mask) != tag) return -1;
     h = (h + 1) & mask;
@@ -260,14 +269,20 @@ __device__ __forceinline__ void fill_local_ids(const FillArgs &f, int64_t tid, i
   (void)gx
 
 // ------------------------------------------------------------------- scans
+// Moves between registers (DPP: four shifts within a row of 16 lanes, then the rows' last lanes broadcast) instead of
+// shuffles, each of which goes through the LDS unit.  The whole wavefront calls.
 __device__ __forceinline__ int wave_inclusive_scan(int v) {
-  const int lane = threadIdx.x & (kWave - 1);
-#pragma unroll
-  for (int d = 1; d < kWave; d <<= 1) {
-    const int t = __shfl_up(v, d, kWave);
-    if (lane >= d) v += t;
-  }
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);  // row_shr:1
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);  // row_shr:2
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);  // row_shr:4
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);  // row_shr:8
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);  // row_bcast:15, into rows 1 and 3
+  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);  // row_bcast:31, into rows 2 and 3
   return v;
+}
+// Sum over the wavefront, in every lane.
+__device__ __forceinline__ int wave_sum(int v) {
+  return __builtin_amdgcn_readlane(wave_inclusive_scan(v), kWave - 1);
 }
 
 // Exclusive scan over a block of BLOCK threads; `total` = sum over the block.

@@ -13,18 +13,11 @@
 // plus an N-entry position map; scans instead of atomics for placement, so the
 // edge order is (node, slot) and local ids follow first occurrence in that order.
 //
-// A hop is three steps:
-//   1. hop_count_sample per-node output counts -> block-CSR row pointers (single-pass
-//                       scan), draw positions, write edges, insert sources into the dedup
-//                       table; for hop 0 it also stages the seeds.  (Also available as
-//                       two kernels, hop_count_scan + hop_sample.)
-//   2. hop_flag_scan    first-occurrence flags -> ranks (single-pass scan); first
-//                       occurrences append their node to ids[] and publish its local id
-//                       in the table; new node count.  The cache lookup of the appended
-//                       nodes (hop 0: of the seeds too) rides along.
-//   3. fill             local id of every edge source = its table slot's value.  Inside a
-//                       batch this rides in extra blocks of the next kernel (the next
-//                       hop's step 1, or the gather); hop_fill_kernel does it alone.
+// A hop is one launch (hop_kernel): per-node output counts -> block-CSR row pointers, draws, edges, inserts of the sources
+// into the dedup table, first occurrences -> ranks, ids[] and local ids of the new nodes, their cache lookup; for hop 0 it
+// also stages the seeds.  What is left is the local id of every edge source = its table slot's value: inside a batch that
+// rides in extra blocks of the next kernel (the next hop, or the gather); hop_fill_kernel does it alone.
+// (Also available as three launches: hop_count_scan, hop_sample, hop_flag_scan.)
 // Batches expected to be small go through one workgroup instead (small.hip).
 #include <algorithm>
 
@@ -42,9 +35,12 @@ struct HopShared {  // what the pipes of a launch have in common
   int max_tiles;
   int stage_seeds;  // hop 0 only: the seeds have not been staged by batch_generate_kernel yet
   int begin;        // hop 0 only: no batch_begin_kernel ran, the parameters are in HopArgs::bp and the state is set up here
-  int tile_blocks;  // hop_count_sample: blocks [0, tile_blocks) own node tiles, the rest fill; hop_flag_scan: own edge
-                    // tiles, the rest look the seeds up
-  // cache lookup of the nodes the hop adds (hop_flag_scan)
+  int tile_blocks;  // hop_kernel: blocks [0, tile_blocks) own tiles, the rest fill; hop_flag_scan: own edge tiles, the rest
+                    // look the seeds up
+  int node_cap;     // nodes a batch can know before the hop
+  int32_t *nodes_seen;  // pinned host memory: receives how many the first batch knew
+  int seed_tiles;   // hop_kernel: the first tiles stage 256 seeds each
+  // cache lookup of the nodes the hop adds
   int look_mode, miss_seg;
   SlotTable cache;
   LruSets lru;  // LOOK_LRU
@@ -56,8 +52,8 @@ struct HopArgs {
   int32_t *agg_src_ids, *agg_dst_off;
   HashSlot *slots;
   int32_t *eslot;   // table slot per edge of this hop (| kKnownRepeat)
-  ScanChain chain_nodes, chain_edges;
-  FillArgs fill;    // the previous hop's last step, carried by hop_count_sample (hop -1: none)
+  unsigned long long *scan_words;
+  FillArgs fill;    // the previous hop's last step, carried by hop_kernel (hop -1: none)
   BatchParams bp;   // HopShared::begin
   int32_t *cache_index;
   int2 *miss_list;
@@ -74,6 +70,15 @@ struct HopGroup {
   int n;
 };
 static_assert(sizeof(HopGroup) <= 4096, "a kernel's arguments");
+// A batch's parameters where the argument segment of a kernel whose first argument is a HopGroup holds them.  Read through
+// this address space because a choice between them and the state's (HopShared::begin), were both behind ordinary pointers,
+// may become a choice of pointers, for which the compiler copies all arguments to scratch memory (a hop took ten times as
+// long).
+typedef const __attribute__((address_space(4))) HopGroup ArgHopGroup;
+typedef const __attribute__((address_space(4))) BatchParams ArgParams;
+__device__ __forceinline__ ArgParams &arg_params(int row) {
+  return ((ArgHopGroup *)__builtin_amdgcn_kernarg_segment_ptr())->p[row].bp;
+}
 struct FillGroup {
   FillArgs p[kMaxGroup];
   int n;
@@ -81,7 +86,7 @@ struct FillGroup {
 struct BeginPipe {
   HashSlot *slots;
   DevState *st;
-  ScanChain chain_nodes, chain_edges;
+  unsigned long long *scan_words;
   BatchParams bp;
 };
 struct BeginGroup {
@@ -91,15 +96,14 @@ struct BeginGroup {
 
 // ------------------------------------------------------------ batch start
 // Clears the dedup table (key = -1, value = INT_MAX), resets the pipe state and
-// the scan chains, and stores the per-batch parameters where later kernels read them.  Most batches do without this
-// launch (2-9 us): their table needs no wiping, the last flag scan of the batch before left chain_nodes clean, every
-// hop's first kernel resets chain_edges, and the first hop's first kernel can set up the state (HopShared::begin).
+// the scan words, and stores the per-batch parameters where later kernels read them.  Most batches do without this
+// launch (2-9 us): their table needs no wiping, scan words of earlier batches mean nothing, and the first hop's kernel can
+// set up the state (HopShared::begin).
 static __global__ __launch_bounds__(256) void batch_begin_kernel(BeginGroup g, int64_t n_slots, int hops,
                                                                  int max_tiles) {
   LMI_GRID_ROW(g.n);
   HashSlot *slots = g.p[row].slots;
   DevState *st = g.p[row].st;
-  const ScanChain chain_nodes = g.p[row].chain_nodes, chain_edges = g.p[row].chain_edges;
   const BatchParams &bp = g.p[row].bp;
   const int64_t tid = (int64_t)bx * blockDim.x + threadIdx.x;
   const int64_t stride = (int64_t)gx * blockDim.x;
@@ -109,10 +113,10 @@ static __global__ __launch_bounds__(256) void batch_begin_kernel(BeginGroup g, i
     int4 *p = reinterpret_cast<int4 *>(slots);
     for (int64_t i = tid; i < n_slots / 2; i += stride) p[i] = fill;
   }
-  scan_chain_reset(chain_nodes, max_tiles, tid, stride);
-  scan_chain_reset(chain_edges, max_tiles, tid, stride);
+  for (int64_t i = tid; i < (int64_t)kScanChains * max_tiles; i += stride) g.p[row].scan_words[i] = 0ull;
   if (tid == 0) {
     state_begin(st, bp, hops);
+    misses_begin(st);
     st->scan_fault = st->bad_id = 0;
   }
 }
@@ -121,14 +125,12 @@ static __global__ __launch_bounds__(256) void batch_begin_kernel(BeginGroup g, i
 // lookup runs before the first hop): ids[i] = seed, labels, table[seed] = min(i).
 // `begin`: the table needs no wiping, and this launch sets the batch up too (hops >= 1), from its arguments.
 static __global__ __launch_bounds__(256) void batch_generate_kernel(int64_t n_nodes, int32_t *ids, int32_t *labels,
-                                                                    int log2cap, BeginPipe p, int begin, int hops,
-                                                                    int max_tiles) {
+                                                                    int log2cap, BeginPipe p, int begin, int hops) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   const BatchParams &bp = p.bp;
-  if (begin) {
-    scan_chain_reset(p.chain_nodes, max_tiles, i, (int64_t)gridDim.x * blockDim.x);
-    scan_chain_reset(p.chain_edges, max_tiles, i, (int64_t)gridDim.x * blockDim.x);
-    if (i == 0) state_begin(p.st, bp, hops);
+  if (begin && i == 0) {
+    state_begin(p.st, bp, hops);
+    misses_begin(p.st);
   }
   if (i >= bp.n_seeds) return;
   const int32_t id = bp.seeds[i];
@@ -155,6 +157,8 @@ static __global__ __launch_bounds__(kScanBlock) void hop_count_scan_kernel(HopGr
   __shared__ int s_prefix;
   DevState *st = a.st;
   const FaultTo fault = fault_to(st);
+  const ScanChain nodes = scan_chain(a.scan_words, g.c.max_tiles, 0);
+  const uint32_t stamp = scan_stamp(fault.serial, g.c.hop);
   const int n = st->node_counter[9 + g.c.hop];
   const int n_tiles = (n + TILE - 1) / TILE;
   if (n_tiles == 0) {
@@ -211,8 +215,8 @@ static __global__ __launch_bounds__(kScanBlock) void hop_count_scan_kernel(HopGr
     }
     int total;
     const int ex = block_exclusive_scan<kScanBlock>(sum, lds, total);
-    if (threadIdx.x == 0) scan_tile_announce(a.chain_nodes, tile, total);
-    const int prefix = scan_tile_prefix(a.chain_nodes, tile, total, &s_prefix, st, fault);
+    if (threadIdx.x == 0) scan_tile_announce(nodes, stamp, tile, total);
+    const int prefix = scan_tile_prefix(nodes, stamp, tile, total, &s_prefix, st, fault);
     if (prefix == kScanFaultPrefix) return;  // the whole block: no offset, no writes
     int run = prefix + ex;
 #pragma unroll
@@ -239,7 +243,6 @@ static __global__ __launch_bounds__(256) void hop_sample_kernel(HopGroup g) {
   const HopArgs &a = g.p[row];  // this block's pipe (mini-batch)
   const DevState *st = a.st;
   const int64_t flat = (int64_t)bx * blockDim.x + threadIdx.x;
-  scan_chain_reset(a.chain_edges, g.c.max_tiles, flat, (int64_t)gx * blockDim.x);
   const uint64_t seed = (uint64_t)st->rng_lo | ((uint64_t)st->rng_hi << 32);
   const int32_t tag = st->table_tag, tag_mask = st->table_mask;
   const int n_prev = st->node_counter[9 + g.c.hop];
@@ -289,7 +292,6 @@ static __global__ __launch_bounds__(256) void hop_sample_lds_kernel(HopGroup g) 
   __shared__ int32_t lds_slot[TAB];
   const DevState *st = a.st;
   const int64_t flat = (int64_t)bx * blockDim.x + threadIdx.x;
-  scan_chain_reset(a.chain_edges, g.c.max_tiles, flat, (int64_t)gx * blockDim.x);
   const uint64_t seed = (uint64_t)st->rng_lo | ((uint64_t)st->rng_hi << 32);
   const int n_prev = st->node_counter[9 + g.c.hop];
   const int eoff = st->edge_counter[12 + g.c.hop + 1];
@@ -352,107 +354,184 @@ static __global__ __launch_bounds__(256) void hop_sample_lds_kernel(HopGroup g) 
   }
 }
 
-// ------------------------------------------------- hop, phases 1 and 2 in one launch
-// One tile of NPB nodes per block.  Wavefront 0 loads the tile's row pointers, scans
-// min(deg, fanout) across its lanes and obtains the tile's edge offset by look-back
-// over the earlier tiles; then the whole block samples the tile's nodes, G lanes per
-// node, from the row bounds kept in LDS.  Same outputs as hop_count_scan_kernel
-// followed by hop_sample_kernel, one launch and one row-pointer read less.
-template <int G, int NPB>
-static __global__ __launch_bounds__(256) void hop_count_sample_kernel(HopGroup g) {
+__device__ __forceinline__ int32_t hop_lookup(const HopGroup &g, const HopArgs &a, int32_t id, int32_t lru_tick) {
+  return g.c.look_mode == LOOK_LRU ? lru_find(g.c.lru, id, lru_tick) : static_find(g.c.cache, id);
+}
+// Cache lookup of the rows a block adds to the batch, ITEMS a thread (`look`): node, row, slot found.  In the kernels that add
+// them because the id is in a register there and the random read of the cache's table hides behind the other tiles'
+// look-back: as a kernel of its own the lookup was a launch and a pass over the ids: 30 us, its part of the last fill
+// included, for a group of four papers100M-shaped batches.
+template <int ITEMS, int BLOCK>
+__device__ __forceinline__ void rows_looked_up(const HopGroup &g, const HopArgs &a, bool seed_rows, const int32_t *node,
+                                               const int32_t *local, const int32_t *slot_of, bool *look, int32_t tag,
+                                               int32_t tag_mask, int *lds, int *lds_at) {
+  int misses = 0;
+#pragma unroll
+  for (int j = 0; j < ITEMS; ++j) {
+    if (look[j]) a.cache_index[local[j]] = slot_of[j];
+    look[j] = look[j] && slot_of[j] < 0 && node[j] >= 0 && node[j] < g.c.n_nodes;  // from here on: a miss
+    misses += look[j] ? 1 : 0;
+  }
+  if (g.c.look_mode == LOOK_LRU) {
+#pragma unroll
+    for (int j = 0; j < ITEMS; ++j) {
+      if (!look[j]) continue;
+      // a repeated seed keeps both rows, but the id is offered for insertion once, by its first row
+      const bool repeat = seed_rows && table_find<true>(a.slots, g.c.log2cap, node[j], tag, tag_mask) != local[j];
+      a.lru_fill[local[j]] = repeat ? -2 : -1;
+      if (!repeat) lru_chain(g.c.lru, a.lru_next, local[j], node[j]);
+    }
+  }
+  if (g.c.look_mode >= LOOK_LIST) {  // one atomic per block: one per wavefront on the same counter costs 24 ns each
+    int total;
+    int at = block_exclusive_scan<BLOCK>(misses, lds, total);
+    if (total == 0) return;
+    if (threadIdx.x == 0) *lds_at = atomicAdd(&a.st->n_miss[g.c.miss_seg], total);
+    __syncthreads();
+    at += *lds_at;
+#pragma unroll
+    for (int j = 0; j < ITEMS; ++j)
+      if (look[j]) a.miss_list[at++] = make_int2(local[j], node[j]);
+  }
+}
+
+// ------------------------------------------------------------- hop, one launch
+// All of a hop by tiles of NPB nodes, G lanes per node: row pointers and counts (wavefront 0), draws and neighbour reads,
+// inserts into the dedup table, the tile's edge offset (look-back), first occurrences and their ranks (look-back), ids and
+// local ids, cache lookup.  An edge is a first occurrence iff no earlier edge and no known node has its source, which the
+// tile can tell as soon as every EARLIER tile has inserted its edges -- later ones hold larger candidates.  So a tile
+// announces its edge count only when its inserts are complete, and the look-back over the counts is that wait too: like the
+// other one it needs no block that has not been dispatched.  The candidates themselves need no offset: i * fanout + slot
+// grows like the edge's index does.  The first hop's seeds, which come before all edges, are staged by tiles of their own
+// ahead of the others (HopShared::seed_tiles).  What tiles tell each other inside the launch -- table slots, scan words, the
+// miss count -- goes through device-scope atomics, which all dies see alike; wait_memory stands between a tile's inserts and
+// its word.
+// Bound by latency: eight dependent reads and two look-backs in a row (800 seeds, 25,10: 13 and 17 us for the two hops), and
+// by random accesses where a hop has 10^5 edges.  As two launches (sampling, then the flags from the edges' slots in memory)
+// a hop paid a launch and three dependent reads more.  us a pass, two launches per hop / one: 800 seeds, 25,10, a third of
+// the rows cached 110.6 / 102.4; 8 000 seeds, all rows cached 80.9 / 73.7; four such batches from a table in HBM 303 / 290;
+// 1 024 seeds, 15,10,5, four batches in a row through the LRU cache 350 / 298.
+template <int G, int BLOCK, int PASSES>
+static __global__ __launch_bounds__(BLOCK) void hop_kernel(HopGroup g) {
   LMI_GRID_ROW(g.n);
   const HopArgs &a = g.p[row];  // this block's pipe (mini-batch)
-  static_assert(NPB <= kWave && NPB >= 256 / G, "tile = one wavefront of nodes at most, one pass at least");
+  constexpr int PER_PASS = BLOCK / G, NPB = PER_PASS * PASSES, WAVES = BLOCK / kWave;
+  static_assert(NPB <= BLOCK, "a thread per node");
   __shared__ int32_t s_id[NPB];
   __shared__ int64_t s_beg[NPB], s_deg[NPB];
   __shared__ int s_row[NPB];
-  __shared__ int s_prefix;
+  __shared__ int s_total, s_edge0, s_rank0, s_miss0;
+  __shared__ int s_cnt[PASSES * WAVES];
+  __shared__ int s_scan[WAVES + 1];
   DevState *st = a.st;
-  const int64_t flat = (int64_t)bx * blockDim.x + threadIdx.x;
-  scan_chain_reset(a.chain_edges, g.c.max_tiles, flat, (int64_t)gx * blockDim.x);
   if (bx >= g.c.tile_blocks) {  // extra blocks: the previous hop's local ids
     fill_local_ids(a.fill, (int64_t)(bx - g.c.tile_blocks) * blockDim.x + threadIdx.x,
                    (int64_t)(gx - g.c.tile_blocks) * blockDim.x);
     return;
   }
+  const int seed_tiles = g.c.seed_tiles;
+  const int tile = bx, t = threadIdx.x;
+  const int my = (tile - seed_tiles) * NPB + t;  // wavefront 0: the thread's node
   // a batch that starts here takes its parameters from the arguments (nobody in this launch may read the state that one
   // of its threads sets up), any other from the state
   const bool begin = g.c.begin != 0;
-  const BatchParams &bp = a.bp;
+  ArgParams &bp = arg_params(row);
+  int32_t id = -1;
+  if (!g.c.stage_seeds && t < NPB && my < g.c.node_cap) id = a.ids[my];  // beside the state, not behind it
   const FaultTo fault = begin ? FaultTo{bp.serial, bp.fault} : fault_to(st);
   const int n_prev = begin ? bp.n_seeds : st->node_counter[9 + g.c.hop];
-  const int n_tiles = (n_prev + NPB - 1) / NPB;
-  if (n_tiles == 0) {
-    if (bx == 0 && threadIdx.x == 0) {
-      if (begin) state_begin(st, bp, g.c.hops);
+  const int n_tiles = seed_tiles + (n_prev + NPB - 1) / NPB;
+  if (tile >= n_tiles) {
+    if (n_tiles == 0 && tile == 0 && t == 0) {
       a.row_ptr[0] = 0;
       scan_epilogue(SCAN_EPI_HOP_EDGES, st, g.c.hop, 0);
+      scan_epilogue(SCAN_EPI_HOP_NODES, st, g.c.hop, 0);
     }
     return;
   }
-  const int tile = bx;
-  if (tile >= n_tiles) return;
-  const int t = threadIdx.x;
-  if (begin && tile == n_tiles - 1 && t == 0) state_begin(st, bp, g.c.hops);  // the thread that updates the headers below
+  const bool last = tile == n_tiles - 1;
+  if (begin && tile == 0 && t == 0) misses_begin(st);  // complete before any tile gets past this one's inserts
+  const uint32_t stamp = scan_stamp(fault.serial, g.c.hop);
+  const ScanChain edges = scan_chain(a.scan_words, g.c.max_tiles, 0), firsts = scan_chain(a.scan_words, g.c.max_tiles, 1);
   const int32_t tag = begin ? bp.table_tag : st->table_tag, tag_mask = begin ? bp.table_mask : st->table_mask;
-  // ---- counts, tile scan (wavefront 0)
-  const int my = tile * NPB + t;
-  int cnt = 0, ex = 0, total = 0;
-  int32_t id = -1;
-  int64_t lo = 0, hi = 0;
-  if (t < kWave) {
-    if (t < NPB && my < n_prev) {
-      if (g.c.stage_seeds) {
-        const int32_t *labels = begin ? bp.labels : st->labels_in;
-        id = (begin ? bp.seeds : st->seeds)[my];
-        a.ids[my] = id;
-        a.labels[my] = labels ? labels[my] : -1;
-      } else {
-        id = a.ids[my];
-      }
-      if (id < 0 || id >= g.c.n_nodes) {
-        if (g.c.stage_seeds) raise_fault(st, kFaultBadId, fault);
-        id = -1;
+  const int32_t *seeds = g.c.stage_seeds ? (begin ? bp.seeds : st->seeds) : nullptr;
+  const int look_mode = g.c.look_mode;
+  int32_t node[PASSES], local[PASSES], slot_of[PASSES];
+  bool look[PASSES];  // a row that the tile adds to the batch
+#pragma unroll
+  for (int u = 0; u < PASSES; ++u) node[u] = local[u] = slot_of[u] = -1, look[u] = false;
+
+  if (tile < seed_tiles) {
+    const int i = tile * BLOCK + t;
+    if (t == 0) scan_tile_announce(firsts, stamp, tile, 0);
+    if (i < n_prev) {
+      const int32_t *labels = begin ? bp.labels : st->labels_in;
+      node[0] = seeds[i];
+      local[0] = i;
+      look[0] = true;
+      a.ids[i] = node[0];
+      a.labels[i] = labels ? labels[i] : -1;
+      if (node[0] < 0 || node[0] >= g.c.n_nodes) raise_fault(st, kFaultBadId, fault);
+      else table_insert_min(a.slots, g.c.log2cap, node[0], i, tag, tag_mask);
+    }
+    wait_memory();
+    __syncthreads();
+    if (t == 0) scan_tile_announce(edges, stamp, tile, 0);
+    if (look_mode != LOOK_NOT && look[0] && node[0] >= 0 && node[0] < g.c.n_nodes)
+      slot_of[0] = hop_lookup(g, a, node[0], begin ? bp.lru_tick : st->lru_tick);
+    if (begin && tile == 0 && t == 0) state_params(st, bp);
+    if (scan_tile_prefix(edges, stamp, tile, 0, &s_edge0, st, fault) == kScanFaultPrefix) return;
+    if (last) {  // no seeds at all
+      if (t == 0) a.row_ptr[0] = 0;
+      if (begin) {
+        if (t < 32) headers_first_hop(st, t, g.c.hops, 0, 0, 0);
+      } else if (t == 0) {
+        scan_epilogue(SCAN_EPI_HOP_EDGES, st, g.c.hop, 0);
+        scan_epilogue(SCAN_EPI_HOP_NODES, st, g.c.hop, 0);
       }
     }
+  } else {
+    // ---- counts
+    if (seeds && t < NPB && my < n_prev) id = seeds[my];
+    if (t >= NPB || my >= n_prev || id < 0 || id >= g.c.n_nodes) id = -1;
+    int64_t lo = 0, hi = 0;
     if (id >= 0) {
       lo = g.c.indptr[id];
       hi = g.c.indptr[id + 1];
-      if (g.c.stage_seeds) table_insert_min(a.slots, g.c.log2cap, id, my, tag, tag_mask);
     }
     const int64_t deg = hi - lo;
-    cnt = (int)(deg < (int64_t)g.c.fanout ? deg : (int64_t)g.c.fanout);
-    const int inc = wave_inclusive_scan(cnt);
-    ex = inc - cnt;
-    total = __shfl(inc, kWave - 1, kWave);
-  }
-  if (t == 0) scan_tile_announce(a.chain_nodes, tile, total);
-  if (t < NPB) {
-    s_id[t] = id;
-    s_beg[t] = lo;
-    s_deg[t] = hi - lo;
-    s_row[t] = ex;
-  }
-  __syncthreads();
-  // ---- sampling.  What is drawn depends on no other tile: the draws are made and the neighbour reads of up to PASSES
-  // nodes per lane group are issued before the look-back, which hides behind them; only where the edges go needs it.
-  const uint64_t seed = begin ? bp.rng_seed : (uint64_t)st->rng_lo | ((uint64_t)st->rng_hi << 32);
-  // the edge offset of the hop is fixed by the hops before it
-  const int eoff = (g.c.hop == 0) ? 0 : st->edge_counter[12 + g.c.hop] + st->edge_counter[9 + g.c.hop];
-  const int fanout = g.c.fanout;
-  const int lane = t & (G - 1);
-  constexpr int PER_PASS = 256 / G, PASSES = NPB / PER_PASS < 4 ? NPB / PER_PASS : 4;
-  int prefix = 0;
-  for (int q0 = t / G; q0 < NPB; q0 += PER_PASS * PASSES) {
-    int32_t nbr[PASSES];
+    const int cnt = (int)(deg < (int64_t)g.c.fanout ? deg : (int64_t)g.c.fanout);
+    if (t < NPB) {
+      s_id[t] = id;
+      s_beg[t] = lo;
+      s_deg[t] = deg;
+    }
+    int ex, total;
+    if constexpr (NPB <= kWave) {
+      ex = wave_inclusive_scan(cnt) - cnt;
+      if (t == kWave - 1) s_total = ex + cnt;
+      if (t < NPB) s_row[t] = ex;
+      __syncthreads();
+      total = s_total;
+    } else {
+      ex = block_exclusive_scan<BLOCK>(cnt, s_scan, total);
+      if (t < NPB) s_row[t] = ex;
+      __syncthreads();
+    }
+    // ---- draws, neighbour reads, inserts
+    const uint64_t seed = begin ? bp.rng_seed : (uint64_t)st->rng_lo | ((uint64_t)st->rng_hi << 32);
+    // the edge offset of the hop is fixed by the hops before it
+    const int eoff = (g.c.hop == 0) ? 0 : st->edge_counter[12 + g.c.hop] + st->edge_counter[9 + g.c.hop];
+    const int fanout = g.c.fanout;
+    const int lane = t & (G - 1);
+    const int node0 = (tile - seed_tiles) * NPB + t / G;  // local id of the lane group's first node
     bool on[PASSES];
 #pragma unroll
     for (int u = 0; u < PASSES; ++u) {
-      const int q = q0 + u * PER_PASS;
+      const int q = t / G + u * PER_PASS;
       const int32_t v = s_id[q];  // -1 behind the last node
       const int64_t beg = s_beg[q], deg = s_deg[q];
       int64_t pick = lane;
-      nbr[u] = -1;
       on[u] = v >= 0 && lane < fanout && (int64_t)lane < deg;
       if (deg > (int64_t)fanout) {
         const uint32_t j = (uint32_t)(deg - fanout) + (uint32_t)lane;
@@ -460,27 +539,84 @@ static __global__ __launch_bounds__(256) void hop_count_sample_kernel(HopGroup g
         if (lane < fanout) d = __umulhi(sample_draw(seed, (uint32_t)g.c.hop, (uint32_t)v, (uint32_t)lane), j + 1u);
         pick = floyd_pick<G>(d, j, lane, fanout);
       }
-      if (on[u]) nbr[u] = g.c.indices[beg + pick];
+      if (on[u]) node[u] = g.c.indices[beg + pick];
     }
-    if (q0 == t / G) {  // the first time round, all threads alike
-      prefix = scan_tile_prefix(a.chain_nodes, tile, total, &s_prefix, st, fault);
-      if (prefix == kScanFaultPrefix) return;  // the whole block: no offset, no writes
-      if (t < NPB && my < n_prev) a.row_ptr[my] = prefix + ex;
-      if (tile == n_tiles - 1 && t == 0) {
-        a.row_ptr[n_prev] = prefix + total;
-        scan_epilogue(SCAN_EPI_HOP_EDGES, st, g.c.hop, prefix + total);
-      }
-    }
+    uint32_t slot[PASSES];
+#pragma unroll
+    for (int u = 0; u < PASSES; ++u)
+      slot[u] = on[u] ? table_insert_min(a.slots, g.c.log2cap, node[u], n_prev + (node0 + u * PER_PASS) * fanout + lane, tag, tag_mask)
+                      : kKnownRepeat;
+    wait_memory();
+    __syncthreads();
+    if (t == 0) scan_tile_announce(edges, stamp, tile, total);
+    const int edge0 = scan_tile_prefix(edges, stamp, tile, total, &s_edge0, st, fault);
+    if (edge0 == kScanFaultPrefix) return;  // the whole block: no offset, no writes
+    // ---- first occurrences, in edge order: pass by pass, threads in order
+    int32_t val[PASSES];
+#pragma unroll
+    for (int u = 0; u < PASSES; ++u)
+      val[u] = (slot[u] & kKnownRepeat) ? -1 : __hip_atomic_load(&a.slots[slot[u]].val, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    uint64_t m[PASSES];
 #pragma unroll
     for (int u = 0; u < PASSES; ++u) {
+      look[u] = !(slot[u] & kKnownRepeat) && val[u] == n_prev + (node0 + u * PER_PASS) * fanout + lane;
+      m[u] = __ballot(look[u]);
+      if ((t & (kWave - 1)) == 0) s_cnt[u * WAVES + t / kWave] = __popcll(m[u]);
+    }
+    __syncthreads();
+    int added = 0;
+    if constexpr (PASSES * WAVES <= 16) {
+#pragma unroll
+      for (int k = 0; k < PASSES * WAVES; ++k) {
+        const int c = s_cnt[k];
+        if (k % WAVES == t / kWave) local[k / WAVES] = added;
+        added += c;
+      }
+    } else {  // at most a wavefront of counts: every wavefront scans them
+      const int lane64 = t & (kWave - 1);
+      const int c = lane64 < PASSES * WAVES ? s_cnt[lane64] : 0;
+      const int inc = wave_inclusive_scan(c);
+      added = __builtin_amdgcn_readlane(inc, kWave - 1);
+#pragma unroll
+      for (int u = 0; u < PASSES; ++u) local[u] = __shfl(inc - c, u * WAVES + t / kWave, kWave);
+    }
+    if (t == 0) scan_tile_announce(firsts, stamp, tile, added);
+    // ---- edges, lookups
+#pragma unroll
+    for (int u = 0; u < PASSES; ++u) {
+      if (look_mode != LOOK_NOT && look[u] && node[u] >= 0 && node[u] < g.c.n_nodes)
+        slot_of[u] = hop_lookup(g, a, node[u], begin ? bp.lru_tick : st->lru_tick);
       if (!on[u]) continue;
-      const int q = q0 + u * PER_PASS;
-      const int e = prefix + s_row[q] + lane;
-      a.agg_src_ids[eoff + e] = nbr[u];
-      a.agg_dst_off[eoff + e] = tile * NPB + q;
-      a.eslot[e] = (int)table_insert_min(a.slots, g.c.log2cap, nbr[u], n_prev + e, tag, tag_mask);
+      const int e = edge0 + s_row[t / G + u * PER_PASS] + lane;
+      a.agg_src_ids[eoff + e] = node[u];
+      a.agg_dst_off[eoff + e] = node0 + u * PER_PASS;
+      a.eslot[e] = (int)slot[u];
+    }
+    if (t < NPB && my < n_prev) a.row_ptr[my] = edge0 + ex;
+    const int rank0 = scan_tile_prefix(firsts, stamp, tile, added, &s_rank0, st, fault);
+    if (rank0 == kScanFaultPrefix) return;  // the whole block: no ranks
+#pragma unroll
+    for (int u = 0; u < PASSES; ++u) {
+      local[u] += n_prev + rank0 + __popcll(m[u] & lanemask_lt());
+      if (look[u]) {
+        a.ids[local[u]] = node[u];
+        // later edges of the same node compare this with their own, larger, candidates either way
+        __hip_atomic_store(&a.slots[slot[u]].val, local[u], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+    }
+    if (last) {
+      if (t == 0) a.row_ptr[n_prev] = edge0 + total;
+      if (begin) {
+        if (t < 32) headers_first_hop(st, t, g.c.hops, n_prev, edge0 + total, rank0 + added);
+      } else if (t == 0) {
+        scan_epilogue(SCAN_EPI_HOP_EDGES, st, g.c.hop, edge0 + total);
+        scan_epilogue(SCAN_EPI_HOP_NODES, st, g.c.hop, rank0 + added);
+      }
     }
   }
+  if (tile == 0 && t == 0 && row == 0 && g.c.nodes_seen) *g.c.nodes_seen = n_prev;  // for the host to shape later launches by
+  if (look_mode != LOOK_NOT)
+    rows_looked_up<PASSES, BLOCK>(g, a, tile < seed_tiles, node, local, slot_of, look, tag, tag_mask, s_scan, &s_miss0);
 }
 
 // ------------------------------------------------------------- hop, step 2
@@ -489,9 +625,6 @@ static __global__ __launch_bounds__(256) void hop_count_sample_kernel(HopGroup g
 // node's place after the n_prev known nodes: the edge appends the node to ids[] and
 // publishes the local id in the table.  Publishing while other tiles still read is safe: a
 // later edge of the same node compares the value with its own, larger, index either way.
-__device__ __forceinline__ int32_t hop_lookup(const HopGroup &g, const HopArgs &a, int32_t id) {
-  return g.c.look_mode == LOOK_LRU ? lru_find(g.c.lru, id, a.st->lru_tick) : static_find(g.c.cache, id);
-}
 template <int ITEMS>
 static __global__ __launch_bounds__(kScanBlock) void hop_flag_scan_kernel(HopGroup g) {
   LMI_GRID_ROW(g.n);
@@ -500,8 +633,6 @@ static __global__ __launch_bounds__(kScanBlock) void hop_flag_scan_kernel(HopGro
   __shared__ int lds[kScanBlock / kWave + 1];
   __shared__ int s_prefix;
   DevState *st = a.st;
-  const int64_t flat = (int64_t)bx * blockDim.x + threadIdx.x;
-  scan_chain_reset(a.chain_nodes, g.c.max_tiles, flat, (int64_t)gx * blockDim.x);  // for the next hop
   int32_t local[ITEMS], node[ITEMS], slot_of[ITEMS];
   bool look[ITEMS];  // a row to look up
 #pragma unroll
@@ -513,10 +644,12 @@ static __global__ __launch_bounds__(kScanBlock) void hop_flag_scan_kernel(HopGro
       node[0] = a.ids[i];
       local[0] = i;
       look[0] = true;
-      if (look_mode != LOOK_NOT && node[0] >= 0 && node[0] < g.c.n_nodes) slot_of[0] = hop_lookup(g, a, node[0]);
+      if (look_mode != LOOK_NOT && node[0] >= 0 && node[0] < g.c.n_nodes) slot_of[0] = hop_lookup(g, a, node[0], st->lru_tick);
     }
   } else {
     const FaultTo fault = fault_to(st);
+    const ScanChain edges = scan_chain(a.scan_words, g.c.max_tiles, 1);
+    const uint32_t stamp = scan_stamp(fault.serial, g.c.hop);
     const int n_prev = st->node_counter[9 + g.c.hop];
     const int n = st->edge_counter[9 + g.c.hop + 1];
     const int eoff = st->edge_counter[12 + g.c.hop + 1];
@@ -545,14 +678,14 @@ static __global__ __launch_bounds__(kScanBlock) void hop_flag_scan_kernel(HopGro
     }
     int total;
     const int ex = block_exclusive_scan<kScanBlock>(sum, lds, total);
-    if (threadIdx.x == 0) scan_tile_announce(a.chain_edges, tile, total);
+    if (threadIdx.x == 0) scan_tile_announce(edges, stamp, tile, total);
 #pragma unroll
     for (int j = 0; j < ITEMS; ++j) {
       look[j] = v[j] != 0;
       if (look_mode != LOOK_NOT && look[j] && node[j] >= 0 && node[j] < g.c.n_nodes)
-        slot_of[j] = hop_lookup(g, a, node[j]);
+        slot_of[j] = hop_lookup(g, a, node[j], st->lru_tick);
     }
-    const int prefix = scan_tile_prefix(a.chain_edges, tile, total, &s_prefix, st, fault);
+    const int prefix = scan_tile_prefix(edges, stamp, tile, total, &s_prefix, st, fault);
     if (prefix == kScanFaultPrefix) return;  // the whole block: no ranks, no writes
     int run = n_prev + prefix + ex;
 #pragma unroll
@@ -568,40 +701,8 @@ static __global__ __launch_bounds__(kScanBlock) void hop_flag_scan_kernel(HopGro
       }
     if (tile == n_tiles - 1 && threadIdx.x == 0) scan_epilogue(SCAN_EPI_HOP_NODES, st, g.c.hop, prefix + total);
   }
-  // ---- cache lookup of the rows the block holds.  In this kernel because the id is in a register here and the random
-  // read of the cache's table hides behind the other tiles' look-back: as a kernel of its own the lookup was a launch
-  // and a pass over the ids: 30 us, its part of the last fill included, for a group of four papers100M-shaped
-  // batches, whose flag scans did not get slower (31 + 12 us).
-  if (look_mode == LOOK_NOT) return;
-  int misses = 0;
-#pragma unroll
-  for (int j = 0; j < ITEMS; ++j) {
-    if (look[j]) a.cache_index[local[j]] = slot_of[j];
-    look[j] = look[j] && slot_of[j] < 0 && node[j] >= 0 && node[j] < g.c.n_nodes;  // from here on: a miss
-    misses += look[j] ? 1 : 0;
-  }
-  if (look_mode == LOOK_LRU) {
-#pragma unroll
-    for (int j = 0; j < ITEMS; ++j) {
-      if (!look[j]) continue;
-      // a repeated seed keeps both rows, but the id is offered for insertion once, by its first row
-      const bool repeat = bx >= g.c.tile_blocks &&
-                          table_find(a.slots, g.c.log2cap, node[j], st->table_tag, st->table_mask) != local[j];
-      a.lru_fill[local[j]] = repeat ? -2 : -1;
-      if (!repeat) lru_chain(g.c.lru, a.lru_next, local[j], node[j]);
-    }
-  }
-  if (look_mode >= LOOK_LIST) {  // one atomic per block: one per wavefront on the same counter costs 24 ns each
-    int total;
-    int at = block_exclusive_scan<kScanBlock>(misses, lds, total);
-    if (total == 0) return;
-    if (threadIdx.x == 0) s_prefix = atomicAdd(&st->n_miss[g.c.miss_seg], total);
-    __syncthreads();
-    at += s_prefix;
-#pragma unroll
-    for (int j = 0; j < ITEMS; ++j)
-      if (look[j]) a.miss_list[at++] = make_int2(local[j], node[j]);
-  }
+  if (look_mode != LOOK_NOT)
+    rows_looked_up<ITEMS, kScanBlock>(g, a, bx >= g.c.tile_blocks, node, local, slot_of, look, st->table_tag, st->table_mask, lds, &s_prefix);
 }
 
 // ------------------------------------------------------------- hop, step 3
@@ -619,8 +720,6 @@ SlotTable slot_table(const Server *s) {
 
 LruSets lru_sets(const Server *s) { return LruSets{s->lru_keys, s->lru_use, s->lru_head, s->lru_sets, s->lru_ways}; }
 
-static ScanChain chain_of(const Pipe &p, int which) { return ScanChain{p.chain_status[which]}; }
-
 static int begin_grid(const Pipe &p) {
   const int64_t n_slots = int64_t(1) << p.dedup.log2cap;
   return (int)std::min<int64_t>(ceil_div(n_slots / 2, 256), 2048);
@@ -632,8 +731,7 @@ static BeginGroup begin_group(Pipe *const *pp, const BatchParams *bps, int n) {
   for (int k = 0; k < n; ++k) {
     g.p[k].slots = pp[k]->dedup.slots;
     g.p[k].st = pp[k]->st;
-    g.p[k].chain_nodes = chain_of(*pp[k], 0);
-    g.p[k].chain_edges = chain_of(*pp[k], 1);
+    g.p[k].scan_words = pp[k]->scan_words;
     g.p[k].bp = bps[k];
   }
   return g;
@@ -650,10 +748,9 @@ int launch_batch_generate(Server *s, Pipe *const *pp, const BatchParams *bps, in
     hipLaunchKernelGGL(batch_begin_kernel, dim3((begin_grid(p0)) * n), dim3(256), 0, st, g, n_slots, s->cfg.hops,
                        p0.max_tiles);
   if (stage_seeds) {
-    const int64_t threads = together ? std::max<int64_t>(s->cfg.batch_size, p0.max_tiles) : s->cfg.batch_size;
     for (int k = 0; k < n; ++k)
-      hipLaunchKernelGGL(batch_generate_kernel, dim3((int)ceil_div(threads, 256)), dim3(256), 0, st, s->n_nodes, pp[k]->ids,
-                         pp[k]->labels, pp[k]->dedup.log2cap, g.p[k], together ? 1 : 0, s->cfg.hops, p0.max_tiles);
+      hipLaunchKernelGGL(batch_generate_kernel, dim3((int)ceil_div(s->cfg.batch_size, 256)), dim3(256), 0, st, s->n_nodes, pp[k]->ids,
+                         pp[k]->labels, pp[k]->dedup.log2cap, g.p[k], together ? 1 : 0, s->cfg.hops);
   }
   LMI_HIP(hipGetLastError());
   for (int k = 0; k < n; ++k) {
@@ -689,6 +786,29 @@ int graph_update_begin(Server *s, Pipe &p, const BatchParams &bp) {
 // Only the fused first kernel of a hop can set the batch up.
 bool hop_sets_up(const Server *s) { return s->fuse_count && !s->lds_dedup; }
 
+// Which tile a hop of n batches takes.  Tiles wait for each other twice, each time the longer the more of them there are:
+// as small as leaves one tile per CU, then several nodes per lane group, with the largest for what does not fit the device
+// anyway.  us a pass by tile (threads x nodes per lane group) and the hop's tiles with it:
+//   800 seeds, fanouts 25,10, second hop (7 068 nodes): 256x1 442 tiles 105.6, 512x1 221 102.8, 1024x1 111 104.1;
+//   8 000 seeds, first hop: 256x1 1 000 83.5, 512x1 500 80.9, 1024x1 250 76.7, 512x4 125 82.8;
+//   their second (31 700 nodes): 1024x1 496 79.6, 512x2 496 74.8, 512x4 248 73.7, 1024x4 124 76.8;
+//   four such batches, second hop: 512x4 1 172 278.6, 1024x4 586 274.7, 256x4 2 344 285.4, 256x1 355.6;
+//   1 024 seeds, 15,10,5, third hop (20 000 nodes): 256x1 625 295.3, 1024x1 157 281.6, 512x4 78 284.7.
+// The nodes of a hop are those that the last batches knew there; before the first, the graph's mean degree tells.
+HopShape hop_shape(const Server *s, int n, int hop, int n_seeds, int G) {
+  const int64_t seen = hop > 0 && s->nodes_seen_host ? s->nodes_seen_host[hop] : 0;
+  int64_t nodes = seen > 0 ? seen : n_seeds;
+  const double mean = s->n_nodes > 0 ? (double)s->n_edges / (double)s->n_nodes : 0;
+  for (int k = 0; k < hop && seen <= 0; ++k) nodes += (int64_t)((double)nodes * std::min<double>(mean, s->cfg.fanout[k]));
+  nodes = std::max<int64_t>(1, std::min(nodes, s->node_cap[hop]));
+  constexpr HopShape kOnePass[] = {{256, 1}, {512, 1}, {1024, 1}}, kMore[] = {{512, 2}, {512, 4}};
+  for (const HopShape &h : kOnePass)
+    if (n * ceil_div(nodes, h.block / G) <= s->n_cu) return h;
+  for (const HopShape &h : kMore)
+    if (n * ceil_div(nodes, h.block / G * h.passes) <= 2 * s->n_cu) return h;
+  return HopShape{1024, 4};
+}
+
 // One hop for each of the n pipes, all in the same launches (the pipes are in step: same hop,
 // same pending fill).
 int launch_hop(Server *s, Pipe *const *pp, int n, hipStream_t st, int hop, bool stage_seeds, bool defer_fill,
@@ -706,6 +826,8 @@ int launch_hop(Server *s, Pipe *const *pp, int n, hipStream_t st, int hop, bool 
   g.c.hops = s->cfg.hops;
   g.c.log2cap = p0.dedup.log2cap;
   g.c.max_tiles = p0.max_tiles;
+  g.c.node_cap = (int)n_max;
+  g.c.nodes_seen = s->nodes_seen_dev ? s->nodes_seen_dev + hop : nullptr;
   g.c.stage_seeds = (hop == 0 && stage_seeds) ? 1 : 0;
   g.c.begin = begin ? 1 : 0;
   g.c.look_mode = look.mode;
@@ -723,8 +845,7 @@ int launch_hop(Server *s, Pipe *const *pp, int n, hipStream_t st, int hop, bool 
     a.agg_dst_off = p.agg_dst_off;
     a.slots = p.dedup.slots;
     a.eslot = p.eslot[hop & 1];
-    a.chain_nodes = chain_of(p, 0);
-    a.chain_edges = chain_of(p, 1);
+    a.scan_words = p.scan_words;
     a.fill.hop = -1;
     a.cache_index = p.cache_index;
     a.miss_list = p.miss_list + miss_list_base(s, look.miss_seg);
@@ -744,30 +865,34 @@ int launch_hop(Server *s, Pipe *const *pp, int n, hipStream_t st, int hop, bool 
   const bool fused = s->fuse_count && !s->lds_dedup;
   if (!fused) LMI_TRY(launch_fill(s, pp, n, st));
   if (fused) {
-    // counts, scan and sampling in one launch, one tile of nodes per block; a hop left
-    // pending gets its local ids filled in by extra blocks behind the tile blocks
-    const int npb = hop_tile_nodes(n_max, G, s->fuse_small_max);
-    const int tile_blocks = (int)ceil_div(std::max<int64_t>(n_max, 1), npb);
-    int grid = tile_blocks;
-    if (p0.fill_pending >= 0) grid += fill_blocks(s->edge_cap[p0.fill_pending], 256);
-    g.c.tile_blocks = tile_blocks;
+    // one tile of nodes per block; a hop left pending gets its local ids filled in by extra blocks behind the tile blocks
+    int n_seeds = 0;
+    for (int k = 0; k < n; ++k) n_seeds = std::max(n_seeds, pp[k]->n_seeds);
+    const auto [block, passes] = hop_shape(s, n, hop, n_seeds, G);
+    const int npb = block / G * passes;
+    g.c.seed_tiles = g.c.stage_seeds ? (int)ceil_div(s->cfg.batch_size, block) : 0;
+    g.c.tile_blocks = g.c.seed_tiles + (int)ceil_div(std::max<int64_t>(n_max, 1), npb);
+    int grid = g.c.tile_blocks;
+    if (p0.fill_pending >= 0) grid += fill_blocks(s->edge_cap[p0.fill_pending], block);
     for (int k = 0; k < n; ++k) {
       if (pp[k]->fill_pending >= 0) g.p[k].fill = fill_args(*pp[k], pp[k]->fill_pending);
       pp[k]->fill_pending = -1;
     }
-#define LMI_FUSED(GG)                                                                                   \
-  if (npb == 64)                                                                                        \
-    hipLaunchKernelGGL((hop_count_sample_kernel<GG, 64>), dim3((grid) * n), dim3(256), 0, st, g);          \
-  else                                                                                                  \
-    hipLaunchKernelGGL((hop_count_sample_kernel<GG, (256 / GG)>), dim3((grid) * n), dim3(256), 0, st, g);
+#define LMI_HOP2(GG, BB, PP) \
+  else if (block == BB && passes == PP) hipLaunchKernelGGL((hop_kernel<GG, BB, PP>), dim3(grid * n), dim3(BB), 0, st, g);
+#define LMI_HOP(GG)                                                                                                         \
+  if (false) {}                                                                                                             \
+  LMI_HOP2(GG, 256, 1) LMI_HOP2(GG, 512, 1) LMI_HOP2(GG, 1024, 1) LMI_HOP2(GG, 512, 2) LMI_HOP2(GG, 512, 4) LMI_HOP2(GG, 1024, 4) \
+  else LMI_FAIL(LMI_ERR_STATE, "no hop kernel of %d threads, %d passes", block, passes);
     switch (G) {
-      case 4: LMI_FUSED(4) break;
-      case 8: LMI_FUSED(8) break;
-      case 16: LMI_FUSED(16) break;
-      case 32: LMI_FUSED(32) break;
-      default: LMI_FUSED(64) break;
+      case 4: LMI_HOP(4) break;
+      case 8: LMI_HOP(8) break;
+      case 16: LMI_HOP(16) break;
+      case 32: LMI_HOP(32) break;
+      default: LMI_HOP(64) break;
     }
-#undef LMI_FUSED
+#undef LMI_HOP
+#undef LMI_HOP2
   } else {
     // one tile per block (blocks past the real item count leave at once); few items per
     // thread while that keeps the tile count near a thousand: the row-pointer reads are
@@ -799,18 +924,18 @@ int launch_hop(Server *s, Pipe *const *pp, int n, hipStream_t st, int hop, bool 
         default: hipLaunchKernelGGL(hop_sample_kernel<64>, dim3((grid) * n), dim3(256), 0, st, g); break;
       }
     }
-  }
-  const int64_t em = std::max<int64_t>(e_max, 1);
-  const int seed_blocks = (hop == 0 && look.mode != LOOK_NOT) ? (int)ceil_div(s->cfg.batch_size, kScanBlock) : 0;
+    const int64_t em = std::max<int64_t>(e_max, 1);
+    const int seed_blocks = (hop == 0 && look.mode != LOOK_NOT) ? (int)ceil_div(s->cfg.batch_size, kScanBlock) : 0;
 #define LMI_FLAG(I_)                                                                                                 \
-  {                                                                                                                  \
-    g.c.tile_blocks = (int)ceil_div(em, kScanBlock * I_);                                                            \
-    hipLaunchKernelGGL(hop_flag_scan_kernel<I_>, dim3((g.c.tile_blocks + seed_blocks) * n), dim3(kScanBlock), 0, st, g); \
-  }
-  if (em <= 1024 * 1024) LMI_FLAG(2)
-  else if (em <= 2560 * 1024) LMI_FLAG(4)
-  else LMI_FLAG(8)
+    {                                                                                                                  \
+      g.c.tile_blocks = (int)ceil_div(em, kScanBlock * I_);                                                            \
+      hipLaunchKernelGGL(hop_flag_scan_kernel<I_>, dim3((g.c.tile_blocks + seed_blocks) * n), dim3(kScanBlock), 0, st, g); \
+    }
+    if (em <= 1024 * 1024) LMI_FLAG(2)
+    else if (em <= 2560 * 1024) LMI_FLAG(4)
+    else LMI_FLAG(8)
 #undef LMI_FLAG
+  }
   LMI_HIP(hipGetLastError());
   if (hop == 0 && look.mode != LOOK_NOT) (look.mode == LOOK_LRU ? s->routes.lru_scan_lookups : s->routes.scan_lookups) += n;
   for (int k = 0; k < n; ++k) {

@@ -38,18 +38,12 @@ __device__ __forceinline__ void tile_reduce_store(int v, int32_t *tile_sums, int
   __syncthreads();
 }
 
-// The state of a batch that starts: headers, counts, and the parameters where later kernels read them.
+// The state of a batch that starts: counts, and the parameters where later kernels read them.
 // scan_fault and bad_id stay as they are: they hold a batch's number, not a flag, and other blocks of the same launch may
 // be raising them.
-__device__ __forceinline__ void state_begin(DevState *st, const BatchParams &bp, int hops) {
-#pragma unroll
-  for (int i = 0; i < 16; ++i) st->node_counter[i] = st->edge_counter[i] = 0;
-#pragma unroll
-  for (int i = 0; i <= LMI_MAX_HOPS; ++i) st->n_miss[i] = 0;
-  st->node_counter[8] = hops;
-  st->node_counter[9] = bp.n_seeds;
-  st->node_counter[1] = st->node_counter[3] = st->node_counter[5] = bp.n_seeds;
-  st->node_counter[7] = bp.n_seeds;
+// `Params`: a BatchParams, or one in the kernel's argument segment (arg_params).
+template <typename Params>
+__device__ __forceinline__ void state_params(DevState *st, const Params &bp) {
   st->serial = bp.serial;
   st->rng_lo = (uint32_t)bp.rng_seed;
   st->rng_hi = (uint32_t)(bp.rng_seed >> 32);
@@ -61,6 +55,22 @@ __device__ __forceinline__ void state_begin(DevState *st, const BatchParams &bp,
   st->labels_in = bp.labels;
   st->fault = bp.fault;
 }
+__device__ __forceinline__ void state_begin(DevState *st, const BatchParams &bp, int hops) {
+#pragma unroll
+  for (int i = 0; i < 16; ++i) st->node_counter[i] = st->edge_counter[i] = 0;
+  st->node_counter[8] = hops;
+  st->node_counter[9] = bp.n_seeds;
+  st->node_counter[1] = st->node_counter[3] = st->node_counter[5] = bp.n_seeds;
+  st->node_counter[7] = bp.n_seeds;
+  state_params(st, bp);
+}
+// Its miss counts, by device-scope stores: other tiles of the same launch may add to them (behind a wait for this).
+__device__ __forceinline__ void misses_begin(DevState *st) {
+#pragma unroll
+  for (int i = 0; i <= LMI_MAX_HOPS; ++i) __hip_atomic_store(&st->n_miss[i], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// Every load, store and atomic of the wavefront so far has completed: device-scope ones are where all dies see them.
+__device__ __forceinline__ void wait_memory() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
 // Header updates that ride on the scan total (thread 0 of the single block).
 // Reference semantics: counter_update, engine/operator_impl.cu:58-91.
@@ -77,6 +87,22 @@ __device__ __forceinline__ void scan_epilogue(int epilogue, DevState *st, int ho
     st->node_counter[0] = st->node_counter[2] = st->node_counter[4] = n_prev;
     st->node_counter[1] = st->node_counter[3] = st->node_counter[5] = total;
     st->node_counter[7] = n_prev + total;
+  }
+}
+
+// Both headers behind the first hop of a batch that the same launch began: what state_begin and the two epilogues leave, one
+// word a lane (t < 32), because one thread's 45 stores in a row held the tile up that all others of the batch wait for.
+__device__ __forceinline__ void headers_first_hop(DevState *st, int t, int hops, int n_seeds, int edges, int added) {
+  const int i = t & 15;
+  if (t < 16) {
+    int v = 0;
+    if (i == 0 || i == 2 || i == 4 || i == 9) v = n_seeds;
+    else if (i == 1 || i == 3 || i == 5) v = added;
+    else if (i == 7 || i == 10) v = n_seeds + added;
+    else if (i == 8) v = hops;
+    st->node_counter[i] = v;
+  } else {
+    st->edge_counter[i] = i == 1 || i == 10 ? edges : 0;
   }
 }
 
@@ -139,43 +165,49 @@ static __global__ __launch_bounds__(kScanBlock) void scan_apply_kernel(const int
 // atomic ticket would drop the reliance on dispatch order, but 500 same-address
 // atomics cost more than the whole scan.)  The wait is bounded all the same.
 //
-// status[t] = (flag << 32) | value in one 64-bit word, written and read with
-// relaxed device-scope atomics (flag and value travel together, nothing else is
-// exchanged): flag 0 = not ready, 1 = value is the tile's own sum, 2 = value is
-// the inclusive prefix up to and including the tile.  The status words must be
-// zeroed by an earlier kernel of the same stream before each use.
+// A word = stamp << 34 | flag << 32 | value, written and read with relaxed device-scope
+// atomics (they travel together, nothing else is exchanged).  flag 1 = value is the tile's
+// own sum, 2 = value is the inclusive prefix up to and including the tile.  A word with
+// another stamp is a word of another batch or hop, that is: not published yet, so nothing
+// has to be cleared between scans (scan_stamp; the words are zeroed when a pipe's batch
+// numbers start over).
 struct ScanChain {
   unsigned long long *status;  // [max_tiles]
 };
+// Chain `which` of the kScanChains that lie one behind the other at `words`.
+constexpr int kScanChains = 2;
+__host__ __device__ inline ScanChain scan_chain(unsigned long long *words, int max_tiles, int which) {
+  return ScanChain{words + (int64_t)which * max_tiles};
+}
 
-constexpr unsigned long long kScanAggregate = 1ull << 32, kScanInclusive = 2ull << 32;
+constexpr unsigned kScanSum = 1, kScanInclusive = 2;
+static_assert(kMaxSerial < (1 << 28) && LMI_MAX_HOPS <= 4, "a stamp takes 30 bits");
+__device__ __forceinline__ uint32_t scan_stamp(int32_t serial, int hop) { return (uint32_t)serial * 4u + (uint32_t)hop; }
 // A tile that waits longer than this for an earlier tile gives up, raises DevState::scan_fault
 // (and the server's sticky fault word) and writes nothing.  Wall-clock ticks, not re-reads: a
 // legitimate wait is microseconds, whatever else shares the device (wall_clock64 counts at a
 // constant 100 MHz: a quarter of a second).  The clock is read once per 1024 re-reads.
 constexpr long long kScanWaitTicks = 25000000;
 constexpr int kScanFaultPrefix = -1;  // what scan_tile_prefix returns to a tile that gave up
+// Windows of 64 tiles that a tile reads at once.  Tiles that announce at about the same time, as behind a wait for the
+// same thing, find no inclusive prefix near them: every window more in a read is one step less in a chain of steps of a
+// microsecond each.
+constexpr int kScanWindows = 4;
 
-// Zeroes a chain for a later kernel; call from any grid with a flat thread index.
-__device__ __forceinline__ void scan_chain_reset(ScanChain c, int max_tiles, int64_t tid, int64_t n_threads) {
-  for (int64_t i = tid; i < max_tiles; i += n_threads) c.status[i] = 0ull;
+__device__ __forceinline__ void scan_publish(ScanChain c, uint32_t stamp, int tile, unsigned flag, int value) {
+  __hip_atomic_store(&c.status[tile], (unsigned long long)stamp << 34 | (unsigned long long)flag << 32 | (unsigned int)value,
+                     __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-
-__device__ __forceinline__ void scan_publish(ScanChain c, int tile, unsigned long long word) {
-  __hip_atomic_store(&c.status[tile], word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-// Publishes this tile's aggregate; one thread of the block calls, as early as the sum is known.
-__device__ __forceinline__ void scan_tile_announce(ScanChain c, int tile, int aggregate) {
-  scan_publish(c, tile, (tile == 0 ? kScanInclusive : kScanAggregate) | (unsigned int)aggregate);
+// Publishes this tile's sum; one thread of the block calls, as early as the sum is known.
+__device__ __forceinline__ void scan_tile_announce(ScanChain c, uint32_t stamp, int tile, int sum) {
+  scan_publish(c, stamp, tile, tile == 0 ? kScanInclusive : kScanSum, sum);
 }
 
 // Returns the exclusive prefix (sum of all earlier tiles) of a tile that was announced to every
 // thread of the block, or kScanFaultPrefix to every thread when the wait ran out: the tile then
-// has no valid offset and must write nothing.
-// Wavefront 0 looks back 64 tiles per step (lookback_window).  lds_prefix is one shared int.
-// Contains __syncthreads.
-__device__ __forceinline__ int scan_tile_prefix(ScanChain c, int tile, int aggregate, int *lds_prefix,
+// has no valid offset and must write nothing.  lds_prefix is one shared int, not written again
+// before every thread has read it.  Contains __syncthreads.
+__device__ __forceinline__ int scan_tile_prefix(ScanChain c, uint32_t stamp, int tile, int sum, int *lds_prefix,
                                                 DevState *st, FaultTo fault) {
   if (threadIdx.x < kWave) {
     const int lane = threadIdx.x;
@@ -183,32 +215,51 @@ __device__ __forceinline__ int scan_tile_prefix(ScanChain c, int tile, int aggre
     if (tile > 0) {
       int base = tile - 1;
       int spins = 0;
-      // after a first fault every later tile gives up almost at once, so a broken chain drains
-      // in milliseconds
-      const bool broken = st->scan_fault == fault.serial;
-      const long long t0 = wall_clock64();
-      while (true) {
-        const int j = base - lane;
-        unsigned long long w = kScanInclusive;  // before tile 0: an inclusive prefix of 0
-        if (j >= 0) w = __hip_atomic_load(&c.status[j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        const unsigned flag = (unsigned)(w >> 32);
-        const LookbackWindow win = lookback_window(__ballot(flag == 2u), __ballot(flag == 0u));
-        if (win.wait) {  // a tile we need has not published yet: read again
-          ++spins;
-          const bool out_of_time = broken ? spins >= 64 : ((spins & 1023) == 0 && wall_clock64() - t0 > kScanWaitTicks);
-          if (!out_of_time) continue;
-          if (lane == 0) raise_fault(st, kFaultScan, fault);  // never expected; bounded so that the grid always drains
-          prefix = kScanFaultPrefix;
-          break;
-        }
-        int contrib = ((win.take >> lane) & 1ull) ? (int)(unsigned)w : 0;
+      bool broken = false;
+      long long t0 = 0;
+      bool done = false;
+      while (!done) {
+        unsigned long long w[kScanWindows];
 #pragma unroll
-        for (int d = kWave / 2; d > 0; d >>= 1) contrib += __shfl_xor(contrib, d, kWave);
-        prefix += contrib;
-        if (win.done) break;
-        base -= kWave;
+        for (int k = 0; k < kScanWindows; ++k) {
+          const int j = base - k * kWave - lane;
+          w[k] = j >= 0 ? __hip_atomic_load(&c.status[j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0ull;
+        }
+        bool wait = false;
+        int mine = 0, windows = 0;
+#pragma unroll
+        for (int k = 0; k < kScanWindows; ++k) {
+          if (done || wait) continue;
+          const int j = base - k * kWave - lane;
+          unsigned flag = (uint32_t)(w[k] >> 34) == stamp ? (unsigned)(w[k] >> 32) & 3u : 0u;
+          if (j < 0) flag = kScanInclusive;  // before tile 0: an inclusive prefix of 0
+          const LookbackWindow win = lookback_window(__ballot(flag == kScanInclusive), __ballot(flag == 0u));
+          wait = win.wait;
+          if (wait) continue;
+          if (j >= 0 && ((win.take >> lane) & 1ull)) mine += (int)(unsigned)w[k];
+          done = win.done;
+          ++windows;
+        }
+        // the windows in front of one that is not complete stay counted
+        if (windows > 0) {
+          prefix += wave_sum(mine);
+          base -= windows * kWave;
+          continue;
+        }
+        if (++spins == 16) {  // no ordinary wait: it is timed from here
+          // after a first fault every later tile gives up almost at once, so a broken chain drains
+          // in milliseconds
+          broken = st->scan_fault == fault.serial;
+          t0 = wall_clock64();
+        }
+        __builtin_amdgcn_s_sleep(1);
+        const bool out_of_time = broken ? spins >= 64 : ((spins & 1023) == 0 && wall_clock64() - t0 > kScanWaitTicks);
+        if (!out_of_time) continue;
+        if (lane == 0) raise_fault(st, kFaultScan, fault);  // never expected; bounded so that the grid always drains
+        prefix = kScanFaultPrefix;
+        break;
       }
-      if (lane == 0 && prefix != kScanFaultPrefix) scan_publish(c, tile, kScanInclusive | (unsigned int)(prefix + aggregate));
+      if (lane == 0 && prefix != kScanFaultPrefix) scan_publish(c, stamp, tile, kScanInclusive, prefix + sum);
     }
     if (lane == 0) *lds_prefix = prefix;
   }

@@ -149,6 +149,7 @@ static __global__ __launch_bounds__(kSmallBlock) void batch_small_kernel(SmallGr
   if (t == 0) {
     *n_miss = *n_draw = 0;
     state_begin(a.st, bp, g.hops);
+    misses_begin(a.st);
   }
   __syncthreads();
   bool full = false;
@@ -252,7 +253,7 @@ static __global__ __launch_bounds__(kSmallBlock) void batch_small_kernel(SmallGr
       scan_epilogue(SCAN_EPI_HOP_EDGES, a.st, hop, n_edges);
     }
     // ---- first occurrences: ranks in edge order, ids, local ids.  An edge is one iff the value of its slot names the
-    // edge (a published local id never does: it is at most the candidate it replaces, see hop_flag_scan_kernel).
+    // edge (a published local id never does: it is at most the candidate it replaces, see hop_kernel).
     int n_new = 0;
     for (int e0 = 0; e0 < n_edges; e0 += kSmallBlock * kSmallItems) {
       const int e = e0 + t * kSmallItems;

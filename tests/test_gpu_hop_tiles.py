@@ -1,0 +1,54 @@
+"""Every tile of the hop kernel (lane group x threads x nodes per lane group) on both of a tile's edges: batches that are one
+node too many for the next smaller tile, repeated seeds among them, and a short last tile."""
+import numpy as np
+import pytest
+
+from conftest import random_graph
+from test_gpu_parity import assert_batch_equal, make_features
+
+pytestmark = pytest.mark.gpu
+
+N_NODES, DIM, CUS = 150_000, 4, 256
+SHAPES = [(256, 1, 1), (512, 1, 1), (1024, 1, 1), (512, 2, 2), (512, 4, 2), (1024, 4, None)]  # threads, nodes, tiles per CU
+
+
+@pytest.fixture(scope="module")
+def world(lmi):
+    rng = np.random.default_rng(11)
+    indptr, indices = random_graph(rng, N_NODES, 14, hubs=400, hub_deg=300)
+    feats = make_features(lmi, rng, N_NODES, DIM)
+    yield rng, indptr, indices, feats
+    feats.free()
+
+
+@pytest.mark.parametrize("shape", range(len(SHAPES)))
+@pytest.mark.parametrize("fanout", [3, 7, 13, 29, 50])   # lane groups of 4, 8, 16, 32, 64
+def test_tiles_match_the_oracle(lmi, oracle, world, fanout, shape):
+    rng, indptr, indices, feats = world
+    lanes = 4
+    while lanes < fanout:
+        lanes *= 2
+    if shape == 0:
+        batch = 3
+    else:   # two batches: a tile per batch more than the tile before may have
+        threads, nodes, per_cu = SHAPES[shape - 1]
+        batch = per_cu * CUS // 2 * (threads // lanes * nodes) + 1
+    srv = lmi.Server(batch, [fanout, 2], DIM, pipes=2, seed=3)
+    try:
+        srv.load_graph(indptr, indices)
+        srv.attach_features(feats)
+        srv.build_static_cache(N_NODES // 3, lmi.TABLE_RANK)
+        srv.tune("small_edges", 0)
+        slot = oracle.static_cache_build(indptr, N_NODES // 3)
+        for it in range(2):   # without and with what the kernels noted of the batch before
+            seeds = [rng.integers(0, N_NODES, batch).astype(np.int32) for _ in range(2)]
+            seeds[1][-1] = seeds[1][0]
+            srv.run_group([0, 1], [0, 0], seeds=seeds, rng_seeds=[5 + it, 6 + it])
+            for k in range(2):
+                g = srv.fetch(pipe=k)
+                assert_batch_equal(g, oracle.sample_batch(indptr, indices, seeds[k], [fanout, 2], 5 + it + k))
+                np.testing.assert_array_equal(g.cache_index, slot[g.ids])
+                assert g.features.tobytes() == feats.array[g.ids].tobytes()
+        srv.status()
+    finally:
+        srv.close()
