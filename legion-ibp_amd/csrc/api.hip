@@ -949,7 +949,7 @@ static int run_group_launches(Server *s, Pipe *const *pp, const BatchParams *bps
   for (int k = 0; k < n; ++k) pipe_begin(*pp[k], st);
   prof_phase(s, st, &s->prof_open, PROF_SAMPLE);
   const bool lru = s->cache_kind == LMI_CACHE_LRU;
-  bool split = false;
+  bool split = false, early = false, done = false;
   if (s->use_graph && st != nullptr && n == 1) {  // the legacy default stream cannot be captured
     Pipe &p = *pp[0];
     LMI_TRY(lru_wait_ready(s, st));  // the lookup sits inside the graph: the whole replay waits
@@ -970,14 +970,18 @@ static int run_group_launches(Server *s, Pipe *const *pp, const BatchParams *bps
     split = s->split_lookup && s->cfg.hops >= 2 && s->feat_loc == LMI_LOC_HOST && s->split_miss == 1 &&
             (s->cache_kind == LMI_CACHE_STATIC || s->cache_kind == LMI_CACHE_INT8) &&
             (s->split_lookup == 1 || (s->split_lookup == 2 && n > 1)) && !in_line;
+    early = early_rows(s, in_line) && !small_batch(s);
     if (lru_rides) LMI_TRY(lru_wait_ready(s, st));
-    LMI_TRY(launch_sampling(s, pp, bps, n, st, false, HopLookup{mode, 0}, HopLookup{mode, split ? 2 : 0}, split));
+    LMI_TRY(launch_sampling(s, pp, bps, n, st, false, HopLookup{mode, 0, early, pp[0]->handover},
+                            HopLookup{mode, split ? 2 : 0, early, pp[0]->handover}, split));
+    done = early && tile_rows(s);
+    if (done) rows_gathered(s, pp, n, pp[0]->handover);
     if (lru && !lru_rides) {
       LMI_TRY(lru_wait_ready(s, st));  // sampling may overlap the previous batch's insertion, the lookup may not
       LMI_TRY(launch_lookup(s, pp, n, st, 0, s->cfg.hops));
     }
   }
-  LMI_TRY(launch_gather_group(s, pp, n, st, split ? 2 : 0, s->cfg.hops, lru ? 1 : 0, false, 0));
+  if (!done) LMI_TRY(launch_gather_group(s, pp, n, st, split ? 2 : 0, s->cfg.hops, lru ? 1 : 0, false, early ? -1 : 0, nullptr, early));
   prof_phase(s, st, &s->prof_open, -1);
   return LMI_OK;
 }
@@ -1092,10 +1096,12 @@ int lmi_run_once_static(lmi_server *h, void *stream, const int32_t *seeds, int32
   const bool prof = s->prof_on;
   s->prof_on = false;  // profiling creates events: not here
   int rc = batch_params(s, p, st, seeds, n, LMI_LOC_DEVICE, 0, LMI_MODE_TRAIN, rng_seed, &bp);
-  const HopLookup look{one_pass_gather(s) ? LOOK_SLOTS : LOOK_LIST, 0};
-  if (rc == LMI_OK) rc = small_batch(s) ? launch_small(s, pp, &bp, 1, st, look) : launch_sampling(s, pp, &bp, 1, st, true, look, look);
+  const bool early = early_rows(s, true) && !small_batch(s);
   const HeaderCopy headers{out->node_counter, out->edge_counter};
-  if (rc == LMI_OK) rc = launch_gather_group(s, pp, 1, st, 0, s->cfg.hops, 0, true, -1, &headers);
+  const HopLookup look{one_pass_gather(s) ? LOOK_SLOTS : LOOK_LIST, 0, early, nullptr, &headers};
+  if (rc == LMI_OK) rc = small_batch(s) ? launch_small(s, pp, &bp, 1, st, look) : launch_sampling(s, pp, &bp, 1, st, true, look, look);
+  if (rc == LMI_OK && early && tile_rows(s)) rows_gathered(s, pp, 1, nullptr);
+  else if (rc == LMI_OK) rc = launch_gather_group(s, pp, 1, st, 0, s->cfg.hops, 0, true, -1, &headers, early);
   s->prof_on = prof;
   return rc;
 }

@@ -19,6 +19,7 @@
 
 #include <hip/hip_ext.h>
 
+#include "gather.hpp"
 #include "scan.hpp"
 
 namespace lmi {
@@ -127,9 +128,7 @@ static __global__ __launch_bounds__(256) void move_rows_kernel(
   }
 }
 
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-typedef u32x4 u32x4_a4 __attribute__((aligned(4)));  // a 16-byte access at a 4-byte-aligned address
 
 // Row mover for rows that a power-of-two lane group does not fit: 400-byte rows (25 chunks of
 // 16 bytes would leave 7 of 32 lanes idle), rows that are no multiple of 16 bytes, rows whose
@@ -265,102 +264,25 @@ static __global__ __launch_bounds__(256) void move_rows_tiled_kernel(
   }
 }
 
-// The HBM gather, for fp32 / fp16 rows of every size from 16 bytes up.  Output rows [first, n)
-// directly, source row = src_index[row] (a cache slot; outside [0, n_src) = nothing to move).  A block takes a
-// tile of consecutive rows and its 256 threads walk the tile's 16-byte units in flat order -- unit f is
-// piece f % upr of row f / upr -- U units per lane and pass: the U slots (lanes of one row read the
-// same word: one cache line per wavefront), then the U row pieces, then the U stores, each step
-// issued whole before the next waits.  Lanes without a unit, or whose row is a miss, issue nothing
-// (every access they would make costs the memory pipeline a cycle whether or not HBM sees it).
-// Nothing else stands between a block and its bytes: no LDS, no barrier.  Measured against the same
-// loop with computed source rows on one output buffer, this shape keeps 90 % of its rate; staging a
-// tile's rows through LDS first kept 70 %.  A row that is no multiple of 16 bytes ends with a unit
-// that overlaps the one before it (both write the same bytes), so every access is 16 bytes wide, at
-// 4-byte alignment when the row length demands it (V16 says which).
-// MISSES: a row without a slot is read from the feature table by its node id in the same pass (gather_in_line says
-// when).  The table may lie behind the host link: the wavefronts that hold such rows then wait for the link, which
-// bounds the launch, while the hits of all others stream past.
-// LOOK: the slots are not known yet: a block looks its tile's rows up first, a thread each, and hands the slots to the
-// others through LDS.  One read in a row more per tile instead of a launch and a pass over the ids.
+// The HBM gather as a launch of its own (gather_rows).  LOOK: the slots are not known yet (`look` there).
 // rows_seen (pinned host memory, or null): the launch leaves each pipe's row count there for the host
 // to size later grids by (see launch_gather_flat).
-constexpr int kFlatTileMax = 256;  // rows per tile
 template <typename V16, int U, bool NT, bool MISSES, bool LOOK>
-static __global__ __launch_bounds__(256) void gather_rows_flat_kernel(MoveGroup g, const uint8_t *__restrict__ src,
-                                                                      uint32_t n_src, const uint8_t *__restrict__ table,
-                                                                      uint32_t n_table, int upr, int last_off,
-                                                                      int rows_per_tile, int64_t src_pitch,
-                                                                      int64_t dst_pitch, unsigned long long *row_counter,
+static __global__ __launch_bounds__(256) void gather_rows_flat_kernel(MoveGroup g, RowSources from, int upr, int last_off,
+                                                                      int rows_per_tile, int64_t dst_pitch,
+                                                                      unsigned long long *row_counter,
                                                                       int32_t *rows_seen, SlotTable look) {
   __shared__ int s_slot[LOOK ? kFlatTileMax : 1];
   LMI_GRID_ROW_TAIL(g);
   const MoveRow &r = g.p[row];
-  const int32_t *__restrict__ src_index = r.src_index;
-  const int32_t *__restrict__ ids = r.ids;
-  uint8_t *__restrict__ dst = r.dst;
   const int n = *r.n_ptr;
   const int first = r.first_ptr ? *r.first_ptr : 0;
   if (bx == 0 && threadIdx.x == 0) {
     if (row_counter && n > first) atomicAdd(row_counter, (unsigned long long)(n - first));  // profiling
     if (rows_seen) rows_seen[row] = n - first;
   }
-  const int dq = (256 * 1) / upr, dr = 256 % upr;  // what 256 units further means in (row, piece)
-  const int r0 = (int)threadIdx.x / upr, u0 = (int)threadIdx.x % upr;
-  const int n_tiles = (n - first + rows_per_tile - 1) / rows_per_tile;
-  for (int tile = bx; tile < n_tiles; tile += gx) {
-    const int row0 = first + tile * rows_per_tile;
-    const int nr = n - row0 < rows_per_tile ? n - row0 : rows_per_tile;
-    const int lim = nr * upr;
-    if constexpr (LOOK) {
-      __syncthreads();  // the tile before is done with its slots
-      if ((int)threadIdx.x < nr) {
-        const int32_t node = ids[row0 + threadIdx.x];
-        const int32_t found = (uint32_t)node < n_table ? static_find(look, node) : -1;
-        s_slot[threadIdx.x] = found;
-        r.look_index[row0 + threadIdx.x] = found;
-      }
-      __syncthreads();
-    }
-    int rr = r0, uu = u0;
-    for (int f0 = threadIdx.x; f0 < lim; f0 += 256 * U) {
-      int slot[U], id[U], off[U];
-      int64_t da[U];
-      V16 v[U];
-#pragma unroll
-      for (int k = 0; k < U; ++k) {
-        const int i = row0 + rr;
-        slot[k] = id[k] = -1;
-        if (f0 + 256 * k < lim) {
-          slot[k] = LOOK ? s_slot[rr] : src_index[i];
-          if (MISSES) id[k] = ids[i];  // beside the slot, not behind it: a miss waits for one read, not for two
-        }
-        off[k] = (uu == upr - 1) ? last_off : 16 * uu;
-        da[k] = (int64_t)i * dst_pitch + off[k];
-        uu += dr;
-        rr += dq;
-        if (uu >= upr) {
-          uu -= upr;
-          ++rr;
-        }
-      }
-      const uint8_t *at[U];
-#pragma unroll
-      for (int k = 0; k < U; ++k) {
-        at[k] = (uint32_t)slot[k] < n_src ? src + (int64_t)slot[k] * src_pitch + off[k] : nullptr;
-        if (MISSES && !at[k] && (uint32_t)id[k] < n_table) at[k] = table + (int64_t)id[k] * src_pitch + off[k];
-      }
-#pragma unroll
-      for (int k = 0; k < U; ++k)
-        if (at[k]) v[k] = __builtin_nontemporal_load(reinterpret_cast<const V16 *>(at[k]));
-#pragma unroll
-      for (int k = 0; k < U; ++k)
-        if (at[k]) {
-          V16 *d = reinterpret_cast<V16 *>(dst + da[k]);
-          if (NT) __builtin_nontemporal_store(v[k], d);
-          else *d = v[k];
-        }
-    }
-  }
+  gather_rows<V16, 256, U, NT, MISSES>(from, r.src_index, r.ids, r.dst, first, n, upr, last_off, rows_per_tile, dst_pitch, bx, gx,
+                                       LOOK, look, r.look_index, s_slot);
 }
 
 // Grid of a gather whose real row count only the device knows.  The worst case of a batch is about
@@ -496,27 +418,26 @@ static int tiled_tile_rows(Server *s, int64_t row_bytes) {
   return t;
 }
 
-// Rows per tile of the flat gather: about 8 KB worth of rows, two at least.
 static int launch_gather_flat(Server *s, hipStream_t st, const MoveArgs &a, bool nt, bool aligned16) {
   const int upr = (int)((a.row_bytes + 15) / 16);
   const int last_off = (int)a.row_bytes - 16;
   const int u_want = s->gather_unroll > 0 ? s->gather_unroll : 2;
   const int U = u_want >= 4 ? 4 : u_want >= 2 ? 2 : 1;
-  int rpt = (int)std::max<int64_t>(2, std::min<int64_t>(64, 8192 / a.row_bytes));
+  int rpt = flat_tile_rows(a.row_bytes);
   if (s->gather_tile_rows > 0) rpt = std::min(s->gather_tile_rows, kFlatTileMax);
   const int64_t want = ceil_div(a.note_rows >= 0 ? hinted_rows(s, a.n_max, a.note_rows) : a.n_max, rpt);
   const int64_t cap = a.max_blocks > 0 ? a.max_blocks : s->gather_blocks > 0 ? s->gather_blocks : (int64_t)s->n_cu * 64;
   const int grid = (int)std::max<int64_t>(1, std::min(want, cap)) + a.g.tail_blocks;
   const SlotTable look = slot_table(s);
+  const RowSources from{a.src, a.table, (uint32_t)a.n_src, (uint32_t)a.n_table, a.src_row_bytes};
 #define LMI_FLAT(V_, U_, NT_, M_, L_)                                                                                      \
   if (a.ev_start || a.ev_stop)                                                                                         \
     hipExtLaunchKernelGGL((gather_rows_flat_kernel<V_, U_, NT_, M_, L_>), dim3(grid * a.g.n), dim3(256), 0, st,             \
-                          a.ev_start, a.ev_stop, 0, a.g, a.src, (uint32_t)a.n_src, a.table, (uint32_t)a.n_table, upr,   \
-                          last_off, rpt, a.src_row_bytes, a.dst_row_bytes, a.row_counter, a.note_rows >= 0 ? s->rows_seen_dev + a.note_rows : nullptr, look); \
+                          a.ev_start, a.ev_stop, 0, a.g, from, upr, last_off, rpt, a.dst_row_bytes, a.row_counter, \
+                          a.note_rows >= 0 ? s->rows_seen_dev + a.note_rows : nullptr, look); \
   else                                                                                                                 \
-    hipLaunchKernelGGL((gather_rows_flat_kernel<V_, U_, NT_, M_, L_>), dim3(grid * a.g.n), dim3(256), 0, st, a.g, a.src,    \
-                       (uint32_t)a.n_src, a.table, (uint32_t)a.n_table, upr, last_off, rpt, a.src_row_bytes,           \
-                       a.dst_row_bytes, a.row_counter, a.note_rows >= 0 ? s->rows_seen_dev + a.note_rows : nullptr, look)
+    hipLaunchKernelGGL((gather_rows_flat_kernel<V_, U_, NT_, M_, L_>), dim3(grid * a.g.n), dim3(256), 0, st, a.g, from, upr, \
+                       last_off, rpt, a.dst_row_bytes, a.row_counter, a.note_rows >= 0 ? s->rows_seen_dev + a.note_rows : nullptr, look)
 #define LMI_FLAT_U(V_, NT_)                        \
   if (a.look) { LMI_FLAT(V_, 2, NT_, true, true); }         \
   else if (a.table) { LMI_FLAT(V_, 2, NT_, true, false); }  \
@@ -1286,6 +1207,39 @@ bool gather_in_line(const Server *s, Pipe *const *pp, int n, int seg_last) {
   return true;
 }
 
+// Whether the hops' launches gather the rows that a batch knows before them (early_rows), and the last hop's tiles the rows
+// they add (tile_rows), in place of a gather behind the hops: where the misses come over the host link on the caller's
+// stream, in one pass with the hits.  The link, which bounds such a batch, then works while the hops are sampled, and starts
+// on a tile's misses while others are still being ranked; a launch and a pass over ids and slots go.  Not with the LRU
+// cache, whose batches miss little, and not from a table in HBM, whose reads the hops' own wait for.  Blocks and tiles of a
+// hop move hits more slowly than a grid of the gather's own, which shows for long rows where most are hits: hence the
+// limits, by the share of the nodes in the cache (us a batch of 800 seeds, 10,5, behind the hops / so, without the limits):
+//   400-byte rows, 20 % 76 / 54, 50 % 70 / 51, 90 % 46 / 38, 99 % 44 / 38;  1 536 bytes, 80 % 50 / 48, 95 % 45 / 46;
+//   2 408 bytes, 20 % 216 / 196, 60 % 82 / 76, 80 % 57 / 55, 90 % 51 / 59;  3 600 bytes, early_rows alone 60 % 101 / 95, both
+//   105;  5 732 bytes, early_rows alone 20 % 453 / 436, 60 % 139 / 134, 90 % 70 / 77, both 20 % 457, 60 % 155;
+//   4 000 seeds, 5,4: 1 536 bytes 80 % 81 / 78, 95 % 61 / 68;  4 096 bytes, early_rows alone 90 % 108 / 103, 95 % 94 / 100.
+struct RowLimits {
+  int64_t early, tile;
+};
+static RowLimits row_limits(const Server *s) {
+  if (s->cache_kind == LMI_CACHE_NONE) return {4096, 4096};  // (longer ones are listed, see one_pass_gather)
+  if (s->cache_rows * 10 > s->n_nodes * 9) return {512, 512};
+  if (s->cache_rows * 4 > s->n_nodes * 3) return {4096, 1536};
+  return {INT64_MAX, 2560};
+}
+bool early_rows(const Server *s, bool in_line) {
+  return in_line && one_pass_gather(s) && s->feat_loc == LMI_LOC_HOST && !no_miss_possible(s) && s->fuse_count && !s->lds_dedup &&
+         (s->cache_kind == LMI_CACHE_STATIC || s->cache_kind == LMI_CACHE_NONE) && s->row_bytes <= row_limits(s).early;
+}
+bool tile_rows(const Server *s) { return s->row_bytes <= row_limits(s).tile; }
+// Their blocks (of 256 threads), for all batches of a launch: a grid that fills the link, as in launch_hits; more where the
+// rows, most of which are hits, would take such a grid longer than a hop takes.
+int early_rows_blocks(const Server *s, int64_t rows) {
+  const int64_t link = s->miss_blocks > 0 ? s->miss_blocks : s->miss_blocks == 0 ? s->n_cu : 96;
+  if (s->cache_kind == LMI_CACHE_NONE) return (int)link;
+  return (int)std::max<int64_t>(link, std::min<int64_t>(ceil_div(rows * s->row_bytes, 1 << 17), 2048));
+}
+
 // Lookup and gather of one segment in one launch (operator by operator; gather_in_line and one_pass_gather hold): a static
 // cache with full-width rows.  The operators of a products-shaped batch: 126 us with
 // three lookup launches (and one more at the start of the batch), 109 without.
@@ -1323,8 +1277,25 @@ int launch_misses_early(Server *s, Pipe *const *pp, int n, hipStream_t st, int s
 // With 1 and 2 the caller's stream does not wait here: the next call on this pipe,
 // or lmi_batch_wait, joins.  A segment of an LRU batch joins at once (a later call
 // inserts the gathered rows).
+// Whether a side stream's join event ends batches like this one: behind that nobody follows the stream that takes a batch, so
+// neither where the gather is in line only because that side stream would have nothing to overlap.
+static bool batch_sided(const Server *s, bool early_fork) {
+  return s->feat_loc == LMI_LOC_HOST && s->cache_kind != LMI_CACHE_NONE && (s->split_miss == 2 || (s->split_miss == 1 && !early_fork));
+}
+static bool early_forked(const Server *s, int n) { return s->early_fork == 1 || (s->early_fork == 2 && n > 1); }
+
+void rows_gathered(Server *s, Pipe *const *pp, int n, hipEvent_t end) {
+  s->routes.one_pass_gathers += n;
+  for (int k = 0; k < n; ++k) {
+    pp[k]->tail_follow = !batch_sided(s, early_forked(s, n));
+    pp[k]->tail_unjoined = true;
+    pp[k]->tail_event = end;
+  }
+}
+
 int launch_gather_group(Server *s, Pipe *const *pp, int n, hipStream_t st, int seg, int seg_last, int lru_lists,
-                        bool same_stream, int hit_seg_first, const HeaderCopy *headers) {
+                        bool same_stream, int hit_seg_first, const HeaderCopy *headers, bool early_rows) {
+  if (early_rows) seg = seg_last;  // the hops' launches took the rows before the last hop's
   const int hit_seg = hit_seg_first >= 0 ? hit_seg_first : seg;  // the hits of segments whose misses went ahead
   const bool have_cache = s->cache_kind != LMI_CACHE_NONE;
   const bool in_line = same_stream || gather_in_line(s, pp, n, seg_last);
@@ -1336,17 +1307,14 @@ int launch_gather_group(Server *s, Pipe *const *pp, int n, hipStream_t st, int s
   // What a batch leaves on the caller's stream ends with a kernel of its gather, which carries an event that says so (the
   // first pipe's for all pipes of a group): recorded behind it the event would be a packet of its own, and recorded when
   // another stream asks it would stand for whatever is queued by then.  Not for a segment: its batch goes on.
-  const bool whole = hit_seg == 0 && seg_last == s->cfg.hops;
+  const bool whole = (hit_seg == 0 || early_rows) && seg_last == s->cfg.hops;
   const hipEvent_t end = whole && !s->prof_on ? pp[0]->handover : nullptr;
   // LRU batches are host-link-bound (a fifth of their rows miss): their host-link gather starts
   // beside the HBM gather instead of behind it.  The insertion that follows it on the side stream
   // only overwrites ways this batch's lookup did not touch, so the hits never read a row it writes.
   const bool early = (lru_lists > 0 && s->lru_early_miss) ||
-                     (lru_lists == 0 && (s->early_fork == 1 || (s->early_fork == 2 && n > 1)));
-  // Behind a side stream's join event nobody follows the stream that takes a batch, so neither where the gather is in
-  // line only because that side stream would have nothing to overlap.
-  const bool sided = s->feat_loc == LMI_LOC_HOST && have_cache && (s->split_miss == 2 || (s->split_miss == 1 && !early));
-  for (int k = 0; k < n; ++k) pp[k]->tail_follow = !sided;
+                     (lru_lists == 0 && early_forked(s, n));
+  for (int k = 0; k < n; ++k) pp[k]->tail_follow = !batch_sided(s, early);
   if (mode == 0) {
     const bool last_hits = lru_lists == 0 && (one_pass_gather(s) || no_miss_possible(s));
     for (int k = 0; k < n; ++k) {

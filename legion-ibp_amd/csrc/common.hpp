@@ -299,10 +299,17 @@ void prof_kernel_events(Server *s, int kind, hipEvent_t *start, hipEvent_t *stop
 // stage_seeds: also run the seed-staging kernel now (otherwise hop 0 stages them itself)
 int launch_batch_generate(Server *s, Pipe *const *pp, const BatchParams *bps, int n, hipStream_t st, bool stage_seeds);
 int graph_update_begin(Server *s, Pipe &p, const BatchParams &bp);
+struct HeaderCopy {
+  int32_t *nodes, *edges;
+};
 // The cache lookup of the nodes a hop adds (hop 0: of the seeds too), in its kernel.
 struct HopLookup {
   int mode = 0;      // LOOK_*
   int miss_seg = 0;  // LOOK_LIST: the miss list that receives them
+  // Blocks of the hop's launch gather the rows known before it, and the last hop's tiles the rows they add (early_rows()).
+  bool early_rows = false;
+  hipEvent_t end = nullptr;                // with early_rows: an event that marks the end of the last hop, and of the batch
+  const HeaderCopy *headers = nullptr;     // with early_rows: see launch_gather_group
 };
 // not at all; cache_index only; cache_index and the miss list; the same in the LRU cache, whose hits are marked and whose
 // misses go on the lists of their sets
@@ -350,15 +357,18 @@ int launch_gather_seg(Server *s, Pipe &p, hipStream_t st, int seg, int seg_last,
 // (group_miss), or all rows in one where the gather is in line (gather_in_line, one_pass_gather).
 // same_stream: everything on `st` whatever the schedule knob says (nothing is left pending).
 // headers: where the caller of the static entry point wants the two 16-int headers (one pipe), or null.
-struct HeaderCopy {
-  int32_t *nodes, *edges;
-};
 int launch_gather_group(Server *s, Pipe *const *pp, int n, hipStream_t st, int seg, int seg_last, int lru_lists,
-                        bool same_stream = false, int hit_seg_first = -1, const HeaderCopy *headers = nullptr);
+                        bool same_stream = false, int hit_seg_first = -1, const HeaderCopy *headers = nullptr,
+                        bool early = false);
+// The pipes of batches whose hops gathered all rows on the caller's stream (early_rows), `end` marking their end.
+void rows_gathered(Server *s, Pipe *const *pp, int n, hipEvent_t end);
 // whether the misses of these batches are gathered on the caller's stream, and whether in the same pass as the hits
 // (no miss list is needed then)
 bool gather_in_line(const Server *s, Pipe *const *pp, int n, int seg_last);
 bool one_pass_gather(const Server *s);
+bool early_rows(const Server *s, bool in_line);
+bool tile_rows(const Server *s);
+int early_rows_blocks(const Server *s, int64_t rows);
 // the host-link gather of segments [seg, seg_last] released now, ahead of the batch's later hops (split_lookup)
 int launch_misses_early(Server *s, Pipe *const *pp, int n, hipStream_t st, int seg, int seg_last);
 // end: an event that marks the end of the insertion, or null

@@ -21,6 +21,9 @@
 // Batches expected to be small go through one workgroup instead (small.hip).
 #include <algorithm>
 
+#include <hip/hip_ext.h>
+
+#include "gather.hpp"
 #include "scan.hpp"
 
 namespace lmi {
@@ -44,12 +47,16 @@ struct HopShared {  // what the pipes of a launch have in common
   int look_mode, miss_seg;
   SlotTable cache;
   LruSets lru;  // LOOK_LRU
+  // hop_kernel: its first blocks gather the rows that the batch knew before the hop and that no launch before gathered
+  int gather_blocks, upr, last_off, rows_per_tile;
+  int tile_rows;  // last hop: every tile gathers the rows it adds and fills in its edges' local ids, and the batch is complete
+  RowSources rows;
 };
 struct HopArgs {
   DevState *st;
   int32_t *ids, *labels;
   int32_t *row_ptr;  // block CSR row pointers of this hop
-  int32_t *agg_src_ids, *agg_dst_off;
+  int32_t *agg_src_ids, *agg_src_off, *agg_dst_off;
   HashSlot *slots;
   int32_t *eslot;   // table slot per edge of this hop (| kKnownRepeat)
   unsigned long long *scan_words;
@@ -58,6 +65,8 @@ struct HopArgs {
   int32_t *cache_index;
   int2 *miss_list;
   int32_t *lru_fill, *lru_next;
+  uint8_t *features;
+  HeaderCopy headers;  // HopShared::tile_rows: where the headers go besides the state (nodes null: nowhere)
 };
 
 // Several mini-batches (pipes) can share every launch of the sampling phase: block b
@@ -395,6 +404,14 @@ __device__ __forceinline__ void rows_looked_up(const HopGroup &g, const HopArgs 
   }
 }
 
+// Copies the headers, which the block has just left in the state, to where the caller wants them too.
+__device__ __forceinline__ void headers_copy(const HopGroup &g, const HopArgs &a, int t) {
+  if (!g.c.tile_rows || !a.headers.nodes) return;
+  __syncthreads();
+  if (t < 16) a.headers.nodes[t] = a.st->node_counter[t];
+  else if (t < 32) a.headers.edges[t - 16] = a.st->edge_counter[t - 16];
+}
+
 // ------------------------------------------------------------- hop, one launch
 // All of a hop by tiles of NPB nodes, G lanes per node: row pointers and counts (wavefront 0), draws and neighbour reads,
 // inserts into the dedup table, the tile's edge offset (look-back), first occurrences and their ranks (look-back), ids and
@@ -411,22 +428,41 @@ __device__ __forceinline__ void rows_looked_up(const HopGroup &g, const HopArgs 
 // a hop paid a launch and three dependent reads more.  us a pass, two launches per hop / one: 800 seeds, 25,10, a third of
 // the rows cached 110.6 / 102.4; 8 000 seeds, all rows cached 80.9 / 73.7; four such batches from a table in HBM 303 / 290;
 // 1 024 seeds, 15,10,5, four batches in a row through the LRU cache 350 / 298.
+// Rows (early_rows, tile_rows say when): blocks ahead of the tiles gather what was known before the hop, the last hop's tiles
+// what they add, and those then fill in their edges' local ids behind a third look-back, for tiles whose rows are published:
+// the batch ends with the hop.  The first of the two cases above is bound by 2.9 MB over the host link (70 us): 102.4 us with
+// a gather of its own, 94.9 with early rows, 89.5 with both.
+// 64 registers and 96 scalar ones at most, so that two blocks of 1024 threads share a CU: the last tiles of a hop otherwise
+// waited for the first to end.
 template <int G, int BLOCK, int PASSES>
-static __global__ __launch_bounds__(BLOCK) void hop_kernel(HopGroup g) {
-  LMI_GRID_ROW(g.n);
+static __global__ __launch_bounds__(BLOCK, 8) void hop_kernel(HopGroup g) {
+  const GridRow grid = grid_row(blockIdx.x, (unsigned)g.n);
+  const int row = grid.row, bx = grid.bx - g.c.gather_blocks, gx = (int)(gridDim.x / (unsigned)g.n) - g.c.gather_blocks;
   const HopArgs &a = g.p[row];  // this block's pipe (mini-batch)
   constexpr int PER_PASS = BLOCK / G, NPB = PER_PASS * PASSES, WAVES = BLOCK / kWave;
   static_assert(NPB <= BLOCK, "a thread per node");
   __shared__ int32_t s_id[NPB];
   __shared__ int64_t s_beg[NPB], s_deg[NPB];
   __shared__ int s_row[NPB];
-  __shared__ int s_total, s_edge0, s_rank0, s_miss0;
+  __shared__ int s_total, s_edge0, s_rank0, s_miss0, s_published;
   __shared__ int s_cnt[PASSES * WAVES];
   __shared__ int s_scan[WAVES + 1];
+  __shared__ int s_slot[kFlatTileMax];
   DevState *st = a.st;
   if (bx >= g.c.tile_blocks) {  // extra blocks: the previous hop's local ids
     fill_local_ids(a.fill, (int64_t)(bx - g.c.tile_blocks) * blockDim.x + threadIdx.x,
                    (int64_t)(gx - g.c.tile_blocks) * blockDim.x);
+    return;
+  }
+  if (bx < 0) {  // the blocks ahead of the tiles: rows known before this hop (early_rows)
+    ArgParams &bp = arg_params(row);
+    const bool first_hop = g.c.hop == 0;
+    const int first = first_hop ? 0 : st->node_counter[9 + g.c.hop - 1];
+    const int n = first_hop && g.c.begin ? bp.n_seeds : st->node_counter[9 + g.c.hop];
+    const int32_t *ids = !first_hop ? a.ids : g.c.begin ? bp.seeds : st->seeds;
+    gather_rows<u32x4_a4, BLOCK, 2, true, true>(g.c.rows, a.cache_index, ids, a.features, first, n, g.c.upr, g.c.last_off,
+                                                g.c.rows_per_tile, g.c.rows.pitch, bx + g.c.gather_blocks, g.c.gather_blocks,
+                                                first_hop, g.c.cache, nullptr, s_slot);
     return;
   }
   const int seed_tiles = g.c.seed_tiles;
@@ -442,17 +478,21 @@ static __global__ __launch_bounds__(BLOCK) void hop_kernel(HopGroup g) {
   const int n_prev = begin ? bp.n_seeds : st->node_counter[9 + g.c.hop];
   const int n_tiles = seed_tiles + (n_prev + NPB - 1) / NPB;
   if (tile >= n_tiles) {
-    if (n_tiles == 0 && tile == 0 && t == 0) {
-      a.row_ptr[0] = 0;
-      scan_epilogue(SCAN_EPI_HOP_EDGES, st, g.c.hop, 0);
-      scan_epilogue(SCAN_EPI_HOP_NODES, st, g.c.hop, 0);
+    if (n_tiles == 0 && tile == 0) {
+      if (t == 0) {
+        a.row_ptr[0] = 0;
+        scan_epilogue(SCAN_EPI_HOP_EDGES, st, g.c.hop, 0);
+        scan_epilogue(SCAN_EPI_HOP_NODES, st, g.c.hop, 0);
+      }
+      headers_copy(g, a, t);
     }
     return;
   }
   const bool last = tile == n_tiles - 1;
   if (begin && tile == 0 && t == 0) misses_begin(st);  // complete before any tile gets past this one's inserts
   const uint32_t stamp = scan_stamp(fault.serial, g.c.hop);
-  const ScanChain edges = scan_chain(a.scan_words, g.c.max_tiles, 0), firsts = scan_chain(a.scan_words, g.c.max_tiles, 1);
+  const ScanChain edges = scan_chain(a.scan_words, g.c.max_tiles, 0), firsts = scan_chain(a.scan_words, g.c.max_tiles, 1),
+                  published = scan_chain(a.scan_words, g.c.max_tiles, 2);
   const int32_t tag = begin ? bp.table_tag : st->table_tag, tag_mask = begin ? bp.table_mask : st->table_mask;
   const int32_t *seeds = g.c.stage_seeds ? (begin ? bp.seeds : st->seeds) : nullptr;
   const int look_mode = g.c.look_mode;
@@ -463,7 +503,10 @@ static __global__ __launch_bounds__(BLOCK) void hop_kernel(HopGroup g) {
 
   if (tile < seed_tiles) {
     const int i = tile * BLOCK + t;
-    if (t == 0) scan_tile_announce(firsts, stamp, tile, 0);
+    if (t == 0) {
+      scan_tile_announce(firsts, stamp, tile, 0);
+      scan_tile_announce(published, stamp, tile, 0);
+    }
     if (i < n_prev) {
       const int32_t *labels = begin ? bp.labels : st->labels_in;
       node[0] = seeds[i];
@@ -590,7 +633,7 @@ static __global__ __launch_bounds__(BLOCK) void hop_kernel(HopGroup g) {
       const int e = edge0 + s_row[t / G + u * PER_PASS] + lane;
       a.agg_src_ids[eoff + e] = node[u];
       a.agg_dst_off[eoff + e] = node0 + u * PER_PASS;
-      a.eslot[e] = (int)slot[u];
+      if (!g.c.tile_rows) a.eslot[e] = (int)slot[u];
     }
     if (t < NPB && my < n_prev) a.row_ptr[my] = edge0 + ex;
     const int rank0 = scan_tile_prefix(firsts, stamp, tile, added, &s_rank0, st, fault);
@@ -613,9 +656,29 @@ static __global__ __launch_bounds__(BLOCK) void hop_kernel(HopGroup g) {
         scan_epilogue(SCAN_EPI_HOP_NODES, st, g.c.hop, rank0 + added);
       }
     }
+    if (g.c.tile_rows) {
+      if (look_mode != LOOK_NOT)
+        rows_looked_up<PASSES, BLOCK>(g, a, false, node, local, slot_of, look, tag, tag_mask, s_scan, &s_miss0);
+      wait_memory();
+      __syncthreads();
+      if (t == 0) scan_tile_announce(published, stamp, tile, 0);
+      const int row0 = n_prev + rank0;
+      gather_rows<u32x4_a4, BLOCK, PASSES == 1 ? 4 : 2, true, true>(g.c.rows, a.cache_index, a.ids, a.features, row0, row0 + added, g.c.upr,
+                                                  g.c.last_off, added, g.c.rows.pitch, 0, 1, false, g.c.cache, nullptr,
+                                                  s_slot);
+      // the first occurrence of an edge's source lies in this tile or in an earlier one
+      if (scan_tile_prefix(published, stamp, tile, 0, &s_published, st, fault) == kScanFaultPrefix) return;
+#pragma unroll
+      for (int u = 0; u < PASSES; ++u) {
+        if (!on[u]) continue;
+        const int e = edge0 + s_row[t / G + u * PER_PASS] + lane;
+        a.agg_src_off[eoff + e] = __hip_atomic_load(&a.slots[slot[u] & ~kKnownRepeat].val, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+    }
   }
+  if (last) headers_copy(g, a, t);
   if (tile == 0 && t == 0 && row == 0 && g.c.nodes_seen) *g.c.nodes_seen = n_prev;  // for the host to shape later launches by
-  if (look_mode != LOOK_NOT)
+  if (look_mode != LOOK_NOT && !(g.c.tile_rows && tile >= seed_tiles))
     rows_looked_up<PASSES, BLOCK>(g, a, tile < seed_tiles, node, local, slot_of, look, tag, tag_mask, s_scan, &s_miss0);
 }
 
@@ -795,12 +858,15 @@ bool hop_sets_up(const Server *s) { return s->fuse_count && !s->lds_dedup; }
 //   four such batches, second hop: 512x4 1 172 278.6, 1024x4 586 274.7, 256x4 2 344 285.4, 256x1 355.6;
 //   1 024 seeds, 15,10,5, third hop (20 000 nodes): 256x1 625 295.3, 1024x1 157 281.6, 512x4 78 284.7.
 // The nodes of a hop are those that the last batches knew there; before the first, the graph's mean degree tells.
-HopShape hop_shape(const Server *s, int n, int hop, int n_seeds, int G) {
+static int64_t hop_nodes(const Server *s, int hop, int n_seeds) {
   const int64_t seen = hop > 0 && s->nodes_seen_host ? s->nodes_seen_host[hop] : 0;
   int64_t nodes = seen > 0 ? seen : n_seeds;
   const double mean = s->n_nodes > 0 ? (double)s->n_edges / (double)s->n_nodes : 0;
   for (int k = 0; k < hop && seen <= 0; ++k) nodes += (int64_t)((double)nodes * std::min<double>(mean, s->cfg.fanout[k]));
-  nodes = std::max<int64_t>(1, std::min(nodes, s->node_cap[hop]));
+  return std::max<int64_t>(1, std::min(nodes, s->node_cap[hop]));
+}
+HopShape hop_shape(const Server *s, int n, int hop, int n_seeds, int G) {
+  const int64_t nodes = hop_nodes(s, hop, n_seeds);
   constexpr HopShape kOnePass[] = {{256, 1}, {512, 1}, {1024, 1}}, kMore[] = {{512, 2}, {512, 4}};
   for (const HopShape &h : kOnePass)
     if (n * ceil_div(nodes, h.block / G) <= s->n_cu) return h;
@@ -842,6 +908,7 @@ int launch_hop(Server *s, Pipe *const *pp, int n, hipStream_t st, int hop, bool 
     a.labels = p.labels;
     a.row_ptr = p.blk_indptr[hop];
     a.agg_src_ids = p.agg_src_ids;
+    a.agg_src_off = p.agg_src_off;
     a.agg_dst_off = p.agg_dst_off;
     a.slots = p.dedup.slots;
     a.eslot = p.eslot[hop & 1];
@@ -851,6 +918,7 @@ int launch_hop(Server *s, Pipe *const *pp, int n, hipStream_t st, int hop, bool 
     a.miss_list = p.miss_list + miss_list_base(s, look.miss_seg);
     a.lru_fill = p.lru_fill;
     a.lru_next = p.lru_next;
+    a.features = (uint8_t *)p.features;
     if (look.mode == LOOK_LRU) p.lru_chained = true;
     if (begin) {
       a.bp = begin[k];
@@ -869,17 +937,31 @@ int launch_hop(Server *s, Pipe *const *pp, int n, hipStream_t st, int hop, bool 
     int n_seeds = 0;
     for (int k = 0; k < n; ++k) n_seeds = std::max(n_seeds, pp[k]->n_seeds);
     const auto [block, passes] = hop_shape(s, n, hop, n_seeds, G);
+    const hipEvent_t end = look.early_rows && hop == s->cfg.hops - 1 && tile_rows(s) ? look.end : nullptr;
     const int npb = block / G * passes;
     g.c.seed_tiles = g.c.stage_seeds ? (int)ceil_div(s->cfg.batch_size, block) : 0;
     g.c.tile_blocks = g.c.seed_tiles + (int)ceil_div(std::max<int64_t>(n_max, 1), npb);
     int grid = g.c.tile_blocks;
     if (p0.fill_pending >= 0) grid += fill_blocks(s->edge_cap[p0.fill_pending], block);
+    if (look.early_rows) {
+      g.c.rows = RowSources{s->cache_data, s->feat, (uint32_t)s->cache_rows, (uint32_t)s->n_nodes, s->row_bytes};
+      g.c.upr = (int)((s->row_bytes + 15) / 16);
+      g.c.last_off = (int)s->row_bytes - 16;
+      g.c.rows_per_tile = flat_tile_rows(s->row_bytes) * (block / 256);
+      g.c.gather_blocks = std::max(1, early_rows_blocks(s, n * hop_nodes(s, hop, n_seeds)) * 256 / block / n);
+      grid += g.c.gather_blocks;
+      g.c.tile_rows = hop == s->cfg.hops - 1 && tile_rows(s) ? 1 : 0;
+      for (int k = 0; k < n && look.headers; ++k) g.p[k].headers = *look.headers;
+    }
     for (int k = 0; k < n; ++k) {
       if (pp[k]->fill_pending >= 0) g.p[k].fill = fill_args(*pp[k], pp[k]->fill_pending);
       pp[k]->fill_pending = -1;
     }
-#define LMI_HOP2(GG, BB, PP) \
-  else if (block == BB && passes == PP) hipLaunchKernelGGL((hop_kernel<GG, BB, PP>), dim3(grid * n), dim3(BB), 0, st, g);
+#define LMI_HOP2(GG, BB, PP)                                                                                       \
+  else if (block == BB && passes == PP) {                                                                          \
+    if (end) hipExtLaunchKernelGGL((hop_kernel<GG, BB, PP>), dim3(grid * n), dim3(BB), 0, st, nullptr, end, 0, g); \
+    else hipLaunchKernelGGL((hop_kernel<GG, BB, PP>), dim3(grid * n), dim3(BB), 0, st, g);                         \
+  }
 #define LMI_HOP(GG)                                                                                                         \
   if (false) {}                                                                                                             \
   LMI_HOP2(GG, 256, 1) LMI_HOP2(GG, 512, 1) LMI_HOP2(GG, 1024, 1) LMI_HOP2(GG, 512, 2) LMI_HOP2(GG, 512, 4) LMI_HOP2(GG, 1024, 4) \
@@ -939,7 +1021,7 @@ int launch_hop(Server *s, Pipe *const *pp, int n, hipStream_t st, int hop, bool 
   LMI_HIP(hipGetLastError());
   if (hop == 0 && look.mode != LOOK_NOT) (look.mode == LOOK_LRU ? s->routes.lru_scan_lookups : s->routes.scan_lookups) += n;
   for (int k = 0; k < n; ++k) {
-    pp[k]->fill_pending = hop;
+    pp[k]->fill_pending = g.c.tile_rows ? -1 : hop;
     pp[k]->hops_done = hop + 1;
   }
   if (!defer_fill) LMI_TRY(launch_fill(s, pp, n, st));

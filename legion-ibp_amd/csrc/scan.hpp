@@ -175,7 +175,7 @@ struct ScanChain {
   unsigned long long *status;  // [max_tiles]
 };
 // Chain `which` of the kScanChains that lie one behind the other at `words`.
-constexpr int kScanChains = 2;
+constexpr int kScanChains = 3;
 __host__ __device__ inline ScanChain scan_chain(unsigned long long *words, int max_tiles, int which) {
   return ScanChain{words + (int64_t)which * max_tiles};
 }
