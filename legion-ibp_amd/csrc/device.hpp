@@ -307,6 +307,21 @@ __device__ __forceinline__ int block_exclusive_scan(int v, int *lds, int &total)
   return res;
 }
 
+// The same with one barrier: every wavefront adds up the others' sums itself.  lds holds BLOCK / 64 ints that are not
+// written again before the block has passed another barrier.
+template <int BLOCK>
+__device__ __forceinline__ int block_exclusive_scan_once(int v, int *lds, int &total) {
+  constexpr int NW = BLOCK / kWave;
+  const int lane = threadIdx.x & (kWave - 1), wid = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int inc = wave_inclusive_scan(v);
+  if (lane == kWave - 1) lds[wid] = inc;
+  __syncthreads();
+  const int w = lane < NW ? lds[lane] : 0;
+  const int winc = wave_inclusive_scan(w);
+  total = __builtin_amdgcn_readlane(winc, kWave - 1);
+  return inc - v + __builtin_amdgcn_readlane(winc - w, wid);
+}
+
 __device__ __forceinline__ uint64_t lanemask_lt() {
   const int lane = threadIdx.x & (kWave - 1);
   return (lane == 0) ? 0ull : (~0ull >> (kWave - lane));

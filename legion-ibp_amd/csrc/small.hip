@@ -6,10 +6,12 @@
 // slots of a hop's edges and the nodes being sampled lie in LDS, the scans are block scans, and one launch per group of
 // batches (a workgroup each) does the seeds, every hop, the relabelling, the cache lookup and the headers.  What is left
 // of HBM is the chain seed -> row pointers -> neighbours -> row pointers ... that no kernel can shorten.
-// us per batch, gather included, on the general path and here: 16 seeds, fanouts 10,5 (445 edges in the last hop): 35 / 20;
-// 64 seeds of a Cora-shaped graph, 25,10 (3 680 edges): 37 / 28; 64 seeds, 10,5 (2 332): 38 / 26, six of them in a
-// group 39 / 27; three hops 5,4,3 (3 918): 54 / 42; 128 seeds of the Cora-shaped graph (6 979): 38 / 38.  1024 threads,
-// because draws and probes fill the CU's four SIMDs: with 512 the second of these takes 33, with 256 50.
+// us per batch, gather included, by the hops' launches and here: 16 seeds, fanouts 10,5 (445 edges in the last hop): 30 / 19;
+// 64 seeds of a Cora-shaped graph, 25,10 (3 680 edges): 27 / 25, 96 (5 185): 28 / 31, 128 (6 979): 30 / 35; 64 seeds, 10,5
+// (2 332): 33 / 26; three hops 5,4,3, 16 seeds (846): 45 / 25, 64 (3 918): 44 / 44; one hop of 20, 128 seeds (1 003): 22 / 18,
+// 256 (1 918): 22 / 25.  1024 threads, because draws and probes fill the CU's four SIMDs: with 512 the second of these took
+// a sixth more, with 256 three quarters.  A barrier of sixteen wavefronts is a tenth of a microsecond: scans take one each
+// (three before: 0.7 us a batch of two hops).
 // Outputs are those of the general path, bit for bit (same draws, same candidates in the dedup table, same ranks).
 #include <algorithm>
 
@@ -50,11 +52,11 @@ struct SmallLds {
                        // next hop, which then starts without a read
   int32_t *key, *val;  // dedup table: id, lowest candidate (later: local id)
   int *base, *node;    // [kSmallBlock] place of the node's first edge, its id
-  int *scan;           // block scans (kSmallScan ints); the last two count misses and the nodes placed in `order`
+  int *scan;           // block scans (kSmallScan ints), which take its halves in turn; the last one counts misses
   uint16_t *order;     // [kSmallBlock] the nodes being sampled, those that draw first
   uint16_t *eslot;     // table slot of each edge of the hop
 };
-constexpr int kSmallScan = 32;
+constexpr int kSmallScan = 2 * kSmallBlock / kWave + 4;
 __host__ __device__ inline int64_t small_lds_bytes(int log2t, int64_t edges) {
   return (int64_t(8) << log2t) + kSmallBlock * 26 + kSmallScan * 4 + 2 * ((edges + 7) / 8 * 8);
 }
@@ -140,14 +142,18 @@ static __global__ __launch_bounds__(kSmallBlock) void batch_small_kernel(SmallGr
   l.scan = l.node + kSmallBlock;
   l.order = reinterpret_cast<uint16_t *>(l.scan + kSmallScan);
   l.eslot = l.order + kSmallBlock;
-  int *n_miss = l.scan + kSmallScan - 1, *n_draw = l.scan + kSmallScan - 2;
+  int *n_miss = l.scan + kSmallScan - 1;
+  int scans = 0;
+  const auto block_scan = [&](int v, int &total) {  // a barrier each
+    return block_exclusive_scan_once<kSmallBlock>(v, l.scan + (scans++ & 1) * (kSmallBlock / kWave), total);
+  };
   const FaultTo fault{bp.serial, bp.fault};
   for (int i = t; i < T; i += kSmallBlock) {
     l.key[i] = kEmptyKey;
     l.val[i] = kIntMax;
   }
   if (t == 0) {
-    *n_miss = *n_draw = 0;
+    *n_miss = 0;
     state_begin(a.st, bp, g.hops);
     misses_begin(a.st);
   }
@@ -222,22 +228,20 @@ static __global__ __launch_bounds__(kSmallBlock) void batch_small_kernel(SmallGr
         l.deg[t] = deg = hi - lo;
         l.node[t] = id;
       }
-      int total;
-      const int base = n_edges + block_exclusive_scan<kSmallBlock>(
-                                     (int)(deg < (int64_t)fanout ? deg : (int64_t)fanout), l.scan, total);
-      if (my < n_known) row_ptr[my] = base;
-      l.base[t] = base;
-      // places in the order: nodes that draw from the front, the others from the back
+      // one scan for the edges (at most 2^16) and, above them, for the places in the order: nodes that draw from the front,
+      // the others from the back
       const int n_here = n_known - c0 < kSmallBlock ? n_known - c0 : kSmallBlock;
       const bool draws = deg > (int64_t)fanout;
-      const uint64_t m = __ballot(draws), m2 = __ballot(!draws && my < n_known);
-      int ahead = 0;
-      if ((t & (kWave - 1)) == 0) ahead = atomicAdd(n_draw, __popcll(m) | (__popcll(m2) << 16));
-      ahead = __shfl(ahead, 0, kWave);
-      if (draws) l.order[(ahead & 0xffff) + __popcll(m & lanemask_lt())] = (uint16_t)t;
-      else if (my < n_known) l.order[n_here - 1 - (ahead >> 16) - __popcll(m2 & lanemask_lt())] = (uint16_t)t;
+      int total;
+      const int ex = block_scan((draws ? fanout | 1 << 20 : (int)deg), total);
+      const int base = n_edges + (ex & 0xfffff), drawn = ex >> 20;
+      total &= 0xfffff;
+      if (my < n_known) {
+        row_ptr[my] = base;
+        l.order[draws ? drawn : n_here - 1 - (t - drawn)] = (uint16_t)t;
+      }
+      l.base[t] = base;
       __syncthreads();
-      if (t == 0) *n_draw = 0;  // for the next nodes, some barriers away
       switch (G) {
         case 4: small_sample<4>(l, g, a, hop, n_here, c0, n_known, eoff, &full); break;
         case 8: small_sample<8>(l, g, a, hop, n_here, c0, n_known, eoff, &full); break;
@@ -265,7 +269,7 @@ static __global__ __launch_bounds__(kSmallBlock) void batch_small_kernel(SmallGr
         sum += first[u];
       }
       int total;
-      int at = n_known + n_new + block_exclusive_scan<kSmallBlock>(sum, l.scan, total);
+      int at = n_known + n_new + block_scan(sum, total);
       n_new += total;
 #pragma unroll
       for (int u = 0; u < kSmallItems; ++u)
@@ -311,14 +315,15 @@ static double small_expected_edges(const Server *s) {
   return most;
 }
 
-// Which batches: those whose largest hop is expected to hold at most small_edges edges (where one workgroup, on one CU,
-// is still faster than launches over the whole device), and whose table and edges fit the LDS of a CU in the worst
+// Which batches: those whose largest hop is expected to hold at most small_edges edges, half as many where it is the only
+// hop (where one workgroup, on one CU, is still faster than a launch a hop over the whole device), and whose table and edges fit the LDS of a CU in the worst
 // case.  Not with the LRU cache: its lookup waits for the insertion before and asks the dedup table in HBM for repeated
 // seeds.
 bool small_batch(const Server *s) {
   const int lg = small_log2t(s);
+  const double most = (double)s->small_edges * (s->cfg.hops == 1 ? 0.5 : 1.0);
   return s->cache_kind != LMI_CACHE_LRU && lg <= 15 && small_lds_bytes(lg, s->max_edges_hop) <= kSmallLds &&
-         small_expected_edges(s) <= (double)s->small_edges && !s->lds_dedup && s->fuse_count;
+         small_expected_edges(s) <= most && !s->lds_dedup && s->fuse_count;
 }
 
 int launch_small(Server *s, Pipe *const *pp, const BatchParams *bps, int n, hipStream_t st, HopLookup look) {
