@@ -432,7 +432,7 @@ int lmi_server_create(const lmi_config *cfg, lmi_server **out) {
       s->fault_dev = (int32_t *)fd;
       s->rows_seen_host = s->fault_host + 8;  // LMI_MAX_GROUP words for whole batches, one for each segment
       s->rows_seen_dev = s->fault_dev ? s->fault_dev + 8 : nullptr;
-      s->nodes_seen_host = s->fault_host + 24;  // LMI_MAX_HOPS words
+      s->nodes_seen_host = s->fault_host + 24;  // one per hop, and one for a batch's rows
       s->nodes_seen_dev = s->fault_dev ? s->fault_dev + 24 : nullptr;
     }
   }
@@ -794,6 +794,7 @@ static int batch_failed(Pipe *const *pp, int n, int rc) {
 // on the first list are gathered over the host link from here on (split lookups).
 static int launch_sampling(Server *s, Pipe *const *pp, const BatchParams *bps, int n, hipStream_t st, bool own_begin,
                            HopLookup early, HopLookup late, bool misses_early = false) {
+  for (int k = 0; k < n; ++k) pp[k]->rows_done = false;
   if (!own_begin && !misses_early && small_batch(s)) return launch_small(s, pp, bps, n, st, early);
   bool begin = own_begin || !hop_sets_up(s);
   for (int k = 0; k < n; ++k) begin = begin || bps[k].clear_table;
@@ -970,11 +971,12 @@ static int run_group_launches(Server *s, Pipe *const *pp, const BatchParams *bps
     split = s->split_lookup && s->cfg.hops >= 2 && s->feat_loc == LMI_LOC_HOST && s->split_miss == 1 &&
             (s->cache_kind == LMI_CACHE_STATIC || s->cache_kind == LMI_CACHE_INT8) &&
             (s->split_lookup == 1 || (s->split_lookup == 2 && n > 1)) && !in_line;
-    early = early_rows(s, in_line) && !small_batch(s);
+    const bool small = small_batch(s);
+    early = small ? in_line && one_pass_gather(s) : early_rows(s, in_line);
     if (lru_rides) LMI_TRY(lru_wait_ready(s, st));
     LMI_TRY(launch_sampling(s, pp, bps, n, st, false, HopLookup{mode, 0, early, pp[0]->handover},
                             HopLookup{mode, split ? 2 : 0, early, pp[0]->handover}, split));
-    done = early && tile_rows(s);
+    done = pp[0]->rows_done;
     if (done) rows_gathered(s, pp, n, pp[0]->handover);
     if (lru && !lru_rides) {
       LMI_TRY(lru_wait_ready(s, st));  // sampling may overlap the previous batch's insertion, the lookup may not
@@ -1100,7 +1102,7 @@ int lmi_run_once_static(lmi_server *h, void *stream, const int32_t *seeds, int32
   const HeaderCopy headers{out->node_counter, out->edge_counter};
   const HopLookup look{one_pass_gather(s) ? LOOK_SLOTS : LOOK_LIST, 0, early, nullptr, &headers};
   if (rc == LMI_OK) rc = small_batch(s) ? launch_small(s, pp, &bp, 1, st, look) : launch_sampling(s, pp, &bp, 1, st, true, look, look);
-  if (rc == LMI_OK && early && tile_rows(s)) rows_gathered(s, pp, 1, nullptr);
+  if (rc == LMI_OK && p.rows_done) rows_gathered(s, pp, 1, nullptr);
   else if (rc == LMI_OK) rc = launch_gather_group(s, pp, 1, st, 0, s->cfg.hops, 0, true, -1, &headers, early);
   s->prof_on = prof;
   return rc;

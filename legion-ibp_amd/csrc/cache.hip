@@ -272,7 +272,7 @@ static __global__ __launch_bounds__(256) void gather_rows_flat_kernel(MoveGroup 
                                                                       int rows_per_tile, int64_t dst_pitch,
                                                                       unsigned long long *row_counter,
                                                                       int32_t *rows_seen, SlotTable look) {
-  __shared__ int s_slot[LOOK ? kFlatTileMax : 1];
+  __shared__ int s_slot[LOOK ? kSlotLds : 1];
   LMI_GRID_ROW_TAIL(g);
   const MoveRow &r = g.p[row];
   const int n = *r.n_ptr;
@@ -293,7 +293,7 @@ static __global__ __launch_bounds__(256) void gather_rows_flat_kernel(MoveGroup 
 // kernels stride over their tiles by the grid, so a grid that turns out small is slower, not wrong.
 // Whole batches use the first LMI_MAX_GROUP words; a gather of one segment (operator by operator) has a word of its own,
 // or the seeds' 800 rows would size the grid of the last hop's 44 000 (284 instead of 190 us for the operators of a batch).
-static int64_t hinted_rows(Server *s, int64_t n_max, int word) {
+int64_t hinted_rows(const Server *s, int64_t n_max, int word) {
   if (!s->rows_seen_host || !s->gather_adaptive) return n_max;
   int32_t seen = 0;
   const int words = word == 0 ? LMI_MAX_GROUP : 1;
@@ -1211,27 +1211,35 @@ bool gather_in_line(const Server *s, Pipe *const *pp, int n, int seg_last) {
 // they add (tile_rows), in place of a gather behind the hops: where the misses come over the host link on the caller's
 // stream, in one pass with the hits.  The link, which bounds such a batch, then works while the hops are sampled, and starts
 // on a tile's misses while others are still being ranked; a launch and a pass over ids and slots go.  Not with the LRU
-// cache, whose batches miss little, and not from a table in HBM, whose reads the hops' own wait for.  Blocks and tiles of a
-// hop move hits more slowly than a grid of the gather's own, which shows for long rows where most are hits: hence the
-// limits, by the share of the nodes in the cache (us a batch of 800 seeds, 10,5, behind the hops / so, without the limits):
-//   400-byte rows, 20 % 76 / 54, 50 % 70 / 51, 90 % 46 / 38, 99 % 44 / 38;  1 536 bytes, 80 % 50 / 48, 95 % 45 / 46;
-//   2 408 bytes, 20 % 216 / 196, 60 % 82 / 76, 80 % 57 / 55, 90 % 51 / 59;  3 600 bytes, early_rows alone 60 % 101 / 95, both
-//   105;  5 732 bytes, early_rows alone 20 % 453 / 436, 60 % 139 / 134, 90 % 70 / 77, both 20 % 457, 60 % 155;
-//   4 000 seeds, 5,4: 1 536 bytes 80 % 81 / 78, 95 % 61 / 68;  4 096 bytes, early_rows alone 90 % 108 / 103, 95 % 94 / 100.
-struct RowLimits {
-  int64_t early, tile;
-};
-static RowLimits row_limits(const Server *s) {
-  if (s->cache_kind == LMI_CACHE_NONE) return {4096, 4096};  // (longer ones are listed, see one_pass_gather)
-  if (s->cache_rows * 10 > s->n_nodes * 9) return {512, 512};
-  if (s->cache_rows * 4 > s->n_nodes * 3) return {4096, 1536};
-  return {INT64_MAX, 2560};
+// cache, whose batches miss little, and not from a table in HBM, whose reads the hops' own wait for.
+// Blocks and tiles of a hop move hits more slowly than a grid of the gather's own, which shows for long rows where most are
+// hits.  So early_rows up to 4 KB, above 512 bytes only where enough rows miss (Server::miss_share; twice that in fact, for
+// the distinct nodes of a batch are drawn more evenly than its edges are), and tile_rows where a thread has few bytes to move
+// and the link is busy for longer than that takes.  us a batch of 800 seeds, 10,5, gathered behind the hops / early_rows / both
+// (bytes a thread of the last hop's tiles, us over the link as estimated here), by bytes of a row and share of nodes cached:
+//   400: 20 % 61 / 57 / 54 (122, 34), 50 % 55 / 54 / 51 (98, 18), 90 % 39 / 38 / 39 (98, 2);  1 024, 4 000 seeds, 5,4: 50 % 113 / 111 / 105
+//   (370, 47);  1 536: 80 % 43 / 38 / 48 (470, 8);  2 408: 20 % 208 / 198 / 196 (736, 207), 60 % 75 / 72 / 70 (736, 38), 70 % 62 / 58 / 62
+//   (736, 23), 80 % 50 / 49 / 59 (736, 12);  4 096: 60 % 102 / 98 / 103 (1 253, 65);  5 732: 20 % 441 / 437 / 449, 80 % 73 / 87 / 118
+//   (1 753, 28);  no cache: 3 072 870 / 857 / 829 (939, 804), 4 096 1 116 / 1 101 / 1 098 (1 253, 1 072);
+//   156 seeds, 10,5, 1 024: 26 % 36 / 28 / 39 (400, 16);  65 seeds, 25,15, 2 408: 62 % 38 / 31 / 50 (815, 9).
+constexpr double kLinkRate = 41e9;  // bytes a second, of 400-byte rows
+static double miss_estimate(const Server *s) {
+  if (s->cache_kind == LMI_CACHE_NONE) return 1.0;
+  return std::min(1.0, s->policy_built == LMI_POLICY_PRESAMPLED ? s->miss_share : 2.2 * s->miss_share);
 }
 bool early_rows(const Server *s, bool in_line) {
   return in_line && one_pass_gather(s) && s->feat_loc == LMI_LOC_HOST && !no_miss_possible(s) && s->fuse_count && !s->lds_dedup &&
-         (s->cache_kind == LMI_CACHE_STATIC || s->cache_kind == LMI_CACHE_NONE) && s->row_bytes <= row_limits(s).early;
+         (s->cache_kind == LMI_CACHE_STATIC || s->cache_kind == LMI_CACHE_NONE) &&
+         (s->row_bytes <= 512 || (s->row_bytes <= 4096 && miss_estimate(s) >= 0.018));
 }
-bool tile_rows(const Server *s) { return s->row_bytes <= row_limits(s).tile; }
+// `n` batches of `added` new rows each, out of `tiles` tiles of `shape` each.
+bool tile_rows(const Server *s, int n, int64_t added, int64_t tiles, const HopShape &shape) {
+  const double bytes = (double)n * (double)added * (double)s->row_bytes;
+  // (with several nodes per lane group a thread has half as much under way)
+  const double thread = bytes / (double)(n * tiles * shape.block) * (shape.passes == 1 ? 1 : 2);
+  const double link_us = bytes * miss_estimate(s) / kLinkRate * 1e6;
+  return thread <= (s->cache_kind == LMI_CACHE_NONE ? 1300 : 450) && link_us >= 0.1 * thread;
+}
 // Their blocks (of 256 threads), for all batches of a launch: a grid that fills the link, as in launch_hits; more where the
 // rows, most of which are hits, would take such a grid longer than a hop takes.
 int early_rows_blocks(const Server *s, int64_t rows) {
@@ -1676,6 +1684,29 @@ static __global__ __launch_bounds__(kScanBlock) void member_flag_kernel(
   }
 }
 
+// sums[0] += keys of the members, sums[1] += all keys: what share of the accesses, were they in proportion to the keys, the
+// cache serves.  One pair of atomics a block.
+static __global__ __launch_bounds__(1024) void key_mass_kernel(const int64_t *indptr, const uint32_t *hot, const int32_t *member,
+                                                               int64_t n, unsigned long long *sums) {
+  __shared__ unsigned long long s_sum[2];
+  if (threadIdx.x < 2) s_sum[threadIdx.x] = 0;
+  __syncthreads();
+  unsigned long long in = 0, all = 0;
+  for (int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; v < n; v += (int64_t)gridDim.x * blockDim.x) {
+    const unsigned long long key = (unsigned long long)rank_key(indptr, hot, v);
+    all += key;
+    if (member[v]) in += key;
+  }
+#pragma unroll
+  for (int d = kWave / 2; d > 0; d >>= 1) in += __shfl_xor(in, d, kWave), all += __shfl_xor(all, d, kWave);
+  if ((threadIdx.x & (kWave - 1)) == 0) {
+    atomicAdd(&s_sum[0], in);
+    atomicAdd(&s_sum[1], all);
+  }
+  __syncthreads();
+  if (threadIdx.x < 2) atomicAdd(&sums[threadIdx.x], s_sum[threadIdx.x]);
+}
+
 static __global__ __launch_bounds__(256) void publish_slots_kernel(const int32_t *member, const int32_t *slot,
                                                                    int64_t n, int table_kind, HashSlot *slots,
                                                                    int log2cap, int32_t *slot_of,
@@ -1851,15 +1882,19 @@ int cache_build_static(Server *s, int64_t capacity_rows, int table_kind, bool in
   } scratch{s};
   const size_t o_bins = scratch.take(kRankBins * 8), o_cnt = scratch.take((N + 1) * 4), o_tie = scratch.take((N + 1) * 4),
                o_slot = scratch.take((N + 1) * 4), o_tiles = scratch.take((ceil_div(N, kScanTile) + 1) * 4),
-               o_n = scratch.take(8), o_cached = scratch.take(cap * 4);
+               o_n = scratch.take(24), o_cached = scratch.take(cap * 4);
   LMI_TRY(cache_buffer(&s->build_scratch, &s->build_scratch_bytes, scratch.bytes));
   scratch.base = (uint8_t *)s->build_scratch;
   unsigned long long *d_bins = (unsigned long long *)(scratch.base + o_bins);
   int32_t *d_cnt = (int32_t *)(scratch.base + o_cnt), *d_tie = (int32_t *)(scratch.base + o_tie),
           *d_slot = (int32_t *)(scratch.base + o_slot), *d_tiles = (int32_t *)(scratch.base + o_tiles),
           *d_n = (int32_t *)(scratch.base + o_n), *d_cached = (int32_t *)(scratch.base + o_cached);
-  const int32_t n32[2] = {(int32_t)N, 0};
-  LMI_HIP(hipMemcpy(d_n, n32, 8, hipMemcpyHostToDevice));
+  struct {  // at d_n: the nodes, the total of a scan, key_mass_kernel's sums
+    int32_t n, total;
+    unsigned long long mass[2];
+  } counts = {(int32_t)N, 0, {0, 0}};
+  static_assert(sizeof(counts) == 24, "o_n");
+  LMI_HIP(hipMemcpy(d_n, &counts, sizeof(counts), hipMemcpyHostToDevice));
 
   int64_t thr = 0, above = 0;
   LMI_TRY(rank_threshold(s, cap, d_bins, &thr, &above));
@@ -1872,9 +1907,13 @@ int cache_build_static(Server *s, int64_t capacity_rows, int table_kind, bool in
   hipLaunchKernelGGL(member_flag_kernel, dim3(grid), dim3(kScanBlock), 0, 0, s->indptr, hot_key, d_n, thr, 1, d_tie,
                      ties_taken, d_cnt, d_tiles);
   LMI_TRY(launch_scan_phases(0, d_cnt, d_slot, d_tiles, d_n, N, SCAN_EPI_NONE, nullptr, 0, d_n + 1));
-  int32_t total = 0;
-  LMI_HIP(hipMemcpy(&total, d_n + 1, 4, hipMemcpyDeviceToHost));
-  if (total != cap) LMI_FAIL(LMI_ERR_HIP, "static cache selection picked %d rows, expected %lld", total, (long long)cap);
+  hipLaunchKernelGGL(key_mass_kernel, dim3(s->n_cu), dim3(1024), 0, 0, s->indptr, hot_key, d_cnt, N,
+                     (unsigned long long *)(d_n + 2));
+  LMI_HIP(hipMemcpy(&counts, d_n, sizeof(counts), hipMemcpyDeviceToHost));
+  if (counts.total != cap)
+    LMI_FAIL(LMI_ERR_HIP, "static cache selection picked %d rows, expected %lld", counts.total, (long long)cap);
+  s->miss_share = counts.mass[1] ? 1.0 - (double)counts.mass[0] / (double)counts.mass[1] : 1.0 - (double)cap / (double)N;
+  s->policy_built = s->policy;
 
   for (int k = 0; k < kCacheBufs; ++k) LMI_TRY(cache_buffer(buf[k], &s->cache_buf[k], want[k]));
   if (table_kind == LMI_TABLE_HASH) {

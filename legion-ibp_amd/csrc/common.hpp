@@ -102,6 +102,7 @@ struct Pipe {
   int id_bits = 0;             // key bits below the epoch tag when that batch ran
   bool table_dirty = true;     // the table (and the scan words) must be wiped before its next use
   bool table_in_lds = false;   // the batch was sampled by one workgroup: `dedup` knows nothing of it, and may never have been wiped
+  bool rows_done = false;      // the batch's sampling launches have gathered all its rows too
   int fill_pending = -1;       // hop whose edge sources still wait for their local ids (launch_fill)
   unsigned long long *scan_words = nullptr;  // look-back scan state: kScanChains chains
   int32_t max_tiles = 0;
@@ -185,6 +186,8 @@ struct Server {
   int cache_kind = LMI_CACHE_NONE;
   int table_kind = LMI_TABLE_HASH;
   int64_t cache_rows = 0;
+  int policy_built = LMI_POLICY_DEGREE;  // ranking key of the cache that was built, and the share of all keys that belongs to
+  double miss_share = 1.0;               // nodes outside it (static / int8)
   int64_t cache_row_bytes = 0;
   uint8_t *cache_data = nullptr;     // [cache_rows][cache_row_bytes]
   float *cache_scale = nullptr;      // int8: per-row scale
@@ -299,6 +302,10 @@ void prof_kernel_events(Server *s, int kind, hipEvent_t *start, hipEvent_t *stop
 // stage_seeds: also run the seed-staging kernel now (otherwise hop 0 stages them itself)
 int launch_batch_generate(Server *s, Pipe *const *pp, const BatchParams *bps, int n, hipStream_t st, bool stage_seeds);
 int graph_update_begin(Server *s, Pipe &p, const BatchParams &bp);
+// Tile of hop_kernel: threads, and nodes per lane group.
+struct HopShape {
+  int block, passes;
+};
 struct HeaderCopy {
   int32_t *nodes, *edges;
 };
@@ -306,7 +313,8 @@ struct HeaderCopy {
 struct HopLookup {
   int mode = 0;      // LOOK_*
   int miss_seg = 0;  // LOOK_LIST: the miss list that receives them
-  // Blocks of the hop's launch gather the rows known before it, and the last hop's tiles the rows they add (early_rows()).
+  // Blocks of the hop's launch gather the rows known before it, and the last hop's tiles the rows they add (early_rows()); a
+  // batch that one workgroup samples has all its rows gathered by others of that launch.
   bool early_rows = false;
   hipEvent_t end = nullptr;                // with early_rows: an event that marks the end of the last hop, and of the batch
   const HeaderCopy *headers = nullptr;     // with early_rows: see launch_gather_group
@@ -367,7 +375,8 @@ void rows_gathered(Server *s, Pipe *const *pp, int n, hipEvent_t end);
 bool gather_in_line(const Server *s, Pipe *const *pp, int n, int seg_last);
 bool one_pass_gather(const Server *s);
 bool early_rows(const Server *s, bool in_line);
-bool tile_rows(const Server *s);
+bool tile_rows(const Server *s, int n, int64_t added, int64_t tiles, const HopShape &shape);
+int64_t hinted_rows(const Server *s, int64_t n_max, int word);
 int early_rows_blocks(const Server *s, int64_t rows);
 // the host-link gather of segments [seg, seg_last] released now, ahead of the batch's later hops (split_lookup)
 int launch_misses_early(Server *s, Pipe *const *pp, int n, hipStream_t st, int seg, int seg_last);
@@ -388,11 +397,5 @@ int pipes_join(Pipe *const *pp, int n, hipStream_t st);
 int cache_dump(Server *s, int32_t *slot_of, int64_t n, int32_t *aux);
 
 inline int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
-
-// Tile of hop_kernel: threads, and nodes per lane group.
-struct HopShape {
-  int block, passes;
-};
-HopShape hop_shape(const Server *s, int n, int hop, int n_seeds, int G);
 
 }  // namespace lmi

@@ -38,13 +38,15 @@ struct RowSources {
 // when).  The table may lie behind the host link: the wavefronts that hold such rows then wait for the link, which
 // bounds the launch, while the hits of all others stream past.
 // look: the slots are not known yet: a block looks its tile's rows up first, a thread each (tiles of at most BLOCK and
-// kFlatTileMax rows), and hands the slots to the others through LDS, and to look_index unless that is null.  One read in a
-// row more per tile instead of a launch and a pass over the ids.
-template <typename V16, int BLOCK, int U, bool NT, bool MISSES>
+// kFlatTileMax rows), and hands slots and ids to the others through LDS (s_rows: kSlotLds ints), and slots to look_index
+// unless that is null.  One read in a row more per tile instead of a launch and a pass over the ids.
+// FRESH (with look): another block of the same launch wrote the ids.
+constexpr int kSlotLds = 2 * kFlatTileMax;
+template <typename V16, int BLOCK, int U, bool NT, bool MISSES, bool FRESH = false>
 __device__ __forceinline__ void gather_rows(const RowSources &from, const int32_t *__restrict__ src_index,
                                             const int32_t *__restrict__ ids, uint8_t *__restrict__ dst, int first, int n,
                                             int upr, int last_off, int rows_per_tile, int64_t dst_pitch, int bx, int gx,
-                                            bool look, const SlotTable &slots, int32_t *look_index, int *s_slot) {
+                                            bool look, const SlotTable &slots, int32_t *look_index, int *s_rows) {
   const int dq = BLOCK / upr, dr = BLOCK % upr;  // what BLOCK units further means in (row, piece)
   const int r0 = (int)threadIdx.x / upr, u0 = (int)threadIdx.x % upr;
   for (int tile = bx; tile * rows_per_tile < n - first; tile += gx) {
@@ -54,9 +56,11 @@ __device__ __forceinline__ void gather_rows(const RowSources &from, const int32_
     if (look) {
       __syncthreads();  // the tile before is done with its slots
       if ((int)threadIdx.x < nr) {
-        const int32_t node = ids[row0 + threadIdx.x];
+        const int32_t node = FRESH ? __hip_atomic_load(&ids[row0 + threadIdx.x], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
+                                   : ids[row0 + threadIdx.x];
         const int32_t found = (uint32_t)node < from.n_table ? static_find(slots, node) : -1;
-        s_slot[threadIdx.x] = found;
+        s_rows[threadIdx.x] = found;
+        s_rows[kFlatTileMax + threadIdx.x] = node;
         if (look_index) look_index[row0 + threadIdx.x] = found;
       }
       __syncthreads();
@@ -71,8 +75,9 @@ __device__ __forceinline__ void gather_rows(const RowSources &from, const int32_
         const int i = row0 + rr;
         slot[k] = id[k] = -1;
         if (f0 + BLOCK * k < lim) {
-          slot[k] = look ? s_slot[rr] : src_index[i];
-          if (MISSES) id[k] = ids[i];  // beside the slot, not behind it: a miss waits for one read, not for two
+          slot[k] = look ? s_rows[rr] : src_index[i];
+          // beside the slot, not behind it: a miss waits for one read, not for two
+          if (MISSES) id[k] = look ? s_rows[kFlatTileMax + rr] : ids[i];
         }
         off[k] = (uu == upr - 1) ? last_off : 16 * uu;
         da[k] = (int64_t)i * dst_pitch + off[k];

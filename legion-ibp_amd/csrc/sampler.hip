@@ -41,7 +41,8 @@ struct HopShared {  // what the pipes of a launch have in common
   int tile_blocks;  // hop_kernel: blocks [0, tile_blocks) own tiles, the rest fill; hop_flag_scan: own edge tiles, the rest
                     // look the seeds up
   int node_cap;     // nodes a batch can know before the hop
-  int32_t *nodes_seen;  // pinned host memory: receives how many the first batch knew
+  int32_t *nodes_seen;  // pinned host memory: receives how many the first batch knew, and behind the last hop its rows
+  int note_total;       // (its rows: only then)
   int seed_tiles;   // hop_kernel: the first tiles stage 256 seeds each
   // cache lookup of the nodes the hop adds
   int look_mode, miss_seg;
@@ -444,10 +445,10 @@ static __global__ __launch_bounds__(BLOCK, 8) void hop_kernel(HopGroup g) {
   __shared__ int32_t s_id[NPB];
   __shared__ int64_t s_beg[NPB], s_deg[NPB];
   __shared__ int s_row[NPB];
-  __shared__ int s_total, s_edge0, s_rank0, s_miss0, s_published;
+  __shared__ int s_total, s_edge0, s_rank0, s_miss0, s_published, s_added;
   __shared__ int s_cnt[PASSES * WAVES];
   __shared__ int s_scan[WAVES + 1];
-  __shared__ int s_slot[kFlatTileMax];
+  __shared__ int s_slot[kSlotLds];
   DevState *st = a.st;
   if (bx >= g.c.tile_blocks) {  // extra blocks: the previous hop's local ids
     fill_local_ids(a.fill, (int64_t)(bx - g.c.tile_blocks) * blockDim.x + threadIdx.x,
@@ -525,6 +526,7 @@ static __global__ __launch_bounds__(BLOCK, 8) void hop_kernel(HopGroup g) {
     if (begin && tile == 0 && t == 0) state_params(st, bp);
     if (scan_tile_prefix(edges, stamp, tile, 0, &s_edge0, st, fault) == kScanFaultPrefix) return;
     if (last) {  // no seeds at all
+      s_added = 0;
       if (t == 0) a.row_ptr[0] = 0;
       if (begin) {
         if (t < 32) headers_first_hop(st, t, g.c.hops, 0, 0, 0);
@@ -648,6 +650,7 @@ static __global__ __launch_bounds__(BLOCK, 8) void hop_kernel(HopGroup g) {
       }
     }
     if (last) {
+      s_added = rank0 + added;
       if (t == 0) a.row_ptr[n_prev] = edge0 + total;
       if (begin) {
         if (t < 32) headers_first_hop(st, t, g.c.hops, n_prev, edge0 + total, rank0 + added);
@@ -677,6 +680,7 @@ static __global__ __launch_bounds__(BLOCK, 8) void hop_kernel(HopGroup g) {
     }
   }
   if (last) headers_copy(g, a, t);
+  if (g.c.note_total && last && t == 0 && row == 0 && g.c.nodes_seen) g.c.nodes_seen[1] = n_prev + s_added;
   if (tile == 0 && t == 0 && row == 0 && g.c.nodes_seen) *g.c.nodes_seen = n_prev;  // for the host to shape later launches by
   if (look_mode != LOOK_NOT && !(g.c.tile_rows && tile >= seed_tiles))
     rows_looked_up<PASSES, BLOCK>(g, a, tile < seed_tiles, node, local, slot_of, look, tag, tag_mask, s_scan, &s_miss0);
@@ -859,7 +863,7 @@ bool hop_sets_up(const Server *s) { return s->fuse_count && !s->lds_dedup; }
 //   1 024 seeds, 15,10,5, third hop (20 000 nodes): 256x1 625 295.3, 1024x1 157 281.6, 512x4 78 284.7.
 // The nodes of a hop are those that the last batches knew there; before the first, the graph's mean degree tells.
 static int64_t hop_nodes(const Server *s, int hop, int n_seeds) {
-  const int64_t seen = hop > 0 && s->nodes_seen_host ? s->nodes_seen_host[hop] : 0;
+  const int64_t seen = hop > 0 && s->nodes_seen_host ? s->nodes_seen_host[hop] : 0;  // hop == hops: the batch's rows
   int64_t nodes = seen > 0 ? seen : n_seeds;
   const double mean = s->n_nodes > 0 ? (double)s->n_edges / (double)s->n_nodes : 0;
   for (int k = 0; k < hop && seen <= 0; ++k) nodes += (int64_t)((double)nodes * std::min<double>(mean, s->cfg.fanout[k]));
@@ -936,8 +940,8 @@ int launch_hop(Server *s, Pipe *const *pp, int n, hipStream_t st, int hop, bool 
     // one tile of nodes per block; a hop left pending gets its local ids filled in by extra blocks behind the tile blocks
     int n_seeds = 0;
     for (int k = 0; k < n; ++k) n_seeds = std::max(n_seeds, pp[k]->n_seeds);
-    const auto [block, passes] = hop_shape(s, n, hop, n_seeds, G);
-    const hipEvent_t end = look.early_rows && hop == s->cfg.hops - 1 && tile_rows(s) ? look.end : nullptr;
+    const HopShape shape = hop_shape(s, n, hop, n_seeds, G);
+    const auto [block, passes] = shape;
     const int npb = block / G * passes;
     g.c.seed_tiles = g.c.stage_seeds ? (int)ceil_div(s->cfg.batch_size, block) : 0;
     g.c.tile_blocks = g.c.seed_tiles + (int)ceil_div(std::max<int64_t>(n_max, 1), npb);
@@ -950,9 +954,16 @@ int launch_hop(Server *s, Pipe *const *pp, int n, hipStream_t st, int hop, bool 
       g.c.rows_per_tile = flat_tile_rows(s->row_bytes) * (block / 256);
       g.c.gather_blocks = std::max(1, early_rows_blocks(s, n * hop_nodes(s, hop, n_seeds)) * 256 / block / n);
       grid += g.c.gather_blocks;
-      g.c.tile_rows = hop == s->cfg.hops - 1 && tile_rows(s) ? 1 : 0;
-      for (int k = 0; k < n && look.headers; ++k) g.p[k].headers = *look.headers;
+      const int64_t nodes = hop_nodes(s, hop, n_seeds);
+      g.c.note_total = hop == s->cfg.hops - 1;
+      g.c.tile_rows = hop == s->cfg.hops - 1 &&
+                      tile_rows(s, n, std::max<int64_t>(1, hop_nodes(s, hop + 1, n_seeds) - nodes), ceil_div(nodes, npb), shape);
+      for (int k = 0; k < n; ++k) {
+        if (look.headers) g.p[k].headers = *look.headers;
+        pp[k]->rows_done = g.c.tile_rows != 0;
+      }
     }
+    const hipEvent_t end = g.c.tile_rows ? look.end : nullptr;
     for (int k = 0; k < n; ++k) {
       if (pp[k]->fill_pending >= 0) g.p[k].fill = fill_args(*pp[k], pp[k]->fill_pending);
       pp[k]->fill_pending = -1;

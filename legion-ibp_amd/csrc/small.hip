@@ -6,7 +6,13 @@
 // slots of a hop's edges and the nodes being sampled lie in LDS, the scans are block scans, and one launch per group of
 // batches (a workgroup each) does the seeds, every hop, the relabelling, the cache lookup and the headers.  What is left
 // of HBM is the chain seed -> row pointers -> neighbours -> row pointers ... that no kernel can shorten.
-// us per batch, gather included, by the hops' launches and here: 16 seeds, fanouts 10,5 (445 edges in the last hop): 30 / 19;
+// Its rows, where they are all gathered in one pass on the caller's stream, are looked up and gathered by other workgroups of
+// the launch, each tile as soon as the sampling workgroup has published its ids: a launch, the lookups of the last hop and the
+// host link's latency for the rows of the hops before leave the chain (us a batch, gather behind / inside: 16 seeds, 10,5, a
+// third cached 18.4 / 16.6, 96 seeds 30.0 / 25.4; one hop of 20, 64 seeds 16.1 / 13.9; 64 seeds of a Cora-shaped graph,
+// 13 MB of rows 25.3 / 23.8, half of them over the link 130 / 116).
+// us per batch, gather behind the launch in both, by the hops' launches and here: 16 seeds, fanouts 10,5 (445 edges in the
+// last hop): 30 / 19;
 // 64 seeds of a Cora-shaped graph, 25,10 (3 680 edges): 27 / 25, 96 (5 185): 28 / 31, 128 (6 979): 30 / 35; 64 seeds, 10,5
 // (2 332): 33 / 26; three hops 5,4,3, 16 seeds (846): 45 / 25, 64 (3 918): 44 / 44; one hop of 20, 128 seeds (1 003): 22 / 18,
 // 256 (1 918): 22 / 25.  1024 threads, because draws and probes fill the CU's four SIMDs: with 512 the second of these took
@@ -15,6 +21,9 @@
 // Outputs are those of the general path, bit for bit (same draws, same candidates in the dedup table, same ranks).
 #include <algorithm>
 
+#include <hip/hip_ext.h>
+
+#include "gather.hpp"
 #include "scan.hpp"
 
 namespace lmi {
@@ -31,6 +40,8 @@ struct SmallPipe {
   int32_t *agg_src_ids, *agg_src_off, *agg_dst_off;
   int32_t *cache_index;
   int2 *miss_list;
+  uint8_t *features;
+  unsigned long long *known;  // with gather workgroups: how many rows they may gather (small_publish)
   BatchParams bp;
 };
 struct SmallGroup {
@@ -42,6 +53,10 @@ struct SmallGroup {
   int log2t;      // LDS dedup table
   int look_mode;
   SlotTable cache;
+  // workgroups per batch that look up and gather its rows, beside the one that samples it; 0: a launch behind this one does
+  int n, workers, upr, last_off, rows_per_tile;
+  RowSources rows;
+  int32_t *rows_seen;  // hinted_rows
   SmallPipe p[LMI_MAX_GROUP];
 };
 static_assert(sizeof(SmallGroup) <= 4096, "a kernel's arguments");
@@ -77,6 +92,12 @@ __device__ __forceinline__ int small_insert(const SmallLds &l, int log2t, int32_
   }
   *full = true;
   return 0;
+}
+
+// `shared`: other workgroups of the launch read the id.
+__device__ __forceinline__ void id_store(int32_t *p, int32_t id, bool shared) {
+  if (shared) __hip_atomic_store(p, id, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  else *p = id;
 }
 
 // Samples the n_here staged nodes, a lane group per node and kSmallNodes nodes in flight, so that their neighbour reads
@@ -127,10 +148,64 @@ __device__ __forceinline__ void small_sample(const SmallLds &l, const SmallGroup
   }
 }
 
+// The rows of a batch whose ids are in memory by now, for the workgroups that gather them: a scan word that only this kernel
+// uses, `last` when there will be no more.  One thread calls, behind wait_memory and a barrier.
+constexpr int kSmallStampHop = 3;  // a hop that no batch has
+__device__ __forceinline__ void small_publish(const SmallPipe &a, int rows, bool last) {
+  scan_publish(ScanChain{a.known}, scan_stamp(a.bp.serial, kSmallStampHop), 0, last ? kScanInclusive : kScanSum, rows);
+}
+
+// A workgroup that gathers: tiles of rows in turn, each as soon as the sampling workgroup has published its ids.  That one has
+// a lower number, so it was dispatched before; the wait is bounded all the same, as in scan_tile_prefix.
+__device__ __forceinline__ void small_gather(const SmallGroup &g, const SmallPipe &a, int worker, int *lds) {
+  const uint32_t stamp = scan_stamp(a.bp.serial, kSmallStampHop);
+  int *s_known = lds + kSlotLds;  // rows, whether they are all
+  int known = 0;
+  bool all = false;
+  for (int64_t row0 = (int64_t)worker * g.rows_per_tile;; row0 += (int64_t)g.workers * g.rows_per_tile) {
+    if (!all && known < row0 + g.rows_per_tile) {
+      __syncthreads();  // everybody has read s_known
+      if (threadIdx.x == 0) {
+        long long t0 = 0;
+        for (int spins = 0;; ++spins) {
+          const unsigned long long w = __hip_atomic_load(a.known, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          if ((uint32_t)(w >> 34) == stamp) {
+            known = (int)(unsigned)w;
+            all = ((unsigned)(w >> 32) & 3u) == kScanInclusive;
+            if (all || known >= row0 + g.rows_per_tile) break;
+          }
+          if (spins == 64) t0 = wall_clock64();
+          if (spins > 64 && (spins & 1023) == 0 && wall_clock64() - t0 > kScanWaitTicks) {
+            raise_fault(a.st, kFaultScan, FaultTo{a.bp.serial, a.bp.fault});
+            known = 0;
+            all = true;
+            break;
+          }
+          __builtin_amdgcn_s_sleep(2);
+        }
+        s_known[0] = known;
+        s_known[1] = all ? 1 : 0;
+      }
+      __syncthreads();
+      known = s_known[0];
+      all = s_known[1] != 0;
+    }
+    if (row0 >= known) return;  // all of them are known by now
+    const int n = (int)(known - row0 < g.rows_per_tile ? known : row0 + g.rows_per_tile);
+    gather_rows<u32x4_a4, kSmallBlock, 2, true, true, true>(g.rows, nullptr, a.ids, a.features, (int)row0, n, g.upr, g.last_off,
+                                                            g.rows_per_tile, g.rows.pitch, 0, 1, true, g.cache, a.cache_index, lds);
+  }
+}
+
 static __global__ __launch_bounds__(kSmallBlock) void batch_small_kernel(SmallGroup g) {
   extern __shared__ __align__(16) unsigned char smem[];
-  const SmallPipe &a = g.p[blockIdx.x];
+  const int row = (int)blockIdx.x % g.n, worker = (int)blockIdx.x / g.n - 1;
+  const SmallPipe &a = g.p[row];
   const BatchParams &bp = a.bp;
+  if (worker >= 0) {
+    small_gather(g, a, worker, reinterpret_cast<int *>(smem));
+    return;
+  }
   const int t = threadIdx.x, T = 1 << g.log2t;
   SmallLds l;
   l.beg = reinterpret_cast<int64_t *>(smem);
@@ -178,7 +253,7 @@ static __global__ __launch_bounds__(kSmallBlock) void batch_small_kernel(SmallGr
         int32_t slot = -1;
         if (g.look_mode != LOOK_NOT && good) slot = static_find(g.cache, id);
         if (hop < 0) {
-          a.ids[i] = id;
+          id_store(&a.ids[i], id, g.workers != 0);
           a.labels[i] = bp.labels ? bp.labels[i] : -1;
           if (i < kSmallBlock) l.node[i] = id;
           if (good) small_insert(l, g.log2t, id, i, &full);
@@ -276,22 +351,30 @@ static __global__ __launch_bounds__(kSmallBlock) void batch_small_kernel(SmallGr
         if (first[u]) {
           const int32_t id = l.key[slot[u]];
           l.val[slot[u]] = at;
-          a.ids[at] = id;
+          id_store(&a.ids[at], id, g.workers != 0);
           if (at < kSmallBlock) l.node[at] = id;
           ++at;
         }
     }
+    const bool last = hop + 1 == g.hops;
+    if (g.workers && last) wait_memory();
     __syncthreads();
+    if (g.workers && last && t == 0) small_publish(a, n_known + n_new, true);
     // ---- local ids of the edges' sources, lookup of the new rows
     for (int e = t; e < n_edges; e += kSmallBlock) a.agg_src_off[eoff + e] = l.val[l.eslot[e]];
-    rows(hop, n_known, n_known + n_new);
+    if (!(g.workers && last)) rows(hop, n_known, n_known + n_new);
     if (t == 0) scan_epilogue(SCAN_EPI_HOP_NODES, a.st, hop, n_new);
     n_known += n_new;
     eoff += n_edges;
+    if (g.workers && !last) wait_memory();  // behind the reads of the new nodes' rows, which took as long
     __syncthreads();  // the next hop overwrites the edges' slots, and reads what was written here
+    if (g.workers && !last && t == 0) small_publish(a, n_known, false);
   }
   if (full) raise_fault(a.st, kFaultBadId, fault);
-  if (t == 0) a.st->n_miss[0] = *n_miss;
+  if (t == 0) {
+    a.st->n_miss[0] = *n_miss;
+    if (g.workers && g.rows_seen) g.rows_seen[row] = n_known;
+  }
 }
 
 // Distinct ids bound the table: a batch's worst case or, in a small graph, its nodes.  Load at most 0.95 in a worst case
@@ -316,8 +399,8 @@ static double small_expected_edges(const Server *s) {
 }
 
 // Which batches: those whose largest hop is expected to hold at most small_edges edges, half as many where it is the only
-// hop (where one workgroup, on one CU, is still faster than a launch a hop over the whole device), and whose table and edges fit the LDS of a CU in the worst
-// case.  Not with the LRU cache: its lookup waits for the insertion before and asks the dedup table in HBM for repeated
+// hop (where one workgroup, on one CU, is still faster than a launch a hop over the whole device), and whose table and edges
+// fit the LDS of a CU in the worst case.  Not with the LRU cache: its lookup waits for the insertion before and asks the dedup table in HBM for repeated
 // seeds.
 bool small_batch(const Server *s) {
   const int lg = small_log2t(s);
@@ -336,6 +419,21 @@ int launch_small(Server *s, Pipe *const *pp, const BatchParams *bps, int n, hipS
   g.log2t = small_log2t(s);
   g.look_mode = look.mode;
   g.cache = slot_table(s);
+  g.n = n;
+  int64_t workers = 0;
+  if (look.early_rows) {
+    g.rows = RowSources{s->cache_data, s->feat, (uint32_t)(s->cache_kind == LMI_CACHE_NONE ? 0 : s->cache_rows),
+                        (uint32_t)s->n_nodes, s->row_bytes};
+    g.upr = (int)((s->row_bytes + 15) / 16);
+    g.last_off = (int)s->row_bytes - 16;
+    g.rows_per_tile = (int)std::max<int64_t>(1, std::min<int64_t>(kFlatTileMax, 16 * 1024 / s->row_bytes));
+    g.rows_seen = s->rows_seen_dev;
+    g.look_mode = LOOK_NOT;
+    workers = std::min<int64_t>(ceil_div(hinted_rows(s, s->max_nodes, 0), g.rows_per_tile), (s->n_cu - n) / n);
+    if (s->cache_kind == LMI_CACHE_NONE && s->feat_loc == LMI_LOC_HOST)  // a grid that fills the link
+      workers = std::min<int64_t>(workers, std::max(1, early_rows_blocks(s, 0) * 256 / kSmallBlock / n));
+  }
+  g.workers = (int)workers;
   for (int k = 0; k < n; ++k) {
     Pipe &p = *pp[k];
     SmallPipe &a = g.p[k];
@@ -348,15 +446,22 @@ int launch_small(Server *s, Pipe *const *pp, const BatchParams *bps, int n, hipS
     a.agg_dst_off = p.agg_dst_off;
     a.cache_index = p.cache_index;
     a.miss_list = p.miss_list;
+    a.features = (uint8_t *)p.features;
+    a.known = p.scan_words;
     a.bp = bps[k];
     p.n_seeds = bps[k].n_seeds;
     p.hops_done = s->cfg.hops;
     p.fill_pending = -1;
     p.table_in_lds = true;
+    p.rows_done = g.workers > 0;
     if (bps[k].clear_table) p.table_dirty = true;  // this batch leaves the table in HBM as it is
   }
-  hipLaunchKernelGGL(batch_small_kernel, dim3(n), dim3(kSmallBlock), (size_t)small_lds_bytes(g.log2t, s->max_edges_hop),
-                     st, g);
+  const dim3 grid(n * (1 + g.workers));
+  const size_t lds = (size_t)small_lds_bytes(g.log2t, s->max_edges_hop);
+  if (look.early_rows && look.end)
+    hipExtLaunchKernelGGL(batch_small_kernel, grid, dim3(kSmallBlock), lds, st, nullptr, look.end, 0, g);
+  else
+    hipLaunchKernelGGL(batch_small_kernel, grid, dim3(kSmallBlock), lds, st, g);
   LMI_HIP(hipGetLastError());
   s->routes.small_batches += n;
   return LMI_OK;
