@@ -950,7 +950,7 @@ static int run_group_launches(Server *s, Pipe *const *pp, const BatchParams *bps
   for (int k = 0; k < n; ++k) pipe_begin(*pp[k], st);
   prof_phase(s, st, &s->prof_open, PROF_SAMPLE);
   const bool lru = s->cache_kind == LMI_CACHE_LRU;
-  bool split = false, early = false, done = false;
+  bool split = false, early = false, small = false, done = false;
   if (s->use_graph && st != nullptr && n == 1) {  // the legacy default stream cannot be captured
     Pipe &p = *pp[0];
     LMI_TRY(lru_wait_ready(s, st));  // the lookup sits inside the graph: the whole replay waits
@@ -971,7 +971,7 @@ static int run_group_launches(Server *s, Pipe *const *pp, const BatchParams *bps
     split = s->split_lookup && s->cfg.hops >= 2 && s->feat_loc == LMI_LOC_HOST && s->split_miss == 1 &&
             (s->cache_kind == LMI_CACHE_STATIC || s->cache_kind == LMI_CACHE_INT8) &&
             (s->split_lookup == 1 || (s->split_lookup == 2 && n > 1)) && !in_line;
-    const bool small = small_batch(s);
+    small = small_batch(s);
     early = small ? in_line && one_pass_gather(s) : early_rows(s, in_line);
     if (lru_rides) LMI_TRY(lru_wait_ready(s, st));
     LMI_TRY(launch_sampling(s, pp, bps, n, st, false, HopLookup{mode, 0, early, pp[0]->handover},
@@ -983,7 +983,7 @@ static int run_group_launches(Server *s, Pipe *const *pp, const BatchParams *bps
       LMI_TRY(launch_lookup(s, pp, n, st, 0, s->cfg.hops));
     }
   }
-  if (!done) LMI_TRY(launch_gather_group(s, pp, n, st, split ? 2 : 0, s->cfg.hops, lru ? 1 : 0, false, early ? -1 : 0, nullptr, early));
+  if (!done) LMI_TRY(launch_gather_group(s, pp, n, st, split ? 2 : 0, s->cfg.hops, lru ? 1 : 0, false, early && !small ? -1 : 0, nullptr, early && !small));
   prof_phase(s, st, &s->prof_open, -1);
   return LMI_OK;
 }

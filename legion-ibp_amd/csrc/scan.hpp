@@ -189,11 +189,6 @@ __device__ __forceinline__ uint32_t scan_stamp(int32_t serial, int hop) { return
 // constant 100 MHz: a quarter of a second).  The clock is read once per 1024 re-reads.
 constexpr long long kScanWaitTicks = 25000000;
 constexpr int kScanFaultPrefix = -1;  // what scan_tile_prefix returns to a tile that gave up
-// Windows of 64 tiles that a tile reads at once.  Tiles that announce at about the same time, as behind a wait for the
-// same thing, find no inclusive prefix near them: every window more in a read is one step less in a chain of steps of a
-// microsecond each.
-constexpr int kScanWindows = 4;
-
 __device__ __forceinline__ void scan_publish(ScanChain c, uint32_t stamp, int tile, unsigned flag, int value) {
   __hip_atomic_store(&c.status[tile], (unsigned long long)stamp << 34 | (unsigned long long)flag << 32 | (unsigned int)value,
                      __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -207,6 +202,11 @@ __device__ __forceinline__ void scan_tile_announce(ScanChain c, uint32_t stamp, 
 // thread of the block, or kScanFaultPrefix to every thread when the wait ran out: the tile then
 // has no valid offset and must write nothing.  lds_prefix is one shared int, not written again
 // before every thread has read it.  Contains __syncthreads.
+// Wavefront 0 looks back 64 tiles per step (lookback_window), not more: tiles that announce at about the same time, as
+// behind a wait for the same thing, find no inclusive prefix near them and would take fewer steps, but all of them read the
+// same few lines again and again until the slowest has announced, and that is what they then wait for (8 000 seeds from a
+// full cache with 8 / 4 / 2 / 1 windows of 64 a step: 82.6 / 76.3 / 75.6 / 73.6 us; four of them from a table in HBM 306 / 275 / 274 /
+// 274).
 __device__ __forceinline__ int scan_tile_prefix(ScanChain c, uint32_t stamp, int tile, int sum, int *lds_prefix,
                                                 DevState *st, FaultTo fault) {
   if (threadIdx.x < kWave) {
@@ -217,47 +217,32 @@ __device__ __forceinline__ int scan_tile_prefix(ScanChain c, uint32_t stamp, int
       int spins = 0;
       bool broken = false;
       long long t0 = 0;
-      bool done = false;
-      while (!done) {
-        unsigned long long w[kScanWindows];
-#pragma unroll
-        for (int k = 0; k < kScanWindows; ++k) {
-          const int j = base - k * kWave - lane;
-          w[k] = j >= 0 ? __hip_atomic_load(&c.status[j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0ull;
+      while (true) {
+        const int j = base - lane;
+        unsigned long long w = 0;
+        unsigned flag = kScanInclusive;  // before tile 0: an inclusive prefix of 0
+        if (j >= 0) {
+          w = __hip_atomic_load(&c.status[j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          flag = (uint32_t)(w >> 34) == stamp ? (unsigned)(w >> 32) & 3u : 0u;
         }
-        bool wait = false;
-        int mine = 0, windows = 0;
-#pragma unroll
-        for (int k = 0; k < kScanWindows; ++k) {
-          if (done || wait) continue;
-          const int j = base - k * kWave - lane;
-          unsigned flag = (uint32_t)(w[k] >> 34) == stamp ? (unsigned)(w[k] >> 32) & 3u : 0u;
-          if (j < 0) flag = kScanInclusive;  // before tile 0: an inclusive prefix of 0
-          const LookbackWindow win = lookback_window(__ballot(flag == kScanInclusive), __ballot(flag == 0u));
-          wait = win.wait;
-          if (wait) continue;
-          if (j >= 0 && ((win.take >> lane) & 1ull)) mine += (int)(unsigned)w[k];
-          done = win.done;
-          ++windows;
+        const LookbackWindow win = lookback_window(__ballot(flag == kScanInclusive), __ballot(flag == 0u));
+        if (win.wait) {  // a tile we need has not published yet: read again
+          if (++spins == 16) {  // no ordinary wait: it is timed from here
+            // after a first fault every later tile gives up almost at once, so a broken chain drains
+            // in milliseconds
+            broken = st->scan_fault == fault.serial;
+            t0 = wall_clock64();
+          }
+          __builtin_amdgcn_s_sleep(1);
+          const bool out_of_time = broken ? spins >= 64 : ((spins & 1023) == 0 && wall_clock64() - t0 > kScanWaitTicks);
+          if (!out_of_time) continue;
+          if (lane == 0) raise_fault(st, kFaultScan, fault);  // never expected; bounded so that the grid always drains
+          prefix = kScanFaultPrefix;
+          break;
         }
-        // the windows in front of one that is not complete stay counted
-        if (windows > 0) {
-          prefix += wave_sum(mine);
-          base -= windows * kWave;
-          continue;
-        }
-        if (++spins == 16) {  // no ordinary wait: it is timed from here
-          // after a first fault every later tile gives up almost at once, so a broken chain drains
-          // in milliseconds
-          broken = st->scan_fault == fault.serial;
-          t0 = wall_clock64();
-        }
-        __builtin_amdgcn_s_sleep(1);
-        const bool out_of_time = broken ? spins >= 64 : ((spins & 1023) == 0 && wall_clock64() - t0 > kScanWaitTicks);
-        if (!out_of_time) continue;
-        if (lane == 0) raise_fault(st, kFaultScan, fault);  // never expected; bounded so that the grid always drains
-        prefix = kScanFaultPrefix;
-        break;
+        prefix += wave_sum((win.take >> lane) & 1ull ? (int)(unsigned)w : 0);
+        if (win.done) break;
+        base -= kWave;
       }
       if (lane == 0 && prefix != kScanFaultPrefix) scan_publish(c, stamp, tile, kScanInclusive, prefix + sum);
     }

@@ -420,18 +420,28 @@ int launch_small(Server *s, Pipe *const *pp, const BatchParams *bps, int n, hipS
   g.look_mode = look.mode;
   g.cache = slot_table(s);
   g.n = n;
+  const int64_t lds = small_lds_bytes(g.log2t, s->max_edges_hop);
   int64_t workers = 0;
   if (look.early_rows) {
     g.rows = RowSources{s->cache_data, s->feat, (uint32_t)(s->cache_kind == LMI_CACHE_NONE ? 0 : s->cache_rows),
                         (uint32_t)s->n_nodes, s->row_bytes};
     g.upr = (int)((s->row_bytes + 15) / 16);
     g.last_off = (int)s->row_bytes - 16;
-    g.rows_per_tile = (int)std::max<int64_t>(1, std::min<int64_t>(kFlatTileMax, 16 * 1024 / s->row_bytes));
-    g.rows_seen = s->rows_seen_dev;
-    g.look_mode = LOOK_NOT;
-    workers = std::min<int64_t>(ceil_div(hinted_rows(s, s->max_nodes, 0), g.rows_per_tile), (s->n_cu - n) / n);
+    // A workgroup's one pass.  A batch of its own takes up to a workgroup per CU (64 seeds of a Cora-shaped graph on 255 / 127 /
+    // 63: 23.8 / 27.8 / 36.0 us).  The sampling workgroups of a group lie on several dies, and launches of several streams that
+    // each filled dies with waiting workgroups could keep the others' sampling ones from being dispatched (the waits would
+    // run out): a group has no more than leave room for four such launches, or a launch behind this one gathers.
+    const int64_t tile_bytes = n == 1 ? 16 * 1024 : 32 * 1024;
+    g.rows_per_tile = (int)std::max<int64_t>(1, std::min<int64_t>(kFlatTileMax, tile_bytes / s->row_bytes));
+    const int64_t tiles = ceil_div(hinted_rows(s, s->max_nodes, 0), g.rows_per_tile);
+    const int64_t room = s->n_cu / (2 * lds <= kSmallLds ? 2 : 4) / n - 1;
+    workers = n == 1 ? std::min<int64_t>(tiles, s->n_cu - 1) : 2 * room >= tiles ? std::min(tiles, room) : 0;
     if (s->cache_kind == LMI_CACHE_NONE && s->feat_loc == LMI_LOC_HOST)  // a grid that fills the link
       workers = std::min<int64_t>(workers, std::max(1, early_rows_blocks(s, 0) * 256 / kSmallBlock / n));
+    if (workers > 0) {
+      g.rows_seen = s->rows_seen_dev;
+      g.look_mode = LOOK_NOT;
+    }
   }
   g.workers = (int)workers;
   for (int k = 0; k < n; ++k) {
@@ -457,11 +467,10 @@ int launch_small(Server *s, Pipe *const *pp, const BatchParams *bps, int n, hipS
     if (bps[k].clear_table) p.table_dirty = true;  // this batch leaves the table in HBM as it is
   }
   const dim3 grid(n * (1 + g.workers));
-  const size_t lds = (size_t)small_lds_bytes(g.log2t, s->max_edges_hop);
-  if (look.early_rows && look.end)
-    hipExtLaunchKernelGGL(batch_small_kernel, grid, dim3(kSmallBlock), lds, st, nullptr, look.end, 0, g);
+  if (workers > 0 && look.end)
+    hipExtLaunchKernelGGL(batch_small_kernel, grid, dim3(kSmallBlock), (size_t)lds, st, nullptr, look.end, 0, g);
   else
-    hipLaunchKernelGGL(batch_small_kernel, grid, dim3(kSmallBlock), lds, st, g);
+    hipLaunchKernelGGL(batch_small_kernel, grid, dim3(kSmallBlock), (size_t)lds, st, g);
   LMI_HIP(hipGetLastError());
   s->routes.small_batches += n;
   return LMI_OK;
