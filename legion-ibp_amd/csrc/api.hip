@@ -972,7 +972,7 @@ static int run_group_launches(Server *s, Pipe *const *pp, const BatchParams *bps
             (s->cache_kind == LMI_CACHE_STATIC || s->cache_kind == LMI_CACHE_INT8) &&
             (s->split_lookup == 1 || (s->split_lookup == 2 && n > 1)) && !in_line;
     small = small_batch(s);
-    early = small ? in_line && one_pass_gather(s) : early_rows(s, in_line);
+    early = small ? in_line && one_pass_gather(s) && !gather_knobs(s) : early_rows(s, in_line);
     if (lru_rides) LMI_TRY(lru_wait_ready(s, st));
     LMI_TRY(launch_sampling(s, pp, bps, n, st, false, HopLookup{mode, 0, early, pp[0]->handover},
                             HopLookup{mode, split ? 2 : 0, early, pp[0]->handover}, split));

@@ -1227,8 +1227,10 @@ static double miss_estimate(const Server *s) {
   if (s->cache_kind == LMI_CACHE_NONE) return 1.0;
   return std::min(1.0, s->policy_built == LMI_POLICY_PRESAMPLED ? s->miss_share : 2.2 * s->miss_share);
 }
+// A gather whose tiles or grid were asked for by a knob stays a launch of its own.
+bool gather_knobs(const Server *s) { return s->gather_tile_rows > 0 || s->gather_blocks > 0; }
 bool early_rows(const Server *s, bool in_line) {
-  return in_line && one_pass_gather(s) && s->feat_loc == LMI_LOC_HOST && !no_miss_possible(s) && s->fuse_count && !s->lds_dedup &&
+  return in_line && !gather_knobs(s) && one_pass_gather(s) && s->feat_loc == LMI_LOC_HOST && !no_miss_possible(s) && s->fuse_count && !s->lds_dedup &&
          (s->cache_kind == LMI_CACHE_STATIC || s->cache_kind == LMI_CACHE_NONE) &&
          (s->row_bytes <= 512 || (s->row_bytes <= 4096 && miss_estimate(s) >= 0.018));
 }
@@ -1907,8 +1909,9 @@ int cache_build_static(Server *s, int64_t capacity_rows, int table_kind, bool in
   hipLaunchKernelGGL(member_flag_kernel, dim3(grid), dim3(kScanBlock), 0, 0, s->indptr, hot_key, d_n, thr, 1, d_tie,
                      ties_taken, d_cnt, d_tiles);
   LMI_TRY(launch_scan_phases(0, d_cnt, d_slot, d_tiles, d_n, N, SCAN_EPI_NONE, nullptr, 0, d_n + 1));
-  hipLaunchKernelGGL(key_mass_kernel, dim3(s->n_cu), dim3(1024), 0, 0, s->indptr, hot_key, d_cnt, N,
-                     (unsigned long long *)(d_n + 2));
+  if (!int8)  // int8 rows are not gathered in the hops, which is what asks for it
+    hipLaunchKernelGGL(key_mass_kernel, dim3((int)std::min<int64_t>(s->n_cu, ceil_div(N, 1024))), dim3(1024), 0, 0, s->indptr,
+                       hot_key, d_cnt, N, (unsigned long long *)(d_n + 2));
   LMI_HIP(hipMemcpy(&counts, d_n, sizeof(counts), hipMemcpyDeviceToHost));
   if (counts.total != cap)
     LMI_FAIL(LMI_ERR_HIP, "static cache selection picked %d rows, expected %lld", counts.total, (long long)cap);

@@ -187,7 +187,7 @@ struct Server {
   int table_kind = LMI_TABLE_HASH;
   int64_t cache_rows = 0;
   int policy_built = LMI_POLICY_DEGREE;  // ranking key of the cache that was built, and the share of all keys that belongs to
-  double miss_share = 1.0;               // nodes outside it (static / int8)
+  double miss_share = 1.0;               // nodes outside it (static)
   int64_t cache_row_bytes = 0;
   uint8_t *cache_data = nullptr;     // [cache_rows][cache_row_bytes]
   float *cache_scale = nullptr;      // int8: per-row scale
@@ -375,6 +375,7 @@ void rows_gathered(Server *s, Pipe *const *pp, int n, hipEvent_t end);
 bool gather_in_line(const Server *s, Pipe *const *pp, int n, int seg_last);
 bool one_pass_gather(const Server *s);
 bool early_rows(const Server *s, bool in_line);
+bool gather_knobs(const Server *s);
 bool tile_rows(const Server *s, int n, int64_t added, int64_t tiles, const HopShape &shape);
 int64_t hinted_rows(const Server *s, int64_t n_max, int word);
 int early_rows_blocks(const Server *s, int64_t rows);
