@@ -1953,6 +1953,11 @@ int cache_build_static(Server *s, int64_t capacity_rows, int table_kind, bool in
     m.note_rows = -1;
     m.src_row_bytes = m.dst_row_bytes = m.row_bytes = s->row_bytes;
     m.n_max = cap;
+    // Over the link a block per CU: more reads in flight cost it a few percent, except of rows so long that few of them are
+    // (us a build on the device's grid / 256 blocks / 96: 735 000 rows of 400 bytes 6 778 / 6 574 / 6 476, of 512 6 985 / 6 785 /
+    // 6 800; 1.2 M of 64 bytes 2 510 / 2 357 / 2 455; 160 000 of 3 072 8 980 / 8 744 / 8 998; 120 000 of 5 732 13 280 / 13 497 /
+    // 14 075).
+    if (s->feat_loc == LMI_LOC_HOST && s->row_bytes <= 4096) m.max_blocks = s->n_cu;
     LMI_TRY(launch_move_rows(s, 0, m, false));
   }
   LMI_HIP(hipDeviceSynchronize());
