@@ -320,6 +320,15 @@ typedef struct lmi_routes {
   int64_t lru_place_copies;  /* LRU insertions in one launch */
 } lmi_routes;
 int lmi_routes_get(lmi_server *s, lmi_routes *out);
+/* The same for the launches that gather rows while they sample, and the tiles of the hops issued last.  Fills the first
+ * out_bytes bytes of `out` (sizeof(lmi_row_routes)). */
+typedef struct lmi_row_routes {
+  int64_t early_rows;  /* batches whose hops' launches gathered the rows known before them */
+  int64_t tile_rows;   /* those of them whose last hop's tiles gathered the rows they added */
+  int64_t small_rows;  /* batches sampled by one workgroup whose rows other workgroups of the launch gathered */
+  int64_t hop_threads[LMI_MAX_HOPS], hop_nodes[LMI_MAX_HOPS];  /* of a tile, in the last kernel issued for each hop */
+} lmi_row_routes;
+int lmi_row_routes_get(lmi_server *s, lmi_row_routes *out, size_t out_bytes);
 /* Tuning knobs by name (e.g. "gather_lanes_per_row", "gather_unroll", "lds_dedup"). */
 int lmi_tune(lmi_server *s, const char *key, int64_t value);
 /* Plain device copy of `bytes` bytes, repeated; returns mean ms per copy

@@ -34,7 +34,7 @@ ABI_SYMBOLS = [
     "lmi_cache_info_get", "lmi_cache_dump", "lmi_op_batch_generate", "lmi_op_random_sample",
     "lmi_op_cache_lookup", "lmi_op_io_submit", "lmi_op_io_complete", "lmi_run_once",
     "lmi_run_group", "lmi_run_once_static", "lmi_batch_wait", "lmi_server_status", "lmi_batch_view_get", "lmi_batch_counters", "lmi_steps_per_epoch", "lmi_profile_enable",
-    "lmi_profile_read", "lmi_routes_get", "lmi_tune", "lmi_bench_copy", "lmi_bench_copy_launch", "lmi_bench_stream", "lmi_bench_row_stream", "lmi_bench_row_stream_shape", "lmi_bench_host_read", "lmi_bench_random_read", "lmi_synth_graph", "lmi_synth_trainset",
+    "lmi_profile_read", "lmi_routes_get", "lmi_row_routes_get", "lmi_tune", "lmi_bench_copy", "lmi_bench_copy_launch", "lmi_bench_stream", "lmi_bench_row_stream", "lmi_bench_row_stream_shape", "lmi_bench_host_read", "lmi_bench_random_read", "lmi_synth_graph", "lmi_synth_trainset",
     "lmi_synth_features",
 ]
 
@@ -70,6 +70,11 @@ class Profile(C.Structure):
 class Routes(C.Structure):
     _fields_ = [(name, C.c_int64) for name in ("small_batches", "scan_lookups", "lru_scan_lookups", "gather_lookups",
                                                "one_pass_gathers", "lru_place_copies")]
+
+
+class RowRoutes(C.Structure):
+    _fields_ = [("early_rows", C.c_int64), ("tile_rows", C.c_int64), ("small_rows", C.c_int64),
+                ("hop_threads", C.c_int64 * MAX_HOPS), ("hop_nodes", C.c_int64 * MAX_HOPS)]
 
 
 class LegionError(RuntimeError):
@@ -143,6 +148,7 @@ def lib():
         L.lmi_profile_enable.argtypes = [C.c_void_p, C.c_int]
         L.lmi_profile_read.argtypes = [C.c_void_p, C.POINTER(Profile), C.c_int]
         L.lmi_routes_get.argtypes = [C.c_void_p, C.POINTER(Routes)]
+        L.lmi_row_routes_get.argtypes = [C.c_void_p, C.POINTER(RowRoutes), C.c_size_t]
         L.lmi_tune.argtypes = [C.c_void_p, C.c_char_p, C.c_int64]
         L.lmi_bench_copy.argtypes = [C.c_size_t, C.c_int, C.POINTER(C.c_double)]
         L.lmi_bench_copy_launch.argtypes = [C.c_size_t, C.c_int, C.POINTER(C.c_double)]
@@ -388,10 +394,12 @@ class Server:
         return p
 
     def routes(self):
-        """How many batches took each launch that is chosen by size, cache and call order (lmi_routes)."""
-        r = Routes()
+        """How many batches took each launch that is chosen by size, cache and call order (lmi_routes, lmi_row_routes)."""
+        r, q = Routes(), RowRoutes()
         check(lib().lmi_routes_get(self.h, C.byref(r)))
-        return {name: int(getattr(r, name)) for name, _ in Routes._fields_}
+        check(lib().lmi_row_routes_get(self.h, C.byref(q), C.sizeof(q)))
+        out = {name: getattr(x, name) for x in (r, q) for name, _ in x._fields_}
+        return {name: v if isinstance(v, int) else list(v) for name, v in out.items()}
 
     def tune(self, key, value):
         check(lib().lmi_tune(self.h, key.encode(), int(value)))

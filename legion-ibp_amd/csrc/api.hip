@@ -1256,6 +1256,13 @@ int lmi_routes_get(lmi_server *h, lmi_routes *out) {
   return LMI_OK;
 }
 
+int lmi_row_routes_get(lmi_server *h, lmi_row_routes *out, size_t out_bytes) {
+  Server *s = reinterpret_cast<Server *>(h);
+  if (!s || !out) LMI_FAIL(LMI_ERR_ARG, "null argument");
+  memcpy(out, &s->row_routes, std::min(out_bytes, sizeof(s->row_routes)));
+  return LMI_OK;
+}
+
 int lmi_tune(lmi_server *h, const char *key, int64_t value) {
   Server *s = reinterpret_cast<Server *>(h);
   if (!s || !key) LMI_FAIL(LMI_ERR_ARG, "null argument");

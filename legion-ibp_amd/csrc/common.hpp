@@ -241,6 +241,7 @@ struct Server {
   std::atomic<int> last_pipe{-1};
   std::atomic<bool> last_taken{true};
   lmi_routes routes{};
+  lmi_row_routes row_routes{};
   hipStream_t side = nullptr;  // server-owned second stream for gathers that must not hold up the caller's stream
   // tuning
   int gather_lpr = 0;     // lanes per row (0 = auto)

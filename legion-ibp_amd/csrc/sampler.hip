@@ -962,7 +962,11 @@ int launch_hop(Server *s, Pipe *const *pp, int n, hipStream_t st, int hop, bool 
         if (look.headers) g.p[k].headers = *look.headers;
         pp[k]->rows_done = g.c.tile_rows != 0;
       }
+      if (hop == 0) s->row_routes.early_rows += n;
+      if (g.c.tile_rows) s->row_routes.tile_rows += n;
     }
+    s->row_routes.hop_threads[hop] = block;
+    s->row_routes.hop_nodes[hop] = npb;
     const hipEvent_t end = g.c.tile_rows ? look.end : nullptr;
     for (int k = 0; k < n; ++k) {
       if (pp[k]->fill_pending >= 0) g.p[k].fill = fill_args(*pp[k], pp[k]->fill_pending);

@@ -480,6 +480,7 @@ int launch_small(Server *s, Pipe *const *pp, const BatchParams *bps, int n, hipS
     hipLaunchKernelGGL(batch_small_kernel<false>, grid, dim3(kSmallBlock), (size_t)lds, st, g);
   LMI_HIP(hipGetLastError());
   s->routes.small_batches += n;
+  if (workers > 0) s->row_routes.small_rows += n;
   return LMI_OK;
 }
 

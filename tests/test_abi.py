@@ -34,6 +34,7 @@ def test_struct_layouts_match_header(lmi):
     assert ctypes.sizeof(lmi.CacheInfo) == 48
     assert ctypes.sizeof(lmi.Profile) == 12 * 8
     assert ctypes.sizeof(lmi.Routes) == 6 * 8
+    assert ctypes.sizeof(lmi.RowRoutes) == (3 + 2 * 3) * 8
 
 
 def test_bad_arguments_are_rejected_without_a_gpu(lmi):

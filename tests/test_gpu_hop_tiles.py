@@ -44,6 +44,9 @@ def test_tiles_match_the_oracle(lmi, oracle, world, fanout, shape):
             seeds = [rng.integers(0, N_NODES, batch).astype(np.int32) for _ in range(2)]
             seeds[1][-1] = seeds[1][0]
             srv.run_group([0, 1], [0, 0], seeds=seeds, rng_seeds=[5 + it, 6 + it])
+            threads, nodes, _ = SHAPES[shape]
+            routes = srv.routes()
+            assert (routes["hop_threads"][0], routes["hop_nodes"][0]) == (threads, threads // lanes * nodes)
             for k in range(2):
                 g = srv.fetch(pipe=k)
                 assert_batch_equal(g, oracle.sample_batch(indptr, indices, seeds[k], [fanout, 2], 5 + it + k))

@@ -53,11 +53,16 @@ def test_rows_and_slots(lmi, oracle, graph, dim, cache, table, fanout):
         after = srv.routes()
         assert after["small_batches"] - before["small_batches"] == len(sizes)
         assert after["one_pass_gathers"] - before["one_pass_gathers"] == (len(sizes) if one_pass else 0)
+        assert after["small_rows"] - before["small_rows"] == (len(sizes) if one_pass else 0)
         for it in range(2):
             seeds = [rng.integers(0, N_NODES, 1 + (5 * k + it) % batch).astype(np.int32) for k in range(n_pipes)]
             srv.run_group(list(range(n_pipes)), [0] * n_pipes, seeds=seeds, rng_seeds=[70 + it + k for k in range(n_pipes)], stream=stream)
             for k in range(n_pipes):
                 check(k, seeds[k], 70 + it + k)
+        # a group that can miss is in line up to 1 MB; eight batches of long rows are more tiles than its share of the device takes
+        worst = batch * int(np.prod([1 + f for f in fanout]))
+        in_line = cache != "static" or n_pipes * worst * dim * 4 <= 1 << 20
+        assert srv.routes()["small_rows"] - after["small_rows"] == (2 * n_pipes if in_line and dim <= 37 else 0)
         srv.status()
     finally:
         srv.close()
