@@ -1291,6 +1291,7 @@ int lmi_tune(lmi_server *h, const char *key, int64_t value) {
   }
   else if (!strcmp(key, "profile_every")) s->prof_every = (int)std::max<int64_t>(1, value);
   else if (!strcmp(key, "small_edges")) s->small_edges = value;
+  else if (!strcmp(key, "small_patience")) s->small_patience = (int)std::max<int64_t>(0, std::min<int64_t>(value, 1 << 20));
   else if (!strcmp(key, "fuse_small_max")) (void)value;  // accepted as before; tiles are chosen by hop_shape
   else if (!strcmp(key, "split_miss")) s->split_miss = (int)value;
   else if (!strcmp(key, "use_graph")) s->use_graph = (int)value;

@@ -262,6 +262,7 @@ struct Server {
   int fuse_count = 1;     // 1: row counts, their scan and the sampling of a hop share one launch
   int64_t small_edges = 7000;  // batches whose largest hop is expected to hold at most this many edges are sampled by one
                                // workgroup (small_batch)
+  int small_patience = 4096;   // reads of the sampling workgroup's word before one that gathers leaves (small_gather)
   int lds_dedup = 0;      // 1: hop_sample stages its probes through an LDS hash table
   int split_miss = 1;     // gather schedule, see launch_gather_group
   int use_graph = 0;      // 1: lmi_run_once replays a captured HIP graph of the sampling kernels (measured

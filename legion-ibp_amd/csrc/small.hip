@@ -41,7 +41,8 @@ struct SmallPipe {
   int32_t *cache_index;
   int2 *miss_list;
   uint8_t *features;
-  unsigned long long *known;  // with gather workgroups: how many rows they may gather (small_publish)
+  unsigned long long *known;  // with gather workgroups: how many rows they may gather (small_publish), and behind it whether
+                              // one of them has left its rows (small_leave)
   BatchParams bp;
 };
 struct SmallGroup {
@@ -55,6 +56,7 @@ struct SmallGroup {
   SlotTable cache;
   // workgroups per batch that look up and gather its rows, beside the one that samples it; 0: a launch behind this one does
   int n, workers, upr, last_off, rows_per_tile;
+  int patience;  // reads of SmallPipe::known before a gather workgroup leaves
   RowSources rows;
   int32_t *rows_seen;  // hinted_rows
   SmallPipe p[LMI_MAX_GROUP];
@@ -155,28 +157,45 @@ __device__ __forceinline__ void small_publish(const SmallPipe &a, int rows, bool
   scan_publish(ScanChain{a.known}, scan_stamp(a.bp.serial, kSmallStampHop), 0, last ? kScanInclusive : kScanSum, rows);
 }
 
-// A workgroup that gathers: tiles of rows in turn, each as soon as the sampling workgroup has published its ids.  That one has
-// a lower number, so it was dispatched before; the wait is bounded all the same, as in scan_tile_prefix.
-__device__ __forceinline__ void small_gather(const SmallGroup &g, const SmallPipe &a, int worker, int *lds) {
+// A gather workgroup leaves, and its rows to the sampling one, where its wait does not end: one of the two has to see what the
+// other has written.  Both are device-scope accesses, each complete before the read of the other's word.
+__device__ __forceinline__ unsigned long long small_known(const SmallPipe &a) {
+  return __hip_atomic_load(a.known, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void small_leave(const SmallPipe &a) {
+  scan_publish(ScanChain{a.known}, scan_stamp(a.bp.serial, kSmallStampHop), 1, kScanInclusive, 0);
+  wait_memory();
+}
+__device__ __forceinline__ bool small_left(const SmallPipe &a) {
+  wait_memory();
+  return (uint32_t)(__hip_atomic_load(a.known + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >> 34) ==
+         scan_stamp(a.bp.serial, kSmallStampHop);
+}
+
+// A workgroup that gathers: every `step`-th tile of rows from `tile` on, each as soon as the sampling workgroup has published
+// its ids (`all`: they all are, `known` of them).
+// The sampling workgroup has a lower number, but each die starts its share of the workgroups by itself: launches of several
+// streams can fill a die with waiting ones while the sampling ones that they wait for stand in line at other dies, filled by
+// one another's.  So a wait that lasts (SmallGroup::patience: half a millisecond; an ordinary one is tens of microseconds)
+// ends with the workgroup leaving, which gives its place to one that somebody waits for, and the sampling workgroup, which
+// waits for nobody, then gathers all the batch's rows itself: some twice, with the same bytes.
+__device__ __forceinline__ void small_gather(const SmallGroup &g, const SmallPipe &a, int tile, int step, int known, bool all,
+                                             int *lds) {
   const uint32_t stamp = scan_stamp(a.bp.serial, kSmallStampHop);
   int *s_known = lds + kSlotLds;  // rows, whether they are all
-  int known = 0;
-  bool all = false;
-  for (int64_t row0 = (int64_t)worker * g.rows_per_tile;; row0 += (int64_t)g.workers * g.rows_per_tile) {
+  for (int64_t row0 = (int64_t)tile * g.rows_per_tile;; row0 += (int64_t)step * g.rows_per_tile) {
     if (!all && known < row0 + g.rows_per_tile) {
       __syncthreads();  // everybody has read s_known
       if (threadIdx.x == 0) {
-        long long t0 = 0;
-        for (int spins = 0;; ++spins) {
-          const unsigned long long w = __hip_atomic_load(a.known, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        for (int reads = 0;; ++reads) {
+          if (reads == g.patience) small_leave(a);
+          const unsigned long long w = small_known(a);
           if ((uint32_t)(w >> 34) == stamp) {
             known = (int)(unsigned)w;
             all = ((unsigned)(w >> 32) & 3u) == kScanInclusive;
-            if (all || known >= row0 + g.rows_per_tile) break;
+            if (all || (known >= row0 + g.rows_per_tile && reads < g.patience)) break;
           }
-          if (spins == 64) t0 = wall_clock64();
-          if (spins > 64 && (spins & 1023) == 0 && wall_clock64() - t0 > kScanWaitTicks) {
-            raise_fault(a.st, kFaultScan, FaultTo{a.bp.serial, a.bp.fault});
+          if (reads >= g.patience) {
             known = 0;
             all = true;
             break;
@@ -197,20 +216,10 @@ __device__ __forceinline__ void small_gather(const SmallGroup &g, const SmallPip
   }
 }
 
-// WORKERS: with gather workgroups (SmallGroup::workers).  Not a branch: a kernel that might gather samples 0.8 us more slowly.
+// The batch's sampling, by one workgroup: the rows it ends with.  WORKERS: others gather them beside it.
 template <bool WORKERS>
-static __global__ __launch_bounds__(kSmallBlock) void batch_small_kernel(SmallGroup g) {
-  extern __shared__ __align__(16) unsigned char smem[];
-  const int row = WORKERS ? (int)blockIdx.x % g.n : (int)blockIdx.x;
-  const SmallPipe &a = g.p[row];
+__device__ __forceinline__ int small_sampled(const SmallGroup &g, const SmallPipe &a, int row, unsigned char *smem) {
   const BatchParams &bp = a.bp;
-  if constexpr (WORKERS) {
-    const int worker = (int)blockIdx.x / g.n - 1;
-    if (worker >= 0) {
-      small_gather(g, a, worker, reinterpret_cast<int *>(smem));
-      return;
-    }
-  }
   const int t = threadIdx.x, T = 1 << g.log2t;
   SmallLds l;
   l.beg = reinterpret_cast<int64_t *>(smem);
@@ -380,6 +389,31 @@ static __global__ __launch_bounds__(kSmallBlock) void batch_small_kernel(SmallGr
     a.st->n_miss[0] = *n_miss;
     if (WORKERS && g.rows_seen) g.rows_seen[row] = n_known;
   }
+  return n_known;
+}
+
+// WORKERS: with gather workgroups (SmallGroup::workers).  Not a branch: a kernel that might gather samples 0.8 us more slowly.
+template <bool WORKERS>
+static __global__ __launch_bounds__(kSmallBlock) void batch_small_kernel(SmallGroup g) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  const int row = WORKERS ? (int)blockIdx.x % g.n : (int)blockIdx.x;
+  const SmallPipe &a = g.p[row];
+  if constexpr (!WORKERS) {
+    small_sampled<false>(g, a, row, smem);
+  } else {
+    int tile = (int)blockIdx.x / g.n - 1, step = g.workers, known = 0;
+    const bool sampler = tile < 0;
+    if (sampler) {
+      known = small_sampled<true>(g, a, row, smem);
+      int *s_left = reinterpret_cast<int *>(smem);
+      if (threadIdx.x == 0) *s_left = small_left(a) ? 1 : 0;
+      __syncthreads();
+      if (*s_left == 0) return;
+      tile = 0;
+      step = 1;
+    }
+    small_gather(g, a, tile, step, known, sampler, reinterpret_cast<int *>(smem));
+  }
 }
 
 // Distinct ids bound the table: a batch's worst case or, in a small graph, its nodes.  Load at most 0.95 in a worst case
@@ -433,13 +467,15 @@ int launch_small(Server *s, Pipe *const *pp, const BatchParams *bps, int n, hipS
     g.upr = (int)((s->row_bytes + 15) / 16);
     g.last_off = (int)s->row_bytes - 16;
     // A workgroup's one pass.  A batch of its own takes up to a workgroup per CU (64 seeds of a Cora-shaped graph on 255 / 127 /
-    // 63: 23.8 / 27.8 / 36.0 us).  The sampling workgroups of a group lie on several dies, and launches of several streams that
-    // each filled dies with waiting workgroups could keep the others' sampling ones from being dispatched (the waits would
-    // run out): a group has no more than leave room for four such launches, or a launch behind this one gathers.
+    // 63: 23.8 / 27.8 / 36.0 us).  A CU has room for one, of sixteen wavefronts with more than 96 scalar registers, and those of
+    // a group wait with several sampling ones: no more of them than leave room for another such launch beside it, or a launch
+    // behind this one gathers (us a group at most half of the CUs / a quarter: eight batches of 32 seeds, 10,5, all rows cached
+    // 17.1 / 19.0, four of 96 23.8 / 27.2; four streams of the first kind, one group each: 40 / 52).  Where yet more streams
+    // wait on each other, small_gather ends it.
     const int64_t tile_bytes = n == 1 ? 16 * 1024 : 32 * 1024;
     g.rows_per_tile = (int)std::max<int64_t>(1, std::min<int64_t>(kFlatTileMax, tile_bytes / s->row_bytes));
     const int64_t tiles = ceil_div(hinted_rows(s, s->max_nodes, 0), g.rows_per_tile);
-    const int64_t room = s->n_cu / (2 * lds <= kSmallLds ? 2 : 4) / n - 1;
+    const int64_t room = s->n_cu / 2 / n - 1;
     workers = n == 1 ? std::min<int64_t>(tiles, s->n_cu - 1) : 2 * room >= tiles ? std::min(tiles, room) : 0;
     if (s->cache_kind == LMI_CACHE_NONE && s->feat_loc == LMI_LOC_HOST)  // a grid that fills the link
       workers = std::min<int64_t>(workers, std::max(1, early_rows_blocks(s, 0) * 256 / kSmallBlock / n));
@@ -449,6 +485,7 @@ int launch_small(Server *s, Pipe *const *pp, const BatchParams *bps, int n, hipS
     }
   }
   g.workers = (int)workers;
+  g.patience = s->small_patience;
   for (int k = 0; k < n; ++k) {
     Pipe &p = *pp[k];
     SmallPipe &a = g.p[k];
