@@ -153,6 +153,7 @@ __device__ __forceinline__ void small_sample(const SmallLds &l, const SmallGroup
 // The rows of a batch whose ids are in memory by now, for the workgroups that gather them: a scan word that only this kernel
 // uses, `last` when there will be no more.  One thread calls, behind wait_memory and a barrier.
 constexpr int kSmallStampHop = 3;  // a hop that no batch has
+static_assert(LMI_MAX_HOPS <= kSmallStampHop, "the stamp would be a hop's");
 __device__ __forceinline__ void small_publish(const SmallPipe &a, int rows, bool last) {
   scan_publish(ScanChain{a.known}, scan_stamp(a.bp.serial, kSmallStampHop), 0, last ? kScanInclusive : kScanSum, rows);
 }
