@@ -1227,8 +1227,12 @@ static double miss_estimate(const Server *s) {
   if (s->cache_kind == LMI_CACHE_NONE) return 1.0;
   return std::min(1.0, s->policy_built == LMI_POLICY_PRESAMPLED ? s->miss_share : 2.2 * s->miss_share);
 }
-// A gather whose tiles or grid were asked for by a knob stays a launch of its own.
-bool gather_knobs(const Server *s) { return s->gather_tile_rows > 0 || s->gather_blocks > 0; }
+// A gather that a knob shapes stays a launch of its own: rows in the hops and beside small batches take their tiles and grid
+// from those launches, and are stored non-temporally.  (Rows in flight per lane follow their knob only without a cache.)
+bool gather_knobs(const Server *s) {
+  return s->gather_tile_rows > 0 || s->gather_blocks > 0 || !s->gather_nt ||
+         (s->gather_unroll > 0 && s->cache_kind == LMI_CACHE_NONE);
+}
 bool early_rows(const Server *s, bool in_line) {
   return in_line && !gather_knobs(s) && one_pass_gather(s) && s->feat_loc == LMI_LOC_HOST && !no_miss_possible(s) && s->fuse_count && !s->lds_dedup &&
          (s->cache_kind == LMI_CACHE_STATIC || s->cache_kind == LMI_CACHE_NONE) &&

@@ -90,6 +90,42 @@ def test_rows_match_the_table(lmi, oracle, graph, dim, cached, fanout):
         feats.free()
 
 
+@pytest.mark.parametrize("small", [False, True])
+@pytest.mark.parametrize("cached", [0.0, 0.3])
+@pytest.mark.parametrize("knob,value", [(None, None), ("gather_nontemporal", 0), ("gather_unroll", 4), ("gather_tile_rows", 5), ("gather_blocks", 40)])
+def test_knobs_keep_a_launch_of_their_own(lmi, oracle, graph, knob, value, cached, small):
+    """A knob of the gather acts on a gather: the rows are in no other launch then."""
+    rng, indptr, indices = graph
+    dim, fanout, batch = 33, [10, 5], 24
+    feats = make_features(lmi, rng, N_NODES, dim)
+    srv = lmi.Server(batch, fanout, dim, pipes=1, seed=3)
+    stream = lmi.stream_create()
+    try:
+        srv.load_graph(indptr, indices)
+        srv.attach_features(feats)
+        if not small:
+            srv.tune("small_edges", 0)
+        if cached:
+            srv.build_static_cache(int(cached * N_NODES), lmi.TABLE_RANK)
+        if knob:
+            srv.tune(knob, value)
+        for it in range(2):
+            seeds = rng.integers(0, N_NODES, batch).astype(np.int32)
+            srv.run_once(seeds, rng_seed=it + 1, stream=stream)
+            g = srv.fetch(stream=stream)
+            assert_batch_equal(g, oracle.sample_batch(indptr, indices, seeds, fanout, it + 1))
+            assert g.features.tobytes() == feats.array[g.ids].tobytes()
+        routes = srv.routes()
+        taken = knob is None or (knob == "gather_unroll" and cached > 0)   # with a cache that knob has never acted on this gather
+        assert routes["small_batches"] == (2 if small else 0)
+        assert routes["one_pass_gathers"] == 2
+        assert routes["small_rows" if small else "early_rows"] == (2 if taken else 0)
+        srv.status()
+    finally:
+        srv.close()
+        feats.free()
+
+
 # threads of a tile, nodes per lane group, tiles per CU that a launch may have of it
 SHAPES = [(256, 1, 1), (512, 1, 1), (1024, 1, 1), (512, 2, 2), (512, 4, 2), (1024, 4, None)]
 
