@@ -424,16 +424,17 @@ int lmi_server_create(const lmi_config *cfg, lmi_server **out) {
     rc = LMI_ERR_HIP;
   if (rc == LMI_OK) {  // sticky fault words: pinned host memory the kernels write and the host reads without a copy
     void *fh = nullptr, *fd = nullptr;
-    if (hipHostMalloc(&fh, 128, hipHostMallocMapped) != hipSuccess) rc = LMI_ERR_HIP;
+    if (hipHostMalloc(&fh, 256, hipHostMallocMapped) != hipSuccess) rc = LMI_ERR_HIP;
     if (rc == LMI_OK) {
-      memset(fh, 0, 128);
+      memset(fh, 0, 256);
       s->fault_host = (volatile int32_t *)fh;
       if (hipHostGetDevicePointer(&fd, fh, 0) != hipSuccess) rc = LMI_ERR_HIP;
       s->fault_dev = (int32_t *)fd;
-      s->rows_seen_host = s->fault_host + 8;  // LMI_MAX_GROUP words for whole batches, one for each segment
-      s->rows_seen_dev = s->fault_dev ? s->fault_dev + 8 : nullptr;
-      s->nodes_seen_host = s->fault_host + 24;  // one per hop, and one for a batch's rows
-      s->nodes_seen_dev = s->fault_dev ? s->fault_dev + 24 : nullptr;
+      s->rows_seen_host = (volatile SeenWord *)(s->fault_host + 8);  // LMI_MAX_GROUP for whole batches, one for each segment
+      s->rows_seen_dev = s->fault_dev ? (SeenWord *)(s->fault_dev + 8) : nullptr;
+      s->nodes_seen_host = s->rows_seen_host + LMI_MAX_GROUP + LMI_MAX_HOPS + 1;  // one per hop, and one for a batch's rows
+      s->nodes_seen_dev = s->rows_seen_dev ? s->rows_seen_dev + LMI_MAX_GROUP + LMI_MAX_HOPS + 1 : nullptr;
+      static_assert(32 + 8 * (LMI_MAX_GROUP + 2 * (LMI_MAX_HOPS + 1)) <= 256, "the pinned words");
     }
   }
   if (rc != LMI_OK) {

@@ -41,6 +41,7 @@ struct MoveRow {
   const int32_t *ids;  // gather_rows_flat_kernel<.., MISSES>: node id per row
   int32_t *look_index; // gather_rows_flat_kernel<.., LOOK>: receives the slot per row
   uint8_t *dst;
+  int note_seeds;  // Pipe::note_seeds
   // the HBM gathers of a batch carry its last steps (MoveGroup::tail_blocks)
   FillArgs fill;        // last hop's local ids (hop -1: already there)
   HeaderCopy headers;   // where the batch's headers go besides its state (nodes null: nowhere)
@@ -271,7 +272,7 @@ template <typename V16, int U, bool NT, bool MISSES, bool LOOK>
 static __global__ __launch_bounds__(256) void gather_rows_flat_kernel(MoveGroup g, RowSources from, int upr, int last_off,
                                                                       int rows_per_tile, int64_t dst_pitch,
                                                                       unsigned long long *row_counter,
-                                                                      int32_t *rows_seen, SlotTable look) {
+                                                                      SeenWord *rows_seen, SlotTable look) {
   __shared__ int s_slot[LOOK ? kSlotLds : 1];
   LMI_GRID_ROW_TAIL(g);
   const MoveRow &r = g.p[row];
@@ -279,7 +280,7 @@ static __global__ __launch_bounds__(256) void gather_rows_flat_kernel(MoveGroup 
   const int first = r.first_ptr ? *r.first_ptr : 0;
   if (bx == 0 && threadIdx.x == 0) {
     if (row_counter && n > first) atomicAdd(row_counter, (unsigned long long)(n - first));  // profiling
-    if (rows_seen) rows_seen[row] = n - first;
+    if (rows_seen && r.note_seeds > 0) note_seen(&rows_seen[row], n - first, r.note_seeds);
   }
   gather_rows<V16, 256, U, NT, MISSES>(from, r.src_index, r.ids, r.dst, first, n, upr, last_off, rows_per_tile, dst_pitch, bx, gx,
                                        LOOK, look, r.look_index, s_slot);
@@ -289,20 +290,18 @@ static __global__ __launch_bounds__(256) void gather_rows_flat_kernel(MoveGroup 
 // ten times what a batch holds, and a block that finds no tile is not free: the device starts about one
 // workgroup per clock, so the 8 000 idle blocks of a worst-case grid cost a 40 us launch a seventh of
 // its time.  The gather kernels leave the row count of every launch in pinned host memory
-// (rows_seen); the largest of the last launch, with an eighth on top, sizes the next grid.  The
+// (rows_seen); the largest of the last launch in proportion to the seeds, with an eighth on top, sizes the next grid.  The
 // kernels stride over their tiles by the grid, so a grid that turns out small is slower, not wrong.
 // Whole batches use the first LMI_MAX_GROUP words; a gather of one segment (operator by operator) has a word of its own,
 // or the seeds' 800 rows would size the grid of the last hop's 44 000 (284 instead of 190 us for the operators of a batch).
-int64_t hinted_rows(const Server *s, int64_t n_max, int word) {
+int64_t hinted_rows(const Server *s, int64_t n_max, int word, Pipe *const *pp, int n) {
   if (!s->rows_seen_host || !s->gather_adaptive) return n_max;
-  int32_t seen = 0;
+  const int seeds = most_seeds(pp, n);
+  int64_t seen = 0;
   const int words = word == 0 ? LMI_MAX_GROUP : 1;
-  for (int k = 0; k < words; ++k) {
-    const int32_t v = s->rows_seen_host[word + k];
-    seen = v > seen ? v : seen;
-  }
+  for (int k = 0; k < words; ++k) seen = std::max(seen, seen_count(&s->rows_seen_host[word + k], seeds));
   if (seen <= 0) return n_max;  // nothing seen yet
-  return std::min<int64_t>(n_max, (int64_t)seen + seen / 8 + 64);
+  return std::min<int64_t>(n_max, seen + seen / 8 + 64);
 }
 
 static int rows_word(const Server *s, int seg, int seg_last) {
@@ -322,7 +321,8 @@ struct MoveArgs {
   const uint8_t *table;             // flat gather: the feature table rows without a slot are read from, or null
   int64_t n_table;                  // node ids below this have a row there
   int look;                         // flat gather with a table: look the slots up on the way
-  int note_rows;                    // flat gather: the word of rows_seen that receives the row counts (hinted_rows), or -1
+  int note_rows;                    // flat gather: the word of rows_seen that receives the row counts, or -1
+  int64_t rows_hint;                // note_rows >= 0: how many rows are expected (hinted_rows)
   int64_t src_row_bytes, dst_row_bytes, row_bytes;  // row_bytes = bytes moved per row
   int64_t n_max;   // per pipe
 };
@@ -425,7 +425,7 @@ static int launch_gather_flat(Server *s, hipStream_t st, const MoveArgs &a, bool
   const int U = u_want >= 4 ? 4 : u_want >= 2 ? 2 : 1;
   int rpt = flat_tile_rows(a.row_bytes);
   if (s->gather_tile_rows > 0) rpt = std::min(s->gather_tile_rows, kFlatTileMax);
-  const int64_t want = ceil_div(a.note_rows >= 0 ? hinted_rows(s, a.n_max, a.note_rows) : a.n_max, rpt);
+  const int64_t want = ceil_div(a.note_rows >= 0 ? a.rows_hint : a.n_max, rpt);
   const int64_t cap = a.max_blocks > 0 ? a.max_blocks : s->gather_blocks > 0 ? s->gather_blocks : (int64_t)s->n_cu * 64;
   const int grid = (int)std::max<int64_t>(1, std::min(want, cap)) + a.g.tail_blocks;
   const SlotTable look = slot_table(s);
@@ -650,7 +650,7 @@ template <typename OUT, int EPL, int U>
 static __global__ __launch_bounds__(256) void gather_int8_tiled_kernel(MoveGroup g, const int8_t *q, const float *scale,
                                                                        int dim, int tile_rows,
                                                                        unsigned long long *row_counter,
-                                                                       int32_t *rows_seen) {
+                                                                       SeenWord *rows_seen) {
   typedef typename RawVec<EPL>::type IN;
   constexpr int OUT_VECS = EPL * (int)sizeof(OUT) / 16;
   constexpr int TILE = 64;
@@ -664,7 +664,8 @@ static __global__ __launch_bounds__(256) void gather_int8_tiled_kernel(MoveGroup
   const int first = g.p[row].first_ptr ? *g.p[row].first_ptr : 0;
   if (bx == 0 && threadIdx.x == 0) {
     if (row_counter && n > first) atomicAdd(row_counter, (unsigned long long)(n - first));
-    if (rows_seen) rows_seen[row] = n - first;  // for the host to size the next grids by (hinted_rows)
+    // for the host to size the next grids by (hinted_rows)
+    if (rows_seen && g.p[row].note_seeds > 0) note_seen(&rows_seen[row], n - first, g.p[row].note_seeds);
   }
   const int units = dim / EPL;
   const int dq = 256 / units, dr = 256 % units;
@@ -966,7 +967,7 @@ int pipes_join(Pipe *const *pp, int n, hipStream_t st) {
 }
 
 // int8 rows: dequantised inside the gather.
-static int launch_hits_int8(Server *s, const MoveGroup &g, hipStream_t st, int seg, int seg_last, hipEvent_t end) {
+static int launch_hits_int8(Server *s, const MoveGroup &g, int64_t rows_hint, hipStream_t st, int seg, int seg_last, hipEvent_t end) {
   const int64_t n_max = s->node_cap[seg_last];
   const int dim = s->cfg.feat_dim;
   const int64_t want = ceil_div(n_max, 4);
@@ -991,7 +992,7 @@ static int launch_hits_int8(Server *s, const MoveGroup &g, hipStream_t st, int s
     // 768-element fp16 rows, share of HBM peak: 8 rows per tile 45 %, 16 51 %, 32 54 %, 64 52 %
     const int tile_rows = s->gather_tile_rows > 0 ? std::min(64, s->gather_tile_rows) : 32;
     // sized by the rows the last launches held (hinted_rows): a block without a tile is not free
-    const int64_t want_f = ceil_div(hinted_rows(s, n_max, rows_word(s, seg, seg_last)), tile_rows);
+    const int64_t want_f = ceil_div(rows_hint, tile_rows);
     const int64_t cap_f = s->gather_blocks > 0 ? s->gather_blocks
                           : s->gather_adaptive ? (int64_t)s->n_cu * 64 : auto_gather_blocks(s, want_f);
     const int grid_f = g.n * ((int)std::max<int64_t>(1, std::min<int64_t>(want_f, cap_f)) + g.tail_blocks);
@@ -1113,10 +1114,13 @@ static int launch_hits(Server *s, Pipe *const *pp, int n, hipStream_t st, int se
     r.ids = p.ids;
     r.look_index = p.cache_index;
     r.dst = (uint8_t *)p.features;
+    r.note_seeds = p.note_seeds;
     r.fill.hop = -1;
   }
   if (carries) tail_args(s, pp, n, headers, &m.g);
-  if (s->cache_kind == LMI_CACHE_INT8) return launch_hits_int8(s, m.g, st, seg, seg_last, end);
+  m.note_rows = rows_word(s, seg, seg_last);
+  m.rows_hint = hinted_rows(s, n_max, m.note_rows, pp, n);
+  if (s->cache_kind == LMI_CACHE_INT8) return launch_hits_int8(s, m.g, m.rows_hint, st, seg, seg_last, end);
   m.src = have_cache ? s->cache_data : s->feat;
   m.n_src = have_cache ? s->cache_rows : s->n_nodes;
   if (misses && have_cache) {
@@ -1131,7 +1135,6 @@ static int launch_hits(Server *s, Pipe *const *pp, int n, hipStream_t st, int se
     const int blocks = s->miss_blocks > 0 ? s->miss_blocks : s->miss_blocks == 0 ? s->n_cu : 96;
     m.max_blocks = std::max(1, (blocks + n - 1) / n);  // per pipe
   }
-  m.note_rows = rows_word(s, seg, seg_last);
   m.src_row_bytes = m.dst_row_bytes = m.row_bytes = s->row_bytes;
   m.n_max = n_max;
   m.row_counter = s->prof_on ? s->d_prof_rows : nullptr;  // all rows of the segment: hits + misses

@@ -135,6 +135,7 @@ struct Pipe {
                                 // then issued this one: its misses have nothing to overlap (gather_in_line)
   int32_t *seed_stage = nullptr;  // [batch_size] host seeds land here
   int32_t n_seeds = 0;
+  int32_t note_seeds = 0;  // n_seeds where the batch's launches leave what they met (SeenWord), else 0
   int32_t hops_done = 0;
   // HIP graph of one whole batch minus the feature gather (captured on first use)
   hipGraphExec_t graph_exec = nullptr;
@@ -154,6 +155,10 @@ struct BatchParams {
   const int32_t *labels;
   int32_t *fault;  // device-visible address of the server's sticky fault words
 };
+
+// What a launch met, for the host to shape later launches by: a count, and how many seeds its batch had, in one word of pinned
+// host memory, so that they travel together.
+typedef unsigned long long SeenWord;  // seeds << 32 | count; 0: nothing seen yet
 
 struct EventPair {  // device time between two recorded events, attributed to `kind`
   hipEvent_t a, b;
@@ -229,11 +234,13 @@ struct Server {
   bool fault_told[2] = {false, false};  // lmi_batch_wait has reported the condition once already
   // row counts the gather kernels leave behind, one word per pipe of a launch (and one per segment gathered by itself),
   // in the same pinned allocation
-  volatile int32_t *rows_seen_host = nullptr;
-  int32_t *rows_seen_dev = nullptr;
-  // nodes that a batch knew before each hop, left there by the hops' kernels
-  volatile int32_t *nodes_seen_host = nullptr;
-  int32_t *nodes_seen_dev = nullptr;
+  volatile SeenWord *rows_seen_host = nullptr;
+  SeenWord *rows_seen_dev = nullptr;
+  // nodes that a batch knew before each hop, and its rows, left there by the hops' kernels
+  volatile SeenWord *nodes_seen_host = nullptr;
+  SeenWord *nodes_seen_dev = nullptr;
+  int32_t noted_seeds = 0;  // of the last batch that leaves such counts, and how many since then do not (pipe_seeds)
+  int unnoted = 0;
   // pipes
   std::vector<Pipe> pipes;
   // the pipe a single batch was last issued on, and whether the caller has taken that batch on its own stream since
@@ -379,7 +386,7 @@ bool one_pass_gather(const Server *s);
 bool early_rows(const Server *s, bool in_line);
 bool gather_knobs(const Server *s);
 bool tile_rows(const Server *s, int n, int64_t added, int64_t tiles, const HopShape &shape);
-int64_t hinted_rows(const Server *s, int64_t n_max, int word);
+int64_t hinted_rows(const Server *s, int64_t n_max, int word, Pipe *const *pp, int n);
 int early_rows_blocks(const Server *s, int64_t rows);
 // the host-link gather of segments [seg, seg_last] released now, ahead of the batch's later hops (split_lookup)
 int launch_misses_early(Server *s, Pipe *const *pp, int n, hipStream_t st, int seg, int seg_last);
@@ -400,5 +407,32 @@ int pipes_join(Pipe *const *pp, int n, hipStream_t st);
 int cache_dump(Server *s, int32_t *slot_of, int64_t n, int32_t *aux);
 
 inline int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
+
+// What a batch of `seeds` seeds meets where another met the count of `word`; 0: nothing seen yet.
+inline int64_t seen_count(const volatile SeenWord *word, int64_t seeds) {
+  const SeenWord w = *word;
+  const int64_t count = (int64_t)(w & 0xFFFFFFFFu), of = (int64_t)(w >> 32);
+  if (count <= 0 || of <= 0) return 0;
+  return ceil_div(count * std::max<int64_t>(1, seeds), of);
+}
+// A batch of n_seeds starts on the pipe.  It leaves its counts for later ones unless it is much shorter than the last that
+// did: in proportion a few seeds tell little of a full batch, and an epoch's short last batch is followed by a full one
+// (the fourth short one in a row counts).  us of a full batch behind one of a single seed, counts taken as they come / in
+// proportion and only from batches of a quarter at least: 8 000 seeds, all rows cached 1 975 / 86, four such batches from a table
+// in HBM 2 970 / 298, 64 seeds of a Cora-shaped graph 57 / 36; a group of those four behind one whose first is short 367 / 296.
+inline void pipe_seeds(Server *s, Pipe &p, int32_t n_seeds) {
+  const bool note = 4 * (int64_t)n_seeds >= s->noted_seeds || ++s->unnoted > 3;
+  if (note) {
+    s->noted_seeds = n_seeds;
+    s->unnoted = 0;
+  }
+  p.n_seeds = n_seeds;
+  p.note_seeds = note ? n_seeds : 0;
+}
+inline int most_seeds(Pipe *const *pp, int n) {
+  int most = 0;
+  for (int k = 0; k < n; ++k) most = std::max(most, pp[k]->n_seeds);
+  return most;
+}
 
 }  // namespace lmi

@@ -103,6 +103,10 @@ __device__ __forceinline__ void raise_fault(DevState *st, int which, FaultTo to)
 }
 __device__ __forceinline__ FaultTo fault_to(const DevState *st) { return FaultTo{st->serial, st->fault}; }
 
+__device__ __forceinline__ void note_seen(SeenWord *word, int count, int seeds) {
+  *word = (SeenWord)(uint32_t)seeds << 32 | (uint32_t)count;
+}
+
 // -------------------------------------------------------------- hash table
 __device__ __forceinline__ uint32_t hash_id(int32_t key, int log2cap) {
   return ((uint32_t)key * 0x9E3779B1u) >> (32 - log2cap);

@@ -41,8 +41,9 @@ struct HopShared {  // what the pipes of a launch have in common
   int tile_blocks;  // hop_kernel: blocks [0, tile_blocks) own tiles, the rest fill; hop_flag_scan: own edge tiles, the rest
                     // look the seeds up
   int node_cap;     // nodes a batch can know before the hop
-  int32_t *nodes_seen;  // pinned host memory: receives how many the first batch knew, and behind the last hop its rows
-  int note_total;       // (its rows: only then)
+  SeenWord *nodes_seen;  // pinned host memory: receives how many the batch `note_row` knew, and behind the last hop its rows
+  int note_row;
+  int note_total;        // (its rows: only then)
   int seed_tiles;   // hop_kernel: the first tiles stage 256 seeds each
   // cache lookup of the nodes the hop adds
   int look_mode, miss_seg;
@@ -680,8 +681,11 @@ static __global__ __launch_bounds__(BLOCK, 8) void hop_kernel(HopGroup g) {
     }
   }
   if (last) headers_copy(g, a, t);
-  if (g.c.note_total && last && t == 0 && row == 0 && g.c.nodes_seen) g.c.nodes_seen[1] = n_prev + s_added;
-  if (tile == 0 && t == 0 && row == 0 && g.c.nodes_seen) *g.c.nodes_seen = n_prev;  // for the host to shape later launches by
+  if (t == 0 && row == g.c.note_row && g.c.nodes_seen) {  // for the host to shape later launches by
+    const int n_seeds = g.c.hop == 0 ? n_prev : st->node_counter[9];
+    if (g.c.note_total && last) note_seen(g.c.nodes_seen + 1, n_prev + s_added, n_seeds);
+    if (tile == 0) note_seen(g.c.nodes_seen, n_prev, n_seeds);
+  }
   if (look_mode != LOOK_NOT && !(g.c.tile_rows && tile >= seed_tiles))
     rows_looked_up<PASSES, BLOCK>(g, a, tile < seed_tiles, node, local, slot_of, look, tag, tag_mask, s_scan, &s_miss0);
 }
@@ -821,7 +825,7 @@ int launch_batch_generate(Server *s, Pipe *const *pp, const BatchParams *bps, in
   }
   LMI_HIP(hipGetLastError());
   for (int k = 0; k < n; ++k) {
-    pp[k]->n_seeds = bps[k].n_seeds;
+    pipe_seeds(s, *pp[k], bps[k].n_seeds);
     pp[k]->hops_done = 0;
     pp[k]->fill_pending = -1;
     pp[k]->table_in_lds = false;
@@ -845,7 +849,7 @@ int graph_update_begin(Server *s, Pipe &p, const BatchParams &bp) {
   kp.kernelParams = args;
   kp.extra = nullptr;
   LMI_HIP(hipGraphExecKernelNodeSetParams(p.graph_exec, p.begin_node, &kp));
-  p.n_seeds = bp.n_seeds;
+  pipe_seeds(s, p, bp.n_seeds);
   p.hops_done = s->cfg.hops;
   return LMI_OK;
 }
@@ -861,9 +865,10 @@ bool hop_sets_up(const Server *s) { return s->fuse_count && !s->lds_dedup; }
 //   their second (31 700 nodes): 1024x1 496 79.6, 512x2 496 74.8, 512x4 248 73.7, 1024x4 124 76.8;
 //   four such batches, second hop: 512x4 1 172 278.6, 1024x4 586 274.7, 256x4 2 344 285.4, 256x1 355.6;
 //   1 024 seeds, 15,10,5, third hop (20 000 nodes): 256x1 625 295.3, 1024x1 157 281.6, 512x4 78 284.7.
-// The nodes of a hop are those that the last batches knew there; before the first, the graph's mean degree tells.
+// The nodes of a hop are in proportion to those that the last batches knew there; before the first, the graph's mean degree
+// tells.
 static int64_t hop_nodes(const Server *s, int hop, int n_seeds) {
-  const int64_t seen = hop > 0 && s->nodes_seen_host ? s->nodes_seen_host[hop] : 0;  // hop == hops: the batch's rows
+  const int64_t seen = hop > 0 && s->nodes_seen_host ? seen_count(&s->nodes_seen_host[hop], n_seeds) : 0;  // hop == hops: the batch's rows
   int64_t nodes = seen > 0 ? seen : n_seeds;
   const double mean = s->n_nodes > 0 ? (double)s->n_edges / (double)s->n_nodes : 0;
   for (int k = 0; k < hop && seen <= 0; ++k) nodes += (int64_t)((double)nodes * std::min<double>(mean, s->cfg.fanout[k]));
@@ -897,7 +902,6 @@ int launch_hop(Server *s, Pipe *const *pp, int n, hipStream_t st, int hop, bool 
   g.c.log2cap = p0.dedup.log2cap;
   g.c.max_tiles = p0.max_tiles;
   g.c.node_cap = (int)n_max;
-  g.c.nodes_seen = s->nodes_seen_dev ? s->nodes_seen_dev + hop : nullptr;
   g.c.stage_seeds = (hop == 0 && stage_seeds) ? 1 : 0;
   g.c.begin = begin ? 1 : 0;
   g.c.look_mode = look.mode;
@@ -926,20 +930,22 @@ int launch_hop(Server *s, Pipe *const *pp, int n, hipStream_t st, int hop, bool 
     if (look.mode == LOOK_LRU) p.lru_chained = true;
     if (begin) {
       a.bp = begin[k];
-      p.n_seeds = begin[k].n_seeds;
+      pipe_seeds(s, p, begin[k].n_seeds);
       p.hops_done = 0;
       p.fill_pending = -1;
       p.table_in_lds = false;
     }
   }
+  for (int k = 1; k < n; ++k)
+    if (pp[k]->note_seeds > pp[g.c.note_row]->note_seeds) g.c.note_row = k;
+  if (s->nodes_seen_dev && pp[g.c.note_row]->note_seeds > 0) g.c.nodes_seen = s->nodes_seen_dev + hop;
   int G = 4;
   while (G < f) G <<= 1;
   const bool fused = s->fuse_count && !s->lds_dedup;
   if (!fused) LMI_TRY(launch_fill(s, pp, n, st));
   if (fused) {
     // one tile of nodes per block; a hop left pending gets its local ids filled in by extra blocks behind the tile blocks
-    int n_seeds = 0;
-    for (int k = 0; k < n; ++k) n_seeds = std::max(n_seeds, pp[k]->n_seeds);
+    const int n_seeds = most_seeds(pp, n);
     const HopShape shape = hop_shape(s, n, hop, n_seeds, G);
     const auto [block, passes] = shape;
     const int npb = block / G * passes;

@@ -43,6 +43,7 @@ struct SmallPipe {
   uint8_t *features;
   unsigned long long *known;  // with gather workgroups: how many rows they may gather (small_publish), and behind it whether
                               // one of them has left its rows (small_leave)
+  int note_seeds;  // Pipe::note_seeds
   BatchParams bp;
 };
 struct SmallGroup {
@@ -58,7 +59,7 @@ struct SmallGroup {
   int n, workers, upr, last_off, rows_per_tile;
   int patience;  // reads of SmallPipe::known before a gather workgroup leaves
   RowSources rows;
-  int32_t *rows_seen;  // hinted_rows
+  SeenWord *rows_seen;  // hinted_rows
   SmallPipe p[LMI_MAX_GROUP];
 };
 static_assert(sizeof(SmallGroup) <= 4096, "a kernel's arguments");
@@ -388,7 +389,7 @@ __device__ __forceinline__ int small_sampled(const SmallGroup &g, const SmallPip
   if (full) raise_fault(a.st, kFaultBadId, fault);
   if (t == 0) {
     a.st->n_miss[0] = *n_miss;
-    if (WORKERS && g.rows_seen) g.rows_seen[row] = n_known;
+    if (WORKERS && g.rows_seen && a.note_seeds > 0) note_seen(&g.rows_seen[row], n_known, a.note_seeds);
   }
   return n_known;
 }
@@ -460,6 +461,7 @@ int launch_small(Server *s, Pipe *const *pp, const BatchParams *bps, int n, hipS
   g.look_mode = look.mode;
   g.cache = slot_table(s);
   g.n = n;
+  for (int k = 0; k < n; ++k) pipe_seeds(s, *pp[k], bps[k].n_seeds);
   const int64_t lds = small_lds_bytes(g.log2t, s->max_edges_hop);
   int64_t workers = 0;
   if (look.early_rows) {
@@ -475,7 +477,7 @@ int launch_small(Server *s, Pipe *const *pp, const BatchParams *bps, int n, hipS
     // wait on each other, small_gather ends it.
     const int64_t tile_bytes = n == 1 ? 16 * 1024 : 32 * 1024;
     g.rows_per_tile = (int)std::max<int64_t>(1, std::min<int64_t>(kFlatTileMax, tile_bytes / s->row_bytes));
-    const int64_t tiles = ceil_div(hinted_rows(s, s->max_nodes, 0), g.rows_per_tile);
+    const int64_t tiles = ceil_div(hinted_rows(s, s->max_nodes, 0, pp, n), g.rows_per_tile);
     const int64_t room = s->n_cu / 2 / n - 1;
     workers = n == 1 ? std::min<int64_t>(tiles, s->n_cu - 1) : 2 * room >= tiles ? std::min(tiles, room) : 0;
     if (s->cache_kind == LMI_CACHE_NONE && s->feat_loc == LMI_LOC_HOST)  // a grid that fills the link
@@ -502,7 +504,7 @@ int launch_small(Server *s, Pipe *const *pp, const BatchParams *bps, int n, hipS
     a.features = (uint8_t *)p.features;
     a.known = p.scan_words;
     a.bp = bps[k];
-    p.n_seeds = bps[k].n_seeds;
+    a.note_seeds = p.note_seeds;
     p.hops_done = s->cfg.hops;
     p.fill_pending = -1;
     p.table_in_lds = true;

@@ -55,3 +55,47 @@ def test_tiles_match_the_oracle(lmi, oracle, world, fanout, shape):
         srv.status()
     finally:
         srv.close()
+
+
+def test_tiles_behind_a_short_batch(lmi, oracle, world):
+    """A full batch takes the same tiles and gathers its rows alike behind a full batch, a short one, and a group whose first
+    batch is short; four short ones in a row are what later ones are shaped by."""
+    rng, indptr, indices, feats = world
+    batch, fanout = 3000, [10, 5]
+    srv = lmi.Server(batch, fanout, DIM, pipes=2, seed=3)
+    stream = lmi.stream_create()
+
+    def batches(sizes, key):
+        """Tiles of the hops, and how many of the batches had the last hop's rows gathered by its tiles."""
+        before = srv.routes()["tile_rows"]
+        seeds = [rng.integers(0, N_NODES, n).astype(np.int32) for n in sizes]
+        if len(sizes) == 1:
+            srv.run_once(seeds[0], rng_seed=key, stream=stream)
+        else:
+            srv.run_group([0, 1], [0, 0], seeds=seeds, rng_seeds=[key, key + 1], stream=stream)
+        for k in range(len(sizes)):
+            g = srv.fetch(pipe=k, stream=stream)
+            assert_batch_equal(g, oracle.sample_batch(indptr, indices, seeds[k], fanout, key + k))
+            assert g.features.tobytes() == feats.array[g.ids].tobytes()
+        r = srv.routes()
+        return r["hop_threads"], r["hop_nodes"], r["tile_rows"] - before
+
+    try:
+        srv.load_graph(indptr, indices)
+        srv.attach_features(feats)
+        srv.tune("small_edges", 0)
+        batches([batch], 1)
+        one, two = batches([batch], 2), batches([batch, batch], 3)
+        for it, before in enumerate([[1], [0], [batch // 5], [1, 1]]):
+            batches(before, 10 + it)
+            assert batches([batch], 20 + it) == one
+        batches([1], 30)
+        assert batches([batch, batch], 31) == two
+        assert batches([1, batch], 33) == two   # the tiles are those of the larger one, and it leaves its counts
+        assert batches([batch, batch], 35) == two
+        for it in range(5):
+            few = batches([3], 40 + it)
+        assert few[0][1] == 256
+        srv.status()
+    finally:
+        srv.close()
