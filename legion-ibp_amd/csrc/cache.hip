@@ -1216,16 +1216,22 @@ bool gather_in_line(const Server *s, Pipe *const *pp, int n, int seg_last) {
 // on a tile's misses while others are still being ranked; a launch and a pass over ids and slots go.  Not with the LRU
 // cache, whose batches miss little, and not from a table in HBM, whose reads the hops' own wait for.
 // Blocks and tiles of a hop move hits more slowly than a grid of the gather's own, which shows for long rows where most are
-// hits.  So early_rows up to 4 KB, above 512 bytes only where enough rows miss (Server::miss_share; twice that in fact, for
-// the distinct nodes of a batch are drawn more evenly than its edges are), and tile_rows where a thread has few bytes to move
-// and the link is busy for longer than that takes.  us a batch of 800 seeds, 10,5, gathered behind the hops / early_rows / both
+// hits.  So early_rows up to 4 KB, above 512 bytes only where enough rows miss, and tile_rows where a thread has few bytes to
+// move and the link is busy for longer than that takes.  The limits are fits, not derived: 512 and 4 096 bytes, 1.8 % of
+// misses, 450 and 1 300 bytes a thread, and a microsecond of link for every ten of these, to the batches below; that 2.2 times
+// the keys outside the cache miss (Server::miss_share; the distinct nodes of a batch are drawn more evenly than its edges are)
+// to synthetic graphs of Zipf-distributed degrees whose neighbours are drawn in proportion to them.  Elsewhere the rules may
+// take the slower way.  us a batch of 800 seeds, 10,5, gathered behind the hops / early_rows / both
 // (bytes a thread of the last hop's tiles, us over the link as estimated here), by bytes of a row and share of nodes cached:
 //   400: 20 % 61 / 57 / 54 (122, 34), 50 % 55 / 54 / 51 (98, 18), 90 % 39 / 38 / 39 (98, 2);  1 024, 4 000 seeds, 5,4: 50 % 113 / 111 / 105
 //   (370, 47);  1 536: 80 % 43 / 38 / 48 (470, 8);  2 408: 20 % 208 / 198 / 196 (736, 207), 60 % 75 / 72 / 70 (736, 38), 70 % 62 / 58 / 62
 //   (736, 23), 80 % 50 / 49 / 59 (736, 12);  4 096: 60 % 102 / 98 / 103 (1 253, 65);  5 732: 20 % 441 / 437 / 449, 80 % 73 / 87 / 118
 //   (1 753, 28);  no cache: 3 072 870 / 857 / 829 (939, 804), 4 096 1 116 / 1 101 / 1 098 (1 253, 1 072);
 //   156 seeds, 10,5, 1 024: 26 % 36 / 28 / 39 (400, 16);  65 seeds, 25,15, 2 408: 62 % 38 / 31 / 50 (815, 9).
-constexpr double kLinkRate = 41e9;  // bytes a second, of 400-byte rows
+
+// Bytes a second, of 400-byte rows, for rows of every length in these rules (aligned rows of 512 bytes come at 55e9, of 200 bytes
+// at 31e9).
+constexpr double kLinkRate = 41e9;
 static double miss_estimate(const Server *s) {
   if (s->cache_kind == LMI_CACHE_NONE) return 1.0;
   return std::min(1.0, s->policy_built == LMI_POLICY_PRESAMPLED ? s->miss_share : 2.2 * s->miss_share);
@@ -1278,22 +1284,6 @@ int launch_misses_early(Server *s, Pipe *const *pp, int n, hipStream_t st, int s
   return LMI_OK;  // the join event that launch_gather_group records behind the batch's last misses covers these
 }
 
-// Gathers the rows [first, last) of a segment into each pipe's feature buffer:
-// cache hits from HBM, misses from the feature table, over the host link where it lies
-// in host memory.  With several pipes, the hits of all are one launch and so are the
-// misses (group_miss).  Schedules (tuning key "split_miss"):
-//   0  both on the caller's stream, in one pass where one_pass_gather allows it;
-//   1  hits on the caller's stream, misses on the server's side stream, where they
-//      overlap the next batch's sampling.  A wide host-link gather beside HBM gathers
-//      cuts their bandwidth by more than half: it runs on a small grid (miss_blocks);
-//   2  both on the side stream (a gather stage behind the sampling stage): the
-//      caller's stream is free for the next batch's sampling as soon as the lookup
-//      is done.
-// gather_in_line says when schedule 0 is taken whatever the knob says: nothing is left
-// then for a side stream to overlap, and a wide grid has no neighbour to slow.
-// With 1 and 2 the caller's stream does not wait here: the next call on this pipe,
-// or lmi_batch_wait, joins.  A segment of an LRU batch joins at once (a later call
-// inserts the gathered rows).
 // Whether a side stream's join event ends batches like this one: behind that nobody follows the stream that takes a batch, so
 // neither where the gather is in line only because that side stream would have nothing to overlap.
 static bool batch_sided(const Server *s, bool early_fork) {
@@ -1310,6 +1300,22 @@ void rows_gathered(Server *s, Pipe *const *pp, int n, hipEvent_t end) {
   }
 }
 
+// Gathers the rows [first, last) of a segment into each pipe's feature buffer:
+// cache hits from HBM, misses from the feature table, over the host link where it lies
+// in host memory.  With several pipes, the hits of all are one launch and so are the
+// misses (group_miss).  Schedules (tuning key "split_miss"):
+//   0  both on the caller's stream, in one pass where one_pass_gather allows it;
+//   1  hits on the caller's stream, misses on the server's side stream, where they
+//      overlap the next batch's sampling.  A wide host-link gather beside HBM gathers
+//      cuts their bandwidth by more than half: it runs on a small grid (miss_blocks);
+//   2  both on the side stream (a gather stage behind the sampling stage): the
+//      caller's stream is free for the next batch's sampling as soon as the lookup
+//      is done.
+// gather_in_line says when schedule 0 is taken whatever the knob says: nothing is left
+// then for a side stream to overlap, and a wide grid has no neighbour to slow.
+// With 1 and 2 the caller's stream does not wait here: the next call on this pipe,
+// or lmi_batch_wait, joins.  A segment of an LRU batch joins at once (a later call
+// inserts the gathered rows).
 int launch_gather_group(Server *s, Pipe *const *pp, int n, hipStream_t st, int seg, int seg_last, int lru_lists,
                         bool same_stream, int hit_seg_first, const HeaderCopy *headers, bool early_rows) {
   if (early_rows) seg = seg_last;  // the hops' launches took the rows before the last hop's

@@ -866,7 +866,10 @@ bool hop_sets_up(const Server *s) { return s->fuse_count && !s->lds_dedup; }
 //   four such batches, second hop: 512x4 1 172 278.6, 1024x4 586 274.7, 256x4 2 344 285.4, 256x1 355.6;
 //   1 024 seeds, 15,10,5, third hop (20 000 nodes): 256x1 625 295.3, 1024x1 157 281.6, 512x4 78 284.7.
 // The nodes of a hop are in proportion to those that the last batches knew there; before the first, the graph's mean degree
-// tells.
+// tells, 2 to 17 times too many on graphs of heavy-tailed degrees: its tiles are larger, and tile_rows decides on the same
+// number (us a pass by that estimate and grids for the worst case, as a call captured on a new server keeps them / by what
+// batches met: 800 seeds into the caller's buffers 111 / 103; 8 000 seeds, all rows cached 92 / 86; two launches a hop, which the
+// worst case shaped, took 127 and 97).
 static int64_t hop_nodes(const Server *s, int hop, int n_seeds) {
   const int64_t seen = hop > 0 && s->nodes_seen_host ? seen_count(&s->nodes_seen_host[hop], n_seeds) : 0;  // hop == hops: the batch's rows
   int64_t nodes = seen > 0 ? seen : n_seeds;

@@ -1,8 +1,8 @@
 // The whole sampling phase of a small batch in one workgroup.
 //
-// A small batch is bound by latency: in the general path every hop is two launches whose blocks pass counts through
-// HBM (look-back) and deduplicate through atomics on a table in HBM, four launches of 5-10 us each for 16 seeds that
-// touch 500 nodes.  One workgroup of 1024 threads has all of it within a barrier's reach instead: the dedup table, the
+// A small batch is bound by latency: in the general path every hop is a launch whose blocks pass counts through
+// HBM (look-back) and deduplicate through atomics on a table in HBM, two launches and a gather of 5-13 us each for 16 seeds
+// that touch 500 nodes.  One workgroup of 1024 threads has all of it within a barrier's reach instead: the dedup table, the
 // slots of a hop's edges and the nodes being sampled lie in LDS, the scans are block scans, and one launch per group of
 // batches (a workgroup each) does the seeds, every hop, the relabelling, the cache lookup and the headers.  What is left
 // of HBM is the chain seed -> row pointers -> neighbours -> row pointers ... that no kernel can shorten.
