@@ -59,16 +59,16 @@ def test_tiles_match_the_oracle(lmi, oracle, world, fanout, shape):
 
 def test_tiles_behind_a_short_batch(lmi, oracle, world):
     """A full batch takes the same tiles and gathers its rows alike behind a full batch, a short one, and a group whose first
-    batch is short; four short ones in a row are what later ones are shaped by."""
+    batch is short; only the fourth short one in a row shapes those behind it."""
     rng, indptr, indices, feats = world
     batch, fanout = 3000, [10, 5]
     srv = lmi.Server(batch, fanout, DIM, pipes=2, seed=3)
     stream = lmi.stream_create()
 
-    def batches(sizes, key):
+    def batches(sizes, key, among=np.arange(N_NODES)):
         """Tiles of the hops, and how many of the batches had the last hop's rows gathered by its tiles."""
         before = srv.routes()["tile_rows"]
-        seeds = [rng.integers(0, N_NODES, n).astype(np.int32) for n in sizes]
+        seeds = [rng.choice(among, n).astype(np.int32) for n in sizes]
         if len(sizes) == 1:
             srv.run_once(seeds[0], rng_seed=key, stream=stream)
         else:
@@ -93,9 +93,14 @@ def test_tiles_behind_a_short_batch(lmi, oracle, world):
         assert batches([batch, batch], 31) == two
         assert batches([1, batch], 33) == two   # the tiles are those of the larger one, and it leaves its counts
         assert batches([batch, batch], 35) == two
-        for it in range(5):
-            few = batches([3], 40 + it)
-        assert few[0][1] == 256
+        alone = np.flatnonzero(np.diff(indptr) == 0)   # three of these meet nobody: so would three thousand
+        for it in range(3):
+            batches([3], 40 + it, alone)
+        assert batches([batch], 43) == one
+        for it in range(4):
+            batches([3], 44 + it, alone)
+        assert batches([batch], 48)[0][1] == 256 != one[0][1]
+        assert batches([batch], 49) == one
         srv.status()
     finally:
         srv.close()
